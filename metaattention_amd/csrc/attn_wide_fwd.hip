@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs 
     for (int k = 0; k < FLY; k++) {
       const int s = s0 + k * AT_ONCE + part;
       const float w = __shfl(e, s & 63, 64);
-      if (s < a.n_split && w > 0.f) {
+      if (s < a.n_split) {   // (a weight of 0 too: every split has written its rows, and 0 x NaN is to stay NaN)
 #pragma unroll
         for (int i = 0; i < 8; i++) acc[i] += w * (float)v[k][i];
       }
@@ -57,14 +57,15 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs 
   for (int d = LPR; d < 64; d *= 2)
 #pragma unroll
     for (int i = 0; i < 8; i++) acc[i] += __shfl_xor(acc[i], d, 64);
-  const float inv = tot > 0.f ? 1.f / tot : 0.f;
+  // (only a row without any key has a sum of exactly 0; one that is NaN makes the row and its scale NaN, as the unsplit kernel does)
+  const float inv = tot == 0.f ? 0.f : 1.f / tot;
   if (part == 0) {
     x8 w;
 #pragma unroll
     for (int i = 0; i < 8; i++) w[i] = (T)(acc[i] * inv);
     *(x8*)((T*)a.o + (int64_t)b * a.osb + (int64_t)m * a.oss + (int64_t)h * a.osh + col) = w;
   }
-  if (a.row_scale && lane == 0) a.row_scale[row] = tot > 0.f ? mx + __logf(tot) : -INFINITY;
+  if (a.row_scale && lane == 0) a.row_scale[row] = tot == 0.f ? -INFINITY : mx + __logf(tot);
 }
 
 // Decode shapes: at most 32 query rows per (batch, head), softmax, no structural mask.  A one-wave workgroup takes one

@@ -458,8 +458,8 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
     if (rs_ptr) *rs_ptr = r_tot;
   } else if constexpr (FAMILY == WF_SOFTMAX) {
     const float tot = r_part + xhalf(r_part);
-    inv = tot > 0.f ? 1.f / tot : 0.f;   // (a row that was left no key at all gives zeros and lse = -inf)
-    if (rs_ptr) *rs_ptr = tot > 0.f ? (row_max + fast_log2(tot)) * kLn2 : -INFINITY;
+    inv = tot == 0.f ? 0.f : 1.f / tot;   // (a row that was left no key at all gives zeros and lse = -inf; NaN stays NaN)
+    if (rs_ptr) *rs_ptr = tot == 0.f ? -INFINITY : (row_max + fast_log2(tot)) * kLn2;
   }
 
   // ---- O: two halves of DV/2 columns through a wave-private LDS block, coalesced 16-byte stores
