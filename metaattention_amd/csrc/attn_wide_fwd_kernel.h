@@ -268,6 +268,9 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
       else if (em_row && !full_next) load_keep(jt * BN, keep_next);
       issue_tile(jt * BN, buf ^ 1);
     }
+    // A tile above this wave's diagonal is for the block's later waves.  (Not only work saved: its probabilities are 0, but
+    // 0 x V is NaN where V is not finite.  Retention has no diagonal of its own, see above.)
+    if (CAUSAL && FAMILY != WF_RETENTION && n0 > m_wave + 31) continue;
     const uint32_t kbase = lds_tiles + buf * STAGE, vbase = kbase + KTILE;
     float ex[16];
     if constexpr (FAMILY != WF_RETENTION) {

@@ -60,3 +60,19 @@ def test_latent_cache_decode(Hq, KV):
         got, got_lse = hb.flash_mla_with_kvcache(bad, k, table, lens, 512, *plan)
         assert got[:, 0][rows].isnan().all() and got_lse[..., 0][rows].isnan().all()
         assert torch.equal(got[:, 0][~rows], out[:, 0][~rows]) and torch.equal(got_lse[..., 0][~rows], lse[..., 0][~rows])
+
+
+@pytest.mark.parametrize("B,H,S,D,DV", [(1, 4, 70, 128, 128), (1, 8, 300, 128, 128), (2, 4, 300, 128, 256), (1, 4, 200, 64, 64), (2, 16, 257, 192, 128), (1, 4, 300, 256, 256)])
+@pytest.mark.parametrize("family", ["softmax", "sigmoid"])
+def test_rows_before_a_value_under_a_causal_mask(B, H, S, D, DV, family):
+    """The rows of the 32-row groups before that of a NaN value do not see it, however many rows a workgroup has."""
+    mod = specs.softmax_attention(B, H, S, D, DV) if family == "softmax" else specs.sigmoid_attention(B, H, S, D, DV, const_bias=-4.0)
+    q, k, v = (_rand(B, S, H, d, dtype=torch.bfloat16) for d in (D, D, DV))
+    out = mod(q, k, v)
+    for key in (S - 1, 63):
+        bad = v.clone()
+        bad[0, key, 1, 3] = NAN
+        got, want, first = mod(q, k, bad), out.clone(), key // 32 * 32
+        assert got[0, key:, 1, 3].isnan().all()
+        got[0, first:, 1, 3] = want[0, first:, 1, 3] = 0
+        assert torch.equal(got, want)
