@@ -99,6 +99,9 @@ int attn_decode_splits(int family, bool causal, int B, int H, int Sq, int Skv, i
   return best;
 }
 
+// The tile DMA of attn_wide_fwd_kernel addresses a tile's 32 rows with 32-bit byte offsets from its first row.
+static constexpr int64_t kWideRowStride = (int64_t)1 << 26;
+
 // Prefill calls whose workgroups of 128 (or 256: attn_fwd.hip) query rows are too few to keep the chip busy: a row block's tiles
 // are then walked by several streams side by side (KVS of attn_wide_fwd_kernel), or the row blocks are smaller.  A step of a
 // stream is a serial chain of about 0.85 us at 128 / 128 whatever else the CU does, 1.08 with a second wave on the SIMD, so the
@@ -107,6 +110,8 @@ int attn_decode_splits(int family, bool causal, int B, int H, int Sq, int Skv, i
 AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, int dv) {
   if (family == WF_RETENTION || a.kv_lens || a.o_part || (a.kv_block_mask && !a.kbm_by_query_head)) return AttnCut::kRows128;
   const bool plain = !a.kv_block_mask && !a.elem_mask && !a.add && !a.slope_q && !a.slope_kv && !(a.softcap > 0.f);
+  const bool persistent = plain && dqk == 128 && (dv == 128 || (dv == 256 && a.Sq >= 256));
+  if (persistent && (a.kss >= kWideRowStride || a.vss >= kWideRowStride)) return AttnCut::kPersistent;   // (the other cuts would refuse them)
   const double k = dqk + dv <= 128 ? 0.75 : dqk == 192 ? 1.25 : 1.0;
   const int64_t bh = (int64_t)a.B * a.H, tiles = ((int64_t)a.Skv + 31) / 32;
   const bool half = causal || a.kv_block_mask || a.elem_mask;   // (what a mask keeps is not known here: taken as a causal one)
@@ -131,7 +136,7 @@ AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, in
     if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 8.8);
     consider(AttnCut::kStreams2x2, 2, 2, 6.5);
   }
-  if (plain && dqk == 128 && (dv == 128 || (dv == 256 && a.Sq >= 256))) {
+  if (persistent) {
     // the persistent kernel: rounds of row blocks of 256 (under a causal mask, pairs of them), 32 keys in 0.6 us, 0.95 once all
     // CUs take part; twice for the two halves of 256 value columns
     const int64_t blocks = ((int64_t)a.Sq + 255) / 256, units = bh * (causal ? (blocks + 1) / 2 : blocks);
@@ -202,9 +207,8 @@ static int wide_dims(const AttnArgs& a, int family, bool causal, int dqk, int dv
 
 // returns 0 ok, -1 launch failure, -2 unsupported
 int attn_wide_fwd_dispatch(const AttnArgs& a, int family, bool causal, bool is_bf16, int dqk, int dv, hipStream_t stream) {
-  // (the tile DMA addresses a tile's 32 rows with 32-bit byte offsets from its first row)
   for (int64_t row_stride : {a.kss, a.vss})
-    if (row_stride < 0 || row_stride >= ((int64_t)1 << 26)) return -2;
+    if (row_stride < 0 || row_stride >= kWideRowStride) return -2;
   const AttnCut cut = attn_prefill_cut(a, family, causal, dqk, dv);
   if (cut == AttnCut::kStreams4x2 || cut == AttnCut::kStreams2x4 || cut == AttnCut::kStreams2x2)
     return (is_bf16 ? attn_streams_bf16 : attn_streams_fp16)(a, cut, family, causal, dqk, dv, stream);

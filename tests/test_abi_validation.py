@@ -96,6 +96,10 @@ CASES = [
     ("ma_attn_fwd", _attn, {"scale": 0.0}, INVALID), ("ma_attn_fwd", _attn, {"scale": float("nan")}, INVALID),
     ("ma_attn_fwd", _attn, {"seqlen_kv": 300}, UNSUPPORTED),                    # causal with unequal lengths
     ("ma_attn_fwd", _attn, {"heads_kv": 3}, INVALID),
+    # rows further apart than the general kernel addresses: few of them, in the persistent kernel (128/128, and 128/256 from 256 queries on)
+    ("ma_attn_fwd", _attn, {"seqlen_q": 16, "seqlen_kv": 16, "k_stride_s": 1 << 27}, LAUNCH),
+    ("ma_attn_fwd", _attn, {"seqlen_q": 256, "seqlen_kv": 16, "mask": hb.MA_MASK_NONE, "dim_v": 256, "v_stride_s": 1 << 26}, LAUNCH),
+    ("ma_attn_fwd", _attn, {"seqlen_q": 16, "seqlen_kv": 16, "dim_qk": 64, "dim_v": 64, "k_stride_s": 1 << 27}, UNSUPPORTED),
     ("ma_attn_fwd", _attn, {"dim_qk": 96, "dim_v": 96}, UNSUPPORTED), ("ma_attn_fwd", _attn, {"dim_qk": 128, "dim_v": 64}, UNSUPPORTED),
     ("ma_attn_fwd", _attn, {"q_stride_s": 4 * 128 + 4}, UNSUPPORTED), ("ma_attn_fwd", _attn, {"k": PTR + 8}, UNSUPPORTED),
     ("ma_attn_fwd", _attn, {"kv_block_mask": PTR + 0x50000000, "kv_block_size": 48, "mask": hb.MA_MASK_NONE}, UNSUPPORTED),
