@@ -25,9 +25,10 @@ struct AttnArgs {
   const uint8_t* elem_mask;
   int64_t em_sb, em_sh, em_sq;
   // split-kv decode (attn_wide_fwd_kernel with one wave per workgroup): n_split kv ranges per (batch, head,
-  // row block), normalised partial outputs [B, n_split, H, Sq, Dv] in the tensor dtype and their fp32
+  // row block), normalised partial outputs [B, n_split, H, Sq, Dv] in fp32 (part_f32) or the tensor dtype and their fp32
   // natural-log row scale [B, n_split, H, Sq], merged by attn_split_combine_kernel
   int n_split;
+  bool part_f32;
   void* o_part;
   float* lse_part;
   float scale, bias;
@@ -46,6 +47,8 @@ struct AttnArgs {
 int attn_wide_fwd_dispatch(const AttnArgs& a, int family, bool causal, bool is_bf16, int dqk, int dv, hipStream_t stream);
 // number of kv splits the decode path would use for these sizes (1: not a decode shape / nothing to gain)
 int attn_decode_splits(int family, bool causal, int B, int H, int Sq, int Skv, int dqk, int dv);
+// whether the partial results of those splits are fp32
+bool attn_decode_partials_f32(int B, int H, int Skv, int dqk, int dv);
 // How a prefill call is cut into workgroups: row blocks of 256 in the persistent kernel (attn_fwd.hip), of 128 in the general one,
 // or the latter's forms with several streams of key tiles per row block (32-row waves x streams).
 enum class AttnCut { kPersistent, kRows128, kStreams4x2, kStreams2x4, kStreams2x2 };

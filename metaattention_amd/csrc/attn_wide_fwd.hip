@@ -12,9 +12,11 @@ namespace ma {
 // partial results, requested before the first have come), so DV / 8 lanes take a row of 16 bytes each and the wave reads
 // 512 / DV splits at a time, four times over.  B9 H32 Hkv8 KV3672 64/64, 26 splits: 12.6 us with a load of every split behind
 // the one before it, DV / 64 columns a lane.
-template <typename T, int DV>
+// P: the partial results' type.
+template <typename T, typename P, int DV>
 __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs a) {
   using x8 = typename Elem<T>::x8;
+  typedef P p8 __attribute__((ext_vector_type(8)));
   constexpr int LPR = DV / 8, AT_ONCE = 64 / LPR, FLY = 4;
   const int lane = threadIdx.x & 63, part = lane / LPR, col = (lane % LPR) * 8;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // (b * H + h) * Sq + m
@@ -22,13 +24,13 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs 
   if (row >= rows) return;
   const int m = (int)(row % a.Sq), h = (int)((row / a.Sq) % a.H), b = (int)(row / ((int64_t)a.Sq * a.H));
   const int64_t part_row = ((int64_t)b * a.n_split * a.H + h) * a.Sq + m, split_stride = (int64_t)a.H * a.Sq;
-  const T* src = (const T*)a.o_part + part_row * DV + col;
-  x8 v[FLY];
+  const P* src = (const P*)a.o_part + part_row * DV + col;
+  p8 v[FLY];
   auto fetch = [&](int s0) {
 #pragma unroll
     for (int k = 0; k < FLY; k++) {
       const int s = s0 + k * AT_ONCE + part;
-      if (s < a.n_split) v[k] = *(const x8*)(src + s * split_stride * DV);
+      if (s < a.n_split) v[k] = *(const p8*)(src + s * split_stride * DV);
     }
   };
   fetch(0);
@@ -68,6 +70,20 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs 
   if (a.row_scale && lane == 0) a.row_scale[row] = tot == 0.f ? -INFINITY : mx + __logf(tot);
 }
 
+// the one-wave workgroups that run side by side on 256 CUs
+static int64_t decode_slots(int dqk, int dv) {
+  const int per_cu = (160 * 1024) / (2 * 32 * (pad_width(dqk) + dv) * 2);
+  return (int64_t)(per_cu > 4 ? 4 : per_cu) * 256;
+}
+
+// Rounding the partial results to the tensor dtype in front of the merge adds a fifth to the error of the output (300 keys, bf16:
+// 2.3e-3 of it unsplit, 2.2e-3 split with fp32 partial results, 2.8e-3 with bf16).  They are fp32 where the call could as well
+// run unsplit: a cache of at most 15 tiles, or (batch, head) pairs that take more than half of the slots by themselves.  Between
+// the few pairs of a long cache they are 16-bit, as the reference's Output_partial is (mla_decode_tl.py:160).
+bool attn_decode_partials_f32(int B, int H, int Skv, int dqk, int dv) {
+  return Skv <= 15 * 32 || 2 * (int64_t)B * H > decode_slots(dqk, dv);
+}
+
 // Decode shapes: at most 32 query rows per (batch, head), softmax, no structural mask.  A one-wave workgroup takes one
 // (batch, head, kv split); a CU holds four of them, or as many as their two tile stages fit into its 160 KB of LDS.  The
 // split count is the one with the shortest schedule, in microseconds: rounds of resident workgroups x (3 for a workgroup's
@@ -78,12 +94,9 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs 
 int attn_decode_splits(int family, bool causal, int B, int H, int Sq, int Skv, int dqk, int dv) {
   if (family != WF_SOFTMAX || causal || Sq > 32) return 1;
   if (!((dqk == 128 && dv == 128) || (dqk == 64 && dv == 64) || (dqk == 128 && dv == 256) || (dqk == 256 && dv == 256) || (dqk == 192 && dv == 128))) return 1;
-  const int64_t tiles = ((int64_t)Skv + 31) / 32, groups = (int64_t)B * H;
-  const int lds = 2 * 32 * (pad_width(dqk) + dv) * 2;
-  int per_cu = (160 * 1024) / lds;
-  if (per_cu > 4) per_cu = 4;
-  const int64_t slots = (int64_t)per_cu * 256;
-  const double stream_us = (double)groups * (double)Skv * (dqk + dv) * 2 / 5.5e6, part_us = (double)groups * Sq * dv * 2 * 1.5 / 5.5e6;
+  const int64_t tiles = ((int64_t)Skv + 31) / 32, groups = (int64_t)B * H, slots = decode_slots(dqk, dv);
+  const int part_bytes = attn_decode_partials_f32(B, H, Skv, dqk, dv) ? 4 : 2;
+  const double stream_us = (double)groups * (double)Skv * (dqk + dv) * 2 / 5.5e6, part_us = (double)groups * Sq * dv * part_bytes * 1.5 / 5.5e6;
   int best = 1;
   double best_us = 0;
   for (int n = 1; n <= 64 && (n == 1 || 2 * n <= tiles); n++) {
@@ -157,7 +170,9 @@ static int wide_family(const AttnArgs& a, int family, bool causal, hipStream_t s
           if (const int rc = launch_wide<T, DQK, DV, WF_SOFTMAX, false, 1>(a, stream)) return rc;
           if (a.n_split > 1) {
             const int64_t rows = (int64_t)a.B * a.H * a.Sq;
-            hipLaunchKernelGGL((attn_split_combine_kernel<T, DV>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, a);
+            const dim3 grid((unsigned)((rows + 3) / 4));
+            if (a.part_f32) hipLaunchKernelGGL((attn_split_combine_kernel<T, float, DV>), grid, dim3(256), 0, stream, a);
+            else hipLaunchKernelGGL((attn_split_combine_kernel<T, T, DV>), grid, dim3(256), 0, stream, a);
           }
           return launch_status();
         }

@@ -465,6 +465,21 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
     if (rs_ptr) *rs_ptr = tot == 0.f ? -INFINITY : (row_max + fast_log2(tot)) * kLn2;
   }
 
+  // ---- a split's partial output in fp32 (attn_decode_partials_f32) as it is: a lane has four consecutive columns of its row at a
+  //      time, and a decode call few rows
+  if constexpr (NW == 1 && KVS == 1) {
+    if (a.part_f32) {
+      float* to = (float*)a.o_part + ((((int64_t)b * a.n_split + split) * a.H + h) * a.Sq + m_lane) * DV + 4 * g;
+      if (m_lane < a.Sq) {
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; q4++)
+            *(f32x4*)(to + 32 * db + 8 * q4) = f32x4{o[db][4 * q4] * inv, o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv};
+      }
+      return;
+    }
+  }
   // ---- O: two halves of DV/2 columns through a wave-private LDS block, coalesced 16-byte stores
   constexpr int HALF = DV / 2, OROW = HALF * 2 + 16;
   const uint32_t ob = lds0 + wave * 32 * OROW;
