@@ -195,3 +195,13 @@ def test_workspace_queries_take_bad_arguments():
     assert lib.ma_linear_bwd_workspace_bytes(ctypes.byref(_linear_bwd(batch=big, heads=1 << 24, heads_q=4, heads_k=4, seqlen=65536))) == 0
     assert lib.ma_linear_workspace_bytes(ctypes.byref(_linear(dim_v=big))) == 0
     assert lib.ma_mla_workspace_bytes(ctypes.byref(_mla(batch=big, heads_q=big, num_split=4))) == 0
+
+
+@pytest.mark.parametrize("heads", [1, 16, 32, 40, 64, 128, 200, 400])
+def test_latent_cache_splits_only_where_half_of_the_cus_would_idle(heads):
+    """(256 CUs are assumed without a device.)  The partial results of splits are rounded: one accumulation from half of the CUs on."""
+    lib, blocks = _lib(), (heads + 127) // 128
+    for batch in (1, 2, 42, 64, 86, 128, 129, 160, 200, 255, 256, 400, 3000):
+        for kv in (64, 200, 4096, 131072):
+            n = lib.ma_mla_choose_split(ctypes.byref(_mla(batch=batch, heads_q=heads, seqlen_kv=kv, num_split=0)))
+            assert n == 1 if 2 * batch * blocks > 256 else 1 <= n <= min(64, (kv + 63) // 64), (batch, kv, n)

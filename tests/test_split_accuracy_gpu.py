@@ -30,3 +30,13 @@ def test_decode(dtype, B, H, Hkv, KV, D, DV):
     ref = (p.unsqueeze(-1) * vr).sum(1)
     whole, cut = (hb.attn_fwd(q, k, v, family=hb.MA_ATTN_SOFTMAX, causal=False, scale=D ** -0.5, split_kv=s)[:, 0] for s in (False, True))
     assert _error(cut, ref) <= ROOM * _error(whole, ref)
+
+
+@pytest.mark.parametrize("B,Hq,KV", [(129, 16, 300), (160, 128, 200)])
+def test_latent_cache_batch(B, Hq, KV):
+    from metaattention_amd import hip_backend as hb
+    q, q_pe, kv, k_pe = (_rand(*s, dtype=torch.bfloat16) for s in ((B, 1, Hq, 512), (B, 1, Hq, 64), (B, KV, 1, 512), (B, KV, 1, 64)))
+    s = torch.matmul(q[:, 0].double(), kv[:, :, 0].double().transpose(1, 2).contiguous()) + torch.matmul(q_pe[:, 0].double(), k_pe[:, :, 0].double().transpose(1, 2).contiguous())
+    ref = torch.matmul(torch.softmax(s * 576 ** -0.5, dim=-1), kv[:, :, 0].double())
+    whole, cut = (hb.mla_decode(q, q_pe, kv, k_pe, scale=576 ** -0.5, num_split=n)[:, 0] for n in (1, 0))
+    assert _error(cut, ref) <= ROOM * _error(whole, ref)
