@@ -205,3 +205,20 @@ def test_latent_cache_splits_only_where_half_of_the_cus_would_idle(heads):
         for kv in (64, 200, 4096, 131072):
             n = lib.ma_mla_choose_split(ctypes.byref(_mla(batch=batch, heads_q=heads, seqlen_kv=kv, num_split=0)))
             assert n == 1 if 2 * batch * blocks > 256 else 1 <= n <= min(64, (kv + 63) // 64), (batch, kv, n)
+
+
+def test_latent_cache_scratch_holds_every_automatic_split():
+    """ma_mla_decode_noalloc serves every call without num_split (here, without a device, it gets as far as asking for one), and a
+    workspace of one round of 128-head workgroups serves ma_mla_decode."""
+    lib = _lib()
+    for heads in (1, 16, 32, 40, 64, 128, 200, 400):
+        for batch in list(range(1, 130)) + [160, 200, 256, 1000]:
+            for kv in (64, 300, 2048, 4096, 8192, 131072):
+                p = _mla(batch=batch, heads_q=heads, seqlen_kv=kv, num_split=0)
+                need = lib.ma_mla_workspace_bytes(ctypes.byref(p))
+                assert need <= lib.ma_mla_noalloc_max_workspace(), (heads, batch, kv, need)
+                rc = lib.ma_mla_decode_noalloc(ctypes.byref(p), None)
+                assert rc == (UNSUPPORTED if need else LAUNCH) and (not need or "device ordinal" in lib.ma_last_error().decode())
+                old = min(256 // (batch * ((heads + 127) // 128)), (kv + 63) // 64, 64) if batch * ((heads + 127) // 128) <= 256 else 1
+                p.workspace, p.workspace_bytes = PTR + 0x50000000, max(old, 1) * batch * heads * (512 * 2 + 4)
+                assert lib.ma_mla_decode(ctypes.byref(p), None) == LAUNCH, (heads, batch, kv, lib.ma_last_error())

@@ -61,3 +61,12 @@ def test_noalloc_rejects_what_does_not_fit():
     hb.mla_decode(q, q_pe, kv, k_pe, scale=SCALE, out=out, no_alloc=True)
     torch.cuda.synchronize()
     assert torch.isfinite(out.float()).all()
+
+
+def test_noalloc_serves_batches_whose_best_split_would_not_fit():
+    """Between two rounds of workgroups (B86: 172 of 256 CUs with two splits) more splits would be faster than the array holds."""
+    from metaattention_amd import hip_backend as hb
+    B, Hq, Skv = 86, 128, 2048
+    q, q_pe, kv, k_pe = (t.cuda() for t in inputs.mla_inputs(B, Hq, Skv, 512, 64, seed=86))
+    (o_ws, lse_ws), (o_na, lse_na) = _both(hb, q, q_pe, kv, k_pe, 0)
+    assert torch.isfinite(o_na.float()).all() and torch.equal(o_ws, o_na) and torch.equal(lse_ws, lse_na)
