@@ -230,7 +230,8 @@ typedef struct ma_linear_bwd_params {
  * q [B,Hq,D], q_pe [B,Hq,Dpe], kv [B,Skv,D], k_pe [B,Skv,Dpe], o [B,Hq,D]
  * (one latent kv head, one query token; the [B,1,Hq,.] / [B,Skv,1,.] tensors
  * of the reference are these with a unit dimension).  Partial outputs are kept in the tensors' dtype, as Output_partial
- * of the reference is (mla_decode_tl.py:160); their log-sum-exp is fp32. */
+ * of the reference is (mla_decode_tl.py:160), except where ma_mla_params.num_splits says otherwise; their log-sum-exp is
+ * fp32. */
 typedef struct ma_mla_params {
   int32_t dtype;
   int32_t batch, heads_q, seqlen_kv, dim, dim_pe;
@@ -253,7 +254,10 @@ typedef struct ma_mla_params {
   /* optional work plan for ragged batches, as written by ma_mla_get_metadata (kv_seqlens is then required and
    * num_split ignored): tile_scheduler_metadata int32 [num_sm_parts, 8], num_splits int32 [batch + 1], device memory.
    * Says that the lengths differ: the workgroups then take equal runs of (batch entry, token range) pieces, which they work
-   * out from kv_seqlens in finer pieces than the plan's, instead of one of num_split equal ranges of one batch entry. */
+   * out from kv_seqlens in finer pieces than the plan's, instead of one of num_split equal ranges of one batch entry.  Of the
+   * plan only num_splits is read: the partial results of an entry that it leaves in one piece are fp32 (or, in a
+   * workspace below ma_mla_workspace_bytes, which any of (batch + num_sm_parts) * heads_q * (2 * dim + 4) bytes serves,
+   * the entry is not cut).  num_sm_parts has no other effect. */
   const int32_t* tile_scheduler_metadata;
   const int32_t* num_splits;
   int32_t num_sm_parts;
@@ -300,8 +304,8 @@ int ma_mla_decode(const ma_mla_params* p, ma_stream_t stream);
  * ignored: the partial results of the kv splits go to an array inside the library, ma_mla_noalloc_max_workspace() bytes
  * (40 MiB) per GPU, held until the process ends -- by every process that loads the library and uses that GPU, whether or
  * not it calls this entry point (the array is part of the code object: 16 processes on one GPU hold 640 MiB); devices
- * beyond ordinal 63 are refused with MA_ERR_UNSUPPORTED.  A call whose ma_mla_workspace_bytes(p) exceeds that returns
- * MA_ERR_WORKSPACE.  The call itself allocates nothing and synchronises nothing.  All calls on one GPU share the array:
+ * beyond ordinal 63 are refused with MA_ERR_UNSUPPORTED.  Every call with num_split 0 fits; one whose num_split, or whose
+ * work plan ((batch + num_sm_parts) * heads_q * (2 * dim + 4) bytes), needs more returns MA_ERR_WORKSPACE.  The call itself allocates nothing and synchronises nothing.  All calls on one GPU share the array:
  * calls that overlap on one GPU (different streams, different threads) race; calls on one stream do not.  Every slot a
  * call reads it has written before, so nothing needs clearing between calls.  The first call on a device looks the
  * array's address up (and, if it is the library's first call, makes the runtime load the code object): make that call

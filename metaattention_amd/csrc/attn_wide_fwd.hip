@@ -16,7 +16,7 @@ namespace ma {
 template <typename T, typename P, int DV>
 __global__ __launch_bounds__(256) void attn_split_combine_kernel(const AttnArgs a) {
   using x8 = typename Elem<T>::x8;
-  typedef P p8 __attribute__((ext_vector_type(8)));
+  typedef P p8 __attribute__((ext_vector_type(8), aligned(16)));
   constexpr int LPR = DV / 8, AT_ONCE = 64 / LPR, FLY = 4;
   const int lane = threadIdx.x & 63, part = lane / LPR, col = (lane % LPR) * 8;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // (b * H + h) * Sq + m

@@ -20,9 +20,13 @@ struct MlaArgs {
   int page_size;
   const int32_t* kv_lens;
   // ragged launch (kv_lens set): `parts` workgroups per block of heads, piece_meta int32 [B, 2] in the workspace (written by
-  // the split kernel, read by the combine kernel); o_part / lse_part then hold B + parts slots
+  // the split kernel, read by the combine kernel); o_part / lse_part then hold B + parts slots.  plan_splits: the caller's plan,
+  // int32 [B + 1], of which it matters whether it leaves an entry in one piece (see RaggedEntry); wide_slots: the slots of
+  // o_part hold fp32 outputs
   int32_t* piece_meta;
   int parts;
+  const int32_t* plan_splits;
+  int wide_slots;
 };
 
 // Blocks of heads of a call (one workgroup serves one), and the workgroups that a device of `cus` CUs runs side by side.

@@ -222,3 +222,20 @@ def test_latent_cache_scratch_holds_every_automatic_split():
                 old = min(256 // (batch * ((heads + 127) // 128)), (kv + 63) // 64, 64) if batch * ((heads + 127) // 128) <= 256 else 1
                 p.workspace, p.workspace_bytes = PTR + 0x50000000, max(old, 1) * batch * heads * (512 * 2 + 4)
                 assert lib.ma_mla_decode(ctypes.byref(p), None) == LAUNCH, (heads, batch, kv, lib.ma_last_error())
+
+
+def test_latent_cache_work_plans_at_scratch_limits():
+    """A plan's own slots, (batch + num_sm_parts) of 16-bit results, serve a call, with the caller's workspace and in the built-in array."""
+    lib = _lib()
+    plan = dict(tile_scheduler_metadata=PTR + 0x50000000, num_splits=PTR + 0x51000000, kv_seqlens=PTR + 0x52000000, workspace=PTR + 0x60000000)
+    for heads in (1, 16, 32, 40, 64, 128, 200):
+        for batch in (1, 16, 62, 200, 511, 762, 1018):
+            for parts in (1, 7, 64, 128, 256, 512, 4000):
+                size = (batch + parts) * heads * (512 * 2 + 4)
+                p = _mla(batch=batch, heads_q=heads, num_sm_parts=parts, workspace_bytes=size, **plan)
+                need = lib.ma_mla_workspace_bytes(ctypes.byref(p))
+                assert lib.ma_mla_decode(ctypes.byref(p), None) == LAUNCH
+                fits = min(size, need) <= lib.ma_mla_noalloc_max_workspace()
+                assert lib.ma_mla_decode_noalloc(ctypes.byref(p), None) == ((UNSUPPORTED if need else LAUNCH) if fits else WORKSPACE)
+                p.workspace_bytes = min(size, need) - 1 if need else 0
+                assert lib.ma_mla_decode(ctypes.byref(p), None) == (WORKSPACE if need else LAUNCH)
