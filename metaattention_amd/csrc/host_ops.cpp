@@ -12,6 +12,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
@@ -31,8 +32,14 @@ using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
 // ------------------------------------------------------------------------------------------------------------- helpers
-// A tensor of exactly torch's own types (Tensor, Parameter); subclasses and functorch wrappers take the Python binding.
-inline const Tensor* tensor_of(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// A plain tensor of torch's own types (Tensor, Parameter).  Subclasses, functorch's wrappers (whose Python type is Tensor), any
+// tensor under a dispatch mode and dual tensors, whose tangents only the binding's autograd functions account for (they refuse
+// forward mode), take the Python binding.
+inline const Tensor* tensor_of(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  return at::isTensorSubclassLike(t) || t._fw_grad(0).defined() ? nullptr : &t;
+}
 
 inline bool on(const Tensor& t, int device) { return t.is_cuda() && t.device().index() == device; }
 
