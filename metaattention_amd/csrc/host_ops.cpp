@@ -18,17 +18,15 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
-#include <torch/csrc/autograd/function.h>
-#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
-#include <torch/csrc/autograd/saved_variable.h>
 
 #include "../../include/metaattention_hip.h"
 
 namespace {
 
 using at::Tensor;
-using torch::autograd::SavedVariable;
+using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 // ------------------------------------------------------------------------------------------------------------- helpers
@@ -152,53 +150,55 @@ bool attn_forward(const AttnPlan& pl, const Tensor& q, const Tensor& k, const Te
   return ma_attn_fwd(&p, st) == MA_OK;
 }
 
-// Backward of the softmax, sigmoid and relu operators: (dq, dk, dv) from what the forward call saved, as _attention.backward
-// (tl_template/attn/attn_tl.py:669-692).
-struct AttnBackward : public torch::autograd::Node {
-  int family = 0;
-  bool causal = false;
-  float scale = 1.f, bias = 0.f;
-  std::shared_ptr<const Masks> masks;
-  SavedVariable q_, k_, v_, o_, rs_;
-
-  std::string name() const override { return "AttentionBackward"; }
-  void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    q_.reset_data(); k_.reset_data(); v_.reset_data(); o_.reset_data(); rs_.reset_data();
+// The softmax, sigmoid and relu operators with gradients.  forward: what has been computed is put on the graph; backward: (dq, dk,
+// dv) from what it saved, as _attention.backward (tl_template/attn/attn_tl.py:669-692).  (A torch::autograd::Function, not a
+// Node of this file's own: it refuses forward mode and works under compiled autograd.)
+struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor* out, const Tensor* row_scale,
+                        const AttnPlan* pl, const Masks* masks) {
+    ctx->save_for_backward({q, k, v, *out, *row_scale});
+    auto& d = ctx->saved_data;
+    d["family"] = (int64_t)pl->family; d["causal"] = pl->causal; d["scale"] = (double)pl->scale; d["bias"] = (double)pl->bias;
+    if (masks) {   // (the operator's, not this call's: no business of saved-tensor hooks)
+      d["elem"] = masks->elem; d["elem_t"] = masks->elem_t; d["blocks"] = masks->blocks; d["blocks_t"] = masks->blocks_t;
+    }
+    return *out;
   }
 
-  variable_list apply(variable_list&& grads) override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
-    const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), o = o_.unpack(shared_from_this()), rs = rs_.unpack();
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &rs = saved[4];
+    auto& d = ctx->saved_data;
     at::AutoDispatchBelowADInplaceOrView no_autograd;
     const Tensor dout = kernel_view(grads[0]);
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     ma_attn_bwd_params p{};
-    p.family = family; p.dtype = dtype_code(q); p.mask = causal ? MA_MASK_CAUSAL : MA_MASK_NONE;
+    p.family = (int)d["family"].toInt(); p.dtype = dtype_code(q); p.mask = d["causal"].toBool() ? MA_MASK_CAUSAL : MA_MASK_NONE;
     p.batch = (int)q.size(0); p.heads = (int)q.size(2); p.heads_kv = (int)k.size(2); p.seqlen_q = (int)q.size(1); p.seqlen_kv = (int)k.size(1);
     p.dim_qk = (int)q.size(3); p.dim_v = (int)v.size(3);
     MA_SET_TENSOR(p, q, q, q); MA_SET_TENSOR(p, k, k, k); MA_SET_TENSOR(p, v, v, v); MA_SET_TENSOR(p, o, o, o);
     MA_SET_TENSOR(p, dout, do, dout); MA_SET_TENSOR(p, dq, dq, dq); MA_SET_TENSOR(p, dk, dk, dk); MA_SET_TENSOR(p, dv, dv, dv);
     if (rs.defined()) p.lse = (const float*)rs.data_ptr();
-    p.scale = scale; p.bias = bias;
-    if (masks) {
-      const Masks& m = *masks;
-      p.elem_mask = (const uint8_t*)m.elem.data_ptr();
-      p.em_stride_b = mask_stride(m.elem, 0); p.em_stride_h = mask_stride(m.elem, 1); p.em_stride_q = m.elem.stride(2);
-      p.elem_mask_t = (const uint8_t*)m.elem_t.data_ptr();
-      p.emt_stride_b = mask_stride(m.elem_t, 0); p.emt_stride_h = mask_stride(m.elem_t, 1); p.emt_stride_k = m.elem_t.stride(2);
-      p.kv_block_mask = (const uint8_t*)m.blocks.data_ptr();
-      p.kbm_stride_b = mask_stride(m.blocks, 0); p.kbm_stride_h = mask_stride(m.blocks, 1); p.kbm_stride_q = m.blocks.stride(2);
-      p.q_block_mask = (const uint8_t*)m.blocks_t.data_ptr();
-      p.qbm_stride_b = mask_stride(m.blocks_t, 0); p.qbm_stride_h = mask_stride(m.blocks_t, 1); p.qbm_stride_k = m.blocks_t.stride(2);
+    p.scale = (float)d["scale"].toDouble(); p.bias = (float)d["bias"].toDouble();
+    if (d.count("elem")) {
+      const Tensor elem = d["elem"].toTensor(), elem_t = d["elem_t"].toTensor(), blocks = d["blocks"].toTensor(), blocks_t = d["blocks_t"].toTensor();
+      p.elem_mask = (const uint8_t*)elem.data_ptr();
+      p.em_stride_b = mask_stride(elem, 0); p.em_stride_h = mask_stride(elem, 1); p.em_stride_q = elem.stride(2);
+      p.elem_mask_t = (const uint8_t*)elem_t.data_ptr();
+      p.emt_stride_b = mask_stride(elem_t, 0); p.emt_stride_h = mask_stride(elem_t, 1); p.emt_stride_k = elem_t.stride(2);
+      p.kv_block_mask = (const uint8_t*)blocks.data_ptr();
+      p.kbm_stride_b = mask_stride(blocks, 0); p.kbm_stride_h = mask_stride(blocks, 1); p.kbm_stride_q = blocks.stride(2);
+      p.q_block_mask = (const uint8_t*)blocks_t.data_ptr();
+      p.qbm_stride_b = mask_stride(blocks_t, 0); p.qbm_stride_h = mask_stride(blocks_t, 1); p.qbm_stride_k = blocks_t.stride(2);
     }
     const size_t need = ma_attn_bwd_workspace_bytes(&p);
     const c10::DataPtr ws = scratch(need);
     p.workspace = ws.get(); p.workspace_bytes = need;
-    NoGil release;
-    TORCH_CHECK(ma_attn_bwd(&p, stream_of(q.device().index())) == MA_OK, ma_last_error());
-    return {dq, dk, dv};
+    {
+      NoGil release;
+      TORCH_CHECK(ma_attn_bwd(&p, stream_of(q.device().index())) == MA_OK, ma_last_error());
+    }
+    return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -240,17 +240,7 @@ PyObject* attention_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   }
   Tensor out, rs;
   if (!attn_forward(pl, q, k, v, mult, gamma, masks.get(), dev, out, rs)) return none();
-  if (grad) {
-    auto node = std::shared_ptr<AttnBackward>(new AttnBackward(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v));
-    node->family = pl.family; node->causal = pl.causal; node->scale = pl.scale; node->bias = pl.bias; node->masks = std::move(masks);
-    node->q_ = SavedVariable(q, false);
-    node->k_ = SavedVariable(k, false);
-    node->v_ = SavedVariable(v, false);
-    if (rs.defined()) node->rs_ = SavedVariable(rs, false);
-    torch::autograd::set_history(out, node);
-    node->o_ = SavedVariable(out, true);
-  }
+  if (grad) out = AttentionFunction::apply(q, k, v, &out, &rs, &pl, masks.get());
   PyObject* r = PyTuple_New(2);
   if (!r) return nullptr;
   PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out));
@@ -400,26 +390,22 @@ bool linear_forward(const LinearPlan& pl, const Tensor& q, const Tensor& k, cons
   return ma_linear_fwd(&p, st) == MA_OK;
 }
 
-// Backward of the chunked operator with respect to q, k, v, the log decay and the value scale, as LinearAttention.backward
-// (tl_template/linear/linear_tl.py:1268-1340).
-struct LinearBackward : public torch::autograd::Node {
-  float q_scale = 1.f;
-  SavedVariable q_, k_, v_, g_, vs_;
-  at::ScalarType g_type = at::kFloat, vs_type = at::kFloat;
-  bool has_vs = false;
-
-  std::string name() const override { return "LinearAttentionBackward"; }
-  void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    q_.reset_data(); k_.reset_data(); v_.reset_data(); g_.reset_data(); vs_.reset_data();
+// The chunked operator with gradients for q, k, v, the log decay and the value scale (if any), as LinearAttention.backward
+// (tl_template/linear/linear_tl.py:1268-1340); see AttentionFunction.
+struct LinearFunction : torch::autograd::Function<LinearFunction> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const std::optional<Tensor>& vs, const Tensor* out,
+                        double q_scale) {
+    ctx->save_for_backward(vs ? variable_list{q, k, v, g, *vs} : variable_list{q, k, v, g});
+    ctx->saved_data["q_scale"] = q_scale;
+    return *out;
   }
 
-  variable_list apply(variable_list&& grads) override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    if (!grads[0].defined()) return variable_list(has_vs ? 5 : 4);
-    const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), g0 = g_.unpack(), vs0 = vs_.unpack();
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const bool has_vs = saved.size() > 4;
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2];
     at::AutoDispatchBelowADInplaceOrView no_autograd;
-    const Tensor g = per_token(g0), vs = has_vs ? per_token(vs0) : Tensor();
+    const Tensor g = per_token(saved[3]), vs = has_vs ? per_token(saved[4]) : Tensor();
     const Tensor dout = grads[0].to(v.scalar_type()).contiguous();
     const Tensor dq = empty(q.sizes(), q.scalar_type(), q.device()), dk = empty(k.sizes(), k.scalar_type(), k.device()),
                  dv = empty(v.sizes(), v.scalar_type(), v.device());
@@ -431,7 +417,7 @@ struct LinearBackward : public torch::autograd::Node {
     p.q = q.data_ptr(); p.k = k.data_ptr(); p.v = v.data_ptr(); p.dout = dout.data_ptr();
     p.log_decay = (const float*)g.data_ptr();
     p.v_scale = has_vs ? (const float*)vs.data_ptr() : nullptr;
-    p.q_scale = q_scale;
+    p.q_scale = (float)ctx->saved_data["q_scale"].toDouble();
     p.dq = dq.data_ptr(); p.dk = dk.data_ptr(); p.dv = dv.data_ptr(); p.dlog_decay = (float*)dg.data_ptr();
     p.dv_scale = has_vs ? (float*)dvs.data_ptr() : nullptr;
     const size_t need = ma_linear_bwd_workspace_bytes(&p);
@@ -441,10 +427,9 @@ struct LinearBackward : public torch::autograd::Node {
       NoGil release;
       TORCH_CHECK(ma_linear_bwd(&p, stream_of(v.device().index())) == MA_OK, ma_last_error());
     }
-    if (g_type != at::kFloat) dg = dg.to(g_type);
-    if (!has_vs) return {dq, dk, dv, dg};
-    if (vs_type != at::kFloat) dvs = dvs.to(vs_type);
-    return {dq, dk, dv, dg, dvs};
+    dg = dg.to(saved[3].scalar_type());
+    if (has_vs) dvs = dvs.to(saved[4].scalar_type());
+    return {dq, dk, dv, dg, dvs, Tensor(), Tensor()};
   }
 };
 
@@ -484,22 +469,7 @@ PyObject* linear_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     at::AutoDispatchBelowADInplaceOrView no_autograd;
     if (!linear_forward(pl, q, k, v, per_token(g), vs.defined() ? per_token(vs) : vs, dev, out)) return none();
   }
-  if (grad) {
-    auto node = std::shared_ptr<LinearBackward>(new LinearBackward(), torch::autograd::deleteNode);
-    node->has_vs = vs.defined();
-    node->set_next_edges(vs.defined() ? torch::autograd::collect_next_edges(q, k, v, g, vs) : torch::autograd::collect_next_edges(q, k, v, g));
-    node->q_scale = pl.q_scale;
-    node->g_type = g.scalar_type();
-    node->q_ = SavedVariable(q, false);
-    node->k_ = SavedVariable(k, false);
-    node->v_ = SavedVariable(v, false);
-    node->g_ = SavedVariable(g, false);
-    if (vs.defined()) {
-      node->vs_type = vs.scalar_type();
-      node->vs_ = SavedVariable(vs, false);
-    }
-    torch::autograd::set_history(out, node);
-  }
+  if (grad) out = LinearFunction::apply(q, k, v, g, vs.defined() ? std::optional<Tensor>(vs) : std::nullopt, &out, (double)pl.q_scale);
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }

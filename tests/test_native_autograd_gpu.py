@@ -4,6 +4,8 @@ import pytest
 import torch
 
 import specs
+from attn_engine import AttentionEngine
+from core import CustomIO, meta_tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +47,65 @@ def test_functorch_transforms_are_refused(which):
         torch.func.grad(lambda x: mod(x, *args[1:]).float().sum())(args[0])
     with pytest.raises((RuntimeError, NotImplementedError)):
         torch.func.jvp(lambda x: mod(x, *args[1:]), (args[0],), (torch.ones_like(args[0]),))
+
+
+def _leaves(args):
+    return [a.detach().clone().requires_grad_(True) for a in args]
+
+
+def _grads(mod, args):
+    leaves = _leaves(args)
+    out = mod(*leaves)
+    out.backward(torch.ones_like(out))
+    return [out.detach()] + [x.grad for x in leaves]
+
+
+@pytest.mark.parametrize("which", OPERATORS + ["window"])
+def test_compiled_autograd(which):
+    from torch._dynamo import compiled_autograd
+    if which == "window":
+        mod = AttentionEngine(tuple(meta_tensor(1, 4, 70, 64, dtype=torch.bfloat16) for _ in range(3)), CustomIO({}),
+                              score_mod=lambda s, io, b, h, q, k: s * 0.125, mask_mod=lambda b, h, q, k: (q >= k) & (q - k < 20),
+                              online_func=specs.OnlineSoftmax())
+        args = tuple(_rand(1, 70, 4, 64) for _ in range(3))
+    else:
+        mod, args = _operators()[which]
+    want = _grads(mod, args)
+    want = _grads(mod, args)                    # (a masked operator's first call builds its masks in the binding)
+    for _ in range(2):
+        with compiled_autograd._enable(lambda gm: gm):
+            got = _grads(mod, args)
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("which", OPERATORS)
+def test_saved_tensor_hooks(which):
+    """What the backward needs goes through the hooks, and through nothing else: the inputs, the output, the row scale."""
+    mod, args = _operators()[which]
+    want, packed = _grads(mod, args), []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        got = _grads(mod, args)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    assert len(packed) == {"softmax": 5, "relu": 4, "gated": 4}[which]
+
+
+@pytest.mark.parametrize("which", OPERATORS)
+def test_backward_twice_and_inputs_changed_in_between(which):
+    mod, args = _operators()[which]
+    leaves = _leaves(args)
+    out = mod(*leaves)
+    first = torch.autograd.grad(out, leaves, torch.ones_like(out), retain_graph=True)
+    again = torch.autograd.grad(out, leaves, torch.ones_like(out))
+    assert all(torch.equal(x, y) for x, y in zip(first, again))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out, leaves, torch.ones_like(out))
+    leaves = _leaves(args)
+    scaled = [x * 1 for x in leaves]
+    out = mod(*scaled)
+    scaled[2].mul_(2)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        out.sum().backward()
