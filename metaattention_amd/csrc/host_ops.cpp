@@ -20,6 +20,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/metaattention_hip.h"
 
@@ -38,6 +39,9 @@ inline const Tensor* tensor_of(PyObject* o) {
   const Tensor& t = THPVariable_Unpack(o);
   return at::isTensorSubclassLike(t) || t._fw_grad(0).defined() ? nullptr : &t;
 }
+
+// torch.jit.trace records the binding's autograd functions, but nothing that happens here (the output would be a constant).
+inline bool traced() { return torch::jit::tracer::isTracing(); }
 
 inline bool on(const Tensor& t, int device) { return t.is_cuda() && t.device().index() == device; }
 
@@ -212,7 +216,7 @@ PyObject* attention_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const AttnPlan& pl = *(const AttnPlan*)PyCapsule_GetPointer(self, kAttnPlan);
   const bool retention = pl.family == MA_ATTN_RETENTION;
-  if (n != (retention ? 4 : 3)) return none();
+  if (n != (retention ? 4 : 3) || traced()) return none();
   const Tensor *qp = tensor_of(args[0]), *kp = tensor_of(args[1]), *vp = tensor_of(args[2]), *mult = retention ? tensor_of(args[3]) : nullptr;
   if (!qp || !kp || !vp || (retention && !mult)) return none();
   const Tensor &q = *qp, &k = *kp, &v = *vp;
@@ -274,7 +278,7 @@ bool mla_launch(ma_mla_params& p, int dev) {
 PyObject* mla_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const MlaPlan& pl = *(const MlaPlan*)PyCapsule_GetPointer(self, kMlaPlan);
-  if (n != 4) return none();
+  if (n != 4 || traced()) return none();
   const Tensor* t[4];
   for (int i = 0; i < 4; i++)
     if (!(t[i] = tensor_of(args[i])) || !t[i]->is_cuda()) return none();
@@ -304,7 +308,7 @@ PyObject* mla_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 // num_splits | None) -> (out [B,1,Hq,D], lse [B,Hq,1]), or None.  The paged interface of flash_mla_with_kvcache.
 PyObject* mla_paged_call(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 8) return none();
+  if (n != 8 || traced()) return none();
   const Tensor *q = tensor_of(args[0]), *kc = tensor_of(args[1]), *bt = tensor_of(args[2]), *sl = tensor_of(args[3]);
   if (!q || !kc || !bt || !sl || !q->is_cuda()) return none();
   const int dev = c10::hip::current_device();
@@ -437,7 +441,7 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
 PyObject* linear_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const LinearPlan& pl = *(const LinearPlan*)PyCapsule_GetPointer(self, kLinearPlan);
-  if (n != 4 + pl.n_custom || n > 12) return none();
+  if (n != 4 + pl.n_custom || n > 12 || traced()) return none();
   const Tensor* t[12];
   for (int i = 0; i < n; i++)
     if (!(t[i] = tensor_of(args[i])) || !t[i]->is_cuda()) return none();

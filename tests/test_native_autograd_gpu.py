@@ -109,3 +109,15 @@ def test_backward_twice_and_inputs_changed_in_between(which):
     scaled[2].mul_(2)
     with pytest.raises(RuntimeError, match="inplace operation"):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("which", OPERATORS)
+@pytest.mark.filterwarnings("ignore")
+def test_trace(which):
+    """A trace made with inputs that get gradients runs the operator, on other inputs than those it was made with as well."""
+    mod, args = _operators()[which]
+    mod(*args)
+    traced = torch.jit.trace(lambda *a: mod(*a) + 0, tuple(_leaves(args)), check_trace=False)
+    other = _leaves([a.flip(0, 1) for a in args])
+    assert torch.equal(traced(*other), mod(*other))
+    assert all(torch.equal(x, y) for x, y in zip(_grads(traced, other), _grads(mod, other)))
