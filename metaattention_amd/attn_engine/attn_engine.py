@@ -131,6 +131,9 @@ class _Attention(torch.autograd.Function):
 
 
 class AttentionEngine:
+    _takes_native = False                # whether the operator has a native call (csrc/host_ops.cpp)
+    _native_fn = _native_mla = None      # made at the first call: see _bind_native, _call_mla
+
     def __init__(self, qkv_meta, custom_fwd_inputs, score_mod, mask_mod, online_func,
                  mask_value="-inf", device=None, backend="tl",
                  tune=False, tune_file="", tune_bwd=False, tune_file_bwd="",
@@ -218,24 +221,33 @@ class AttentionEngine:
         # the native call takes q, k, v (and retention's multiplier); score functions with other custom inputs or index terms
         # go through _call_prefill
         plain = not (form.extra or form.softcap is not None or form.bias_tensor)
-        self._native = self._bind_native if plain and len(self.names) == (fam == "retention") else None
+        self._takes_native = plain and len(self.names) == (fam == "retention")
 
-    def _bind_native(self, *args):
-        """First call: makes the operator's native callable (csrc/host_ops.cpp), which takes this place."""
+    def _bind_native(self):
+        """First call: makes the operator's native callable."""
         from hip_backend import host, MA_BF16, MA_FP16
         form = self.score_form
-        native = host().attention_plan(_FAMILY_CODE[self.family], MA_BF16 if self.dtype == torch.bfloat16 else MA_FP16,
-                                       self.mask_kind == "causal", self.mask_kind.startswith("other"), form.scale, form.bias)
-        self._native_fn = native
-        self._native = self._native_retention if self.family == "retention" else native
-        return self._native(*args)
+        self._native_fn = host().attention_plan(_FAMILY_CODE[self.family], MA_BF16 if self.dtype == torch.bfloat16 else MA_FP16,
+                                                self.mask_kind == "causal", self.mask_kind.startswith("other"), form.scale, form.bias)
+        if self._mask_tensors is not None:      # (built by the operator that this one is a copy of)
+            self._register_masks()
+        return self._native_fn
 
-    def _native_retention(self, *args):
+    def __getstate__(self):
+        """For pickle and copy: without the native callables, which a copy makes anew (its masks are its own), and without the
+        decays remembered per tensor object."""
+        return {k: v for k, v in self.__dict__.items() if k not in ("_native_fn", "_native_mla", "_gamma_cache")}
+
+    def _native_call(self, *args):
+        """The native call's (out, row scale or None), or None where the binding has to serve."""
+        fn = self._native_fn or self._bind_native()
+        if self.family != "retention":
+            return fn(*args)
         if len(args) != 4 or any(t.dim() != 4 for t in args):
             return None
         q, k, v, mask = args
         gamma = self._gamma_for(q, k, v, mask)
-        res = self._native_fn(q, k, v, mask if gamma is None else gamma)
+        res = fn(q, k, v, mask if gamma is None else gamma)
         if res is not None:
             self.last_call_generated_mask = gamma is not None
         return res
@@ -470,11 +482,10 @@ class AttentionEngine:
 
     def _register_masks(self):
         """Hands the dense masks of the current shape to the native call."""
-        fn = getattr(self, "_native_fn", None)
-        if fn is not None:
+        if self._native_fn is not None:
             from hip_backend import host
             (B, H, Sq, Skv, _), elem, _, t, blocks = self._mask_tensors
-            host().attention_masks(fn, B, H, Sq, Skv, elem, blocks, *(t if t is not None else (None, None)))
+            host().attention_masks(self._native_fn, B, H, Sq, Skv, elem, blocks, *(t if t is not None else (None, None)))
 
     # ------------------------------------------------------------------ MLA decode
     def _init_mla(self, backend="tl"):
@@ -488,7 +499,6 @@ class AttentionEngine:
         # (core/lower/lower_decode_mla.py:25-38): fixed softmax, scale (d + d_pe)^-0.5
         self.mla_scale = 1.0 / math.sqrt(m["Dqk"])
         self.attention = self._call_mla
-        self._native_mla = None
         if backend in ("cute", "cute_v2"):
             # the paged interface of the reference's second MLA backend (attn_engine.py:196-224): mod(q [B,1,Hq,576],
             # k_cache [B * Skv / 64, 64, 1, 576]) -> (out, lse), every sequence full, pages in order
@@ -551,9 +561,8 @@ class AttentionEngine:
         return mla_decode(*(_kernel_view(t) for t in (q, q_pe, kv, k_pe)), scale=self.mla_scale)
 
     def __call__(self, *args, **kargs):
-        native = getattr(self, "_native", None) if not kargs else None
-        if native is not None:
-            res = native(*args)
+        if self._takes_native and not kargs:
+            res = self._native_call(*args)
             if res is not None:
                 out, self.final_rowscales = res
                 return out

@@ -42,6 +42,9 @@ class _LinearAttention(torch.autograd.Function):
 
 
 class LinearAttentionEngine:
+    _takes_native = False      # whether the native call (csrc/host_ops.cpp) evaluates the operator's decay_mod
+    _native_fn = None          # made at the first call: see _bind_native
+
     def __init__(self, qkv_meta, q_mod=None, k_mod=None, v_mod=None, decay_mod=None, custom_io=None,
                  tune=False, tune_filename="tune_result", tune_bwd=False, chunk_size=None):
         # tune* select the reference's tile search; fixed CDNA4 tiles here.
@@ -58,17 +61,21 @@ class LinearAttentionEngine:
         self.attention = self._call
         # the native call evaluates these decay_mods; any other is evaluated here, see _log_decay
         plan = self.plan
-        self._native = self._bind_native if plan.decay_sym is None or plan.decay_kind in ("log", "mul_head") else None
+        self._takes_native = plan.decay_sym is None or plan.decay_kind in ("log", "mul_head")
 
-    def _bind_native(self, *args):
-        """First call: makes the operator's native callable (csrc/host_ops.cpp), which takes this place."""
+    def _bind_native(self):
+        """First call: makes the operator's native callable."""
         from hip_backend import host
         plan = self.plan
         kind = "identity" if plan.decay_sym is None else plan.decay_kind
-        self._native = host().linear_plan({"identity": 0, "log": 1, "mul_head": 2}[kind],
-                                          self.names.index(plan.decay_head_tensor) if kind == "mul_head" else -1,
-                                          self.names.index(plan.v_scale_tensor) if plan.v_scale_tensor else -1, len(self.names), plan.q_scale)
-        return self._native(*args)
+        self._native_fn = host().linear_plan({"identity": 0, "log": 1, "mul_head": 2}[kind],
+                                             self.names.index(plan.decay_head_tensor) if kind == "mul_head" else -1,
+                                             self.names.index(plan.v_scale_tensor) if plan.v_scale_tensor else -1, len(self.names), plan.q_scale)
+        return self._native_fn
+
+    def __getstate__(self):
+        """For pickle and copy: without the native callable, which a copy makes anew."""
+        return {k: v for k, v in self.__dict__.items() if k != "_native_fn"}
 
     def _log_decay(self, decay, given):
         """decay_mod evaluated on the [B,H,T] fp32 decay input.  Like the
@@ -102,8 +109,8 @@ class LinearAttentionEngine:
         return linear_fwd(q, k, v, g, q_scale=self.plan.q_scale, v_scale=v_scale, chunk=self.chunk_size)
 
     def __call__(self, *args, **kargs):
-        if self._native is not None and not kargs:
-            out = self._native(*args)
+        if self._takes_native and not kargs:
+            out = (self._native_fn or self._bind_native())(*args)
             if out is not None:
                 return out
         return self.attention(*args, **kargs)
