@@ -79,3 +79,55 @@ def test_mla_and_decode(Hq, KV):
     out = dec(q, k, v)
     scales = dec.final_rowscales
     assert torch.equal(out, dec.attention(q, k, v)) and torch.equal(scales, dec.final_rowscales)
+
+
+def _binding_is_off(monkeypatch):
+    import hip_backend
+
+    def refuse(*args, **kwargs):
+        raise AssertionError("the binding was called")
+    for name in ("attn_fwd", "attn_bwd", "linear_fwd", "linear_bwd", "mla_decode", "_require_gpu"):
+        monkeypatch.setattr(hip_backend, name, refuse)
+
+
+def test_ordinary_calls_are_served_natively(monkeypatch):
+    """Forward and, through the native autograd functions, backward of the ordinary calls never reach the Python binding."""
+    from hip_backend import flash_mla_with_kvcache, get_mla_metadata
+    lens = torch.tensor([100, 64], dtype=torch.int32, device="cuda")
+    plan = get_mla_metadata(lens, 16, 1)
+    window = specs.softmax_attention(2, 4, 65, 64, 64)
+    window.mask_kind, window.mask_mod = "other", _window
+    q, k, v = _rand(2, 65, 4, 64), _rand(2, 65, 2, 64), _rand(2, 65, 2, 64)
+    want = _grads(window, (q, k, v))                     # (the first call builds the masks, in the binding)
+    _binding_is_off(monkeypatch)
+    assert all(torch.equal(x, y) for x, y in zip(_grads(window, (q, k, v)), want))
+    for mod in (specs.softmax_attention(2, 4, 65, 64, 64), specs.relu_attention(2, 4, 65, 64, 64), specs.sigmoid_attention(2, 4, 65, 64, 64, const_bias=-1.0)):
+        _grads(mod, (q, k, v))
+    decay = torch.rand(2, 4, 65, device="cuda") * 0.1 + 0.5
+    lin = _rand(2, 4, 65, 64, gain=0.1), _rand(2, 4, 65, 64, gain=0.1), _rand(2, 4, 65, 64)
+    _grads(specs.retnet_recurrent(2, 4, 65, 64, 64), (*lin, decay))
+    _grads(specs.gated_retention(2, 4, 65, 64, 64), (*lin, -decay))
+    _grads(specs.mamba2(2, 1, 65, 64, 64, HV=4), (lin[0][:, :1].contiguous(), lin[1][:, :1].contiguous(), lin[2], decay, -torch.rand(1, 4, device="cuda"), decay.bfloat16()))
+    specs.softmax_attention_decode(2, 4, 1, 300, 64, 64, dtype=torch.bfloat16, HKV=2)(q[:, :1].contiguous(), _rand(2, 300, 2, 64), _rand(2, 300, 2, 64))
+    specs.mla_decode(2, 16, 100, 576, 512)(_rand(2, 1, 16, 512), _rand(2, 1, 16, 64), _rand(2, 100, 1, 512), _rand(2, 100, 1, 64))
+    table = torch.arange(4, dtype=torch.int32, device="cuda").view(2, 2)
+    for p in ((), plan):
+        flash_mla_with_kvcache(_rand(2, 1, 16, 576), _rand(4, 64, 1, 576), table, lens, 512, *p)
+    ret = specs.retention_parallel(1, 2, 68, 256, 512)
+    ret(_rand(1, 68, 2, 256, gain=0.1), _rand(1, 68, 2, 256, gain=0.1), _rand(1, 68, 2, 512), _rand(1, 2, 68, 68))
+
+
+def test_what_the_native_call_hands_over_it_does_not_launch():
+    """Such calls return None at the checks, before anything is allocated for a launch; the operator then serves them once."""
+    mod = specs.softmax_attention(1, 4, 70, 64, 64)
+    q, k, v = _rand(1, 70, 4, 64), _rand(1, 70, 4, 64), _rand(1, 70, 4, 64)
+    out = mod(q, k, v)
+    wide = torch.zeros(1, 70, 4, 65, dtype=q.dtype, device="cuda")[..., :64]
+    wide.copy_(q)
+    odd = {"unaligned view": (wide, k, v), "another dtype": (q.half(), k.half(), v.half()), "too many": (q, k, v, q), "not on the GPU": (q.cpu(), k, v),
+           "a subclass": (torch.Tensor._make_subclass(type("Mine", (torch.Tensor,), {}), q), k, v)}
+    for name, args in odd.items():
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        assert mod._native_fn(*args) is None, name
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before, name
+    assert torch.equal(mod(*odd["unaligned view"]), out)
