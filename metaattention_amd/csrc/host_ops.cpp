@@ -160,7 +160,9 @@ bool attn_forward(const AttnPlan& pl, const Tensor& q, const Tensor& k, const Te
 struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor* out, const Tensor* row_scale,
                         const AttnPlan* pl, const Masks* masks) {
-    ctx->save_for_backward({q, k, v, *out, *row_scale});
+    // (the output without its history: a saved-tensor hook that raises, as checkpointing's does to stop a recomputation, leaves what
+    // was to be saved in the node, and with a history that would be a cycle that keeps the whole graph)
+    ctx->save_for_backward({q, k, v, out->detach(), *row_scale});
     auto& d = ctx->saved_data;
     d["family"] = (int64_t)pl->family; d["causal"] = pl->causal; d["scale"] = (double)pl->scale; d["bias"] = (double)pl->bias;
     if (masks) {   // (the operator's, not this call's: no business of saved-tensor hooks)

@@ -121,3 +121,54 @@ def test_trace(which):
     other = _leaves([a.flip(0, 1) for a in args])
     assert torch.equal(traced(*other), mod(*other))
     assert all(torch.equal(x, y) for x, y in zip(_grads(traced, other), _grads(mod, other)))
+
+
+@pytest.mark.parametrize("which", OPERATORS)
+def test_checkpointing_leaves_nothing_behind(which):
+    """A recomputation ends in the middle of saving, by an exception: what was computed is freed with the graph all the same."""
+    from torch.utils.checkpoint import checkpoint
+    mod, args = _operators()[which]
+    leaves = _leaves(args)
+
+    def step():
+        out = checkpoint(mod, *leaves, use_reentrant=False)
+        return torch.autograd.grad(out, leaves, torch.ones_like(out))
+    want = torch.autograd.grad(mod(*leaves), leaves, torch.ones_like(args[0]))
+    assert all(torch.equal(x, y) for x, y in zip(step(), want))
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        step()
+    assert torch.cuda.memory_allocated() == before
+    edge = torch.autograd.graph.get_gradient_edge(leaves[0]).node      # (made anew when no graph holds it)
+    assert "seen" not in edge.metadata
+    edge.metadata["seen"] = True
+    del edge
+    assert "seen" not in torch.autograd.graph.get_gradient_edge(leaves[0]).node.metadata
+
+
+@pytest.mark.parametrize("which", OPERATORS)
+def test_training_pass_in_a_graph(which):
+    mod, args = _operators()[which]
+    leaves, dout = _leaves(args), torch.ones_like(args[0])
+
+    def step():
+        return torch.autograd.grad(mod(*leaves), leaves, dout)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for seed in range(3):
+        with torch.no_grad():
+            for x, a in zip(leaves, args):
+                x.copy_(a.roll(seed, 0).flip(1))
+        want = step()
+        for x in got:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
