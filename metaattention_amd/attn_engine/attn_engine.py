@@ -238,11 +238,7 @@ class AttentionEngine:
         decays remembered per tensor object."""
         return {k: v for k, v in self.__dict__.items() if k not in ("_native_fn", "_native_mla", "_gamma_cache")}
 
-    def _native_call(self, *args):
-        """The native call's (out, row scale or None), or None where the binding has to serve."""
-        fn = self._native_fn or self._bind_native()
-        if self.family != "retention":
-            return fn(*args)
+    def _native_retention(self, fn, *args):
         if len(args) != 4 or any(t.dim() != 4 for t in args):
             return None
         q, k, v, mask = args
@@ -562,7 +558,8 @@ class AttentionEngine:
 
     def __call__(self, *args, **kargs):
         if self._takes_native and not kargs:
-            res = self._native_call(*args)
+            fn = self._native_fn or self._bind_native()
+            res = fn(*args) if self.family != "retention" else self._native_retention(fn, *args)
             if res is not None:
                 out, self.final_rowscales = res
                 return out

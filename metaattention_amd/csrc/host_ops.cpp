@@ -162,9 +162,9 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
                         const AttnPlan* pl, const Masks* masks) {
     // (the output without its history: a saved-tensor hook that raises, as checkpointing's does to stop a recomputation, leaves what
     // was to be saved in the node, and with a history that would be a cycle that keeps the whole graph)
-    ctx->save_for_backward({q, k, v, out->detach(), *row_scale});
+    ctx->save_for_backward({q, k, v, out->tensor_data(), *row_scale});
     auto& d = ctx->saved_data;
-    d["family"] = (int64_t)pl->family; d["causal"] = pl->causal; d["scale"] = (double)pl->scale; d["bias"] = (double)pl->bias;
+    d["plan"] = std::vector<double>{(double)pl->family, pl->causal ? 1. : 0., pl->scale, pl->bias};
     if (masks) {   // (the operator's, not this call's: no business of saved-tensor hooks)
       d["elem"] = masks->elem; d["elem_t"] = masks->elem_t; d["blocks"] = masks->blocks; d["blocks_t"] = masks->blocks_t;
     }
@@ -175,17 +175,18 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
     const variable_list saved = ctx->get_saved_variables();
     const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &rs = saved[4];
     auto& d = ctx->saved_data;
+    const std::vector<double> plan = d["plan"].toDoubleVector();
     at::AutoDispatchBelowADInplaceOrView no_autograd;
     const Tensor dout = kernel_view(grads[0]);
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     ma_attn_bwd_params p{};
-    p.family = (int)d["family"].toInt(); p.dtype = dtype_code(q); p.mask = d["causal"].toBool() ? MA_MASK_CAUSAL : MA_MASK_NONE;
+    p.family = (int)plan[0]; p.dtype = dtype_code(q); p.mask = plan[1] != 0 ? MA_MASK_CAUSAL : MA_MASK_NONE;
     p.batch = (int)q.size(0); p.heads = (int)q.size(2); p.heads_kv = (int)k.size(2); p.seqlen_q = (int)q.size(1); p.seqlen_kv = (int)k.size(1);
     p.dim_qk = (int)q.size(3); p.dim_v = (int)v.size(3);
     MA_SET_TENSOR(p, q, q, q); MA_SET_TENSOR(p, k, k, k); MA_SET_TENSOR(p, v, v, v); MA_SET_TENSOR(p, o, o, o);
     MA_SET_TENSOR(p, dout, do, dout); MA_SET_TENSOR(p, dq, dq, dq); MA_SET_TENSOR(p, dk, dk, dk); MA_SET_TENSOR(p, dv, dv, dv);
     if (rs.defined()) p.lse = (const float*)rs.data_ptr();
-    p.scale = (float)d["scale"].toDouble(); p.bias = (float)d["bias"].toDouble();
+    p.scale = (float)plan[2]; p.bias = (float)plan[3];
     if (d.count("elem")) {
       const Tensor elem = d["elem"].toTensor(), elem_t = d["elem_t"].toTensor(), blocks = d["blocks"].toTensor(), blocks_t = d["blocks_t"].toTensor();
       p.elem_mask = (const uint8_t*)elem.data_ptr();
