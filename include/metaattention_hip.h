@@ -19,6 +19,9 @@
  *     case ma_last_error() (thread local) describes the problem;
  *   - strides are in ELEMENTS of the tensor's dtype; the innermost (feature)
  *     dimension of every tensor must be contiguous;
+ *   - a call gives the same bits every time; the order of its sums follows from all of its sizes, batch and heads
+ *     included (how many workgroups, splits, runs or segments there are), so that a batch entry may differ in the last bits
+ *     from the same entry in a call of its own;
  *   - tensors may be larger than 4 GiB (bases are 64-bit).  The kernels count work items and rows in 32 bits:
  *     sequence lengths up to 2^24 (2^30 for the chunked and the MLA operators), batch x heads x ceil(seqlen / 32)
  *     below 2^30, and whatever else a call's description names; sizes beyond that come back as MA_ERR_UNSUPPORTED.
@@ -113,7 +116,7 @@ typedef struct ma_attn_params {
    *   x = s * scale + bias + score_add[b, h, q, kv] + pos_slope_q[h] * q + pos_slope_kv[h] * kv,
    * score_add fp32 (score_add_fp32 != 0) or `dtype`, addressed with ELEMENT strides, 0 for an axis the tensor does not
    * have; pos_slope_* fp32 [heads].  softcap > 0 (SOFTMAX only): x is replaced by softcap * tanh(x) before the row
-   * function.  The backward kernels do not take these. */
+   * function.  (Gradients through them: the same fields of ma_attn_bwd_params.) */
   const void* score_add; int64_t sa_stride_b, sa_stride_h, sa_stride_q, sa_stride_kv; int32_t score_add_fp32;
   const float* pos_slope_q; const float* pos_slope_kv;
   float softcap;

@@ -1241,9 +1241,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_reduce_kernel(const AttnBwdA
 // ------------------------------------------------------------------------------------------------
 // Two streams of key tiles in the dq kernel where row blocks are few: a tile is a serial chain of about a microsecond, and with
 // at most one workgroup of four waves per CU half of the wave slots are empty.  Under a causal mask (heaviest blocks first)
-// the chains of the longest blocks still bind at 1.5 row blocks per CU.  Forward + backward, one and two streams: B1 H8 S2048
-// 128/128 causal (128 blocks) 145.8, 132.6 us; B2 H16 S1000 192/128 (256) 151.7, 145.5; B4 H12 S1024 64/64 causal (384) 83.6,
-// 78.6; beyond the line B8 H12 S600 64/64 causal (480) 74.5, 76.3 and B4 H12 S1024 128/128 without a mask (384) 163.4, 174.3.
+// the chains of the longest blocks still bind at 1.5 row blocks per CU, and about there the sizes cross.  Forward + backward,
+// two streams against one at 320, 384, 416 and 448 row blocks: 128/128 S1024 0.96, 0.99, 1.01, 1.03, 192/128 S1024 0.97, 0.99, 1.02,
+// 1.02, 64/64 S600 0.93, 1.01, 1.04, .. (480) 1.02; longer chains cross later (64/64 S1024 0.91, 0.93, 0.96, 0.98; 128/128 S2048 0.93,
+// 0.94, 0.97, 0.98).  Without a mask, at 192, 256 and 288: 128/128 0.97, 0.99, 1.08, 64/64 0.92, 0.91, 1.06.
 inline bool dq_two_streams(int64_t blocks, bool causal) { return 2 * blocks <= (causal ? 3 : 2) * (int64_t)device_cus(); }
 
 template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL>

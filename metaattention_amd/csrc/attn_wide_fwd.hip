@@ -143,7 +143,8 @@ AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, in
   };
   const bool sizes = (dqk == 64 && dv == 64) || (dqk == 128 && dv == 128) || (dqk == 192 && dv == 128);
   consider(AttnCut::kRows128, 4, 1, 6.2);
-  // (only where row blocks of 128 leave slots empty: a batch that fills them gives every entry the bits it has alone)
+  // (only where row blocks of 128 leave slots empty.  With batch x heads in the rule, a row's sums, and so its last bits, may be
+  // formed in another order in a batch than in a call of its own)
   if (sizes && bh * (((int64_t)a.Sq + 127) / 128) < (dqk + dv <= 128 ? 768 : 512)) {
     consider(AttnCut::kStreams4x2, 4, 2, 6.5);
     if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 8.8);

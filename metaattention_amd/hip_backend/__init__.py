@@ -449,9 +449,11 @@ def mla_decode(q, q_pe, kv, k_pe, *, scale: float, num_split: int = 0, out=None,
 def get_mla_metadata(cache_seqlens, num_heads_per_head_k: int, num_heads_k: int, num_sm_parts: int = 0):
     """get_mla_metadata of the paged MLA interface (cute_template_kvshared/flash_mla_interface.py:57-72): the work plan
     for a ragged batch, computed on the device from cache_seqlens (int32 [B]) by the greedy scheme of
-    kernels/get_mla_metadata.cu:8-75.  Returns (tile_scheduler_metadata int32 [num_sm_parts, 8], num_splits int32 [B + 1]);
-    flash_mla_with_kvcache hands every workgroup the run of (batch entry, token range) pieces its part names.
-    num_sm_parts defaults to one part per CU and block of 128 query heads."""
+    kernels/get_mla_metadata.cu:8-75.  Returns (tile_scheduler_metadata int32 [num_sm_parts, 8], num_splits int32 [B + 1]).
+    To flash_mla_with_kvcache a plan says that the lengths differ: its workgroups then take equal runs of pieces that they
+    work out from cache_seqlens themselves, and of the plan read only which entries num_splits leaves in one piece
+    (their partial results are fp32).  num_sm_parts, one part per CU and block of 128 query heads by default, sizes the plan
+    and nothing else."""
     _require_gpu(cache_seqlens)
     assert num_heads_k == 1, "one latent kv head"
     lib = load_library()
@@ -498,7 +500,7 @@ def flash_mla_with_kvcache(q, k_cache, block_table, cache_seqlens, head_dim_v: i
     p.kv_seqlens = seqlens.data_ptr()
     p.block_table, p.block_table_stride, p.page_size = block_table.data_ptr(), block_table.stride(0), page
     if tile_scheduler_metadata is not None and tile_scheduler_metadata.dim() == 2 and tile_scheduler_metadata.shape[1] == 8:
-        # the plan of get_mla_metadata: every workgroup walks a run of pieces
+        # the plan of get_mla_metadata: the launch for ragged batches
         assert num_splits is not None and num_splits.shape == (B + 1,), "num_splits of get_mla_metadata goes with its metadata"
         assert tile_scheduler_metadata.dtype == torch.int32 and num_splits.dtype == torch.int32
         assert tile_scheduler_metadata.is_contiguous() and num_splits.is_contiguous()
