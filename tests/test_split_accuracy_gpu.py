@@ -42,19 +42,14 @@ def test_latent_cache_batch(B, Hq, KV):
     assert _error(cut, ref) <= ROOM * _error(whole, ref)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("Hq,lens", [(16, [300]), (32, [20 + 20 * i for i in range(16)]), (64, [300 - 4 * i for i in range(64)]), (128, [150] * 40), (40, [320, 1, 0, 200, 33])])
-def test_latent_cache_entries_that_the_plan_leaves_whole(dtype, Hq, lens):
-    """With a workspace as asked for (fp32 partial results), and with one that holds the plan's own parts (no cuts, or fewer parts)."""
-    import ctypes
+def _paged(dtype, Hq, lens):
+    """A paged batch through the C ABI: (parameters, tensors to keep, output in 64 bits, the plan)."""
     from metaattention_amd import hip_backend as hb
     B, page = len(lens), 64
     per_seq = -(-max(lens) // page)
     q, pool = _rand(B, 1, Hq, 576, dtype=dtype), _rand(B * per_seq, page, 1, 576, dtype=dtype)
     table = torch.randperm(B * per_seq, generator=torch.Generator().manual_seed(B)).to(torch.int32).cuda().view(B, per_seq)
     seqlens = torch.tensor(lens, dtype=torch.int32, device="cuda")
-    meta, splits = hb.get_mla_metadata(seqlens, Hq, 1)
-    assert int((splits[1:] - splits[:-1]).max()) == 1
     ref = torch.zeros(B, Hq, 512, dtype=torch.float64, device="cuda")
     for b, n in enumerate(lens):
         kv = pool[table[b].long()].reshape(-1, 576)[:n].double()
@@ -67,25 +62,61 @@ def test_latent_cache_entries_that_the_plan_leaves_whole(dtype, Hq, lens):
     p.kv, p.kv_stride_s, p.k_pe, p.kpe_stride_s = pool.data_ptr(), 576, pool.data_ptr() + 1024, 576
     p.scale, p.kv_seqlens, p.block_table, p.block_table_stride, p.page_size = 576 ** -0.5, seqlens.data_ptr(), table.data_ptr(), per_seq, page
     p.o_stride_b, p.o_stride_h = Hq * 512, 512
+    return p, (q, pool, table, seqlens), ref, hb.get_mla_metadata(seqlens, Hq, 1)
+
+
+def _run(p, dtype, plan, parts, size):
+    """plan None: unsplit.  size: bytes of workspace (None: what is asked for, "array": the built-in one)."""
+    import ctypes
+    from metaattention_amd import hip_backend as hb
     lib = hb.load_library()
-
-    def run(plan, parts, size):
-        out, lse = torch.full((B, Hq, 512), float("nan"), dtype=dtype, device="cuda"), torch.full((B, Hq), float("nan"), device="cuda")
-        p.o, p.lse, p.num_split = out.data_ptr(), lse.data_ptr(), 0 if plan else 1
-        p.tile_scheduler_metadata, p.num_splits, p.num_sm_parts = (meta.data_ptr(), splits.data_ptr(), parts) if plan else (None, None, 0)
-        size = lib.ma_mla_workspace_bytes(ctypes.byref(p)) if size is None else size
-        ws = torch.full((size + 256,), 255, dtype=torch.uint8, device="cuda")      # (all NaN; what lies behind the workspace stays as it is)
-        p.workspace, p.workspace_bytes = ws.data_ptr(), size
-        hb._check(lib.ma_mla_decode(ctypes.byref(p), None))
+    out, lse = torch.full((p.batch, p.heads_q, 512), float("nan"), dtype=dtype, device="cuda"), torch.full((p.batch, p.heads_q), float("nan"), device="cuda")
+    p.o, p.lse, p.num_split = out.data_ptr(), lse.data_ptr(), 0 if plan else 1
+    p.tile_scheduler_metadata, p.num_splits, p.num_sm_parts = (plan[0].data_ptr(), plan[1].data_ptr(), parts) if plan else (None, None, 0)
+    if size == "array":
+        hb._check(lib.ma_mla_decode_noalloc(ctypes.byref(p), None))
         torch.cuda.synchronize()
-        assert (ws[size:] == 255).all()
         return out, lse
+    size = lib.ma_mla_workspace_bytes(ctypes.byref(p)) if size is None else size
+    ws = torch.full((size + 256,), 255, dtype=torch.uint8, device="cuda")      # (all NaN; what lies behind the workspace stays as it is)
+    p.workspace, p.workspace_bytes = ws.data_ptr(), size
+    hb._check(lib.ma_mla_decode(ctypes.byref(p), None))
+    torch.cuda.synchronize()
+    assert (ws[size:] == 255).all()
+    return out, lse
 
-    one, lse_one = run(False, 0, 0)
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,lens", [(16, [300]), (32, [20 + 20 * i for i in range(16)]), (64, [300 - 4 * i for i in range(64)]), (128, [150] * 40), (40, [320, 1, 0, 200, 33])])
+def test_latent_cache_entries_that_the_plan_leaves_whole(dtype, Hq, lens):
+    """With a workspace as asked for (fp32 partial results), and with ones that hold the plan's own parts (no cuts, or fewer parts)."""
+    B = len(lens)
+    p, keep, ref, plan = _paged(dtype, Hq, lens)
+    parts, splits = plan[0].shape[0], plan[1]
+    assert int((splits[1:] - splits[:-1]).max()) == 1
+    one, lse_one = _run(p, dtype, None, 0, 0)
     slot = Hq * (2 * 512 + 4)
-    for parts, size in ((meta.shape[0], None), (meta.shape[0], (B + meta.shape[0]) * slot), (7, (B + 7) * slot), (1, (B + 1) * slot)):
-        out, lse = run(True, parts, size)
-        assert _error(out, ref) <= ROOM * _error(one, ref), (parts, size)
+    for n, size in ((parts, None), (parts, (B + parts) * slot), (7, (B + 7) * slot), (1, (B + 1) * slot), (parts, "array")):
+        out, lse = _run(p, dtype, plan, n, size)
+        assert _error(out, ref) <= ROOM * _error(one, ref), (n, size)
         torch.testing.assert_close(lse, lse_one, rtol=1e-5, atol=1e-5)
         empty = [b for b, n in enumerate(lens) if n == 0]
         assert torch.count_nonzero(out[empty]) == 0 and (lse[empty] == float("-inf")).all()
+
+
+@pytest.mark.parametrize("Hq,lens", [(128, [64 + 250 * i for i in range(16)]), (32, [3000, 5, 0, 700, 64, 2049, 130, 31] * 3), (64, [4000] + [90] * 50), (200, [1500, 100, 900, 320])])
+def test_latent_cache_plan_of_mixed_lengths(Hq, lens):
+    """Entries that the plan cuts beside entries that it leaves whole, in every kind of workspace: the former may round their partial
+    results (at most the square root of two of the unsplit error), the latter not."""
+    dtype, B = torch.bfloat16, len(lens)
+    p, keep, ref, plan = _paged(dtype, Hq, lens)
+    parts, pieces = plan[0].shape[0], plan[1][1:] - plan[1][:-1]
+    whole = (pieces == 1).cpu() & torch.tensor([n > 0 for n in lens])
+    assert whole.any() and (pieces > 1).any()
+    one, lse_one = _run(p, dtype, None, 0, 0)
+    slot = Hq * (2 * 512 + 4)
+    for n, size in ((parts, None), (parts, (B + parts) * slot), (16, (B + 16) * slot), (min(parts, 256), "array")):
+        out, lse = _run(p, dtype, plan, n, size)
+        assert _error(out[whole], ref[whole]) <= ROOM * _error(one[whole], ref[whole]), (n, size)
+        assert _error(out, ref) <= 2 ** 0.5 * ROOM * _error(one, ref), (n, size)
+        torch.testing.assert_close(lse, lse_one, rtol=1e-5, atol=1e-5)
