@@ -125,6 +125,21 @@ __device__ __forceinline__ void dma16_so(const void* base_uniform, uint32_t lane
       : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(lane_off), "s"(sb)
       : "memory");
 }
+// Same for the lanes of a wave-uniform mask; the whole wave must be active.
+__device__ __forceinline__ void dma16_masked(const void* base_uniform, uint32_t lane_off, uint32_t lds_base, uint64_t lanes) {
+  const uint64_t b = (uint64_t)(uintptr_t)base_uniform;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  const uint32_t mlo = __builtin_amdgcn_readfirstlane((uint32_t)lanes), mhi = __builtin_amdgcn_readfirstlane((uint32_t)(lanes >> 32));
+  const uint64_t sb = ((uint64_t)hi << 32) | lo, mask = ((uint64_t)mhi << 32) | mlo;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_mov_b64 exec, %3\n\t"
+      "global_load_lds_dwordx4 %1, %2\n\t"
+      "s_mov_b64 exec, -1\n\t"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(lane_off), "s"(sb), "s"(mask)
+      : "memory");
+}
 __device__ __forceinline__ void dma4_so(const void* base_uniform, uint32_t lane_off, uint32_t lds_base) {
   const uint64_t b = (uint64_t)(uintptr_t)base_uniform;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));

@@ -20,7 +20,7 @@ struct LinArgs {
   // Hv = heads of v (dividing H: head h reads v head h / (H / Hv)).
   int rev, Hv;
   int64_t q_row, k_row, v_row;
-  // qk_cols (general addressing only; 0: all Dk): the q and k operands hold only this many columns (a multiple of 8); the
+  // qk_cols (general addressing only; 0: all Dk): the q and k operands hold only this many columns (a multiple of 32); the
   // rest of the Dk-wide contraction is zeros that are never loaded (the tiles' LDS is cleared once, the loads of the missing
   // columns are switched off).
   int qk_cols;

@@ -15,14 +15,20 @@
 // sequence is walked in chunks of 32 tokens; per chunk and wave, with
 // g = chunk-local cumsum of the log decay, everything is computed TRANSPOSED so
 // each lane owns one token column:
-//   A^T = K Q^T                      [32 x 32]   (every wave, redundantly: it is the B operand below)
+//   A^T = K Q^T                      [32 x 32]
 //   P^T = A^T * q_scale * exp(g_i - g_j) * vs_j * [j <= i]
 //   O^T = h^T (Q^T) * exp(g_i) q_scale + V^T P^T          [32 dv x 32 tokens]
 //   h   = exp(g_last) h + K^T (V * vs * exp(g_last - g))  [DK x 32 dv]
 // The state accumulator of K^T V (lane = value column, rows = key dims) is,
 // register for register, the A operand of h^T Q^T, so the state never moves.
-// Q/K/V chunk tiles arrive by direct-to-LDS DMA, double buffered, with a single
-// workgroup barrier per chunk.
+// Q/K/V chunk tiles arrive by direct-to-LDS DMA with a single workgroup barrier per chunk.
+//
+// Where a workgroup has four waves or more and produces outputs the chunk loop is pipelined (see PIPE): P^T, which is the
+// same for every wave of a head, is made once, by three waves and a chunk ahead, the chunk's scalars two chunks ahead by a
+// fourth, tiles arrive two or three chunks ahead.  Vector issue bounds this loop (61 % of the cycles of a chunk at 256 / 512
+// with P^T formed by every wave, the matrix pipe 23 %), so what pays is fewer vector instructions per wave: 650 -> 450 a chunk.
+// 8 x 16 heads, 2048 tokens, 256 / 512: 290 -> 222 us a pass.  At that rate the clock gives way (2.1 -> 1.65 GHz with random
+// operands): 9500 -> 6000 clocks a chunk.
 //
 // Heads that share their q and k head (Mamba2: one B/C group for all heads) can be
 // grouped HG to a workgroup, which then shares the Q/K tiles in LDS.
@@ -44,6 +50,11 @@ namespace ma {
 
 namespace {
 constexpr int L = 32;  // tokens per chunk
+// What the waves of a head share in the pipelined loop.  P^T of two chunks, as the B operand of V^T P^T: slice 0 64 lanes x 16 bytes,
+// slice 1 its 32 lanes of tokens 16..31.  Scalars of three chunks: running log2 decay and value scale x q_scale of the tokens, factors
+// of the state update's rows and of the tokens' inter-chunk term, decay of the chunk.
+constexpr int kPipeP1 = 1024, kPipeP = 1536, kScalG = 0, kScalV = 4 * L, kScalW = 8 * L, kScalE = 12 * L, kScalD = 16 * L, kPipeScal = kScalD + 16;
+constexpr int pipe_shared(int heads) { return heads * (2 * kPipeP + 3 * kPipeScal) + 16; }     // (the last 16 bytes: zeros)
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {
@@ -62,20 +73,37 @@ __device__ __forceinline__ X8 scale_bf16x8(X8 v, const float (&w)[8]) {
 }
 }  // namespace
 
-// minimum waves per SIMD asked of the register allocator: 8 waves of one workgroup need 2; the
-// two-heads-per-workgroup configuration is meant to run three workgroups of 4 waves per CU
-template <int DK, int NWH, int HG>
-constexpr int min_waves_per_simd() { return HG > 1 ? 3 : (NWH == 4 && DK > 128 ? 1 : 2); }
+// The pipelined chunk loop (P^T shared by the waves of a head and made one chunk ahead): workgroups of four waves or more that
+// produce outputs.
+template <int NWH, int HG, int MODE>
+constexpr bool pipelined() { return NWH * HG >= 4 && MODE != 1; }
+// ... and where a workgroup has four state waves of at most 128 key dims by four waves of their own (`helpers`), one beside each state
+// wave of a SIMD, which write the outputs too.  A chunk of a state wave alone takes 1900 clocks, that of its helper 2300; without them
+// P^T, scalars and outputs stand in the state waves' chain (4700 clocks) and only further workgroups on the CU, with sequence
+// segments to supply them, hide it.  8 x 64 heads sharing q and k, 2048 tokens, 128 / 64: three workgroups a CU in three segments
+// 127 us, one with helpers in a single pass 87 us; 8 x 16 heads, 128 / 128, forward and backward 386 -> 363 us.
+template <int DK, int NWH, int HG, int MODE>
+constexpr int helpers() { return pipelined<NWH, HG, MODE>() && NWH * HG == 4 && DK <= 128 ? 4 : 0; }
+// waves of a workgroup
+template <int DK, int NWH, int HG, int MODE>
+constexpr int workgroup_waves() { return NWH * HG + helpers<DK, NWH, HG, MODE>(); }
+// minimum waves per SIMD asked of the register allocator: the eight waves of a workgroup need two
+template <int DK, int NWH, int HG, int MODE>
+constexpr int min_waves_per_simd() { return HG > 1 && MODE == 1 ? 3 : NWH == 4 && DK > 128 ? 1 : 2; }
 
 // GEN: the operands' general addressing (reversed time, row strides, v head broadcast) of LinArgs; without it the
 // addressing is the plain one, with compile-time row sizes.
 // GEN 1: one scan, 2: the scans of a LinScans, one blockIdx.y each (with the arguments behind an index the single scan takes 1 %
 // longer: B8 H16 T2048 256 / 512 forward + backward 1516, 1530 us).
 template <int DK, int NWH, int HG, int MODE, int GEN = 0>
-__global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>())) void linear_fwd_kernel(const std::conditional_t<GEN == 2, LinScans, LinArgs> all) {
+__global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_waves_per_simd<DK, NWH, HG, MODE>())) void linear_fwd_kernel(const std::conditional_t<GEN == 2, LinScans, LinArgs> all) {
   const LinArgs& a = one_scan(all, GEN == 2 ? (int)blockIdx.y : 0);
   constexpr int NW = NWH * HG;
-  constexpr bool ALIAS_OST = HG > 1;     // output staging block inside the wave's own (already consumed) V columns
+  constexpr bool PIPE = pipelined<NWH, HG, MODE>();
+  constexpr bool HELP = helpers<DK, NWH, HG, MODE>() > 0;
+  constexpr int NT = 64 * workgroup_waves<DK, NWH, HG, MODE>();
+  static_assert(!HELP || NWH * HG == 4, "helper w serves state wave w");
+  constexpr bool ALIAS_OST = HG > 1 || PIPE;     // output staging block inside the wave's own (already consumed) V columns
   using T = __bf16;
   using E = Elem<T>;
   using x8 = typename E::x8;
@@ -90,22 +118,16 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
   constexpr int SCAL_BYTES = 3 * L * 4;            // per-wave g / pv*q_scale / w
   constexpr int NIQ = QT / 1024, NIV = VT / 1024;  // DMA instructions per tile
   static_assert(CPRQ >= 16, "DK < 128 needs its own Q/K swizzle");
-  // Every wave of the workgroup needs the same 32 x 32 tile A^T = K Q^T.  With four or more waves it is computed
-  // once: in 16 x 16 quadrants (v_mfma_f32_16x16x32; the quadrant of keys 16..31 x queries 0..15 lies above the
-  // diagonal and is left out), each over 1 / KP of the key dims, one (quadrant, part) per wave, exchanged
-  // through LDS.  16 MFMAs of 32x32x16 and 2 x DK / 16 KB of operand reads per wave become at most 4 half-size
-  // MFMAs plus a 1 KB write and 4 KP KB of reads, for one more barrier per chunk.
-  constexpr bool SHARE_A = NW >= 4 && MODE != 1;
-  constexpr int KP = NW >= 8 ? 2 : 1;               // parts of the key dims per quadrant
-  constexpr int A_ITEMS = 3 * KP;
-
   extern __shared__ __align__(16) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool helper = HELP && wave_id >= NW;
+  const int wave = helper ? wave_id - NW : wave_id;       // (a helper's: the state wave whose outputs it writes)
   const int r0 = lane & 31;
-  const uint32_t lds_scal = lds0 + 2 * STAGE + wave * SCAL_BYTES;
-  const uint32_t lds_ost = lds0 + 2 * STAGE + NW * SCAL_BYTES + wave * (L * OROW);   // (unused with ALIAS_OST)
-  const uint32_t lds_apart = lds0 + 2 * STAGE + NW * SCAL_BYTES + (ALIAS_OST ? 0 : NW * (L * OROW));   // A^T quadrants, 1 KB each
+  constexpr int NST = HELP ? 4 : PIPE ? 3 : 2;             // stages of chunk tiles
+  const uint32_t lds_scal = lds0 + NST * STAGE + wave * SCAL_BYTES;                                     // (unused with PIPE)
+  const uint32_t lds_ost = lds0 + NST * STAGE + NW * SCAL_BYTES + wave * (L * OROW);   // (unused with ALIAS_OST)
+  const uint32_t lds_p = lds0 + NST * STAGE, lds_scalars = lds_p + HG * 2 * kPipeP, lds_zero = lds_scalars + HG * 3 * kPipeScal;   // PIPE: [slot][head] (see kPipeP)
 
   // workgroup -> (head group, value slice, segment); the workgroups of one head group share
   // id % 8 (one XCD, shared L2)
@@ -169,13 +191,35 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
   // (columns beyond the operand's are zeros: the 16- and 32-wide slices of the contraction that hold nothing else are skipped)
   const int qk_used = GEN && a.qk_cols > 0 ? a.qk_cols : DK;
   if (GEN && qk_chunks < (uint32_t)CPRQ) {
-    // the Q and K tiles of both stages start as zeros: the missing columns are never written
-    for (uint32_t off = (uint32_t)tid * 16; off < (uint32_t)(2 * QT); off += 64 * NW * 16) {
-      lds_write<u32x4>(lds0 + off, u32x4{0u, 0u, 0u, 0u});
-      lds_write<u32x4>(lds0 + STAGE + off, u32x4{0u, 0u, 0u, 0u});
-    }
+    // the Q and K tiles of all stages start as zeros: the missing columns are never written
+    for (uint32_t off = (uint32_t)tid * 16; off < (uint32_t)(2 * QT); off += NT * 16)
+#pragma unroll
+      for (int st = 0; st < NST; st++) lds_write<u32x4>(lds0 + st * STAGE + off, u32x4{0u, 0u, 0u, 0u});
     __syncthreads();
   }
+  // a partial chunk: rows beyond the sequence are clamped to its last row
+  auto issue_rows = [&](int t0, uint32_t base) {
+    constexpr int NQK = MODE == 1 ? NIQ : 2 * NIQ;      // (the state-only pass needs no Q)
+#pragma unroll 1
+    for (int ii = wave; ii < NQK + NIV; ii += NW) {
+      if (ii < NQK) {
+        const int which = MODE == 1 ? 1 : ii >= NIQ, i2 = (MODE != 1 && which) ? ii - NIQ : ii;
+        const int row = i2 * (1024 / RBQ) + lane / CPRQ, c = lane % CPRQ;
+        const int tpos = min(t0 + row, Tn - 1), trow = rev ? Tn - 1 - tpos : tpos;
+        const uint32_t lc = (uint32_t)(c ^ swz_tile<CPRQ>(row));
+        const char* src = (which ? kb + (int64_t)trow * k_rb : qb + (int64_t)trow * q_rb) + (lc << 4);
+        if (!GEN || lc < qk_chunks) dma16(src, base + which * QT + i2 * 1024);
+      } else {
+        const int i2 = ii - NQK;
+        const int row = i2 * (1024 / RBV) + lane / CPRV, c = lane % CPRV;
+        const int tpos = min(t0 + row, Tn - 1), trow = rev ? Tn - 1 - tpos : tpos;
+        const int lc = c ^ swz_tile<CPRV>(row);          // logical 16-byte chunk: head lc / (4 NWH), then its columns
+        const char* src = vb + (int64_t)trow * v_row_bytes + ((lc % (4 * NWH)) << 4);
+        if (HG > 1) src += (lc / (4 * NWH)) * v_head_bytes;
+        dma16(src, base + 2 * QT + i2 * 1024);
+      }
+    }
+  };
   auto issue_chunk = [&](int t0, int buf) {
     const uint32_t base = lds0 + buf * STAGE;
     constexpr int NQK = MODE == 1 ? NIQ : 2 * NIQ;      // (the state-only pass needs no Q)
@@ -223,28 +267,7 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
       }
       return;
     }
-    // last, partial chunk: rows beyond the sequence are clamped to its last row
-#pragma unroll 1
-    for (int it = 0; it < (NQK + NIV + NW - 1) / NW; it++) {
-      const int ii = wave + NW * it;
-      if ((NQK + NIV) % NW != 0 && ii >= NQK + NIV) break;
-      if (ii < NQK) {
-        const int which = MODE == 1 ? 1 : ii >= NIQ, i2 = (MODE != 1 && which) ? ii - NIQ : ii;
-        const int row = i2 * RQ + lane / CPRQ, c = lane % CPRQ;
-        const int tpos = min(t0 + row, Tn - 1), trow = rev ? Tn - 1 - tpos : tpos;
-        const uint32_t lc = (uint32_t)(c ^ swz_tile<CPRQ>(row));
-        const char* src = (which ? kb + (int64_t)trow * k_rb : qb + (int64_t)trow * q_rb) + (lc << 4);
-        if (!GEN || lc < qk_chunks) dma16(src, base + which * QT + i2 * 1024);
-      } else {
-        const int i2 = ii - NQK;
-        const int row = i2 * RV + lane / CPRV, c = lane % CPRV;
-        const int tpos = min(t0 + row, Tn - 1), trow = rev ? Tn - 1 - tpos : tpos;
-        const int lc = c ^ swz_tile<CPRV>(row);          // logical 16-byte chunk: head lc / (4 NWH), then its columns
-        const char* src = vb + (int64_t)trow * v_row_bytes + ((lc % (4 * NWH)) << 4);
-        if (HG > 1) src += (lc / (4 * NWH)) * v_head_bytes;
-        dma16(src, base + 2 * QT + i2 * 1024);
-      }
-    }
+    issue_rows(t0, base);
   };
 
   f32x16 hst[KB];
@@ -256,20 +279,24 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
   // scalars of the chunk about to be processed (loaded one chunk ahead)
   const int ti = r0;
   float ld_next = 0.f, vs_next = 1.f;
-  if (c_begin * L + ti < Tn) {
+  if (!PIPE && c_begin * L + ti < Tn) {
     ld_next = ldp[c_begin * L + ti];
     if (vsp) vs_next = vsp[c_begin * L + ti];
   }
-  if (c_begin < c_end) issue_chunk(c_begin * L, 0);
+  if (!helper) {
+    if (c_begin < c_end) issue_chunk(c_begin * L, 0);
+    if (PIPE && c_begin + 1 < c_end) issue_chunk((c_begin + 1) * L, 1);
+    if (HELP && c_begin + 2 < c_end) issue_chunk((c_begin + 2) * L, 2);
+  }
 
-  if (MODE == 2 && seg > 0 && a.ws_entering) {
+  if (MODE == 2 && !helper && seg > 0 && a.ws_entering) {
     // entering state, formed by linear_states_kernel
     const float* src = ws_mine + (seg - 1) * WS_SEG;
 #pragma unroll
     for (int i = 0; i < KB; i++)
 #pragma unroll
       for (int j = 0; j < 16; j++) hst[i][j] = src[(i * 16 + j) * 64];
-  } else if (MODE == 2 && seg > 0) {
+  } else if (MODE == 2 && !helper && seg > 0) {
     // entering state: the local end states of the earlier segments, each decayed by the segments between
     const float* dec = a.ws_decay + (int64_t)(bh - a.bg0 * HG) * (a.nseg - 1);
     float acc_log = 0.f;
@@ -297,6 +324,401 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
   }
   float seg_log = 0.f;   // MODE 1: total log decay of the segment
 
+  auto write_out = [&](const f32x16& o, int t0, uint32_t vbase) {
+    // ---- write this wave's [32 tokens x 32 columns] block: stage (wave private), then 16-byte row pieces.
+    //      With ALIAS_OST the staging block is the wave's own 4 chunks per row of the V tile just consumed
+    //      (only this wave reads them, and the next DMA into this buffer is issued behind the next barrier).
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int r = ln & 31, g = ln >> 5;
+    if (MODE != 1 && a.out_f32) {
+      // fp32 outputs (used by the backward pass, whose decay gradient is a difference of sums over these
+      // values): the same staging block, 16 columns at a time
+      const int sw_r = swz_tile<CPRV>(r);
+      float* ob32 = (float*)a.o + (int64_t)piece * a.piece_o + (int64_t)bh * Tn * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH);
+#pragma unroll
+      for (int half = 0; half < 2; half++) {
+#pragma unroll
+        for (int q2 = 0; q2 < 2; q2++) {
+          const int q4 = 2 * half + q2;
+          f32x4 w;
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            w[i] = o[4 * q4 + i];
+          if (ALIAS_OST) lds_write<f32x4>(vbase + r * RBV + (uint32_t)(((4 * wave + 2 * q2 + g) ^ sw_r) << 4), w);
+          else lds_write<f32x4>(lds_ost + r * OROW + (8 * q2 + 4 * g) * 4, w);
+        }
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+          const int ci = ln + 64 * it, row = ci >> 2, cc = ci & 3;
+          const u32x4 w = ALIAS_OST ? lds_read<u32x4>(vbase + row * RBV + (uint32_t)(((4 * wave + cc) ^ swz_tile<CPRV>(row)) << 4))
+                                    : lds_read<u32x4>(lds_ost + row * OROW + cc * 16);
+          if (t0 + row < Tn) {
+            f32x4* dst = (f32x4*)(ob32 + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + 16 * half + cc * 4);
+            f32x4 val = __builtin_bit_cast(f32x4, w);
+            if (a.out_f32 == 2) val += *dst;   // (a contraction cut into pieces: the pieces' outputs add up)
+            *dst = val;
+          }
+        }
+      }
+    } else if constexpr (MODE != 1) {
+      const int sw_r = swz_tile<CPRV>(r);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          w[i] = (T)o[4 * q4 + i];
+        if (ALIAS_OST) lds_write<x4>((vbase + r * RBV + (uint32_t)(((4 * wave) ^ sw_r) << 4) + g * 8) ^ (uint32_t)(q4 << 4), w);
+        else lds_write<x4>(lds_ost + r * OROW + (8 * q4 + 4 * g) * 2, w);
+      }
+      // (rows 16 apart share their swizzle)
+      const uint32_t ra = vbase + (ln >> 2) * RBV + (uint32_t)(((4 * wave + (ln & 3)) ^ swz_tile<CPRV>(ln >> 2)) << 4);
+#pragma unroll
+      for (int it = 0; it < 2; it++) {
+        const int ci = ln + 64 * it, row = ci >> 2, cc = ci & 3;
+        const u32x4 w = ALIAS_OST ? lds_read<u32x4>(ra + 16 * it * RBV) : lds_read<u32x4>(lds_ost + row * OROW + cc * 16);
+        if (t0 + row < Tn) *(u32x4*)(ob + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + cc * 8) = w;
+      }
+    }
+  };
+  if constexpr (PIPE) {
+    constexpr int RQ = 1024 / RBQ, RV = 1024 / RBV, NLQ = NIQ / NW, NLV = NIV / NW, NL = 2 * NLQ + NLV;
+    static_assert(NIQ % NW == 0 && NIV % NW == 0, "every wave moves the same number of instructions");
+    constexpr int JOBS = 4;        // waves 0..2: a quadrant of P^T each, wave 3: scalars
+    auto scalars_of = [&](int cn) { return lds_scalars + (uint32_t)((cn - c_begin) % 3) * (HG * kPipeScal); };
+
+    // ---- Scalars of chunk cn, lane: token lane % 32, head lane / 32 of the group (one head: both halves alike).  ld, vs: its log
+    //      decay and value scale.  Inclusive scan over the tokens (DPP: shifts within rows of 16 lanes, then lane 15 of rows 0
+    //      and 2 carried into rows 1 and 3), in the log2 domain.
+    const int64_t lane_head = (int64_t)(bh0 + (HG > 1 ? lane >> 5 : 0)) * Tn;
+    auto load_scalars = [&](int cn, float& ld, float& vs) {
+      const int t = cn * L + r0;
+      ld = 0.f;
+      vs = 1.f;
+      if (cn < c_end && t < Tn) {
+        ld = a.log_decay[lane_head + t];
+        if (a.v_scale) vs = a.v_scale[lane_head + t];
+      }
+    };
+    auto publish = [&](int cn, float ld, float vs) {
+      const bool valid = cn * L + r0 < Tn;
+      float x = valid ? ld : 0.f;
+      x += dpp_f32<0x111>(x);   // row_shr:1, lanes shifted in from outside the row read 0
+      x += dpp_f32<0x112>(x);
+      x += dpp_f32<0x114>(x);
+      x += dpp_f32<0x118>(x);
+      x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x142, 0xa, 0xf, false));   // row_bcast:15
+      const float gi2 = x * kLog2e;
+      const float last0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gi2), 31));
+      const float last1 = HG > 1 ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gi2), 63)) : last0;
+      const float g_last2 = HG > 1 && lane >= 32 ? last1 : last0;
+      if (HG > 1 || lane < 32) {
+        const uint32_t at = scalars_of(cn) + (HG > 1 ? (uint32_t)(lane >> 5) * kPipeScal : 0u) + (uint32_t)r0 * 4;
+        lds_write<float>(at + kScalG, gi2);
+        lds_write<float>(at + kScalV, valid ? vs * a.q_scale : 0.f);
+        lds_write<float>(at + kScalW, valid ? vs * fast_exp2(g_last2 - gi2) : 0.f);
+        lds_write<float>(at + kScalE, fast_exp2(gi2) * a.q_scale);
+        if (r0 == 0) lds_write<float>(at + kScalD, fast_exp2(g_last2));
+      }
+    };
+
+    // ---- A 16 x 16 quadrant of
+    //        P^T = (K Q^T) * q_scale * exp(g_i - g_j) * vs_j * [j <= i]
+    //      of chunk cn (wave 0: keys 0..15 x queries 0..15, 1: keys 0..15 x queries 16..31, 2: keys 16..31 x queries 16..31; the
+    //      fourth lies above the diagonal), for every head of the group, straight into the B operand layout of V^T P^T.  A / B
+    //      operand of the 16 x 16 MFMA: lane holds row (column) lane % 16, k = 8 (lane / 16) .. +7 of a 32-wide slice; C: lane holds
+    //      column lane % 16, rows 4 (lane / 16) + {0..3}.
+    //      Every wave of a head used to take A^T and form all of P^T for itself: 200 of its 650 vector instructions a
+    //      chunk, in a loop that vector issue bounds.
+    auto make_p = [&](int cn, int stage) {
+      int la = lane;
+      asm volatile("" : "+v"(la));
+      const int kq = wave >> 1, qq = wave > 0;        // key and query half of the quadrant
+      const int rr = la & 15, kg = la >> 4;
+      const uint32_t qbase = lds0 + stage * STAGE, kbase = qbase + QT;
+      // (tile bases and row offsets are multiples of the row size, so the swizzled chunk index occupies its own
+      // address bits: one XOR with a constant per read moves to another slice)
+      const uint32_t c0 = (uint32_t)((kg ^ swz16(rr)) << 4);
+      const uint32_t ka = kbase + (16 * kq + rr) * RBQ + c0, qa = qbase + (16 * qq + rr) * RBQ + c0;
+      f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      // (operands are requested three slices ahead: read as they are needed they cost an LDS latency each)
+      constexpr int NS = DK / 32, AH = 3;
+      x8 kf[AH + 1], qf[AH + 1];
+      auto request = [&](int s2) {
+        kf[s2 % (AH + 1)] = lds_read<x8>(ka ^ (uint32_t)(s2 * 64));
+        qf[s2 % (AH + 1)] = lds_read<x8>(qa ^ (uint32_t)(s2 * 64));
+      };
+#pragma unroll
+      for (int s2 = 0; s2 < AH; s2++) request(s2);
+      const uint32_t sc = scalars_of(cn);
+      float gq[HG];
+      f32x4 gk[HG], pk[HG];
+#pragma unroll
+      for (int h = 0; h < HG; h++) {
+        gq[h] = lds_read<float>(sc + h * kPipeScal + kScalG + (uint32_t)(16 * qq + rr) * 4);
+        gk[h] = lds_read<f32x4>(sc + h * kPipeScal + kScalG + (uint32_t)(16 * kq + 4 * kg) * 4);
+        pk[h] = lds_read<f32x4>(sc + h * kPipeScal + kScalV + (uint32_t)(16 * kq + 4 * kg) * 4);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s2 = 0; s2 < NS; s2++) {
+        if (GEN && s2 * 32 >= qk_used) break;
+        if (s2 + AH < NS) request(s2 + AH);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[s2 & 1] = E::mfma16(kf[s2 % (AH + 1)], qf[s2 % (AH + 1)], acc[s2 & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const bool low[4] = {wave == 1 || 4 * kg <= rr, wave == 1 || 4 * kg + 1 <= rr, wave == 1 || 4 * kg + 2 <= rr, wave == 1 || 4 * kg + 3 <= rr};
+#pragma unroll
+      for (int h = 0; h < HG; h++) {
+        float p[4];
+        x4 w;
+        // (above the diagonal the exponent is positive and the product may be inf or NaN: the select drops it)
+#pragma unroll
+        for (int t = 0; t < 4; t++) p[t] = (acc[0][t] + acc[1][t]) * fast_exp2(gq[h] - gk[h][t]) * pk[h][t];
+        asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));   // computed for every lane, then selected: no branch per element
+#pragma unroll
+        for (int t = 0; t < 4; t++) w[t] = (T)(low[t] ? p[t] : 0.f);
+        // keys 16 kq + 4 kg + {0..3} of token i: slice kq, lane half kg % 2, elements 4 (kg / 2) ..
+        const uint32_t at = lds_p + (uint32_t)(((cn - c_begin) & 1) * HG + h) * kPipeP + (uint32_t)(kg >> 1) * 8 +
+                            (kq ? kPipeP1 + (uint32_t)(rr + 16 * (kg & 1)) * 16 : (uint32_t)(16 * qq + rr + 32 * (kg & 1)) * 16);
+        lds_write<x4>(at, w);
+      }
+    };
+    // what waves 0..3 (or the helpers) prepare while chunk c is under way: P^T of c + 1, scalars of c + 2
+    auto prepare = [&](int c, int buf, float ld, float vs) {
+      if (wave < 3) {
+        if (c + 1 < c_end) make_p(c + 1, buf == NST - 1 ? 0 : buf + 1);
+      } else if (c + 2 < c_end) {
+        publish(c + 2, ld, vs);
+      }
+    };
+
+    // ---- Loads of a chunk inside the loop: each wave moves instructions wave, wave + NW .. of each tile.  Bases are the tile's
+    //      first row (reversed time: its last, the lowest address) plus the instruction's rows, lane offsets do not change; what is
+    //      not to be loaded is switched off in the execution mask, without a branch.
+    const int ln_q = wave * RQ + lane / CPRQ, ln_v = wave * RV + lane / CPRV;        // the lane's row in instruction 0
+    const uint32_t lcq = (uint32_t)((lane % CPRQ) ^ swz_tile<CPRQ>(ln_q)), lcv = (uint32_t)((lane % CPRV) ^ swz_tile<CPRV>(ln_v));
+    const uint32_t row_q = (uint32_t)(rev ? L - 1 - ln_q : ln_q) * (uint32_t)q_rb, row_k = GEN ? (uint32_t)(rev ? L - 1 - ln_q : ln_q) * (uint32_t)k_rb : row_q;
+    const uint32_t row_v = (uint32_t)(rev ? L - 1 - ln_v : ln_v) * (uint32_t)v_row_bytes + (HG > 1 ? (lcv / (4 * NWH)) * (uint32_t)v_head_bytes : 0u);
+    const uint64_t qk_lanes = GEN ? (uint64_t)__ballot(lcq < qk_chunks) : ~(uint64_t)0;      // (qk_chunks is a multiple of 4: the same lanes in every load)
+    auto load_one = [&](int x, int t2, uint32_t base2, uint64_t on) {
+      const int64_t first = rev ? Tn - t2 - L : t2;
+      if (x < 2 * NLQ) {
+        const int j = x % NLQ;
+        const bool is_k = x >= NLQ;
+        const int64_t rows = first + (rev ? -1 : 1) * j * NW * RQ;
+        const uint32_t ch = (lcq ^ (uint32_t)swz_tile<CPRQ>(j * NW * RQ)) << 4;
+        dma16_masked(is_k ? kb + rows * k_rb : qb + rows * q_rb, (is_k ? row_k : row_q) + ch, base2 + (is_k ? QT : 0) + (wave + NW * j) * 1024, on & qk_lanes);
+      } else {
+        const int j = x - 2 * NLQ;
+        const int64_t rows = first + (rev ? -1 : 1) * j * NW * RV;
+        const uint32_t ch = ((lcv ^ (uint32_t)swz_tile<CPRV>(j * NW * RV)) % (4 * NWH)) << 4;
+        dma16_masked(vb + rows * v_row_bytes, row_v + ch, base2 + 2 * QT + (wave + NW * j) * 1024, on);
+      }
+    };
+
+    float ld_next = 0.f, vs_next = 1.f;      // of the next chunk to be published
+    const bool jobs = HELP ? helper : wave < JOBS;
+    if (tid == 0) lds_write<u32x4>(lds_zero, u32x4{0u, 0u, 0u, 0u});
+    if (jobs && wave == 3) {
+      load_scalars(c_begin, ld_next, vs_next);
+      publish(c_begin, ld_next, vs_next);
+      load_scalars(c_begin + 1, ld_next, vs_next);
+      publish(c_begin + 1, ld_next, vs_next);
+      load_scalars(c_begin + 2, ld_next, vs_next);
+    }
+    wait_dma();
+    __syncthreads();
+    if (jobs && wave < 3 && c_begin < c_end) make_p(c_begin, 0);
+    __syncthreads();
+
+    // HELP: [chunk parity][wave] blocks of 32 tokens x 32 columns fp32 on their way out, rows padded by 16 bytes
+    constexpr uint32_t OSTR = 128 + 16;
+    auto out_block = [&](int c) { return lds_zero + 16 + (uint32_t)(((c - c_begin) & 1) * NW + wave) * (L * OSTR); };
+    auto write_block = [&](int c) {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int t0 = c * L;
+      const uint32_t from = out_block(c);
+      if (a.out_f32) {
+        float* ob32 = (float*)a.o + (int64_t)piece * a.piece_o + (int64_t)bh * Tn * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH);
+#pragma unroll
+        for (int it = 0; it < 4; it++) {
+          const int row = 8 * it + (ln >> 3), cc = ln & 7;
+          f32x4 val = lds_read<f32x4>(from + row * OSTR + cc * 16);
+          if (t0 + row < Tn) {
+            f32x4* dst = (f32x4*)(ob32 + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + cc * 4);
+            if (a.out_f32 == 2) val += *dst;   // (a contraction cut into pieces: the pieces' outputs add up)
+            *dst = val;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+          const int row = 16 * it + (ln >> 2), cc = ln & 3;
+          const f32x4 lo = lds_read<f32x4>(from + row * OSTR + cc * 32), hi = lds_read<f32x4>(from + row * OSTR + cc * 32 + 16);
+          x8 w;
+#pragma unroll
+          for (int i = 0; i < 4; i++) { w[i] = (T)lo[i]; w[4 + i] = (T)hi[i]; }
+          if (t0 + row < Tn) *(x8*)(ob + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + cc * 8) = w;
+        }
+      }
+    };
+
+    f32x16 o_out;         // outputs of chunk c - 1, written while chunk c is under way: nobody waits for the stores
+    // a state wave's work of chunk c
+    auto run_chunk = [&](int c, int buf) {
+      const int t0 = c * L;
+      const uint32_t base = lds0 + buf * STAGE, qbase = base, kbase = base + QT, vbase = base + 2 * QT;
+      // the loads of this chunk: chunk c + NST - 1, into the stage that chunk c - 1 has left
+      const int t2 = t0 + (NST - 1) * L;
+      const uint32_t base2 = lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE;
+      const bool loads = c + NST - 1 < c_end, whole = t2 + L <= Tn && v_head_bytes < ((int64_t)1 << 31);
+      const uint64_t on = loads && whole ? ~(uint64_t)0 : 0;
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int r = ln & 31, g = ln >> 5;
+      const int jr = (ln & 15) >> 2, lc = (((ln >> 4) & 1) << 1) | ((ln & 3) >> 1);
+      constexpr int X8 = 2;          // swz(row + 8) ^ swz(row); rows 16 apart share their swizzle
+      // ---- V^T fragments (rows = this wave's 32 value columns; k-slot i of slice s is token
+      //      16s + 8(i/4) + 4g + i%4, the order P^T comes in)
+      x8 vf[2];
+      {
+        const uint32_t va = vbase + (4 * g + jr) * RBV + (ln & 1) * 8 + (uint32_t)(((4 * wave + lc) ^ swz_tile<CPRV>(4 * g + jr)) << 4);
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const x4 lo = lds_read_tr4<T>(va + 16 * s * RBV), hi = lds_read_tr4<T>((va ^ (uint32_t)(X8 << 4)) + (16 * s + 8) * RBV);
+          vf[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      }
+      const uint32_t ph = lds_p + (uint32_t)(((c - c_begin) & 1) * HG + hl) * kPipeP, sh = scalars_of(c) + hl * kPipeScal;
+      const x8 pf0 = lds_read<x8>(ph + ln * 16);
+      const x8 pf1 = lds_read<x8>(r >= 16 ? ph + kPipeP1 + (r - 16 + 16 * g) * 16 : lds_zero);
+      const float eg = lds_read<float>(sh + kScalE + r * 4);
+      float decay_all = lds_read<float>(sh + kScalD);
+      f32x4 w4[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) w4[i] = lds_read<f32x4>(sh + kScalW + 16 * g + 32 * i);
+      if (!HELP && c > c_begin) write_out(o_out, t0 - L, vbase);
+
+      const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      f32x16 o_intra = E::mfma32(vf[0], pf0, zero16);
+      o_intra = E::mfma32(vf[1], pf1, o_intra);
+      // value-scaled V^T for the state update
+      x8 vsf[2];
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const float w8[8] = {w4[2 * s][0], w4[2 * s][1], w4[2 * s][2], w4[2 * s][3], w4[2 * s + 1][0], w4[2 * s + 1][1], w4[2 * s + 1][2], w4[2 * s + 1][3]};
+        vsf[s] = scale_bf16x8(vf[s], w8);
+      }
+      if (!HELP && wave < JOBS) {
+        prepare(c, buf, ld_next, vs_next);
+        if (wave == 3) load_scalars(c + 3, ld_next, vs_next);
+      }
+
+      // ---- per 32-row state block: inter-chunk product with the OLD state (as bf16 operand), decay, state update.  The
+      //      conversion and the decay of the next block are dealt into the gaps behind the four MFMAs of this block, operands
+      //      are requested one block ahead.
+      if (loads && !whole) issue_rows(t2, base2);
+      const uint32_t qpa = qbase + r * RBQ + (uint32_t)(((2 * g) ^ swz16(r)) << 4);
+      const uint32_t kta = kbase + (4 * g + jr) * RBQ + ((ln >> 1) & 1) * 8 + (uint32_t)(((((ln & 1) << 1) | ((ln >> 4) & 1)) ^ swz16(4 * g + jr)) << 4);
+      f32x16 o_inter;
+      {
+        x8 qf[2][2];
+        x4 klo[2][2], khi[2][2];
+        u32x4 hf[2];       // (slice s of the next block's operand is written behind the MFMA that reads this block's)
+        auto request = [&](int bb) {
+#pragma unroll
+          for (int s = 0; s < 2; s++) {
+            qf[bb % 2][s] = lds_read<x8>(qpa ^ (uint32_t)((4 * bb + s) << 4));
+            klo[bb % 2][s] = lds_read_tr4<T>((kta ^ (uint32_t)((4 * bb) << 4)) + 16 * s * RBQ);
+            khi[bb % 2][s] = lds_read_tr4<T>((kta ^ (uint32_t)(((4 * bb) ^ X8) << 4)) + (16 * s + 8) * RBQ);
+          }
+        };
+        auto convert = [&](int bb, int part) {      // a quarter of block bb: operand in bf16, then decayed in place
+          typename E::x2 x, y;
+#pragma unroll
+          for (int i = 0; i < 2; i++) { x[i] = (T)hst[bb][4 * part + i]; y[i] = (T)hst[bb][4 * part + 2 + i]; }
+          uint32_t lo = __builtin_bit_cast(uint32_t, x), hi = __builtin_bit_cast(uint32_t, y);
+          // (pinned here, the products through their factor: the compiler otherwise gathers the vector work of a block in
+          // front of its MFMAs)
+          asm volatile("" : "+v"(lo), "+v"(hi), "+v"(decay_all));
+#pragma unroll
+          for (int i = 0; i < 4; i++) hst[bb][4 * part + i] *= decay_all;
+          hf[part >> 1][2 * (part & 1)] = lo;
+          hf[part >> 1][2 * (part & 1) + 1] = hi;
+        };
+        request(0);
+#pragma unroll
+        for (int part = 0; part < 4; part++) convert(0, part);
+#pragma unroll
+        for (int bb = 0; bb < KB; bb++) {
+          const bool used = !GEN || bb * 32 < qk_used, more = bb + 1 < KB;
+          if (used) {
+            if (more) request(bb + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+              o_inter = E::mfma32(__builtin_bit_cast(x8, hf[s]), qf[bb % 2][s], bb == 0 && s == 0 ? zero16 : o_inter);
+              __builtin_amdgcn_sched_barrier(0);
+              if (more) convert(bb + 1, s);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+              const x8 kf = __builtin_shufflevector(klo[bb % 2][s], khi[bb % 2][s], 0, 1, 2, 3, 4, 5, 6, 7);
+              hst[bb] = E::mfma32(kf, vsf[s], hst[bb]);
+              __builtin_amdgcn_sched_barrier(0);
+              if (more) convert(bb + 1, 2 + s);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+#pragma unroll
+          for (int x = 0; x < NL; x++)
+            if (x * KB / NL == bb) load_one(x, t2, base2, on);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 16; j++) o_out[j] = o_inter[j] * eg + o_intra[j];
+      if constexpr (HELP) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+          const f32x4 w = {o_out[4 * q4], o_out[4 * q4 + 1], o_out[4 * q4 + 2], o_out[4 * q4 + 3]};
+          lds_write<f32x4>(out_block(c) + r * OSTR + (8 * q4 + 4 * g) * 4, w);
+        }
+      }
+      // chunk c + 2 must be there for P^T of c + 2, made in c + 1: with four stages it was asked for a chunk ago and the loads of this
+      // chunk may go on; with three, its V, not read before c + 2, may
+      if (loads && !whole) wait_dma();
+      else wait_vm<HELP ? NL : NLV>();
+    };
+    // a helper's: scalars' loads of chunk c + 3, outputs of c - 1, P^T of c + 1 or scalars of c + 2
+    auto help_chunk = [&](int c, int buf) {
+      const float ld_now = ld_next, vs_now = vs_next;
+      if (wave == 3) load_scalars(c + 3, ld_next, vs_next);
+      if (c > c_begin) write_block(c - 1);
+      prepare(c, buf, ld_now, vs_now);
+    };
+    int buf = 0;          // stage of chunk c
+    if (HELP && helper) {
+      for (int c = c_begin; c < c_end; c++) {
+        help_chunk(c, buf);
+        __syncthreads();
+        buf = buf == NST - 1 ? 0 : buf + 1;
+      }
+      if (c_begin < c_end) write_block(c_end - 1);
+    } else {
+      for (int c = c_begin; c < c_end; c++) {
+        run_chunk(c, buf);
+        __syncthreads();
+        buf = buf == NST - 1 ? 0 : buf + 1;
+      }
+      if (!HELP && c_begin < c_end) write_out(o_out, (c_end - 1) * L, lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE + 2 * QT);
+    }
+  }
+  if constexpr (!PIPE) {
   for (int c = c_begin; c < c_end; c++) {
     const int buf = (c - c_begin) & 1, t0 = c * L;
     wait_dma();
@@ -316,30 +738,6 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
     const uint32_t base = lds0 + buf * STAGE;
     const uint32_t qbase = base, kbase = base + QT, vbase = base + 2 * QT;
 
-    // ---- this wave's share of A^T = K Q^T: quadrant slot 0 = keys 0..15 x queries 0..15, 1 = keys 0..15 x queries
-    //      16..31, 2 = keys 16..31 x queries 16..31; A / B operand: lane holds row (column) lane % 16, k = 8 (lane / 16) .. +7
-    //      of a 32-wide slice; C: lane holds column lane % 16, rows 4 (lane / 16) + {0..3}
-    if constexpr (SHARE_A) {
-      if (wave < A_ITEMS) {
-        const int slot = wave / KP, kp = wave % KP;
-        int la = lane;
-        asm volatile("" : "+v"(la));
-        const int rr = la & 15, kg = la >> 4;
-        // (tile bases and row offsets are multiples of the row size, so the swizzled chunk index occupies its own
-        // address bits: one XOR with a constant per read moves to another slice)
-        constexpr int NS16 = DK / 32 / KP;
-        const uint32_t c0 = (uint32_t)((kg ^ swz16(rr)) << 4) ^ (uint32_t)(kp * NS16 * 64);
-        const uint32_t ka = kbase + (16 * (slot >> 1) + rr) * RBQ + c0, qa = qbase + (16 * (slot > 0) + rr) * RBQ + c0;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s2 = 0; s2 < NS16; s2++) {
-          if (GEN && (kp * NS16 + s2) * 32 >= qk_used) break;
-          acc = E::mfma16(lds_read<x8>(ka ^ (uint32_t)(s2 * 64)), lds_read<x8>(qa ^ (uint32_t)(s2 * 64)), acc);
-        }
-        lds_write<f32x4>(lds_apart + wave * 1024 + la * 16, acc);
-      }
-    }
-
     // ---- per-lane LDS read offsets.  They are loop invariant; left outside the loop, they (and every
     //      swizzled address derived from them, dozens) stay in registers across chunks, which the state
     //      accumulator leaves no room for.  The lane id is laundered so that they are rebuilt per chunk.
@@ -349,14 +747,20 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
     // K rows / Q rows as MFMA operands of A^T = K Q^T: row r, logical chunk 2ks + g
     const uint32_t qk_row = r * RBQ;
     const int qk_c0 = g ^ swz16(r);
-    // Q^T operand of h^T Q^T: token r, key dims 32b + 16s + 4g + {0..3} and + 8: chunk 4b + 2s (+1), half g
-    const uint32_t qp_row = r * RBQ + g * 8;
-    const int qp_swz = swz16(r);
+    // A 32-row block of the state holds its key dims in an order that makes the Q^T operand of h^T Q^T one 128-bit read per
+    // slice: accumulator rows 8q + 4g + {0..3} of lane half g are key dims 16g + 4q + {0..3}, so slice s (q = 2s, 2s + 1) of
+    // lane half g is the eight dims of chunk 4b + 2g + s.  (In the rows' own order it was two 64-bit reads that left half of the
+    // banks idle and met twice in the other half: SQ_LDS_BANK_CONFLICT 15.7 M -> 7.3 M a pass at 8 x 16 heads, 2048 tokens,
+    // 256 / 512, 290 -> 280 us before anything else changed.)
+    const uint32_t qp_row = r * RBQ;
+    const int qp_c0 = (2 * g) ^ swz16(r);
     // transposing reads (K^T and V^T): lane block lane/16 -> (row group g, column half), rows 16s + 4g + jr (+8)
     const int jr = (ln & 15) >> 2;
     const int lc = (((ln >> 4) & 1) << 1) | ((ln & 3) >> 1);
-    const uint32_t kt_row = (4 * g + jr) * RBQ + (ln & 1) * 8;
-    const int kt_c0 = lc ^ swz16(4 * g + jr);                      // rows +8 / +16: see HALF_XOR below
+    // (K^T: the four columns that become rows 4m .. 4m + 3 of a state block, m = 4 ((ln >> 4) & 1) + ln % 4, are its dims
+    // 16 (m % 2) + 4 (m / 2) ..: chunk 2 (m % 2) + m / 4, half (m / 2) % 2)
+    const uint32_t kt_row = (4 * g + jr) * RBQ + ((ln >> 1) & 1) * 8;
+    const int kt_c0 = (((ln & 1) << 1) | ((ln >> 4) & 1)) ^ swz16(4 * g + jr);                      // rows +8 / +16: see Q_X8 below
     const uint32_t vt_row = (4 * g + jr) * RBV + (ln & 1) * 8;
     const int vt_c0 = (4 * wave + lc) ^ swz_tile<CPRV>(4 * g + jr);
     // swz(row + 8) ^ swz(row) and swz(row + 16) ^ swz(row) for rows < 8
@@ -389,30 +793,13 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
     // ---- A^T = K Q^T (lane: token i = r, rows j = 8(jj/4) + 4g + jj%4)
     // two accumulation chains, so that consecutive MFMAs do not wait for each other, where registers
     // allow (with three waves per SIMD the other waves fill those gaps)
-    constexpr bool TWO_CHAINS = HG == 1 && !SHARE_A;
+    constexpr bool TWO_CHAINS = HG == 1;
     // (a chain's first MFMA takes the constant zero as its accumulator input: no registers to clear)
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     f32x16 sacc, sacc2;
 #pragma unroll
     for (int j = 0; j < 16; j++) { sacc[j] = 0.f; sacc2[j] = 0.f; }
-    if constexpr (SHARE_A) {
-      // gather the quadrants: this lane's rows 8 q4 + 4g + {0..3} of column r sit in lane (r % 16) + 16 (2 (q4 % 2) + g)
-      // of quadrant slot (q4 / 2) + (r / 16); for the quadrant that was left out this reads its neighbour, and the
-      // causal select below discards it
-      __syncthreads();
-#pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) {
-        const uint32_t src = lds_apart + (uint32_t)(((q4 >> 1) + (r >> 4)) * KP) * 1024 + (uint32_t)((r & 15) + 16 * (2 * (q4 & 1) + g)) * 16;
-        f32x4 t = lds_read<f32x4>(src);
-        if constexpr (KP == 2) {
-          const f32x4 t2 = lds_read<f32x4>(src + 1024);
-#pragma unroll
-          for (int i = 0; i < 4; i++) t[i] += t2[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) sacc[4 * q4 + i] = t[i];
-      }
-    } else if constexpr (MODE != 1) {
+    if constexpr (MODE != 1) {
       constexpr int NS = DK / 16, AH = 2, RING = 3;
       x8 kf[RING], qf[RING];
       const uint32_t kq_a = kbase + qk_row + (uint32_t)(qk_c0 << 4), qq_a = qbase + qk_row + (uint32_t)(qk_c0 << 4);
@@ -501,16 +888,13 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
     {
       // per 32-row state block b: inter-chunk product with the OLD state, then the state update
       constexpr int RING = 2;
-      x4 qlo[RING][2], qhi[RING][2], klo[RING][2], khi[RING][2];
-      const uint32_t qpa = qbase + qp_row + (uint32_t)(qp_swz << 4), kta = kbase + kt_row + (uint32_t)(kt_c0 << 4);
+      x8 qf[RING][2];
+      x4 klo[RING][2], khi[RING][2];
+      const uint32_t qpa = qbase + qp_row + (uint32_t)(qp_c0 << 4), kta = kbase + kt_row + (uint32_t)(kt_c0 << 4);
       auto request = [&](int bb) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-          const int lcq = 4 * bb + 2 * s;
-          if constexpr (MODE != 1) {
-            qlo[bb % RING][s] = lds_read<x4>(qpa ^ (uint32_t)(lcq << 4));
-            qhi[bb % RING][s] = lds_read<x4>(qpa ^ (uint32_t)((lcq + 1) << 4));
-          }
+          if constexpr (MODE != 1) qf[bb % RING][s] = lds_read<x8>(qpa ^ (uint32_t)((4 * bb + s) << 4));
           const int cx = s ? Q_X16 : 0;
           klo[bb % RING][s] = lds_read_tr4<T>((kta ^ (uint32_t)(((4 * bb) ^ cx) << 4)) + 16 * s * RBQ);
           khi[bb % RING][s] = lds_read_tr4<T>((kta ^ (uint32_t)(((4 * bb) ^ cx ^ Q_X8) << 4)) + (16 * s + 8) * RBQ);
@@ -541,9 +925,8 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
         if constexpr (MODE != 1) {
 #pragma unroll
           for (int s = 0; s < 2; s++) {
-            x8 qf = __builtin_shufflevector(qlo[bb % RING][s], qhi[bb % RING][s], 0, 1, 2, 3, 4, 5, 6, 7);
-            if (DK < 256 && HG == 1 && s) o_inter2 = E::mfma32(hf[s], qf, bb == 0 ? zero16 : o_inter2);   // (a second chain where registers allow)
-            else o_inter = E::mfma32(hf[s], qf, (bb == 0 && (s == 0 || (DK < 256 && HG == 1))) ? zero16 : o_inter);
+            if (DK < 256 && HG == 1 && s) o_inter2 = E::mfma32(hf[s], qf[bb % RING][s], bb == 0 ? zero16 : o_inter2);   // (a second chain where registers allow)
+            else o_inter = E::mfma32(hf[s], qf[bb % RING][s], (bb == 0 && (s == 0 || (DK < 256 && HG == 1))) ? zero16 : o_inter);
           }
         }
 #pragma unroll
@@ -555,59 +938,13 @@ __global__ __launch_bounds__(64 * NWH * HG, (min_waves_per_simd<DK, NWH, HG>()))
       }
     }
 
-    // ---- write this wave's [32 tokens x 32 columns] block: stage (wave private), then 16-byte row pieces.
-    //      With ALIAS_OST the staging block is the wave's own 4 chunks per row of the V tile just consumed
-    //      (only this wave reads them, and the next DMA into this buffer is issued behind the next barrier).
-    if (MODE != 1 && a.out_f32) {
-      // fp32 outputs (used by the backward pass, whose decay gradient is a difference of sums over these
-      // values): the same staging block, 16 columns at a time
-      const int sw_r = swz_tile<CPRV>(r);
-      float* ob32 = (float*)a.o + (int64_t)piece * a.piece_o + (int64_t)bh * Tn * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH);
+    if constexpr (MODE != 1) {
+      f32x16 o;
 #pragma unroll
-      for (int half = 0; half < 2; half++) {
-#pragma unroll
-        for (int q2 = 0; q2 < 2; q2++) {
-          const int q4 = 2 * half + q2;
-          f32x4 w;
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-            w[i] = (DK < 256 && HG == 1 ? o_inter[4 * q4 + i] + o_inter2[4 * q4 + i] : o_inter[4 * q4 + i]) * eg + o_intra[4 * q4 + i];
-          if (ALIAS_OST) lds_write<f32x4>(vbase + r * RBV + (uint32_t)(((4 * wave + 2 * q2 + g) ^ sw_r) << 4), w);
-          else lds_write<f32x4>(lds_ost + r * OROW + (8 * q2 + 4 * g) * 4, w);
-        }
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-          const int ci = ln + 64 * it, row = ci >> 2, cc = ci & 3;
-          const u32x4 w = ALIAS_OST ? lds_read<u32x4>(vbase + row * RBV + (uint32_t)(((4 * wave + cc) ^ swz_tile<CPRV>(row)) << 4))
-                                    : lds_read<u32x4>(lds_ost + row * OROW + cc * 16);
-          if (t0 + row < Tn) {
-            f32x4* dst = (f32x4*)(ob32 + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + 16 * half + cc * 4);
-            f32x4 val = __builtin_bit_cast(f32x4, w);
-            if (a.out_f32 == 2) val += *dst;   // (a contraction cut into pieces: the pieces' outputs add up)
-            *dst = val;
-          }
-        }
-      }
-    } else if constexpr (MODE != 1) {
-      const int sw_r = swz_tile<CPRV>(r);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) {
-        x4 w;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          w[i] = (T)((DK < 256 && HG == 1 ? o_inter[4 * q4 + i] + o_inter2[4 * q4 + i] : o_inter[4 * q4 + i]) * eg + o_intra[4 * q4 + i]);
-        if (ALIAS_OST) lds_write<x4>((vbase + r * RBV + (uint32_t)(((4 * wave) ^ sw_r) << 4) + g * 8) ^ (uint32_t)(q4 << 4), w);
-        else lds_write<x4>(lds_ost + r * OROW + (8 * q4 + 4 * g) * 2, w);
-      }
-      // (rows 16 apart share their swizzle)
-      const uint32_t ra = vbase + (ln >> 2) * RBV + (uint32_t)(((4 * wave + (ln & 3)) ^ swz_tile<CPRV>(ln >> 2)) << 4);
-#pragma unroll
-      for (int it = 0; it < 2; it++) {
-        const int ci = ln + 64 * it, row = ci >> 2, cc = ci & 3;
-        const u32x4 w = ALIAS_OST ? lds_read<u32x4>(ra + 16 * it * RBV) : lds_read<u32x4>(lds_ost + row * OROW + cc * 16);
-        if (t0 + row < Tn) *(u32x4*)(ob + (int64_t)(rev_o ? Tn - 1 - (t0 + row) : t0 + row) * a.Dv + cc * 8) = w;
-      }
+      for (int j = 0; j < 16; j++) o[j] = (DK < 256 && HG == 1 ? o_inter[j] + o_inter2[j] : o_inter[j]) * eg + o_intra[j];
+      write_out(o, t0, vbase);
     }
+  }
   }
   if (MODE == 1) {
     // the state this segment ends in when entered with zeros, and its total log decay
@@ -661,7 +998,10 @@ template <int DK, int NWH, int HG>
 struct Config {
   static constexpr int NW = NWH * HG;
   static constexpr size_t stage = (size_t)L * (4 * DK + 2 * 32 * NW);
-  static constexpr size_t lds = 2 * stage + NW * (3 * L * 4) + (HG > 1 ? 0 : NW * (L * 80)) + (NW >= 4 ? 3 * (NW >= 8 ? 2 : 1) * 1024 : 0);
+  static constexpr int waves = workgroup_waves<DK, NWH, HG, 0>();      // of a workgroup that produces outputs
+  static constexpr size_t lds_states = 2 * stage + NW * (3 * L * 4);
+  static constexpr size_t lds = pipelined<NWH, HG, 0>() ? (waves > NW ? 4 : 3) * stage + pipe_shared(HG) + (waves > NW ? 2 * NW * L * 144 : 0) : lds_states + NW * (L * 80);
+  static_assert(lds <= 160 * 1024, "a workgroup's LDS");
   static constexpr int64_t ws_wave_floats = (int64_t)(DK / 32) * 16 * 64;
 
   static bool prepare(int& resident, int& cus) {
@@ -677,7 +1017,7 @@ struct Config {
     if (cus <= 0) return false;
     int r = s_resident.load(std::memory_order_relaxed);
     if (r < 0) {
-      if (hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, linear_fwd_kernel<DK, NWH, HG, 2>, 64 * NW, lds)) != 0) return false;
+      if (hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, linear_fwd_kernel<DK, NWH, HG, 2>, 64 * waves, lds)) != 0) return false;
       r = r < 1 ? 1 : r;
       s_resident.store(r, std::memory_order_relaxed);
     }
@@ -753,7 +1093,7 @@ struct Config {
     if (a.v_row == 0) a.v_row = a.Dv;
     if (a.Hv == 0) a.Hv = a.H;
     if (a.q_row % 8 != 0 || a.k_row % 8 != 0 || a.v_row % (32 * NWH) != 0 || a.Hv <= 0 || a.H % a.Hv != 0) return -2;
-    if (a.qk_cols < 0 || a.qk_cols > DK || a.qk_cols % 8 != 0) return -2;
+    if (a.qk_cols < 0 || a.qk_cols > DK || a.qk_cols % 32 != 0) return -2;
     if (HG > 1 && a.Hv != a.H) return -2;
     if (a.n_pieces > 1 && !a.out_f32) return -2;
     return 0;
@@ -769,9 +1109,9 @@ struct Config {
       const unsigned w = (unsigned)(heads * a.dv_blocks * (a.n_pieces > 1 ? a.n_pieces : 1) * (MODE == 0 ? 1 : MODE == 1 ? a.nseg - 1 : a.nseg));
       width = w > width ? w : width;
     }
-    if (n > 1) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 2>), dim3(width, (unsigned)n), dim3(64 * NW), lds, stream, all);
-    else if (gen) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 1>), dim3(width), dim3(64 * NW), lds, stream, all.s[0]);
-    else hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE>), dim3(width), dim3(64 * NW), lds, stream, all.s[0]);
+    if (n > 1) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 2>), dim3(width, (unsigned)n), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all);
+    else if (gen) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 1>), dim3(width), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all.s[0]);
+    else hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE>), dim3(width), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all.s[0]);
   }
 
   // n scans side by side (see linear_scans_dispatch; more than one: all with the general addressing).
@@ -803,7 +1143,11 @@ struct Config {
     const Tail tail = nseg <= 1 && n == 1 ? tail_plan(a, want_segments, resident, cus) : Tail{0, 0, 1, 0};
     size_t need = 0;
     for (int i = 0; i < n; i++) need += ws_bytes(all.s[i], nseg);
-    if (query) { *query = tail.tail_bg > 0 ? tail_ws_bytes(tail, a.dv_blocks) : need; return 0; }
+    if (query) {
+      // (an automatic choice asks for some workspace also where it is a single pass: 0 is the answer for segments = 1)
+      *query = tail.tail_bg > 0 ? tail_ws_bytes(tail, a.dv_blocks) : need > 0 || want_segments != 0 ? need : 256;
+      return 0;
+    }
     if (nseg > 1 && (!ws || ws_size < need || ((uintptr_t)ws & 3) != 0)) nseg = 1;   // no workspace: single pass
     if (nseg <= 1 && tail.tail_bg > 0 && ws && ws_size >= tail_ws_bytes(tail, a.dv_blocks) && ((uintptr_t)ws & 3) == 0) {
       // the full rounds in a single pass, then the tail in segments (see tail_plan)

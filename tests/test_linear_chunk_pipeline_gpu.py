@@ -1,0 +1,90 @@
+"""The pipelined chunk loop of the linear scan (tiles two or three chunks ahead, P^T one chunk ahead, scalars two): sequence lengths
+around its start and its end, with each workgroup layout (eight state waves; four with four helpers; two heads with four helpers)
+and each form of operand addressing, and what a chunk must not let through from later tokens.
+
+Outputs are compared chunk by chunk in the 2-norm: P^T, the state as an operand and the output are rounded to bf16 (2^-9 each, at
+most), fp32 sums add nothing that shows, so a chunk's relative error stays below 3 * 2^-9 = 5.9e-3 but for what cancels in it; a
+wrong tile, chunk or factor is of the order of 1."""
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+BOUND = 1e-2
+# B, Hq, H, Dk, Dv: <256, 8>, <128, 8>, <256, 4>, <128, 4>, two heads of <128, 2>, key widths that are padded
+LAYOUTS = [(1, 2, 2, 256, 256), (1, 1, 2, 128, 256), (1, 2, 2, 256, 128), (2, 1, 1, 128, 128), (1, 1, 4, 128, 64), (1, 2, 2, 192, 256), (1, 2, 2, 64, 128)]
+
+
+def _hb():
+    from metaattention_amd import hip_backend as hb
+    hb.load_library()
+    return hb
+
+
+def _case(B, Hq, H, T, Dk, Dv, scaled, seed):
+    g = torch.Generator().manual_seed(seed)
+    q, k = (torch.randn(B, Hq, T, Dk, generator=g).mul(Dk ** -0.25).bfloat16() for _ in range(2))
+    v = torch.randn(B, H, T, Dv, generator=g).bfloat16()
+    ld = torch.nn.functional.logsigmoid(torch.randn(B, H, T, generator=g) + 2.0)
+    vs = torch.rand(B, H, T, generator=g) + 0.1 if scaled else None
+    return q, k, v, ld, vs
+
+
+def _reference(q, k, v, ld, vs, chunk):
+    pad = -q.shape[2] % chunk
+    p = lambda t: torch.nn.functional.pad(t, (0, 0, 0, pad) if t.dim() == 4 else (0, pad))   # noqa: E731
+    o = oracle.linear_attention_chunked(p(q), p(k), p(v), p(ld), chunk=chunk, v_scale=None if vs is None else p(vs), compute_dtype=torch.float64)
+    return o[:, :, :q.shape[2]]
+
+
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 96, 97, 128, 161])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_lengths_around_the_pipeline(layout, T):
+    hb = _hb()
+    B, Hq, H, Dk, Dv = layout
+    q, k, v, ld, vs = _case(B, Hq, H, T, Dk, Dv, T % 2 == 1, T)
+    print(f"pipeline {layout} T{T}", flush=True)
+    ref = _reference(q, k, v, ld, vs, 32)
+    for segments in (1, 3):
+        o = hb.linear_fwd(q.cuda(), k.cuda(), v.cuda(), ld.cuda(), v_scale=None if vs is None else vs.cuda(), segments=segments)
+        torch.cuda.synchronize()
+        err = (o.double().cpu() - ref).pow(2)
+        for t in range(0, T, 32):
+            rel = (err[:, :, t:t + 32].sum(dim=(2, 3)) / ref[:, :, t:t + 32].pow(2).sum(dim=(2, 3))).sqrt()
+            assert rel.max() < BOUND, (segments, t, rel)
+
+
+@pytest.mark.parametrize("T", [33, 96, 130])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_gradients_around_the_pipeline(layout, T):
+    """The scans on reversed operands, column slices and shared heads, fp32 outputs among them."""
+    hb = _hb()
+    B, Hq, H, Dk, Dv = layout
+    q, k, v, ld, vs = _case(B, Hq, H, T, Dk, Dv, Hq != H, T + 1)
+    dout = torch.randn(B, H, T, Dv, generator=torch.Generator().manual_seed(T)).bfloat16()
+    print(f"pipeline gradients {layout} T{T}", flush=True)
+    ref = oracle.linear_attention_grads(q, k, v, ld, dout, v_scale=vs)
+    out = hb.linear_bwd(q.cuda(), k.cuda(), v.cuda(), ld.cuda(), dout.cuda(), v_scale=None if vs is None else vs.cuda())
+    torch.cuda.synchronize()
+    for name, x, r in zip(("dq", "dk", "dv"), out[:3], ref[:3]):
+        err = (x.double().cpu() - r).norm() / r.norm()
+        assert err < BOUND, (name, float(err))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_later_keys_and_decays_stay_out(layout, bad):
+    """A key, a decay or a value scale that is not finite changes nothing before its own token, inside its chunk too."""
+    hb = _hb()
+    B, Hq, H, Dk, Dv = layout
+    T, at = 96, 45
+    q, k, v, ld, vs = _case(B, Hq, H, T, Dk, Dv, True, 7)
+    good = hb.linear_fwd(q.cuda(), k.cuda(), v.cuda(), ld.cuda(), v_scale=vs.cuda(), segments=1)
+    for which in ("k", "ld", "vs"):
+        k2, ld2, vs2 = k.clone(), ld.clone(), vs.clone()
+        {"k": k2, "ld": ld2, "vs": vs2}[which][:, :, at] = bad
+        print(f"later {which} = {bad} {layout}", flush=True)
+        o = hb.linear_fwd(q.cuda(), k2.cuda(), v.cuda(), ld2.cuda(), v_scale=vs2.cuda(), segments=1)
+        torch.cuda.synchronize()
+        assert torch.equal(o[:, :, :at], good[:, :, :at]), which
