@@ -295,6 +295,10 @@ int ma_linear_fwd(const ma_linear_params* p, ma_stream_t stream);
 /* linear_tl.py:1268-1340 */
 size_t ma_linear_bwd_workspace_bytes(const ma_linear_bwd_params* p);
 int ma_linear_bwd(const ma_linear_bwd_params* p, ma_stream_t stream);
+/* The gradients of q, k and v alone: dlog_decay and dv_scale are not read and may be NULL.  A workspace of its own query, never more
+ * than ma_linear_bwd's. */
+size_t ma_linear_bwd_qkv_workspace_bytes(const ma_linear_bwd_params* p);
+int ma_linear_bwd_qkv(const ma_linear_bwd_params* p, ma_stream_t stream);
 
 /* mla_decode_tl.py:293-303 (`main_split`) */
 int ma_mla_choose_split(const ma_mla_params* p);

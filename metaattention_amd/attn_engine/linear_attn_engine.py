@@ -35,10 +35,11 @@ class _LinearAttention(torch.autograd.Function):
         from hip_backend import linear_bwd
         q, k, v, g, *rest = ctx.saved_tensors
         vs = rest[0] if ctx.has_vs else None
-        dq, dk, dv, dg, dvs = linear_bwd(q, k, v, g, dout, q_scale=ctx.q_scale, v_scale=vs)
+        with_decay = ctx.needs_input_grad[3] or (vs is not None and ctx.needs_input_grad[4])
+        dq, dk, dv, dg, dvs = linear_bwd(q, k, v, g, dout, q_scale=ctx.q_scale, v_scale=vs, with_decay=with_decay)
         if dvs is not None:
             dvs = dvs.to(vs.dtype)
-        return dq, dk, dv, dg.to(g.dtype), dvs, None, None
+        return dq, dk, dv, dg.to(g.dtype) if dg is not None else None, dvs, None, None
 
 
 class LinearAttentionEngine:

@@ -416,8 +416,11 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
     const Tensor dout = grads[0].to(v.scalar_type()).contiguous();
     const Tensor dq = empty(q.sizes(), q.scalar_type(), q.device()), dk = empty(k.sizes(), k.scalar_type(), k.device()),
                  dv = empty(v.sizes(), v.scalar_type(), v.device());
-    Tensor dg = empty(g.sizes(), at::kFloat, v.device()), dvs;
-    if (has_vs) dvs = empty(vs.sizes(), at::kFloat, v.device());
+    // (nobody asks for the decay's gradient or the value scale's: a call that leaves them out)
+    const bool with_decay = ctx->needs_input_grad(3) || (has_vs && ctx->needs_input_grad(4));
+    Tensor dg, dvs;
+    if (with_decay) dg = empty(g.sizes(), at::kFloat, v.device());
+    if (with_decay && has_vs) dvs = empty(vs.sizes(), at::kFloat, v.device());
     ma_linear_bwd_params p{};
     p.dtype = MA_BF16;
     linear_sizes(q, k, v, p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v);
@@ -425,17 +428,17 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
     p.log_decay = (const float*)g.data_ptr();
     p.v_scale = has_vs ? (const float*)vs.data_ptr() : nullptr;
     p.q_scale = (float)ctx->saved_data["q_scale"].toDouble();
-    p.dq = dq.data_ptr(); p.dk = dk.data_ptr(); p.dv = dv.data_ptr(); p.dlog_decay = (float*)dg.data_ptr();
-    p.dv_scale = has_vs ? (float*)dvs.data_ptr() : nullptr;
-    const size_t need = ma_linear_bwd_workspace_bytes(&p);
+    p.dq = dq.data_ptr(); p.dk = dk.data_ptr(); p.dv = dv.data_ptr(); p.dlog_decay = dg.defined() ? (float*)dg.data_ptr() : nullptr;
+    p.dv_scale = dvs.defined() ? (float*)dvs.data_ptr() : nullptr;
+    const size_t need = with_decay ? ma_linear_bwd_workspace_bytes(&p) : ma_linear_bwd_qkv_workspace_bytes(&p);
     const c10::DataPtr ws = scratch(need);
     p.workspace = ws.get(); p.workspace_bytes = need;
     {
       NoGil release;
-      TORCH_CHECK(ma_linear_bwd(&p, stream_of(v.device().index())) == MA_OK, ma_last_error());
+      TORCH_CHECK((with_decay ? ma_linear_bwd : ma_linear_bwd_qkv)(&p, stream_of(v.device().index())) == MA_OK, ma_last_error());
     }
-    dg = dg.to(saved[3].scalar_type());
-    if (has_vs) dvs = dvs.to(saved[4].scalar_type());
+    if (dg.defined()) dg = dg.to(saved[3].scalar_type());
+    if (dvs.defined()) dvs = dvs.to(saved[4].scalar_type());
     return {dq, dk, dv, dg, dvs, Tensor(), Tensor()};
   }
 };

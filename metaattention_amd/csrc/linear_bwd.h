@@ -9,7 +9,8 @@ struct LinBwdArgs {
   const float* log_decay;   // [B,H,T]
   const float* v_scale;     // [B,H,T] or null
   void* dq; void* dk; void* dv;   // bf16, shaped like q, k, v
-  float* dlog_decay;        // [B,H,T]
+  bool wants_decay;         // the gradients of the decay and of the value scale are wanted
+  float* dlog_decay;        // [B,H,T] or null
   float* dv_scale;          // [B,H,T] or null
   float q_scale;
   int B, H, Hq, Hk, T, Dk, Dv;

@@ -331,11 +331,20 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return o; };
   // (a contraction of equal pieces that are all read in place runs its pieces side by side, each with an output of its own)
   const bool side_by_side = sl.n > 1 && a.Dv % sl.w[0] == 0 && sl.w[sl.n - 1] == sl.w[0];
-  const int np = side_by_side ? sl.n : 1;
-  const int64_t piece_stride = BHT * a.Dk;
-  const size_t o_dqh = take((size_t)np * BHT * a.Dk * 4), o_dkh = take((size_t)np * BHT * a.Dk * 4), o_du = take((size_t)BHT * a.Dv * 4);
-  const size_t o_dG = take((size_t)BHT * 4), o_grev = take((size_t)BHT * 4);
   const bool direct_dv = !a.v_scale && !a.dv_scale;     // dv is du itself, and the scan writes it: bf16, rows back in time order
+  // Without the decay's gradient nothing but dq and dk themselves is made of the dq and dk scans.  Where every head has its own q and k
+  // and there is no v_scale the scans write them, bf16 and in time order: those of one piece at once; of equal pieces the first
+  // leaves fp32, which the last takes in before it rounds, the pieces of dq beside those of dk in one launch each, as long as
+  // that fills the device (below that, pieces side by side are the shorter chain).  8 x 16 heads, 2048 tokens, 256 / 512, forward and
+  // backward 1248 -> 1043 us: two launches of 337 us where two of 260 were followed by 285 us of adding up.
+  const bool own_heads = !a.wants_decay && direct_dv && a.Hq == a.H && a.Hk == a.H;
+  const bool in_turn = own_heads && side_by_side && a.Dk % 128 == 0 && (int64_t)2 * a.B * a.H >= device_cus();
+  const bool direct_qk = in_turn || (own_heads && sl.n == 1);
+  const int np = side_by_side && !in_turn ? sl.n : 1;
+  const int64_t piece_stride = BHT * a.Dk;
+  const size_t part = direct_qk && !in_turn ? 0 : (size_t)np * BHT * a.Dk * 4;
+  const size_t o_dqh = take(part), o_dkh = take(part), o_du = take(direct_dv ? 0 : (size_t)BHT * a.Dv * 4);
+  const size_t o_dG = take((size_t)BHT * 4), o_grev = take((size_t)BHT * 4);
   // Heads in groups that share q and k, with a v_scale and a contraction of one piece (Mamba2): the dk scan leaves bf16 in
   // time order (see grads_shared_kernel).
   const bool dk_bf16 = a.Hq == a.Hk && a.Hq != a.H && !direct_dv && sl.n == 1;
@@ -359,9 +368,19 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   // the columns of piece s that exist (a last piece may reach beyond the value columns: the scan kernel pads with zeros)
   auto piece_cols = [&](int s) { return sl.c0[s] + sl.w[s] <= a.Dv ? 0 : a.Dv - sl.c0[s]; };
   // dq (per head) = LA(do, v, k; v_scale), contraction over the value columns; k is read with its own heads
+  // (direct_qk: dq itself, bf16; in turn: its pieces add up in `out`, and the last leaves dq)
+  auto direct = [&](LinArgs la, int s, void* grad, float* out, bool reversed) {
+    if (!direct_qk) return la;
+    la.rev_o = reversed ? 1 : 0;
+    if (s + 1 < sl.n) return la;
+    la.o = grad;
+    la.out_f32 = 0;
+    la.o_add = in_turn ? out : nullptr;
+    return la;
+  };
   auto dq_scan = [&](int s, float* out) {
-    return scan(Operand{do_p + sl.c0[s], a.H, a.Dv}, Operand{v_p + sl.c0[s], a.H, a.Dv}, Operand{k_p, a.Hk, a.Dk}, false, sl.w[s], a.Dk, a.log_decay, a.v_scale,
-                out, s > 0, np, np > 1 ? 0 : piece_cols(s));
+    return direct(scan(Operand{do_p + sl.c0[s], a.H, a.Dv}, Operand{v_p + sl.c0[s], a.H, a.Dv}, Operand{k_p, a.Hk, a.Dk}, false, sl.w[s], a.Dk, a.log_decay, a.v_scale,
+                out, s > 0, np, np > 1 ? 0 : piece_cols(s)), s, a.dq, out, false);
   };
   // du (reversed) = LA(R k, R q, R do), contraction over the key columns: the operands are read in reversed time in place
   auto du_scan = [&](const float* grev, float* out) {
@@ -370,8 +389,8 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   };
   // dk (per head, reversed, before its v_scale factor) = LA(R v, R do, R q), contraction over the value columns
   auto dk_scan = [&](int s, const float* grev, float* out) {
-    return scan(Operand{v_p + sl.c0[s], a.H, a.Dv}, Operand{do_p + sl.c0[s], a.H, a.Dv}, Operand{q_p, a.Hq, a.Dk}, true, sl.w[s], a.Dk, grev, nullptr, out, s > 0,
-                np, np > 1 ? 0 : piece_cols(s), dk_bf16);
+    return direct(scan(Operand{v_p + sl.c0[s], a.H, a.Dv}, Operand{do_p + sl.c0[s], a.H, a.Dv}, Operand{q_p, a.Hq, a.Dk}, true, sl.w[s], a.Dk, grev, nullptr, out, s > 0,
+                np, np > 1 ? 0 : piece_cols(s), dk_bf16), s, a.dk, out, true);
   };
   // The three scans are independent of each other.  Where their contractions are one piece (or pieces side by side) dq and dk go
   // out in one launch, and du with them where it runs in the same instantiation: one short call of few heads is three
@@ -383,7 +402,7 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   {
     size_t need = 0;
     LinArgs la[3] = {dq_scan(0, nullptr), dk_scan(0, nullptr, nullptr), du_scan(nullptr, nullptr)};
-    with_du = whole && sl.w[0] == DKP && linear_scans_together(la, 3, DKP);
+    with_du = whole && !in_turn && sl.w[0] == DKP && linear_scans_together(la, 3, DKP);
     if (whole && linear_scans_dispatch(la, with_du ? 3 : 2, sl.w[0], nullptr, 0, nullptr, &need) == 0 && need > scan_ws) scan_ws = need;
     for (int s = 0; s < sl.n && !whole; s++) {
       la[0] = dq_scan(s, nullptr);
@@ -402,12 +421,12 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   // (dk last: the epilogue finds part of what it wrote in the memory-side cache)
   if (!with_du)
     if (const int rc = linear_fwd_dispatch(du_scan(grev, du), DKP, 0, scan_at, scan_ws, stream, nullptr)) return rc;
-  if (whole) {
+  for (int s = 0; s < (in_turn ? sl.n : 1) && whole; s++) {
     LinArgs la[kLinScans];
     int n = 0;
-    la[n++] = dq_scan(0, dqh);
+    la[n++] = dq_scan(s, dqh);
     if (with_du) la[n++] = du_scan(grev, du);
-    la[n++] = dk_scan(0, grev, dkh);
+    la[n++] = dk_scan(s, grev, dkh);
     if (const int rc = linear_scans_dispatch(la, n, sl.w[0], scan_at, scan_ws, stream, nullptr)) return rc;
   }
   for (int s = 0; s < sl.n && !whole; s++) {
@@ -415,6 +434,7 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
     if (const int rc = linear_fwd_dispatch(dk_scan(s, grev, dkh), sl.w[s], 0, scan_at, scan_ws, stream, nullptr)) return rc;
   }
   if (direct_dv) du = nullptr;
+  if (direct_qk) return launch_status();
 
   if (a.Hq == a.Hk && a.Hq != a.H) {
     // heads in groups that share q and k: gradients, group sums and conversions in one pass over the scan outputs
@@ -429,7 +449,7 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
     else if (a.Dk > 128) launch(grads_shared_kernel<64>, 4);
     else if (dk_bf16) launch(grads_shared_kernel<32, true>, 8);
     else launch(grads_shared_kernel<32>, 8);
-    hipLaunchKernelGGL(suffix_sum_kernel, dim3((unsigned)(a.B * a.H)), dim3(256), 0, stream, a.dlog_decay, (const float*)dG, a.T);
+    if (a.wants_decay) hipLaunchKernelGGL(suffix_sum_kernel, dim3((unsigned)(a.B * a.H)), dim3(256), 0, stream, a.dlog_decay, (const float*)dG, a.T);
     return launch_status();
   }
   if ((a.Dk > a.Dv ? a.Dk : a.Dv) >= 256)
@@ -448,7 +468,7 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
     hipLaunchKernelGGL(group_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, (__bf16*)a.dk, (const float*)dkh, a.v_scale, a.H, a.Hk,
                        a.T, a.Dk, 1, n4, np, piece_stride);
   }
-  hipLaunchKernelGGL(suffix_sum_kernel, dim3((unsigned)(a.B * a.H)), dim3(256), 0, stream, a.dlog_decay, (const float*)dG, a.T);
+  if (a.wants_decay) hipLaunchKernelGGL(suffix_sum_kernel, dim3((unsigned)(a.B * a.H)), dim3(256), 0, stream, a.dlog_decay, (const float*)dG, a.T);
   return launch_status();
 }
 

@@ -32,6 +32,9 @@ struct LinArgs {
   // (fp32) by p * piece_o elements; the caller adds the pieces' outputs up.
   int n_pieces;
   int64_t piece_qk, piece_o;
+  // o_add (general addressing and the pipelined chunk loop only, bf16 outputs; null: none): fp32 [B,H,T,Dv], in the rows' own order where
+  // rev_o says so, added to the outputs before they are rounded (the last piece of a contraction takes in the earlier ones).
+  const float* o_add;
   float* ws_state;
   float* ws_decay;
   int ws_entering;   // ws_state holds, in slot s, the state that segment s + 1 is entered with (linear_states_kernel), not the one segment s ends in

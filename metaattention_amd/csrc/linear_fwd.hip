@@ -568,6 +568,25 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
     };
 
     f32x16 o_out;         // outputs of chunk c - 1, written while chunk c is under way: nobody waits for the stores
+    // What is added to a chunk's outputs (o_add) is asked for when they are there and the state loop's operand registers are free
+    // again, and waited for where they are written, behind the next chunk's first reads.
+    f32x4 add[4];
+    const bool adds = GEN && !HELP && a.o_add != nullptr;
+    auto load_add = [&](int t0) {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int r = ln & 31, g = ln >> 5, t = min(t0 + r, Tn - 1);
+      const float* src = a.o_add + ((int64_t)bh * Tn + (rev_o ? Tn - 1 - t : t)) * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH) + 4 * g;
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) add[q4] = *(const f32x4*)(src + 8 * q4);
+    };
+    auto finish = [&](int t0, uint32_t vbase) {
+      if (adds) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) o_out[j] += add[j >> 2][j & 3];
+      }
+      write_out(o_out, t0, vbase);
+    };
     // a state wave's work of chunk c
     auto run_chunk = [&](int c, int buf) {
       const int t0 = c * L;
@@ -601,7 +620,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       f32x4 w4[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) w4[i] = lds_read<f32x4>(sh + kScalW + 16 * g + 32 * i);
-      if (!HELP && c > c_begin) write_out(o_out, t0 - L, vbase);
+      if (!HELP && c > c_begin) finish(t0 - L, vbase);
 
       const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       f32x16 o_intra = E::mfma32(vf[0], pf0, zero16);
@@ -691,7 +710,14 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       }
       // chunk c + 2 must be there for P^T of c + 2, made in c + 1: with four stages it was asked for a chunk ago and the loads of this
       // chunk may go on; with three, its V, not read before c + 2, may
+      if (adds) {
+        load_add(t0);
+      } else {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) add[q4] = f32x4{0.f, 0.f, 0.f, 0.f};     // (not carried through the chunk)
+      }
       if (loads && !whole) wait_dma();
+      else if (adds) wait_vm<NLV + 4>();
       else wait_vm<HELP ? NL : NLV>();
     };
     // a helper's: scalars' loads of chunk c + 3, outputs of c - 1, P^T of c + 1 or scalars of c + 2
@@ -715,7 +741,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
         __syncthreads();
         buf = buf == NST - 1 ? 0 : buf + 1;
       }
-      if (!HELP && c_begin < c_end) write_out(o_out, (c_end - 1) * L, lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE + 2 * QT);
+      if (!HELP && c_begin < c_end) finish((c_end - 1) * L, lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE + 2 * QT);
     }
   }
   if constexpr (!PIPE) {
@@ -1084,7 +1110,7 @@ struct Config {
   // general operand addressing: defaults for what is left at zero; the row distances must be multiples of the tile
   // rows (the kernel XORs the swizzle of an instruction's first row onto the finished lane offset)
   static bool general(const LinArgs& a) {
-    return a.rev != 0 || a.q_row != 0 || a.k_row != 0 || a.v_row != 0 || (a.Hv != 0 && a.Hv != a.H) || a.qk_cols != 0 || a.n_pieces > 1 || a.rev_o != 0;
+    return a.rev != 0 || a.q_row != 0 || a.k_row != 0 || a.v_row != 0 || (a.Hv != 0 && a.Hv != a.H) || a.qk_cols != 0 || a.n_pieces > 1 || a.rev_o != 0 || a.o_add != nullptr;
   }
   static int fill(LinArgs& a) {
     a.dv_blocks = a.Dv / (32 * NWH);
@@ -1096,6 +1122,7 @@ struct Config {
     if (a.qk_cols < 0 || a.qk_cols > DK || a.qk_cols % 32 != 0) return -2;
     if (HG > 1 && a.Hv != a.H) return -2;
     if (a.n_pieces > 1 && !a.out_f32) return -2;
+    if (a.o_add && (!pipelined<NWH, HG, 0>() || helpers<DK, NWH, HG, 0>() > 0 || a.out_f32)) return -2;
     return 0;
   }
 

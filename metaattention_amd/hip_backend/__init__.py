@@ -28,6 +28,7 @@ MA_MASK_NONE, MA_MASK_CAUSAL = 0, 1
 EXPORTED_SYMBOLS = (
     "ma_version", "ma_last_error", "ma_attn_workspace_bytes", "ma_attn_fwd", "ma_attn_bwd_workspace_bytes", "ma_attn_bwd",
     "ma_linear_workspace_bytes", "ma_linear_fwd", "ma_linear_bwd_workspace_bytes", "ma_linear_bwd",
+    "ma_linear_bwd_qkv_workspace_bytes", "ma_linear_bwd_qkv",
     "ma_mla_choose_split", "ma_mla_workspace_bytes", "ma_mla_decode", "ma_mla_num_sm_parts", "ma_mla_get_metadata",
     "ma_mla_noalloc_max_workspace", "ma_mla_decode_noalloc",
 )
@@ -164,6 +165,10 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.ma_linear_bwd_workspace_bytes.restype = c_size_t
     lib.ma_linear_bwd.argtypes = [POINTER(LinearBwdParams), c_void_p]
     lib.ma_linear_bwd.restype = c_int
+    lib.ma_linear_bwd_qkv_workspace_bytes.argtypes = [POINTER(LinearBwdParams)]
+    lib.ma_linear_bwd_qkv_workspace_bytes.restype = c_size_t
+    lib.ma_linear_bwd_qkv.argtypes = [POINTER(LinearBwdParams), c_void_p]
+    lib.ma_linear_bwd_qkv.restype = c_int
     lib.ma_mla_choose_split.argtypes = [POINTER(MlaParams)]
     lib.ma_mla_choose_split.restype = c_int
     lib.ma_mla_workspace_bytes.argtypes = [POINTER(MlaParams)]
@@ -565,11 +570,12 @@ def linear_fwd(q, k, v, log_decay, *, q_scale: float = 1.0, v_scale=None, chunk=
     return out
 
 
-def linear_bwd(q, k, v, log_decay, dout, *, q_scale: float = 1.0, v_scale=None, workspace=None):
+def linear_bwd(q, k, v, log_decay, dout, *, q_scale: float = 1.0, v_scale=None, workspace=None, with_decay: bool = True):
     """Gradients of linear_fwd with respect to q, k, v, log_decay and v_scale (None when no v_scale):
     (dq, dk, dv, dlog_decay, dv_scale) with dq, dk, dv in the tensors' dtype (the gradients of heads that share a
     q / k head summed, as LinearAttention.backward does, linear_tl.py:1300-1303) and the two per-token gradients in
-    fp32 [B,H,T].  One call of ma_linear_bwd; the workspace it needs is allocated here unless one is passed."""
+    fp32 [B,H,T].  One call of ma_linear_bwd; the workspace it needs is allocated here unless one is passed.
+    ``with_decay`` False: dlog_decay and dv_scale are not wanted (None, and ma_linear_bwd_qkv is called)."""
     _require_gpu(q, k, v, log_decay, dout, v_scale, workspace)
     B, H, T, Dv = v.shape
     Hq, Hk, Dk = q.shape[1], k.shape[1], q.shape[-1]
@@ -583,8 +589,8 @@ def linear_bwd(q, k, v, log_decay, dout, *, q_scale: float = 1.0, v_scale=None, 
         assert v_scale.shape == (B, H, T)
         vs = v_scale.to(torch.float32).contiguous()
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dld = torch.empty(B, H, T, dtype=torch.float32, device=v.device)
-    dvs = torch.empty(B, H, T, dtype=torch.float32, device=v.device) if vs is not None else None
+    dld = torch.empty(B, H, T, dtype=torch.float32, device=v.device) if with_decay else None
+    dvs = torch.empty(B, H, T, dtype=torch.float32, device=v.device) if with_decay and vs is not None else None
     p = LinearBwdParams()
     p.dtype = _dtype_code(v.dtype)
     p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v = B, H, Hq, Hk, T, Dk, Dv
@@ -592,15 +598,16 @@ def linear_bwd(q, k, v, log_decay, dout, *, q_scale: float = 1.0, v_scale=None, 
     p.log_decay = g.data_ptr()
     p.v_scale = vs.data_ptr() if vs is not None else None
     p.q_scale = float(q_scale)
-    p.dq, p.dk, p.dv, p.dlog_decay = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dld.data_ptr()
+    p.dq, p.dk, p.dv, p.dlog_decay = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dld.data_ptr() if dld is not None else None
     p.dv_scale = dvs.data_ptr() if dvs is not None else None
     lib = load_library()
-    need = lib.ma_linear_bwd_workspace_bytes(ctypes.byref(p))
+    query, call = (lib.ma_linear_bwd_workspace_bytes, lib.ma_linear_bwd) if with_decay else (lib.ma_linear_bwd_qkv_workspace_bytes, lib.ma_linear_bwd_qkv)
+    need = query(ctypes.byref(p))
     if need > 0:
         if workspace is None:
             workspace = torch.empty(need, dtype=torch.uint8, device=v.device)
         p.workspace, p.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()   # (a small one is refused by the library)
-    _check(lib.ma_linear_bwd(ctypes.byref(p), _stream()))
+    _check(call(ctypes.byref(p), _stream()))
     return dq, dk, dv, dld, dvs
 
 

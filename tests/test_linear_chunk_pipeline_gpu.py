@@ -88,3 +88,27 @@ def test_later_keys_and_decays_stay_out(layout, bad):
         o = hb.linear_fwd(q.cuda(), k2.cuda(), v.cuda(), ld2.cuda(), v_scale=vs2.cuda(), segments=1)
         torch.cuda.synchronize()
         assert torch.equal(o[:, :, :at], good[:, :, :at]), which
+
+
+@pytest.mark.parametrize("T", [1, 33, 96, 130])
+@pytest.mark.parametrize("B,Hq,H,Dk,Dv,scaled", [
+    (1, 2, 2, 256, 256, False), (2, 2, 2, 128, 128, False), (1, 2, 2, 64, 64, False), (1, 2, 2, 192, 256, False),   # one piece: the scans write dq and dk
+    (8, 16, 16, 256, 512, False), (4, 32, 32, 128, 512, False), (8, 16, 16, 256, 768, False),                       # equal pieces in turn
+    (1, 2, 2, 256, 512, False), (8, 16, 16, 192, 512, False), (1, 2, 2, 256, 320, False),                           # pieces side by side, unequal pieces
+    (2, 1, 4, 128, 64, True), (1, 2, 2, 256, 512, True),                                                            # shared heads, a value scale
+])
+def test_gradients_without_the_decays(B, Hq, H, Dk, Dv, scaled, T):
+    """dq, dk, dv of the call that leaves the decay's gradient out: the same fp32 sums, each rounded to bf16 once, in two arrangements
+    (2^-9 each against the other's value where a sum falls on the other side of a rounding edge)."""
+    hb = _hb()
+    q, k, v, ld, vs = _case(B, Hq, H, T, Dk, Dv, scaled, T + 3)
+    dout = torch.randn(B, H, T, Dv, generator=torch.Generator().manual_seed(T)).bfloat16()
+    args = [t.cuda() for t in (q, k, v, ld, dout)]
+    kw = dict(v_scale=None if vs is None else vs.cuda())
+    print(f"gradients without the decay's B{B} H{Hq}/{H} T{T} {Dk}/{Dv}", flush=True)
+    full, some = hb.linear_bwd(*args, **kw), hb.linear_bwd(*args, **kw, with_decay=False)
+    torch.cuda.synchronize()
+    assert some[3] is None and some[4] is None
+    for name, x, y in zip(("dq", "dk", "dv"), some[:3], full[:3]):
+        x, y = x.double(), y.double()
+        assert torch.isfinite(x).all() and (x - y).norm() <= 2 ** -8 * y.norm(), name
