@@ -38,9 +38,18 @@ namespace {
 enum { WF_SOFTMAX = 0, WF_SIGMOID = 1, WF_RELU = 2, WF_RETENTION = 3 };   // = MA_ATTN_* of the C interface
 }
 
+// Whether a causal kernel has a tile of zeros behind its stages (see ZERO_V).
+constexpr bool wide_zero_tile(int dqk, int dv, int family, bool causal) { return causal && family != WF_RETENTION && dqk + dv >= 512; }
+
 // NW x KVS waves: NW of them own 32 query rows each and walk every KVS-th tile of keys, KVS such streams side by side with their
 // own tile stages; at the end the streams' sums are merged through LDS.
-template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, int NW, int KVS>
+// TERMS: what a call brings beside s * scale + bias and the structural mask.  0: score terms of any kind and masks, 1: masks alone,
+// 2: nothing.  Without the code for the rest a kernel needs 30 to 40 registers less (64/64 158 -> 122: four waves on a SIMD instead of
+// three; 128/256 19 spilled -> 1) and half of its loop's branches: B2 H32 S2000 256/256 causal 246 -> 185 us, 64/64 relu 85 -> 68,
+// B1 H16 S700 128/256 causal 40 -> 25, 128/128 causal 14.9 -> 12.7.
+enum { WT_ALL = 0, WT_MASKS = 1, WT_NONE = 2 };
+
+template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, int NW, int KVS, int TERMS>
 __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad_width(DQK) + DV >= 384)) ? 1 : 2)) void attn_wide_fwd_kernel(const AttnArgs a) {
   using E = Elem<T>;
   using x8 = typename E::x8;
@@ -53,6 +62,8 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   constexpr int NIK = KTILE / 1024, NIV = VTILE / 1024;
   static_assert(CPRK >= 8 && CPRV >= 8 && DQK % 16 == 0 && DV % 64 == 0, "head size");
 
+  constexpr bool MASKED = TERMS != WT_NONE, PLAIN = TERMS != WT_ALL;
+  constexpr bool ZERO_V = wide_zero_tile(DQK, DV, FAMILY, CAUSAL);
   extern __shared__ __align__(16) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -90,11 +101,12 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   const int m_ld = min(m_lane, a.Sq - 1);
 
   x8 qf[KS];
-  {
+  auto load_q = [&]() {
     const T* qp = (const T*)a.q + (int64_t)b * a.qsb + (int64_t)m_ld * a.qss + (int64_t)h * a.qsh + 8 * g;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) qf[ks] = *(const x8*)(qp + 16 * ks);
-  }
+  };
+  if constexpr (KVS == 1) load_q();
   const char* kb = (const char*)((const T*)a.k + (int64_t)b * a.ksb + (int64_t)(h / a.kv_group) * a.ksh);
   const char* vb = (const char*)((const T*)a.v + (int64_t)b * a.vsb + (int64_t)(h / a.kv_group) * a.vsh);
   const int64_t k_row_bytes = a.kss * 2, v_row_bytes = a.vss * 2;
@@ -106,12 +118,25 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   int n_tiles = (skv + BN - 1) / BN;
   if (CAUSAL) n_tiles = min(n_tiles, (mb * BM + BM + BN - 1) / BN);
   // tiles whose block of keys is switched off for this (batch, kv head) are skipped (:57-64)
-  const uint8_t* bm_row = a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb +
+  const uint8_t* bm_row = MASKED && a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb +
                                                 (int64_t)(a.kbm_by_query_head ? h : h / a.kv_group) * a.kbm_sh + (int64_t)(mb * BM / 128) * a.kbm_sq
                                           : nullptr;
+  // (BITS: see next_tile; with 256 value columns and more the accumulators leave no registers for them, scalar ones included)
+  constexpr bool BITS = DV <= 128;
+  static_assert(BITS || KVS == 1, "");
+  const int tiles_per_block = a.kv_block / BN;
+  // this workgroup's share of the tiles
+  const int tiles_per_split = (n_tiles + a.n_split - 1) / a.n_split;
+  const int t_begin = split * tiles_per_split;
+  n_tiles = min(n_tiles, t_begin + tiles_per_split);
+  // (several streams: the first entries of the block mask are asked for before the Q rows, whose many lines stand in the way of what
+  // comes after)
+  const int first_entry = BITS && bm_row && t_begin + lane < n_tiles ? bm_row[(t_begin + lane) / tiles_per_block] : 0;
+
+  if constexpr (KVS > 1) load_q();
   // element-wise keep mask of this lane's row (any mask_mod, evaluated densely by the host: blockattn_tl.py:176-190
   // generates its code into the kernel instead); the four bytes of a lane's four consecutive keys come as one word
-  const uint8_t* em_row = a.elem_mask ? a.elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_ld * a.em_sq : nullptr;
+  const uint8_t* em_row = MASKED && a.elem_mask ? a.elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_ld * a.em_sq : nullptr;
   auto load_keep = [&](int n0, uint32_t (&kp)[4]) {
 #pragma unroll
     for (int q4 = 0; q4 < 4; q4++) {
@@ -130,9 +155,9 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   // lower.py:561-615 loads them per q tile, per kv step or as [block_M, block_N] tiles depending on their shape: here
   // one strided tensor covers all of those shapes) and terms linear in the indices; folded into the raw score as
   // extra / scale, so that everything after sees s * scale + bias + extra
-  const bool has_extra = a.add || a.slope_q || a.slope_kv;
+  const bool has_extra = !PLAIN && (a.add || a.slope_q || a.slope_kv);
   const float inv_scale = 1.f / a.scale;
-  const float sl_q = a.slope_q ? a.slope_q[h] * (float)m_ld : 0.f, sl_kv = a.slope_kv ? a.slope_kv[h] : 0.f;
+  const float sl_q = !PLAIN && a.slope_q ? a.slope_q[h] * (float)m_ld : 0.f, sl_kv = !PLAIN && a.slope_kv ? a.slope_kv[h] : 0.f;
   const int64_t add_row = (int64_t)b * a.add_sb + (int64_t)h * a.add_sh + (int64_t)m_ld * a.add_sq;
   auto load_extra = [&](int n0, float (&ex)[16]) {
 #pragma unroll
@@ -143,39 +168,63 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
       ex[jj] = e * inv_scale;
     }
   };
-  const int tiles_per_block = a.kv_block / BN;
-  // this workgroup's share of the tiles
-  const int tiles_per_split = (n_tiles + a.n_split - 1) / a.n_split;
-  const int t_begin = split * tiles_per_split;
-  n_tiles = min(n_tiles, t_begin + tiles_per_split);
+  // The block mask is read 64 tiles at a time, a tile per lane, and walked as bits: kept (entry not 0) and full (entry 2, beside an
+  // element-wise mask: that mask keeps every score of the block and is not read for it) of tiles win .. win + 63.  Read tile by tile
+  // each step began with a memory latency or two.
+  uint64_t kept = 0, full_bits = 0, mine = 0;      // mine: the lanes of this stream's tiles, the same in every 64
+  int win = t_begin;
+  static_assert(64 % KVS == 0, "a stream has the same lanes in every group of 64 tiles");
+#pragma unroll
+  for (int l = 0; l < 64; l += KVS) mine |= 1ull << l;
+  auto take_window = [&](int e, uint64_t& some, uint64_t& all) {
+    some = __ballot(e != 0);
+    all = em_row ? __ballot(e >= 2) : 0;
+  };
+  auto read_window = [&](int t0, uint64_t& some, uint64_t& all) {
+    take_window(t0 + lane < n_tiles ? bm_row[(t0 + lane) / tiles_per_block] : 0, some, all);
+  };
   auto next_tile = [&](int jt) {
-    if (bm_row)
-      while (jt < n_tiles && !bm_row[jt / tiles_per_block]) jt += KVS;
-    return jt;
+    if (!bm_row) return jt;
+    if constexpr (!BITS) {
+      while (jt < n_tiles && !bm_row[jt / tiles_per_block]) jt++;
+      return jt;
+    }
+    for (;;) {
+      if (jt >= n_tiles) return jt;
+      if (jt - win >= 64) {
+        win += 64;
+        read_window(win, kept, full_bits);
+      }
+      if (jt - win < 64) {
+        const uint64_t ahead = (kept & (mine << stream)) >> (jt - win);
+        if (ahead) return jt + (int)__builtin_ctzll(ahead);
+        jt = win + 64 + stream;
+      }
+    }
+  };
+  auto tile_full = [&](int jt) {
+    if constexpr (!BITS) return em_row && bm_row && bm_row[jt / tiles_per_block] >= 2;
+    return bm_row && ((full_bits >> (jt - win)) & 1) != 0;
   };
   // (KVS > 1) steps of the longest stream: the barriers are everybody's
-  int n_steps = 0;
-  if constexpr (KVS > 1) {
-    n_steps = (n_tiles - t_begin + KVS - 1) / KVS;
-    if (bm_row) {
-      static_assert(64 % KVS == 0, "a stream has the same lanes in every group of 64 tiles");
-      uint64_t mine = 0;
-      for (int l = 0; l < 64; l += KVS) mine |= 1ull << l;
+  int n_steps = KVS > 1 ? (n_tiles - t_begin + KVS - 1) / KVS : 0;
+  if (BITS && bm_row) {
+    take_window(first_entry, kept, full_bits);
+    if constexpr (KVS > 1) {
       int count[KVS];
+      uint64_t some = kept, all;
 #pragma unroll
-      for (int st = 0; st < KVS; st++) count[st] = 0;
-      for (int t0 = t_begin; t0 < n_tiles; t0 += 64) {
-        const uint64_t kept = __ballot(t0 + lane < n_tiles && bm_row[min(t0 + lane, n_tiles - 1) / tiles_per_block] != 0);
+      for (int st = 0; st < KVS; st++) count[st] = __popcll(some & (mine << st));
+      for (int t0 = t_begin + 64; t0 < n_tiles; t0 += 64) {
+        read_window(t0, some, all);
 #pragma unroll
-        for (int st = 0; st < KVS; st++) count[st] += __popcll(kept & (mine << st));
+        for (int st = 0; st < KVS; st++) count[st] += __popcll(some & (mine << st));
       }
       n_steps = 0;
 #pragma unroll
       for (int st = 0; st < KVS; st++) n_steps = max(n_steps, count[st]);
     }
   }
-  // (block mask entry 2, beside an element-wise mask: that mask keeps every score of the block and is not read for it)
-  auto tile_full = [&](int jt) { return em_row && bm_row && bm_row[jt / tiles_per_block] >= 2; };
 
   // DMA of one tile: each instruction moves 1 KB (1024 / row bytes tile rows); lane i fetches the
   // 16-byte chunk that belongs at physical position i of that KB.  Rows beyond the sequence are clamped
@@ -226,6 +275,10 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   const uint32_t v_row_off = (4 * g + jr) * VROW + (lane & 1) * 8;
   const int v_c0 = lc ^ swz_tile<CPRV>(4 * g + jr);
 
+  if constexpr (ZERO_V) {      // (read behind the first step's barrier)
+    static_assert(KVS == 1, "behind the one stream's stages");
+    for (uint32_t off = (uint32_t)tid * 16; off < (uint32_t)VTILE; off += 64 * NW * 16) lds_write<u32x4>(lds0 + 2 * STAGE + off, u32x4{0u, 0u, 0u, 0u});
+  }
   f32x16 o[DB];
 #pragma unroll
   for (int i = 0; i < DB; i++)
@@ -239,20 +292,18 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   x4 mk_next[4];
   uint32_t keep_next[4] = {0, 0, 0, 0};
   bool full_next = false;
-  int jt = next_tile(t_begin + stream);
+  int jt = next_tile(t_begin + stream);      // the tile of the step under way
   if (jt < n_tiles) {
     issue_tile(jt * BN, 0);
     full_next = tile_full(jt);
     if constexpr (FAMILY == WF_RETENTION) load_mask(jt * BN, mk_next);
     else if (em_row && !full_next) load_keep(jt * BN, keep_next);
   }
-
   for (int it = 0; KVS > 1 ? it < n_steps : jt < n_tiles; it++) {
     const int buf = it & 1, n0 = jt * BN;
     wait_dma();
     __syncthreads();
     if (KVS > 1 && jt >= n_tiles) continue;   // (this stream is done)
-    jt = next_tile(jt + KVS);   // from here on: the tile after this one
     x4 mk[4];
     if constexpr (FAMILY == WF_RETENTION) {
 #pragma unroll
@@ -262,6 +313,7 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
 #pragma unroll
     for (int q4 = 0; q4 < 4; q4++) keep[q4] = keep_next[q4];
     const bool full = full_next;
+    jt = next_tile(jt + KVS);   // from here on: the tile after this one
     if (jt < n_tiles) {
       full_next = tile_full(jt);
       if constexpr (FAMILY == WF_RETENTION) load_mask(jt * BN, mk_next);
@@ -269,9 +321,12 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
       issue_tile(jt * BN, buf ^ 1);
     }
     // A tile above this wave's diagonal is for the block's later waves.  (Not only work saved: its probabilities are 0, but
-    // 0 x V is NaN where V is not finite.  Retention has no diagonal of its own, see above.)
-    if (CAUSAL && FAMILY != WF_RETENTION && n0 > m_wave + 31) continue;
-    const uint32_t kbase = lds_tiles + buf * STAGE, vbase = kbase + KTILE;
+    // 0 x V is NaN where V is not finite.  Retention has no diagonal of its own, see above.)  With accumulators of 256 registers the
+    // paths that meet behind a `continue` make the compiler move them (256/256 438 registers for 328, 256/512 216 spilled ones for
+    // none), so that those waves take such a tile with V from a tile of zeros instead.
+    const bool above = CAUSAL && FAMILY != WF_RETENTION && n0 > m_wave + 31;
+    if (!ZERO_V && above) continue;
+    const uint32_t kbase = lds_tiles + buf * STAGE, vbase = ZERO_V && above ? lds0 + 2 * STAGE : kbase + KTILE;
     float ex[16];
     if constexpr (FAMILY != WF_RETENTION) {
       if (has_extra) load_extra(n0, ex);
@@ -282,7 +337,7 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
 #pragma unroll
     for (int j = 0; j < 16; j++) s[j] = 0.f;
     {
-      constexpr int AH = 2, RING = 3;
+      constexpr int AH = KVS == 1 ? 2 : DQK > 128 ? 3 : 5, RING = AH + 1;      // (several streams are few waves: further ahead)
       x8 kf[RING];
 #pragma unroll
       for (int ks = 0; ks < AH; ks++) kf[ks] = lds_read<x8>(kbase + k_row_off + (uint32_t)((k_c0 ^ (2 * ks)) << 4));
@@ -308,7 +363,7 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
 #pragma unroll
         for (int jj = 0; jj < 16; jj++) s[jj] += ex[jj];
       }
-      if (a.softcap > 0.f) {   // x -> softcap * tanh(x), x = s * scale + bias;  tanh(x) = 1 - 2 / (1 + e^(2x))
+      if (!PLAIN && a.softcap > 0.f) {   // x -> softcap * tanh(x), x = s * scale + bias;  tanh(x) = 1 - 2 / (1 + e^(2x))
 #pragma unroll
         for (int jj = 0; jj < 16; jj++) {
           const float x = s[jj] * a.scale + bias;
@@ -414,46 +469,64 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
   }
   __syncthreads();   // every wave is done with the K/V buffers: they become output staging
 
+  // Streams: each keeps DB / KVS of a row block's 32-column accumulators, hands the others to their streams through LDS and takes in
+  // theirs; the outputs go out the same way.  (Halving the streams step by step, with the last one writing all of the outputs, took
+  // two rounds of twice the data at four streams: 6100 clocks behind the last tile at 128 columns.)
+  constexpr int OWN = DB > KVS ? DB / KVS : 1, OWNERS = DB / OWN;      // (more streams than column blocks: the last ones keep none)
+  static_assert(DB % OWN == 0, "a stream's share of the columns");
   if constexpr (KVS > 1) {
-    // the upper half of the streams hand their sums to the lower half, until one is left: 16 bytes a lane, lane-major
-    constexpr int SUMS = DB * 4096, PAIR = SUMS + 512;   // per wave: the accumulators, then row_max and r_part
+    constexpr uint32_t PART = (OWNERS == KVS ? DB - OWN : DB) * 4096, ROWS = KVS * NW * PART;      // a wave's column blocks; then row_max and r_part of all
+    const uint32_t out = lds0 + wave_all * PART + lane * 16, rows = lds0 + ROWS + wave * 512 + lane * 8;
 #pragma unroll
-    for (int half = KVS / 2; half >= 1; half /= 2) {
-      const uint32_t at = lds0 + ((stream % half) * NW + wave) * PAIR + lane * 16;
-      if (stream >= half && stream < 2 * half) {
+    for (int i = 0; i < DB; i++) {
+      if (i / OWN == stream) continue;
 #pragma unroll
-        for (int i = 0; i < DB; i++)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; q4++)
-            lds_write<f32x4>(at + (4 * i + q4) * 1024, f32x4{o[i][4 * q4], o[i][4 * q4 + 1], o[i][4 * q4 + 2], o[i][4 * q4 + 3]});
-        lds_write<f32x2>(at + SUMS - lane * 8, f32x2{row_max, r_part});
-      }
-      __syncthreads();
-      if (stream < half) {
-        const f32x2 other = lds_read<f32x2>(at + SUMS - lane * 8);
-        float c_mine = 1.f, c_other = 1.f;
-        if constexpr (FAMILY == WF_SOFTMAX) {
-          const float m = fmaxf(row_max, other[0]);
-          c_mine = fast_exp2(row_max - m);
-          c_other = fast_exp2(other[0] - m);
-          row_max = m;
-        }
-        r_part = r_part * c_mine + other[1] * c_other;
-#pragma unroll
-        for (int i = 0; i < DB; i++)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; q4++) {
-            const f32x4 x = lds_read<f32x4>(at + (4 * i + q4) * 1024);
-#pragma unroll
-            for (int j = 0; j < 4; j++) o[i][4 * q4 + j] = o[i][4 * q4 + j] * c_mine + x[j] * c_other;
-          }
-      }
-      __syncthreads();
+      for (int q4 = 0; q4 < 4; q4++)
+        lds_write<f32x4>(out + (i - (OWNERS == KVS && i / OWN > stream ? OWN : 0)) * 4096 + q4 * 1024, f32x4{o[i][4 * q4], o[i][4 * q4 + 1], o[i][4 * q4 + 2], o[i][4 * q4 + 3]});
     }
-    if (stream > 0) return;
+    lds_write<f32x2>(rows + stream * (NW * 512), f32x2{row_max, r_part});
+    __syncthreads();
+    // (stream 0's blocks in front: a stream's own are the compile-time first ones from here on)
+#pragma unroll
+    for (int st = 1; st < OWNERS; st++)
+      if (stream == st)
+#pragma unroll
+        for (int i = 0; i < OWN; i++) o[i] = o[st * OWN + i];
+    auto sums_of = [&](int st) { return lds_read<f32x2>(rows + st * (NW * 512)); };
+    float m = row_max;
+    if constexpr (FAMILY == WF_SOFTMAX) {
+#pragma unroll
+      for (int st = 0; st < KVS; st++) m = fmaxf(m, sums_of(st)[0]);
+    }
+    auto coef = [&](float of) { return FAMILY == WF_SOFTMAX ? fast_exp2(of - m) : 1.f; };
+    const float c_mine = coef(row_max);
+    row_max = m;
+    r_part = 0.f;
+#pragma unroll
+    for (int st = 0; st < KVS; st++) r_part += sums_of(st)[1] * coef(sums_of(st)[0]);      // (in one order, so that every stream has the same sum)
+#pragma unroll
+    for (int i = 0; i < OWN; i++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) o[i][j] *= c_mine;
+#pragma unroll
+    for (int d = 1; d < KVS; d++) {
+      const int from = (stream + d) % KVS;
+      const float c = coef(sums_of(from)[0]);
+      const uint32_t at = lds0 + (from * NW + wave) * PART + (uint32_t)(stream >= OWNERS ? 0 : OWNERS == KVS && stream > from ? stream - 1 : stream) * (OWN * 4096) + lane * 16;
+#pragma unroll
+      for (int i = 0; i < OWN; i++)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+          const f32x4 x = lds_read<f32x4>(at + (4 * i + q4) * 1024);
+#pragma unroll
+          for (int j = 0; j < 4; j++) o[i][4 * q4 + j] += x[j] * c;
+        }
+    }
+    __syncthreads();
+    if (stream >= OWNERS) return;
   }
   float inv = 1.f;
-  float* rs_ptr = a.row_scale && g == 0 && m_lane < a.Sq ? a.row_scale + ((int64_t)b * a.H + h) * a.Sq + m_lane : nullptr;
+  float* rs_ptr = a.row_scale && g == 0 && stream == 0 && m_lane < a.Sq ? a.row_scale + ((int64_t)b * a.H + h) * a.Sq + m_lane : nullptr;
   if (a.n_split > 1) rs_ptr = g == 0 && m_lane < a.Sq ? a.lse_part + (((int64_t)b * a.n_split + split) * a.H + h) * a.Sq + m_lane : nullptr;
   if constexpr (FAMILY == WF_RETENTION) {
     const float r_tot = fmaxf(r_part + xhalf(r_part), 1.f);
@@ -480,24 +553,25 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
       return;
     }
   }
-  // ---- O: two halves of DV/2 columns through a wave-private LDS block, coalesced 16-byte stores
-  constexpr int HALF = DV / 2, OROW = HALF * 2 + 16;
-  const uint32_t ob = lds0 + wave * 32 * OROW;
-  T* obase = (T*)a.o + (int64_t)b * a.osb + (int64_t)h * a.osh;
+  // ---- O: the wave's columns (a stream's share of them) in two halves, or one where that is 32, through a wave-private LDS block;
+  //      coalesced 16-byte stores
+  constexpr int NH = OWN >= 2 ? 2 : 1, HB = OWN / NH, HALF = 32 * HB, OROW = HALF * 2 + 16;
+  const uint32_t ob = lds0 + wave_all * 32 * OROW;
+  T* obase = (T*)a.o + (int64_t)b * a.osb + (int64_t)h * a.osh + stream * (OWN * 32);
   int64_t o_row_stride = a.oss;
   if (a.n_split > 1) {
-    obase = (T*)a.o_part + ((((int64_t)b * a.n_split + split) * a.H + h) * a.Sq) * DV;
+    obase = (T*)a.o_part + ((((int64_t)b * a.n_split + split) * a.H + h) * a.Sq) * DV + stream * (OWN * 32);
     o_row_stride = DV;
   }
 #pragma unroll
-  for (int hf = 0; hf < 2; hf++) {
+  for (int hf = 0; hf < NH; hf++) {
 #pragma unroll
-    for (int dbl = 0; dbl < DB / 2; dbl++)
+    for (int dbl = 0; dbl < HB; dbl++)
 #pragma unroll
       for (int q4 = 0; q4 < 4; q4++) {
         x4 w;
 #pragma unroll
-        for (int i = 0; i < 4; i++) w[i] = (T)(o[hf * (DB / 2) + dbl][4 * q4 + i] * inv);
+        for (int i = 0; i < 4; i++) w[i] = (T)(o[hf * HB + dbl][4 * q4 + i] * inv);
         lds_write<x4>(ob + r * OROW + (32 * dbl + 8 * q4 + 4 * g) * 2, w);
       }
 #pragma unroll
@@ -511,19 +585,28 @@ __global__ __launch_bounds__(64 * NW * KVS, ((DQK + DV >= 512 || (NW == 1 && pad
 
 template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, int NW = 4, int KVS = 1>
 static int launch_wide(const AttnArgs& a, hipStream_t stream) {
-  constexpr size_t tiles = KVS * 2 * (size_t)32 * (pad_width(DQK) + DV) * 2;
-  constexpr size_t merge = KVS > 1 ? KVS / 2 * NW * (size_t)(DV * 128 + 512) : 0;
-  constexpr size_t ostage = NW * 32 * (size_t)(DV + 16);
+  constexpr size_t tiles = KVS * 2 * (size_t)32 * (pad_width(DQK) + DV) * 2 + (wide_zero_tile(DQK, DV, FAMILY, CAUSAL) ? 32 * DV * 2 : 0);
+  constexpr size_t merge = KVS > 1 ? KVS * NW * (size_t)((DV >= 32 * KVS ? DV - DV / KVS : DV) * 128 + 512) : 0;
+  constexpr int own = DV > 32 * KVS ? DV / KVS : 32;      // columns that a wave writes, in two halves where they are more than 32
+  constexpr size_t ostage = NW * KVS * 32 * (size_t)((own >= 64 ? own / 2 : own) * 2 + 16);
   constexpr size_t most = tiles > merge ? tiles : merge, lds = most > ostage ? most : ostage;
   static_assert(lds <= 160 * 1024, "LDS of a CU");
-  auto kern = attn_wide_fwd_kernel<T, DQK, DV, FAMILY, CAUSAL, NW, KVS>;
-  static std::atomic<uint64_t> lds_ok{0};
-  if (allow_lds(lds_ok, lds, kern) != 0) return -1;
   AttnArgs args = a;
   if (args.n_split < 1) args.n_split = 1;
   args.num_m_blocks = (a.Sq + 32 * NW - 1) / (32 * NW);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(args.num_m_blocks * a.B * a.H * args.n_split)), dim3(64 * NW * KVS), lds, stream, args);
-  return launch_status();
+  auto launch = [&](auto kern, std::atomic<uint64_t>& lds_ok) {
+    if (allow_lds(lds_ok, lds, kern) != 0) return -1;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(args.num_m_blocks * a.B * a.H * args.n_split)), dim3(64 * NW * KVS), lds, stream, args);
+    return launch_status();
+  };
+  static std::atomic<uint64_t> ok[3];
+  if constexpr (FAMILY != WF_RETENTION) {
+    if (!a.add && !a.slope_q && !a.slope_kv && !(a.softcap > 0.f)) {
+      if (!a.kv_block_mask && !a.elem_mask) return launch(attn_wide_fwd_kernel<T, DQK, DV, FAMILY, CAUSAL, NW, KVS, WT_NONE>, ok[WT_NONE]);
+      return launch(attn_wide_fwd_kernel<T, DQK, DV, FAMILY, CAUSAL, NW, KVS, WT_MASKS>, ok[WT_MASKS]);
+    }
+  }
+  return launch(attn_wide_fwd_kernel<T, DQK, DV, FAMILY, CAUSAL, NW, KVS, WT_ALL>, ok[WT_ALL]);
 }
 
 }  // namespace ma
