@@ -44,6 +44,15 @@ struct AttnBwdArgs {
   float* dkv_part;
 };
 
+// The fused dk / dv kernel at 64 / 64, where two of its waves share a SIMD: a workgroup of two streams of four waves takes one key
+// block, every other tile a stream, and their sums meet in LDS; heaviest blocks first under a causal mask.  With few key blocks
+// the persistent kernel of one stream (two workgroups a CU, under a causal mask pairs of key blocks) leaves SIMDs idle: it takes
+// 1.0 us a tile alone on its SIMD and 0.64 a tile in company, and a pair brings two beginnings and ends of about 5 us one after the
+// other.  Backward, one stream against two: causal, B4 H12 S600 (240 blocks) 41.5 and 33.5 us, S1024 (384) 59.2 and 51.9, B2 H32
+// S1024 (512) 64 and 61.5, B4 H32 S1000 (1024) 95 and 108 (its ends are then covered by the other workgroup); without a mask B4 H12
+// S600 33.5 and 30.5, S1024 (384) 61 and 68; a window of a third of S 41.6 and 40.4, 66 and 73.5.
+inline bool dkv_two_streams(int64_t workgroups, bool causal) { return workgroups <= (causal ? 2 : 1) * (int64_t)device_cus(); }
+
 // How many runs the steps of a key block's dk / dv are cut into (attn_bwd_kernels.h), and the bytes of partial sums that takes.
 // half: the call has a causal or another mask.
 int attn_bwd_parts(const AttnBwdArgs& a, bool half, int dqk, int dv);

@@ -29,6 +29,25 @@ int attn_bwd_parts(const AttnBwdArgs& a, bool half, int dqk, int dv) {
   const double step_us = 1.2 * (dqk + dv) / 256, sum_us = 2.0 * (double)attn_bwd_part_bytes(a, 1, dqk, dv) / 4e6;
   int best = 1;
   double best_us = 0;
+  if (dqk + dv <= 128) {
+    // two streams a workgroup and a key block each (dkv_two_streams; beyond that rule one run): 0.64 us a tile, about 4.5 a
+    // workgroup; the longest block or all of them over the CUs, in whole rounds where they weigh the same.  Backward of B1 H16 S700
+    // causal, 96 blocks: 35.5 us in one run, 38 in two, 42 in three; B1 H4 S2000 causal, 64 blocks: 71.5, 62, 58, 56.5 in four, 59 in
+    // six; H16 Hkv4: 180, 117, 95, 83, 78 in six.
+    const bool causal = half && !a.elem_mask_t && !a.q_block_mask;
+    const int64_t blocks_all = blocks * a.B * a.Hkv, most = tiles * a.kv_group;
+    if (!dkv_two_streams(blocks_all, causal)) return 1;
+    for (int n = 1; n <= 16 && (n == 1 || (most >= 4 * n && blocks_all * n <= 4 * (int64_t)cus)); n++) {
+      const double longest = 6.5 + 0.64 * (double)((most + n - 1) / n), mean = (half ? 0.5 : 1.0) * 0.64 * (double)most / n + 4.5;
+      const double rounds = causal ? (double)(blocks_all * n) / cus : (double)((blocks_all * n + cus - 1) / cus), all = 2 + mean * rounds;
+      const double us = (longest > all ? longest : all) + (n > 1 ? 4 + n * sum_us : 0);
+      if (n == 1 || us < best_us) {
+        best_us = us;
+        best = n;
+      }
+    }
+    return best;
+  }
   for (int n = 1; n <= 16 && (n == 1 || steps >= 4 * n); n++) {
     const double us = (double)((items * n + cus - 1) / cus) * ((double)((steps + n - 1) / n) + 6) * step_us + (n > 1 ? 4 + n * sum_us : 0);
     if (n == 1 || us < best_us) {

@@ -243,8 +243,11 @@ constexpr size_t dq_lds(int dqk, int dv, int family) {
 }
 
 // KVS: two streams of four waves walk every other tile each, side by side with their own stages, and their sums meet in LDS.
-template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool EXTRA = false, int KVS = 1>
-__global__ __launch_bounds__(256 * KVS, (DQK + DV >= 512 ? 1 : 2)) void attn_bwd_dq_kernel(const AttnBwdArgs a) {
+// MASKS: with the code for element-wise and tile masks.  Without it the kernel loses registers and branches of every step, and
+// 64 / 64 fits four waves on a SIMD: dq of B4 H12 S1024 64/64 sigmoid causal 29 -> 27 us; forward + backward of B2 H32 S1600 64/64 relu
+// 260 -> 228, 256/256 causal 770 -> 709, B1 H16 S700 128/256 causal 142 -> 124.
+template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool MASKS, bool EXTRA = false, int KVS = 1>
+__global__ __launch_bounds__(256 * KVS, (DQK + DV >= 512 ? 1 : DQK + DV <= 128 && !MASKS ? 4 : 2)) void attn_bwd_dq_kernel(const AttnBwdArgs a) {
   using E = Elem<T>;
   using x8 = typename E::x8;
   constexpr int BM = 128, BN = 32;
@@ -317,8 +320,9 @@ __global__ __launch_bounds__(256 * KVS, (DQK + DV >= 512 ? 1 : 2)) void attn_bwd
   // a partial last tile, or a tensor whose rows are not 16-byte aligned, is read from global memory as it is needed
   constexpr int MULT = 2 * STAGE;
   const bool mult_ok = FAMILY == BF_RETENTION && (a.sm_sq & 7) == 0 && (a.sm_sb & 7) == 0 && (a.sm_sh & 7) == 0 && ((uintptr_t)a.smask & 15) == 0;
-  const bool keep_ok = FAMILY != BF_RETENTION && a.elem_mask && ((a.em_sq | a.em_sb | a.em_sh | (int64_t)(uintptr_t)a.elem_mask) & 15) == 0;
-  const uint8_t* bm_full = a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb + (int64_t)h * a.kbm_sh + (int64_t)mb * a.kbm_sq : nullptr;
+  const uint8_t* elem_mask = MASKS ? a.elem_mask : nullptr;
+  const bool keep_ok = FAMILY != BF_RETENTION && elem_mask && ((a.em_sq | a.em_sb | a.em_sh | (int64_t)(uintptr_t)elem_mask) & 15) == 0;
+  const uint8_t* bm_full = MASKS && a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb + (int64_t)h * a.kbm_sh + (int64_t)mb * a.kbm_sq : nullptr;
   auto tile_full = [&](int jt_) { return bm_full && bm_full[jt_] >= 2; };   // the element-wise mask keeps every score of the tile
   TileDma<KROW, 4, DQK / 8> k_dma;
   TileDma<VROW, 4> v_dma;
@@ -340,7 +344,7 @@ __global__ __launch_bounds__(256 * KVS, (DQK + DV >= 512 ? 1 : 2)) void attn_bwd
       // element-wise keep mask: whole tiles of a 16-byte aligned mask come with the K/V tile (same area, 1 KB per wave and
       // stage); a tile the block mask marks as kept in full (entry 2) needs none of it
       if (keep_ok && n0 + BN <= a.Skv && m_wave < a.Sq && !tile_full(n0 / BN))
-        keep_dma(a.elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_wave * a.em_sq + n0, a.em_sq, a.Sq - m_wave,
+        keep_dma(elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_wave * a.em_sq + n0, a.em_sq, a.Sq - m_wave,
                  lds0 + MULT + (buf * 4 + wave) * 1024, lane);
     }
   };
@@ -355,10 +359,10 @@ __global__ __launch_bounds__(256 * KVS, (DQK + DV >= 512 ? 1 : 2)) void attn_bwd
   lse2 = c_bias - lse2;   // what the row function adds to s * c_scale
 
   // element-wise keep mask of this lane's query row
-  const uint8_t* em_row = a.elem_mask ? a.elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_ld * a.em_sq : nullptr;
+  const uint8_t* em_row = elem_mask ? elem_mask + (int64_t)b * a.em_sb + (int64_t)h * a.em_sh + (int64_t)m_ld * a.em_sq : nullptr;
 
   // tiles in which the mask keeps nothing for this workgroup's rows are never fetched
-  const uint8_t* bm_row = a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb + (int64_t)h * a.kbm_sh + (int64_t)mb * a.kbm_sq : nullptr;
+  const uint8_t* bm_row = MASKS && a.kv_block_mask ? a.kv_block_mask + (int64_t)b * a.kbm_sb + (int64_t)h * a.kbm_sh + (int64_t)mb * a.kbm_sq : nullptr;
   auto next_tile = [&](int jt) {
     if (bm_row)
       while (jt < n_tiles && !bm_row[jt]) jt++;
@@ -842,9 +846,11 @@ struct PhaseF {
   static constexpr bool is_s(int j) { return j < 2 * KMIN ? j % 2 == 0 : KS > VS; }
   static constexpr int slice(int j) { return j < 2 * KMIN ? j / 2 : KMIN + (j - 2 * KMIN); }
 };
+// STREAMS 2 (64 / 64, see dkv_two_streams): two streams of four waves walk every other tile of the workgroup's steps each, with
+// stages of their own, as two runs would; at the end one keeps dk and the other dv, and each hands the other one over through LDS.
 // PARTS: n_parts > 1 (an instantiation of its own: the walk over a run's tiles costs the one-run loop 3 % at 64 / 64).
-template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool MASKS, bool PARTS>
-__global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused_kernel(const AttnBwdArgs a) {
+template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool MASKS, bool PARTS, int STREAMS = 1>
+__global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused_kernel(const AttnBwdArgs a) {
   using E = Elem<T>;
   using x8 = typename E::x8;
   using x4 = typename E::x4;
@@ -858,6 +864,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
   constexpr int NST = MASKS ? 4 : fused_stages(pad_width(DQK), DV), LA = NST == 8 ? 4 : 3, ROWVALS = NST * STAGE;
   // (MASKS) behind the row values: 1 KB of mask bytes per stage and wave, then the step list and its length
   constexpr int KEEP = ROWVALS + NST * 512, LIST = KEEP + NST * 4 * 1024, LIST_N = LIST + FUSED_LIST_MAX * 4;
+  constexpr int STREAM_LDS = (MASKS ? LIST_N + 4 : ROWVALS + NST * 512) + 1023 & ~1023;
   // the MFMAs of a step and the fragment ring
   constexpr int NF = KS + VS, NV = 2 * VB, NK = 2 * QB, NTOT = NF + NV + NK;
   constexpr int RING = 8, AH = !ROWS_AHEAD && FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
@@ -865,21 +872,31 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
   using PhF = PhaseF<KS, VS>;
 
   extern __shared__ __align__(16) char smem[];
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr bool WALK = PARTS || STREAMS > 1;
+  static_assert(STREAMS == 1 || (STREAMS == 2 && !ROWS_AHEAD), "two streams share a SIMD");
+  const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int stream = STREAMS > 1 ? wave_all >> 2 : 0, wave = STREAMS > 1 ? wave_all & 3 : wave_all;   // wave: within its stream
+  const uint32_t lds_all = (uint32_t)(uintptr_t)(MA_LDS char*)smem, lds0 = lds_all + (STREAMS > 1 ? stream * (uint32_t)STREAM_LDS : 0u);
   const int r = lane & 31, g = lane >> 5;
 
-  // Persistent: the grid is one workgroup per CU, and every workgroup walks items  item = blockIdx.x, + gridDim.x, ...  An
+  // STREAMS 2: an item, a workgroup of its own, is one key block (or a run of it).
+  // STREAMS 1 is persistent: the grid is one workgroup per CU, and every workgroup walks items  item = blockIdx.x, + gridDim.x, ...  An
   // item is a (batch, kv head) and, under a causal mask, the PAIR of key blocks (k, n - 1 - k), which together see the
   // same number of query tiles whatever k is: every item weighs the same.  Items that follow each other on an XCD
   // (item % 8) belong to the same (batch, kv head) pairs, whose Q and dO tiles then come from that XCD's L2.
   const int nnb = a.num_blocks, BHK = a.B * a.Hkv, n_parts = PARTS ? a.n_parts : 1;
   // With n_parts > 1 an item is one of the n_parts runs of each block's steps, whose fp32 sums go to the workspace
   // (attn_bwd_dkv_reduce_kernel adds the runs up).
-  const int per_bh = (CAUSAL ? (nnb + 1) / 2 : nnb) * n_parts, n_items = BHK * per_bh;
+  const int per_bh = (CAUSAL && STREAMS == 1 ? (nnb + 1) / 2 : nnb) * n_parts, n_items = BHK * per_bh;
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
   int bhk, ki, run;
-  if ((BHK & 7) == 0) {
+  if (STREAMS > 1) {
+    // the heaviest blocks of all heads first
+    const int xcds = (BHK & 7) == 0 ? 8 : 1, slot = item / xcds, heads = BHK / xcds;
+    run = slot % n_parts;
+    bhk = (slot / n_parts) % heads * xcds + item % xcds;
+    ki = slot / (n_parts * heads);
+  } else if ((BHK & 7) == 0) {
     const int slot = item >> 3;
     bhk = (slot / per_bh) * 8 + (item & 7);
     ki = slot % per_bh;
@@ -896,7 +913,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
     if (!CAUSAL) ki = (ki + bhk) % nnb;
   }
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
-  for (int part = 0; part < (CAUSAL && ki != nnb - 1 - ki ? 2 : 1); part++) {
+  for (int part = 0; part < (STREAMS == 1 && CAUSAL && ki != nnb - 1 - ki ? 2 : 1); part++) {
   const int nb = part == 0 ? ki : nnb - 1 - ki;
   const int n_wave = nb * BNW + wave * 32, n_lane = n_wave + r;
   const int n_ld = min(n_lane, a.Skv - 1);
@@ -928,13 +945,24 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
   const int t_count = (a.Sq + BMT - 1) / BMT - t_first;
   int n_steps = t_count > 0 ? t_count * a.kv_group : 0;
   DkvWalk first{0, 0, 0};
-  if (PARTS && !MASKS && n_steps > 0) {
-    first.skip = ((run - t_first) % n_parts + n_parts) % n_parts;
-    n_steps = 0;
-    const int each = t_count / n_parts, more = t_count % n_parts;
-    for (int hg = 0, skip = first.skip; hg < a.kv_group; hg++, skip = skip == 0 ? n_parts - 1 : skip - 1) n_steps += each + (skip < more ? 1 : 0);
-    first.to_tile(first.skip, n_parts, t_count, a.kv_group);
+  // (the streams of a workgroup are runs side by side, whose sums meet in LDS)
+  const int n_runs = n_parts * STREAMS;
+  int n_bodies = 0;      // (STREAMS > 1) steps of the longer stream: the barriers are everybody's
+  if (WALK && !MASKS && n_steps > 0) {
+    const int each = t_count / n_runs, more = t_count % n_runs;
+    auto steps_of = [&](int skip) {
+      int n = 0;
+      for (int hg = 0; hg < a.kv_group; hg++, skip = skip == 0 ? n_runs - 1 : skip - 1) n += each + (skip < more ? 1 : 0);
+      return n;
+    };
+    const int mine = run * STREAMS + stream;
+    auto skip_of = [&](int any_run) { return ((any_run - t_first) % n_runs + n_runs) % n_runs; };
+    first.skip = skip_of(mine);
+    n_steps = steps_of(first.skip);
+    if (STREAMS > 1) n_bodies = max(n_steps, steps_of(skip_of(mine ^ 1)));
+    first.to_tile(first.skip, n_runs, t_count, a.kv_group);
   }
+  if (STREAMS == 1) n_bodies = n_steps;
   const bool keep_ok = MASKS && a.elem_mask_t && ((a.emt_sk | a.emt_sb | a.emt_sh | (int64_t)(uintptr_t)a.elem_mask_t) & 15) == 0;
   if constexpr (MASKS) {
     // the step list: entry = tile | head of the group << 16 | kept in full << 31
@@ -948,7 +976,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
         if (i < n_steps) {
           const int hg = i / t_count, t = i - hg * t_count;
           const uint8_t e = qbm ? qbm[(int64_t)(hk * a.kv_group + hg) * a.qbm_sh + t_first + t] : (uint8_t)1;
-          keep = e != 0 && (!PARTS || (t_first + t + hg) % n_parts == run);
+          keep = e != 0 && (!WALK || (t_first + t + hg) % n_runs == run * STREAMS + stream);
           entry = (uint32_t)t | ((uint32_t)hg << 16) | (e >= 2 || !a.elem_mask_t ? 0x80000000u : 0u);
         }
         const uint64_t votes = __ballot(keep);
@@ -959,6 +987,8 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
     }
     __syncthreads();
     n_steps = __builtin_amdgcn_readfirstlane((int)lds_read<uint32_t>(lds0 + LIST_N));
+    n_bodies = n_steps;
+    if (STREAMS > 1) n_bodies = max(n_steps, __builtin_amdgcn_readfirstlane((int)lds_read<uint32_t>(lds_all + (stream ^ 1) * (uint32_t)STREAM_LDS + LIST_N)));
   }
   // (list entries are requested a step before they are used and made wave-uniform only then: a read that is waited for
   // at once would drain the ring of operand fragments)
@@ -1044,7 +1074,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
     }
   };
 
-  if (n_steps > 0) {
+  if (n_bodies > 0) {
     // the next tile to fetch
     DkvWalk fetch = first, at = first;   // (without MASKS) the next tile to fetch, the current step's
     int i_n = 0;
@@ -1058,7 +1088,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
       } else {
         issue_tile(fetch.hg, fetch.t, i_n & (NST - 1));
         i_n++;
-        fetch.template next<PARTS>(n_parts, t_count, a.kv_group);
+        fetch.template next<WALK>(n_runs, t_count, a.kv_group);
       }
     };
 #pragma unroll
@@ -1066,6 +1096,10 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
       if (i_n < n_steps) issue_next();
     // (the padding step of an odd number of steps evaluates S, dP, lse and delta of the stage behind the last tile's:
     // where no earlier tile has been there, tile 0 goes there, so that what it computes is finite)
+    if constexpr (STREAMS > 1) {
+      // (here one for every step that the other stream has more, and a stream may have none at all: tile 0 of the group's first head)
+      for (int i = n_steps; i < ((n_bodies + 1) & ~1) && i < NST; i++) issue_tile(0, 0, i);
+    } else {
     if ((n_steps & 1) && n_steps < NST) {
       if constexpr (MASKS) {
         const uint32_t e = uniform(list_request(0));
@@ -1073,6 +1107,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
       } else {
         issue_tile(first.hg, first.t, n_steps);
       }
+    }
     }
     wait_dma();
     __syncthreads();
@@ -1089,11 +1124,11 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
       const bool real = u < n_steps;                 // (the padding step: the last tile once more, everything masked)
       const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
       if constexpr (MASKS) c_next = list_request(u + 1);
-      const uint32_t cur_tile = lds0 + (uint32_t)(((real ? u : n_steps - 1) & (NST - 1)) * STAGE);
+      const uint32_t cur_tile = lds0 + (uint32_t)(((real ? u : max(n_steps, 1) - 1) & (NST - 1)) * STAGE);
       const uint32_t nxt_tile = lds0 + (uint32_t)(((u + 1) & (NST - 1)) * STAGE);
       const uint32_t nn_tile = lds0 + (uint32_t)(((u + 2) & (NST - 1)) * STAGE);
       const int m0 = real ? (t_first + (MASKS ? (int)(c_entry & 0xffffu) : at.t)) * BMT : a.Sq;
-      if (!MASKS) at.template next<PARTS>(n_parts, t_count, a.kv_group);
+      if (!MASKS) at.template next<WALK>(n_runs, t_count, a.kv_group);
       if (ROWS_AHEAD) rowvals((u + 1) & (NST - 1), nxt);   // (requested here, needed in the next step)
       else row_lse(u & (NST - 1), cur);
       // the tiles that touch the diagonal, an end of the sequences or an element-wise mask (the test is wave-uniform)
@@ -1174,7 +1209,7 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
         __builtin_amdgcn_sched_barrier(0);
       });
     };
-    for (int u = 0; u < n_steps; u += 2) {
+    for (int u = 0; u < n_bodies; u += 2) {
       body(u, ra, rb);
       body(u + 1, rb, ra);
     }
@@ -1182,6 +1217,40 @@ __global__ __launch_bounds__(256, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused
   wait_dma();
   __syncthreads();   // every wave is done with the tiles: they become output staging
 
+  if constexpr (STREAMS > 1) {
+    // stream 0 keeps dk and stream 1 dv: each hands the other one over, 16 bytes a lane, lane-major
+    static_assert(QB == VB && 8 * QB * 4096 <= STREAMS * STREAM_LDS, "LDS of the sums");
+    const uint32_t out = lds_all + wave_all * (QB * 4096) + lane * 16, in = lds_all + (wave_all ^ 4) * (QB * 4096);
+#pragma unroll
+    for (int i = 0; i < QB; i++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        const f32x16& x = stream == 0 ? dv[i] : dk[i];
+        lds_write<f32x4>(out + (i * 4 + q4) * 1024, f32x4{x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]});
+      }
+    __syncthreads();
+    if (stream == 1) {
+#pragma unroll
+      for (int i = 0; i < QB; i++) dk[i] = dv[i];
+    }
+#pragma unroll
+    for (int i = 0; i < QB; i++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        const f32x4 x = lds_read<f32x4>(in + lane * 16 + (i * 4 + q4) * 1024);
+#pragma unroll
+        for (int j = 0; j < 4; j++) dk[i][4 * q4 + j] += x[j];      // (from here on a stream's own output)
+      }
+    if constexpr (PARTS) {
+      partial_store<QB>(dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4 + (stream == 0 ? 0 : 32 * DQK), dk);
+    } else {
+      // (staged where only this wave has read)
+      T* base = stream == 0 ? (T*)a.dk + (int64_t)b * a.dksb + (int64_t)hk * a.dksh : (T*)a.dv + (int64_t)b * a.dvsb + (int64_t)hk * a.dvsh;
+      store_rows<T, DQK>(dk, stream == 0 ? a.scale : 1.f, in, base, stream == 0 ? a.dkss : a.dvss, n_wave, a.Skv, lane);
+    }
+    __syncthreads();   // the sums have left the stages: the next key block's tiles may arrive
+    continue;
+  }
   if constexpr (PARTS) {
     float* to = dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4;
     partial_store<QB>(to, dk);
@@ -1252,7 +1321,10 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   constexpr int DMAX = DQK > DV ? DQK : DV;
   constexpr size_t ostage = 4 * 32 * (size_t)(DMAX + 16);
   constexpr size_t lds = dq_lds(DQK, DV, FAMILY);
-  auto k1 = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL>;
+  constexpr bool NOT_RETENTION = FAMILY != BF_RETENTION;      // (which takes no masks)
+  const bool masked = a.elem_mask || a.kv_block_mask;
+  auto k1 = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, false>;
+  auto k1m = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, NOT_RETENTION>;
   // one dk/dv launch where both accumulators fit beside a second wave, else one launch each (at 256 / 256 the single launch
   // held both 128-register accumulators in a 512-register wave and spilled 170 registers: the whole backward at B4 H16 S4096
   // took 9.7 ms under the causal mask and 6.2 ms without; with one launch each 3.3 ms and 4.8 ms)
@@ -1260,14 +1332,14 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   auto k2 = attn_bwd_dkv_kernel<T, DQK, DV, FAMILY, CAUSAL, SPLIT ? 1 : 3>;
   auto k3 = attn_bwd_dkv_kernel<T, DQK, DV, FAMILY, CAUSAL, 2>;
   static std::atomic<uint64_t> lds_ok{0};
-  if (allow_lds(lds_ok, lds, k1, k2, k3) != 0) return -1;
+  if (allow_lds(lds_ok, lds, k1, k1m, k2, k3) != 0) return -1;
   AttnBwdArgs args = a;
   if (a.add || a.slope_q || a.slope_kv || a.softcap != 0.f) {
     // additive score terms / soft-capping: instantiations of their own (not for the retention family, whose score function
     // is the multiplier tensor; soft-capping goes with softmax only, as in the forward), dk and dv by the two-launch kernels
     if constexpr (FAMILY != BF_RETENTION) {
       if (a.softcap != 0.f && FAMILY != BF_SOFTMAX) return -2;
-      auto e1 = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, true>;
+      auto e1 = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, true, true>;
       auto e2 = attn_bwd_dkv_kernel<T, DQK, DV, FAMILY, CAUSAL, SPLIT ? 1 : 3, true>;
       auto e3 = attn_bwd_dkv_kernel<T, DQK, DV, FAMILY, CAUSAL, 2, true>;
       static std::atomic<uint64_t> elds_ok{0};
@@ -1286,14 +1358,15 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   bool dq_done = false;
   if constexpr (FAMILY != BF_RETENTION && DQK + DV <= 320) {   // (128 / 256: measured no faster)
     if (dq_two_streams(args.num_blocks * (int64_t)a.B * a.H, CAUSAL)) {
-      auto k1s = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, false, 2>;
+      auto k1s = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false, 2>;
+      auto k1sm = attn_bwd_dq_kernel<T, DQK, DV, FAMILY, CAUSAL, true, false, 2>;
       static std::atomic<uint64_t> slds_ok{0};
-      if (allow_lds(slds_ok, 2 * lds, k1s) != 0) return -1;
-      hipLaunchKernelGGL(k1s, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(512), 2 * lds, stream, args);
+      if (allow_lds(slds_ok, 2 * lds, k1s, k1sm) != 0) return -1;
+      hipLaunchKernelGGL(masked ? k1sm : k1s, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(512), 2 * lds, stream, args);
       dq_done = true;
     }
   }
-  if (!dq_done) hipLaunchKernelGGL(k1, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(256), lds, stream, args);
+  if (!dq_done) hipLaunchKernelGGL(masked ? k1m : k1, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(256), lds, stream, args);
   args.num_blocks = (a.Skv + 127) / 128;
   // (128 / 256 would fit the fused kernel's registers only with 60-90 spilled: measured no faster than its two launches)
   if constexpr (FAMILY != BF_RETENTION && (DQK + DV <= 256 || (DQK == 192 && DV == 128))) {
@@ -1305,18 +1378,37 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
       constexpr size_t fmax = ftiles > mtiles ? ftiles : mtiles, flds = fmax > ostage ? fmax : ostage;
       if (!a.dkv_part) args.n_parts = 1;
       const bool parts = args.n_parts > 1;
-      auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
-      auto kfp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, true>;
-      auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false>;   // (masks go with MA_MASK_NONE)
-      auto kmp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, true>;
-      if (CAUSAL && masks) return -2;
-      static std::atomic<uint64_t> flds_ok{0};
-      if (allow_lds(flds_ok, flds, kf, kfp, km, kmp) != 0) return -1;
-      const int cus = device_cus();
-      if (cus <= 0) return -1;
-      const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
-      const int slots = cus * fused_per_cu(DQK, DV);
-      hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
+      if (CAUSAL && masks) return -2;   // (masks go with MA_MASK_NONE)
+      const int64_t workgroups = (int64_t)args.num_blocks * a.B * a.Hkv * args.n_parts;
+      constexpr bool TWO = fused_per_cu(DQK, DV) == 2;
+      bool launched = false;
+      if constexpr (TWO) {
+        if (parts || dkv_two_streams(workgroups, CAUSAL)) {
+          auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false, 2>;
+          auto kfp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, true, 2>;
+          auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false, 2>;
+          auto kmp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, true, 2>;
+          constexpr size_t slds = 2 * ((flds + 1023) & ~(size_t)1023);
+          static std::atomic<uint64_t> slds_ok{0};
+          if (allow_lds(slds_ok, slds, kf, kfp, km, kmp) != 0) return -1;
+          hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)workgroups), dim3(512), slds, stream, args);
+          launched = true;
+        }
+      }
+      if (!launched) {
+        constexpr bool RUNS = !TWO;      // (at 64 / 64 several runs are always two streams a workgroup)
+        auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
+        auto kfp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, RUNS>;
+        auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false>;
+        auto kmp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, RUNS>;
+        static std::atomic<uint64_t> flds_ok{0};
+        if (allow_lds(flds_ok, flds, kf, kfp, km, kmp) != 0) return -1;
+        const int cus = device_cus();
+        if (cus <= 0) return -1;
+        const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
+        const int slots = cus * fused_per_cu(DQK, DV);
+        hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
+      }
       if (parts) {
         const dim3 grid((unsigned)(args.num_blocks * a.B * a.Hkv), 2);
         hipLaunchKernelGGL((attn_bwd_dkv_reduce_kernel<T, DQK, DV>), grid, dim3(256), 0, stream, args);
