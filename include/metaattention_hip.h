@@ -291,6 +291,11 @@ int ma_attn_bwd(const ma_attn_bwd_params* p, ma_stream_t stream);
 /* linear_tl.py:1240-1269 */
 size_t ma_linear_workspace_bytes(const ma_linear_params* p);
 int ma_linear_fwd(const ma_linear_params* p, ma_stream_t stream);
+/* The same with what the decay_mod and v_mod of an operator do in front of it: log_decay holds the decay itself where decay_is_exp is
+ * not 0 (its logarithm is taken), the log decay over decay_head[h] where decay_head (fp32 [H]) is not NULL; v_scale is fp32
+ * (MA_LINEAR_FP32) or bf16 (MA_BF16).  dim_k 128 and 256. */
+#define MA_LINEAR_FP32 (-1)
+int ma_linear_fwd_factors(const ma_linear_params* p, int32_t decay_is_exp, const float* decay_head, int32_t v_scale_dtype, ma_stream_t stream);
 
 /* linear_tl.py:1268-1340 */
 size_t ma_linear_bwd_workspace_bytes(const ma_linear_bwd_params* p);

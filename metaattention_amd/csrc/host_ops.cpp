@@ -380,7 +380,9 @@ void linear_sizes(const Tensor& q, const Tensor& k, const Tensor& v, int32_t& B,
 // fp32, contiguous, the heads and tokens as they are: what the kernels take per-token factors as
 Tensor per_token(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
 
-bool linear_forward(const LinearPlan& pl, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& vs, int dev, Tensor& out) {
+// g: the log decay, or what the kernel makes it from (decay_kind); vs: fp32 or bf16
+bool linear_forward(const LinearPlan& pl, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& vs, int dev, Tensor& out,
+                    int decay_kind = DECAY_AS_IS, const float* decay_head = nullptr) {
   out = empty(v.sizes(), v.scalar_type(), v.device());
   ma_linear_params p{};
   p.dtype = MA_BF16;
@@ -388,13 +390,14 @@ bool linear_forward(const LinearPlan& pl, const Tensor& q, const Tensor& k, cons
   p.q = q.data_ptr(); p.k = k.data_ptr(); p.v = v.data_ptr(); p.o = out.data_ptr();
   p.log_decay = (const float*)g.data_ptr();
   p.v_scale = vs.defined() ? (const float*)vs.data_ptr() : nullptr;
+  const int32_t vs_dtype = vs.defined() && vs.scalar_type() == at::kBFloat16 ? MA_BF16 : MA_LINEAR_FP32;
   p.q_scale = pl.q_scale;
   const size_t need = ma_linear_workspace_bytes(&p);
   const c10::DataPtr ws = scratch(need);
   p.workspace = ws.get(); p.workspace_bytes = need;
   const ma_stream_t st = stream_of(dev);
   NoGil release;
-  return ma_linear_fwd(&p, st) == MA_OK;
+  return ma_linear_fwd_factors(&p, decay_kind == DECAY_LOG, decay_head, vs_dtype, st) == MA_OK;
 }
 
 // The chunked operator with gradients for q, k, v, the log decay and the value scale (if any), as LinearAttention.backward
@@ -461,11 +464,27 @@ PyObject* linear_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   const int64_t B = v.size(0), H = v.size(1), T = v.size(2);
   if (q.size(0) != B || k.size(0) != B || q.size(2) != T || k.size(2) != T || q.size(3) != k.size(3) || B > (1 << 30) || H > (1 << 30) || T > (1 << 30)) return none();
   if (decay.dim() != 3 || decay.size(0) != B || decay.size(1) != H || decay.size(2) != T) return none();
-  Tensor g = decay.to(at::kFloat), vs;
+  Tensor vs;
   if (pl.v_scale_arg >= 0) {
     vs = *t[4 + pl.v_scale_arg];
     if (vs.dim() != 3 || vs.size(0) != B || vs.size(1) != H || vs.size(2) != T) return none();
   }
+  // Without gradients the kernel takes the decay, a head's factor and a bf16 value scale as they are (a launch less each)
+  bool wanted = false;
+  for (int i = 0; i < n; i++) wanted = wanted || t[i]->requires_grad();
+  if (!(wanted && at::GradMode::is_enabled())) {
+    const Tensor* head = pl.decay_kind == DECAY_MUL_HEAD ? t[4 + pl.decay_head_arg] : nullptr;
+    const bool plain = (q.size(3) == 128 || q.size(3) == 256) && decay.scalar_type() == at::kFloat && decay.layout() == at::kStrided && decay.is_contiguous() &&
+                       (!vs.defined() || ((vs.scalar_type() == at::kFloat || vs.scalar_type() == at::kBFloat16) && vs.is_contiguous())) &&
+                       (!head || (head->scalar_type() == at::kFloat && head->is_contiguous() && head->numel() == H));
+    if (plain) {
+      Tensor out;
+      at::AutoDispatchBelowADInplaceOrView no_autograd;
+      if (!linear_forward(pl, q, k, v, decay, vs, dev, out, pl.decay_kind, head ? (const float*)head->data_ptr() : nullptr)) return none();
+      return THPVariable_Wrap(out);
+    }
+  }
+  Tensor g = decay.to(at::kFloat);
   if (pl.decay_kind == DECAY_LOG) {
     g = g.log();
   } else if (pl.decay_kind == DECAY_MUL_HEAD) {

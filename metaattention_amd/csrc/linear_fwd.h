@@ -7,7 +7,7 @@ namespace ma {
 struct LinArgs {
   const void* q; const void* k; const void* v; void* o;
   const float* log_decay;  // [B,H,T]
-  const float* v_scale;    // [B,H,T] or null
+  const float* v_scale;    // [B,H,T] or null (v_scale_bf16: bf16)
   float q_scale;
   int B, H, Hq, Hk, T, Dv, dv_blocks;
   // sequence segments (see linear_fwd.hip): nseg segments of seg_chunks 32-token chunks; local end
@@ -41,6 +41,10 @@ struct LinArgs {
   // head-group range of this launch (a workgroup handles head group bg0 + its own index; bg_n groups in all; bg_n = 0: every
   // group, from 0).  The workspace of a launch with sequence segments is indexed by the launch's own group index.
   int bg0, bg_n;
+  // (not with general addressing) what log_decay holds where it is not the log decay itself: its exponential (decay_log), or the log decay over a head's factor
+  // (decay_head [H] or null)
+  int v_scale_bf16, decay_log;
+  const float* decay_head;
 };
 
 // Scans that go out in one launch (general addressing): scan i is blockIdx.y = i.

@@ -173,7 +173,21 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
   const int64_t v_head_bytes = (int64_t)Tn * v_row_bytes;
   T* ob = (T*)a.o + (int64_t)bh * Tn * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH);
   const float* ldp = a.log_decay + (int64_t)bh * Tn;
-  const float* vsp = a.v_scale ? a.v_scale + (int64_t)bh * Tn : nullptr;
+  const int64_t tok0 = (int64_t)bh * Tn;
+  // A token's value scale, and its log decay from what log_decay holds.  As passes of their own in front of this kernel the
+  // conversion of a bf16 scale and the product with a head's factor were 9.8 of 99 us at 8 x 64 heads, 2048 tokens, 128 / 64.
+  // (Not with general addressing: the code alone cost the two-head kernels of a 64-wide key 2 %, 42.9 -> 44.1 us at 8 x 16 heads,
+  // 1024 tokens.)
+  // (The scale is loaded as it is and converted where it is used: a conversion behind the load, in a branch, waits for it there,
+  // 12 us of that pass.)
+  auto v_scale_at = [&](int64_t i) {
+    return GEN == 0 && a.v_scale_bf16 ? __builtin_bit_cast(float, (uint32_t)((const uint16_t*)a.v_scale)[i]) : a.v_scale[i];
+  };
+  auto v_scale_of = [&](float x) { return GEN == 0 && a.v_scale_bf16 ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) << 16) : x; };
+  auto log_decay_of = [&](float x, float head_factor) {
+    if (GEN == 0 && a.decay_log) x = logf(x);
+    return GEN == 0 && a.decay_head ? x * head_factor : x;
+  };
   const int n_chunks_all = (Tn + L - 1) / L;
   const int c_begin = MODE == 0 ? 0 : seg * a.seg_chunks;
   const int c_end = MODE == 0 ? n_chunks_all : min(c_begin + a.seg_chunks, n_chunks_all);
@@ -281,7 +295,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
   float ld_next = 0.f, vs_next = 1.f;
   if (!PIPE && c_begin * L + ti < Tn) {
     ld_next = ldp[c_begin * L + ti];
-    if (vsp) vs_next = vsp[c_begin * L + ti];
+    if (a.v_scale) vs_next = v_scale_at(tok0 + c_begin * L + ti);
   }
   if (!helper) {
     if (c_begin < c_end) issue_chunk(c_begin * L, 0);
@@ -392,18 +406,20 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
     //      decay and value scale.  Inclusive scan over the tokens (DPP: shifts within rows of 16 lanes, then lane 15 of rows 0
     //      and 2 carried into rows 1 and 3), in the log2 domain.
     const int64_t lane_head = (int64_t)(bh0 + (HG > 1 ? lane >> 5 : 0)) * Tn;
+    const float head_factor = GEN == 0 && a.decay_head ? a.decay_head[h0 + (HG > 1 ? lane >> 5 : 0)] : 1.f;
     auto load_scalars = [&](int cn, float& ld, float& vs) {
       const int t = cn * L + r0;
       ld = 0.f;
       vs = 1.f;
       if (cn < c_end && t < Tn) {
         ld = a.log_decay[lane_head + t];
-        if (a.v_scale) vs = a.v_scale[lane_head + t];
+        if (a.v_scale) vs = v_scale_at(lane_head + t);
       }
     };
-    auto publish = [&](int cn, float ld, float vs) {
+    auto publish = [&](int cn, float ld, float vs_loaded) {
+      const float vs = v_scale_of(vs_loaded);
       const bool valid = cn * L + r0 < Tn;
-      float x = valid ? ld : 0.f;
+      float x = valid ? log_decay_of(ld, head_factor) : 0.f;
       x += dpp_f32<0x111>(x);   // row_shr:1, lanes shifted in from outside the row read 0
       x += dpp_f32<0x112>(x);
       x += dpp_f32<0x114>(x);
@@ -745,11 +761,12 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
     }
   }
   if constexpr (!PIPE) {
+  const float head_factor = GEN == 0 && a.decay_head ? a.decay_head[h0 + hl] : 1.f;
   for (int c = c_begin; c < c_end; c++) {
     const int buf = (c - c_begin) & 1, t0 = c * L;
     wait_dma();
     __syncthreads();
-    const float ld = ld_next, vs = vs_next;
+    const float ld = ld_next, vs = v_scale_of(vs_next);
     const bool has_next = c + 1 < c_end;
     if (has_next) {
       const int tn = t0 + L + ti;
@@ -757,7 +774,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       vs_next = 1.f;
       if (tn < Tn) {
         ld_next = ldp[tn];
-        if (vsp) vs_next = vsp[tn];
+        if (a.v_scale) vs_next = v_scale_at(tok0 + tn);
       }
     }
     if (has_next) issue_chunk(t0 + L, buf ^ 1);
@@ -798,7 +815,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
     const bool valid = t0 + ti < Tn;
     // (DPP: shifts within rows of 16 lanes, then lane 15 of rows 0 and 2 carried into rows 1 and 3; the
     // two halves of the wave scan the same 32 values)
-    float gi = valid ? ld : 0.f;
+    float gi = valid ? log_decay_of(ld, head_factor) : 0.f;
     gi += dpp_f32<0x111>(gi);   // row_shr:1, lanes shifted in from outside the row read 0
     gi += dpp_f32<0x112>(gi);
     gi += dpp_f32<0x114>(gi);

@@ -27,7 +27,7 @@ MA_MASK_NONE, MA_MASK_CAUSAL = 0, 1
 
 EXPORTED_SYMBOLS = (
     "ma_version", "ma_last_error", "ma_attn_workspace_bytes", "ma_attn_fwd", "ma_attn_bwd_workspace_bytes", "ma_attn_bwd",
-    "ma_linear_workspace_bytes", "ma_linear_fwd", "ma_linear_bwd_workspace_bytes", "ma_linear_bwd",
+    "ma_linear_workspace_bytes", "ma_linear_fwd", "ma_linear_fwd_factors", "ma_linear_bwd_workspace_bytes", "ma_linear_bwd",
     "ma_linear_bwd_qkv_workspace_bytes", "ma_linear_bwd_qkv",
     "ma_mla_choose_split", "ma_mla_workspace_bytes", "ma_mla_decode", "ma_mla_num_sm_parts", "ma_mla_get_metadata",
     "ma_mla_noalloc_max_workspace", "ma_mla_decode_noalloc",
@@ -161,6 +161,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.ma_linear_workspace_bytes.restype = c_size_t
     lib.ma_linear_fwd.argtypes = [POINTER(LinearParams), c_void_p]
     lib.ma_linear_fwd.restype = c_int
+    lib.ma_linear_fwd_factors.argtypes = [POINTER(LinearParams), c_int32, c_void_p, c_int32, c_void_p]
+    lib.ma_linear_fwd_factors.restype = c_int
     lib.ma_linear_bwd_workspace_bytes.argtypes = [POINTER(LinearBwdParams)]
     lib.ma_linear_bwd_workspace_bytes.restype = c_size_t
     lib.ma_linear_bwd.argtypes = [POINTER(LinearBwdParams), c_void_p]
