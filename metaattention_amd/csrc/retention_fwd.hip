@@ -120,7 +120,35 @@ __global__ __launch_bounds__(64 * RP_NW, 2) void retention_cols_fwd_kernel(const
   // DMA of one tile: each instruction moves 1 KB (two rows of K or of this half of V); lane i fetches the 16-byte
   // chunk that belongs at physical position i of that KB.  Rows beyond the sequence are clamped to its last row
   // (their scores are multiplied by a zero of M).
+  // GAMMA: a wave's two instructions of K (V) are 16 rows apart, so that one lane offset, the same for every tile, serves both, on
+  // a base in scalar registers; a last tile that ends inside, and rows that 32-bit offsets do not reach, go row by row.  (With
+  // 64-bit addresses made for every instruction B8 H16 S2048 took 627 us, 570 like this.  A multiplier that is read as it is
+  // used keeps them: those instructions are asm statements, which the compiler's waits for the multiplier cover too, 792 us
+  // and 1075; with the multiplier by DMA as well, two instructions more a tile, 1098.)
+  const int d_row = GAMMA ? 2 * wave + (lane >> 5) : 0;      // (made for a multiplier that is read, the compiler would keep them through the loop)
+  static_assert(RP_CPRK == 32 && RP_CPRV == 32 && RP_NW == 8 && NI == 4, "two rows an instruction, 16 a round of the waves");
+  const uint32_t d_chunk = GAMMA ? (uint32_t)(((lane & 31) ^ swz_tile<32>(d_row)) << 4) : 0u;      // (the swizzle repeats every 16 rows)
+  const uint32_t k_lane = (uint32_t)d_row * (uint32_t)k_row_bytes + d_chunk, v_lane = (uint32_t)d_row * (uint32_t)v_row_bytes + d_chunk;
+  const int whole_tiles = k_row_bytes < (1 << 26) && v_row_bytes < (1 << 26) ? skv / RP_BN : 0;
+  auto issue_by_rows = [&](int jt) {
+#pragma unroll 1
+    for (int it = 0; it < NI; it++) {
+      const bool is_k = it < 2;
+      const int64_t row = min(jt * RP_BN + 16 * (it & 1) + d_row, skv - 1);
+      dma16(is_k ? kb + row * k_row_bytes + d_chunk : vb + row * v_row_bytes + d_chunk,
+            lds0 + (jt % RP_NST) * RP_STAGE + (is_k ? 0 : RP_KTILE) + (wave + RP_NW * (it & 1)) * 1024);
+    }
+  };
   auto issue_one = [&](int jt, int it) __attribute__((always_inline)) {
+    if constexpr (GAMMA) {
+      const bool is_k = it < 2;
+      const uint32_t to = lds0 + (jt % RP_NST) * RP_STAGE + (is_k ? 0 : RP_KTILE) + (wave + RP_NW * (it & 1)) * 1024;
+      const int first = jt * RP_BN + 16 * (it & 1);
+      const char* base = is_k ? kb : vb;
+      const int64_t row_bytes = is_k ? k_row_bytes : v_row_bytes;
+      dma16_so(base + first * row_bytes, is_k ? k_lane : v_lane, to);
+      return;
+    }
     const uint32_t base = lds0 + (jt % RP_NST) * RP_STAGE;
     const int n0 = jt * RP_BN;
     {
@@ -138,6 +166,9 @@ __global__ __launch_bounds__(64 * RP_NW, 2) void retention_cols_fwd_kernel(const
     }
   };
   auto issue_tile = [&](int jt) __attribute__((always_inline)) {
+    if constexpr (GAMMA) {
+      if (jt >= whole_tiles) return issue_by_rows(jt);
+    }
 #pragma unroll
     for (int it = 0; it < NI; it++) issue_one(jt, it);
   };
@@ -180,8 +211,16 @@ __global__ __launch_bounds__(64 * RP_NW, 2) void retention_cols_fwd_kernel(const
       // this wave's loads of tile jt have landed (they complete in order: only those of tile jt+1 may be in flight)
       if (jt + 1 < n_tiles) __builtin_amdgcn_s_waitcnt(0x0F70 | NI); else wait_dma();
       __syncthreads();   // tile jt has landed for every wave; every wave is done with tile jt-1, whose stage tile jt+2 takes
-      const bool load_ahead = jt + 2 < n_tiles;
-      if (jt >= my_tiles) {
+      if constexpr (GAMMA) {
+        if (jt >= my_tiles) {
+          if (jt + 2 < n_tiles) issue_tile(jt + 2);
+          continue;
+        }
+      }
+      const bool load_ahead = jt + 2 < (GAMMA ? min(n_tiles, whole_tiles) : n_tiles);
+      if constexpr (GAMMA) {
+        if (jt + 2 < n_tiles && !load_ahead) issue_by_rows(jt + 2);
+      } else if (jt >= my_tiles) {
         if (load_ahead) issue_tile(jt + 2);
         continue;
       }
