@@ -28,6 +28,10 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
+# -amdgpu-mfma-vgpr-form: kernels of more than 256 registers otherwise put every MFMA's result in accumulation registers, the
+# scores too, which the vector ALU then moves out one by one (the pipelined dk / dv kernel: see attn_bwd_kernels.h)
+UNIT_FLAGS = {"attn_bwd_128.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+
 
 def _hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), "/opt/rocm/bin/hipcc", "hipcc"):
@@ -46,7 +50,7 @@ def _run(cmd: list, what: str, verbose: bool) -> None:
 
 def _compile(src: str, verbose: bool) -> str:
     obj = os.path.join(OBJ_DIR, os.path.basename(src).replace(".hip", ".o"))
-    cmd = [_hipcc(), *HIPCC_FLAGS, "-c", src, "-o", obj]
+    cmd = [_hipcc(), *HIPCC_FLAGS, *UNIT_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
     _run(cmd, f"hipcc of {src}", verbose)
     return obj
 

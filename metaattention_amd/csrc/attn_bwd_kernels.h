@@ -867,7 +867,10 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
   constexpr int STREAM_LDS = (MASKS ? LIST_N + 4 : ROWVALS + NST * 512) + 1023 & ~1023;
   // the MFMAs of a step and the fragment ring
   constexpr int NF = KS + VS, NV = 2 * VB, NK = 2 * QB, NTOT = NF + NV + NK;
-  constexpr int RING = 8, AH = !ROWS_AHEAD && FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
+  // (128 / 128 in runs, whose loop has the registers for it: further ahead, 205 -> 199 us at B2 H32 Hkv8 S2047; without runs the longer
+  // ring moves accumulators about, 161 -> 182 at B2 H32 S1600)
+  constexpr bool LONG = DQK == 128 && DV == 128 && PARTS && !MASKS;
+  constexpr int RING = LONG ? 16 : 8, AH = LONG ? 8 : !ROWS_AHEAD && FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
   static_assert(NTOT % RING == 0 && AH < RING && AH <= NK && AH <= NF, "fragment ring");
   using PhF = PhaseF<KS, VS>;
 
@@ -926,6 +929,16 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
     const T* vp = (const T*)a.v + (int64_t)b * a.vsb + (int64_t)n_ld * a.vss + (int64_t)hk * a.vsh + 8 * g;
 #pragma unroll
     for (int sl = 0; sl < VS; sl++) vf[sl] = *(const x8*)(vp + 16 * sl);
+    if constexpr (ROWS_AHEAD && DQK + DV <= 256) {      // (192 / 128, which spills either way, is no faster)
+      // (in accumulation registers, where only MFMAs read them: the scores then get vector registers, which the row function reads
+      // without moves.  One wave on a SIMD issues an instruction at a time, and that bounds the loop: of 412 k clocks a wave at B2
+      // H32 Hkv8 S2047, 250 k were issue, 140 k of those MFMAs' time.  With the MFMAs in their vector-register form, which the build
+      // asks for in this file's unit of 128 / 128: 214 -> 205 us)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) asm volatile("" : "+a"(kf[ks]));
+#pragma unroll
+      for (int sl = 0; sl < VS; sl++) asm volatile("" : "+a"(vf[sl]));
+    }
   }
   f32x16 dk[QB], dv[VB];
 #pragma unroll

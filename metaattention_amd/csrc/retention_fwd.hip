@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * RP_NW, 2) void retention_cols_fwd_kernel(const
   static_assert(RP_CPRK == 32 && RP_CPRV == 32 && RP_NW == 8 && NI == 4, "two rows an instruction, 16 a round of the waves");
   const uint32_t d_chunk = GAMMA ? (uint32_t)(((lane & 31) ^ swz_tile<32>(d_row)) << 4) : 0u;      // (the swizzle repeats every 16 rows)
   const uint32_t k_lane = (uint32_t)d_row * (uint32_t)k_row_bytes + d_chunk, v_lane = (uint32_t)d_row * (uint32_t)v_row_bytes + d_chunk;
-  const int whole_tiles = k_row_bytes < (1 << 26) && v_row_bytes < (1 << 26) ? skv / RP_BN : 0;
+  const int whole_tiles = (uint64_t)k_row_bytes < (1 << 26) && (uint64_t)v_row_bytes < (1 << 26) ? skv / RP_BN : 0;
   auto issue_by_rows = [&](int jt) {
 #pragma unroll 1
     for (int it = 0; it < NI; it++) {
