@@ -117,47 +117,55 @@ static constexpr int64_t kWideRowStride = (int64_t)1 << 26;
 
 // Prefill calls whose workgroups of 128 (or 256: attn_fwd.hip) query rows are too few to keep the chip busy: a row block's tiles
 // are then walked by several streams side by side (KVS of attn_wide_fwd_kernel), or the row blocks are smaller.  A step of a
-// stream is a serial chain of about 0.85 us at 128 / 128 whatever else the CU does, 1.08 with a second wave on the SIMD, so the
+// stream is a serial chain of about 0.78 us at 128 / 128 whatever else the CU does, 1.0 with a second wave on the SIMD, so the
 // cut is the one with the shortest schedule in microseconds: the longest workgroup, or all of them over the slots where that is
-// more; measured constants, right to about 15 % for 1 to 4 rounds of workgroups.
+// more.  The constants are fitted to all cuts' times at 354 shapes (64/64, 128/128, 192/128; 4 to 128 heads of 64 to 4096 rows,
+// causal and not): the choice costs 0.9 % over the best cut on average, 14 % at the worst.
+// 128 / 256 is always row blocks of 128: the persistent kernel, which takes the value columns in two halves, lost at every size
+// once the general kernel had its registers to itself (B1 H16 S300 28 us and 14.5, B2 H32 S1653 causal 139 and 84, B8 H32 S4096 2087
+// and 1736, without a mask 3710 and 2988); it is left with the rows that are too far apart for the general kernel.
 AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, int dv) {
   if (family == WF_RETENTION || a.kv_lens || a.o_part || (a.kv_block_mask && !a.kbm_by_query_head)) return AttnCut::kRows128;
   const bool plain = !a.kv_block_mask && !a.elem_mask && !a.add && !a.slope_q && !a.slope_kv && !(a.softcap > 0.f);
   const bool persistent = plain && dqk == 128 && (dv == 128 || (dv == 256 && a.Sq >= 256));
   if (persistent && (a.kss >= kWideRowStride || a.vss >= kWideRowStride)) return AttnCut::kPersistent;   // (the other cuts would refuse them)
-  const double k = dqk + dv <= 128 ? 0.75 : dqk == 192 ? 1.25 : 1.0;
+  const bool small = dqk + dv <= 128;
+  const double step_alone = small ? 0.65 : dqk == 192 ? 1.15 : 0.78, step_two = small ? 0.81 : dqk == 192 ? 1.35 : 1.0;
   const int64_t bh = (int64_t)a.B * a.H, tiles = ((int64_t)a.Skv + 31) / 32;
   const bool half = causal || a.kv_block_mask || a.elem_mask;   // (what a mask keeps is not known here: taken as a causal one)
   AttnCut best = AttnCut::kRows128;
   double best_us = 1e30;
   auto consider = [&](AttnCut cut, int nw, int kvs, double fixed) {
-    const int64_t blocks = ((int64_t)a.Sq + 32 * nw - 1) / (32 * nw), n = bh * blocks, slots = nw * kvs == 8 ? 256 : dqk + dv <= 128 ? 768 : 512;
-    const bool alone = nw * kvs == 4 && n <= 256;
-    const double step = dqk == 128 && dv == 256 ? (alone ? 1.5 : 2.7) : k * (alone ? 0.85 : 1.08), longest = (double)((tiles + kvs - 1) / kvs);
+    const int64_t blocks = ((int64_t)a.Sq + 32 * nw - 1) / (32 * nw), n = bh * blocks;
+    // (64 / 64: the LDS of six streams; 192 / 128: of two)
+    const int64_t slots = dqk == 192 && kvs > 1 ? 256 : (small ? 768 : 512) * 4 / (nw * kvs);
+    const double step = nw * kvs == 4 && n <= 256 ? step_alone : step_two, longest = (double)((tiles + kvs - 1) / kvs);
     const double mean = half ? longest * (double)(blocks + 1) / (double)(2 * blocks) : longest;
-    const double one = fixed + longest * step, all = 1.1 * (fixed + mean * step) * (double)n / (double)slots, us = one > all ? one : all;
+    // (one workgroup to a CU, all of a weight: whole rounds)
+    const double rounds = dqk == 192 && kvs > 1 && !causal ? (double)((n + slots - 1) / slots) : 0, part = 1.15 * (double)n / (double)slots;
+    const double one = fixed + longest * step, all = (fixed + mean * step) * (rounds > part ? rounds : part), us = one > all ? one : all;
     if (us < best_us) {
       best_us = us;
       best = cut;
     }
   };
   const bool sizes = (dqk == 64 && dv == 64) || (dqk == 128 && dv == 128) || (dqk == 192 && dv == 128);
-  consider(AttnCut::kRows128, 4, 1, 6.2);
+  consider(AttnCut::kRows128, 4, 1, 4.9);
   // (only where row blocks of 128 leave slots empty.  With batch x heads in the rule, a row's sums, and so its last bits, may be
   // formed in another order in a batch than in a call of its own)
-  if (sizes && bh * (((int64_t)a.Sq + 127) / 128) < (dqk + dv <= 128 ? 768 : 512)) {
-    consider(AttnCut::kStreams4x2, 4, 2, 6.5);
-    if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 8.8);
-    consider(AttnCut::kStreams2x2, 2, 2, 6.5);
+  if (sizes && bh * (((int64_t)a.Sq + 127) / 128) <= (small ? 768 : 512)) {
+    consider(AttnCut::kStreams4x2, 4, 2, 8.9);
+    if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 7.3);
+    consider(AttnCut::kStreams2x2, 2, 2, 5.5);
   }
-  if (persistent) {
-    // the persistent kernel: rounds of row blocks of 256 (under a causal mask, pairs of them), 32 keys in 0.6 us, 0.95 once all
-    // CUs take part; twice for the two halves of 256 value columns
+  if (persistent && dv == 128) {
+    // the persistent kernel: rounds of row blocks of 256 (under a causal mask, pairs of them), 32 keys in 0.64 us, 0.92 once all
+    // CUs take part
     const int64_t blocks = ((int64_t)a.Sq + 255) / 256, units = bh * (causal ? (blocks + 1) / 2 : blocks);
     const double steps = causal && blocks > 1 ? (double)(8 * blocks + 8) : (double)tiles;
     const double busy = units <= 128 ? 0.0 : units >= 256 ? 1.0 : (double)(units - 128) / 128.0;
-    const double us = (5 + (double)((units + 255) / 256) * (3 + (steps < 2 * tiles ? steps : 2 * tiles) * (0.6 + 0.35 * busy))) * (dv == 256 ? 2 : 1);
-    if (0.95 * us < best_us) best = AttnCut::kPersistent;
+    const double us = 5.3 + (double)((units + 255) / 256) * (3.1 + (steps < 2 * tiles ? steps : 2 * tiles) * (0.64 + 0.28 * busy));
+    if (us < best_us) best = AttnCut::kPersistent;
   }
   return best;
 }
