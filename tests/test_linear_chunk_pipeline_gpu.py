@@ -112,3 +112,19 @@ def test_gradients_without_the_decays(B, Hq, H, Dk, Dv, scaled, T):
     for name, x, y in zip(("dq", "dk", "dv"), some[:3], full[:3]):
         x, y = x.double(), y.double()
         assert torch.isfinite(x).all() and (x - y).norm() <= 2 ** -8 * y.norm(), name
+
+
+@pytest.mark.parametrize("B,Hq,H,T,Dk,Dv", [(1, 1, 4, 300, 128, 64), (2, 2, 2, 200, 256, 512), (8, 1, 64, 256, 128, 64), (1, 2, 2, 100, 64, 128)])
+def test_backward_workspace_is_a_matter_of_sizes(B, Hq, H, T, Dk, Dv):
+    """What the query says of sizes alone serves a call with a value scale and one without, with the decay's gradient and without."""
+    import ctypes
+    hb = _hb()
+    lib, p = hb.load_library(), hb.LinearBwdParams()
+    p.dtype, p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v = hb.MA_BF16, B, H, Hq, Hq, T, Dk, Dv
+    q, k, v, ld, vs = (t.cuda() for t in _case(B, Hq, H, T, Dk, Dv, True, T))
+    for query, with_decay in ((lib.ma_linear_bwd_workspace_bytes, True), (lib.ma_linear_bwd_qkv_workspace_bytes, False)):
+        ws = torch.empty(query(ctypes.byref(p)), dtype=torch.uint8, device="cuda")
+        for scale in (None, vs):
+            got = hb.linear_bwd(q, k, v, ld, torch.ones_like(v), v_scale=scale, workspace=ws, with_decay=with_decay)
+            want = hb.linear_bwd(q, k, v, ld, torch.ones_like(v), v_scale=scale, with_decay=with_decay)
+            assert all(a is None and b is None or torch.equal(a, b) for a, b in zip(got, want))
