@@ -153,7 +153,7 @@ AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, in
   consider(AttnCut::kRows128, 4, 1, 4.9);
   // (only where row blocks of 128 leave slots empty.  With batch x heads in the rule, a row's sums, and so its last bits, may be
   // formed in another order in a batch than in a call of its own)
-  if (sizes && bh * (((int64_t)a.Sq + 127) / 128) <= (small ? 768 : 512)) {
+  if (sizes && bh * (((int64_t)a.Sq + 127) / 128) < (small ? 768 : 512)) {
     consider(AttnCut::kStreams4x2, 4, 2, 8.9);
     if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 7.3);
     consider(AttnCut::kStreams2x2, 2, 2, 5.5);
