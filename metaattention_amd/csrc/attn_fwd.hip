@@ -618,9 +618,8 @@ int attn_fwd_dispatch(const AttnArgs& a, int family, bool causal, bool is_bf16, 
   if (attn_prefill_cut(a, family, causal, dqk, dv) == AttnCut::kPersistent) {
     if (dv == 128)
       return is_bf16 ? dispatch_family<__bf16, 128, 128>(a, family, causal, stream) : dispatch_family<_Float16, 128, 128>(a, family, causal, stream);
-    // 128 / 256: two launches, one per half of the value columns (given the probabilities the columns are independent; the
-    // scores are computed twice, which this kernel still does in less time than the general kernel needs once: 0.78 against
-    // 1.46 ms at B8 H12 S4096).  Both launches write the same row scales.
+    // 128 / 256, rows that are too far apart for the general kernel's tile offsets: two launches, one per half of the value columns
+    // (given the probabilities the columns are independent; the scores are computed twice).  Both write the same row scales.
     for (int half = 0; half < 2; half++) {
       AttnArgs h = a;
       h.v = (const char*)a.v + half * 128 * 2;
