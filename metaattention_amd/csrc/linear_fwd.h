@@ -7,7 +7,7 @@ namespace ma {
 struct LinArgs {
   const void* q; const void* k; const void* v; void* o;
   const float* log_decay;  // [B,H,T]
-  const float* v_scale;    // [B,H,T] or null (v_scale_bf16: bf16)
+  const float* v_scale;    // [B,H,T] or null (v_scale_bf16, set only with a scale: bf16)
   float q_scale;
   int B, H, Hq, Hk, T, Dv, dv_blocks;
   // sequence segments (see linear_fwd.hip): nseg segments of seg_chunks 32-token chunks; local end

@@ -44,6 +44,28 @@ def test_factors(T, B, Hq, H, Dk, Dv, log, head, half):
     assert lib.ma_linear_fwd_factors(ctypes.byref(p), 1, None, -1, None) < 0
 
 
+@pytest.mark.parametrize("T,Hq,H,Dk,Dv,segments", [(40, 2, 2, 256, 256, 1), (200, 1, 4, 128, 64, 3), (33, 2, 2, 256, 64, 1), (300, 1, 3, 128, 128, 4)])
+@pytest.mark.parametrize("half", [False, True])
+def test_no_value_scale(T, Hq, H, Dk, Dv, segments, half):
+    """Without a value scale the type that one would have says nothing: the plain call's kernels and numbers, to the bit."""
+    from metaattention_amd import hip_backend as hb
+    lib, g = hb.load_library(), torch.Generator().manual_seed(T)
+    q, k = (torch.randn(1, Hq, T, Dk, generator=g).mul(Dk ** -0.5).bfloat16().cuda() for _ in range(2))
+    v = torch.randn(1, H, T, Dv, generator=g).bfloat16().cuda()
+    decay = torch.rand(1, H, T, generator=g).cuda() * -0.3
+    want = hb.linear_fwd(q, k, v, decay, segments=segments, out_fp32=True)
+    out = torch.full_like(want, float("nan"))
+    p = hb.LinearParams()
+    p.dtype, p.out_fp32, p.segments, p.q_scale = hb.MA_BF16, 1, segments, 1.0
+    p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v = 1, H, Hq, Hq, T, Dk, Dv
+    p.q, p.k, p.v, p.o, p.log_decay = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), decay.data_ptr()
+    ws = torch.empty(max(lib.ma_linear_workspace_bytes(ctypes.byref(p)), 1), dtype=torch.uint8, device="cuda")
+    p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+    print(f"no value scale T{T} {(Hq, H, Dk, Dv)} half={half} segments={segments}", flush=True)
+    assert lib.ma_linear_fwd_factors(ctypes.byref(p), 0, None, hb.MA_BF16 if half else -1, torch.cuda.current_stream().cuda_stream) == 0, lib.ma_last_error()
+    assert torch.count_nonzero(want) > 0 and torch.equal(out, want)
+
+
 @pytest.mark.parametrize("Dk", [128, 64])
 def test_engine_with_and_without_gradients(Dk):
     """The same operator through its native call: factors in the kernel, and (with gradients) as tensors in front of it."""
