@@ -1108,11 +1108,8 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
     for (int i = 0; i < LA; i++)
       if (i_n < n_steps) issue_next();
     // (the padding step of an odd number of steps evaluates S, dP, lse and delta of the stage behind the last tile's:
-    // where no earlier tile has been there, tile 0 goes there, so that what it computes is finite)
-    if constexpr (STREAMS > 1) {
-      // (here one for every step that the other stream has more, and a stream may have none at all: tile 0 of the group's first head)
-      for (int i = n_steps; i < ((n_bodies + 1) & ~1) && i < NST; i++) issue_tile(0, 0, i);
-    } else {
+    // where no earlier tile has been there, the first one goes there, so that what it computes is 0 unless a tile that this key block
+    // sees is not finite)
     if ((n_steps & 1) && n_steps < NST) {
       if constexpr (MASKS) {
         const uint32_t e = uniform(list_request(0));
@@ -1120,7 +1117,6 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
       } else {
         issue_tile(first.hg, first.t, n_steps);
       }
-    }
     }
     wait_dma();
     __syncthreads();
@@ -1137,7 +1133,7 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
       const bool real = u < n_steps;                 // (the padding step: the last tile once more, everything masked)
       const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
       if constexpr (MASKS) c_next = list_request(u + 1);
-      const uint32_t cur_tile = lds0 + (uint32_t)(((real ? u : max(n_steps, 1) - 1) & (NST - 1)) * STAGE);
+      const uint32_t cur_tile = lds0 + (uint32_t)(((real ? u : n_steps - 1) & (NST - 1)) * STAGE);
       const uint32_t nxt_tile = lds0 + (uint32_t)(((u + 1) & (NST - 1)) * STAGE);
       const uint32_t nn_tile = lds0 + (uint32_t)(((u + 2) & (NST - 1)) * STAGE);
       const int m0 = real ? (t_first + (MASKS ? (int)(c_entry & 0xffffu) : at.t)) * BMT : a.Sq;
@@ -1222,10 +1218,14 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
         __builtin_amdgcn_sched_barrier(0);
       });
     };
-    for (int u = 0; u < n_bodies; u += 2) {
+    for (int u = 0; u < n_steps; u += 2) {
       body(u, ra, rb);
       body(u + 1, rb, ra);
     }
+    // (the steps that only the other stream has: their barriers and nothing else.  No tile stands in for them, as this stream may have
+    // none that its key block sees, and zeros times a tile that is not finite are not 0)
+    if (STREAMS > 1)
+      for (int u = (n_steps + 1) & ~1; u < ((n_bodies + 1) & ~1); u++) __builtin_amdgcn_s_barrier();
   }
   wait_dma();
   __syncthreads();   // every wave is done with the tiles: they become output staging

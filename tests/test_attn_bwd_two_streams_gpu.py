@@ -71,6 +71,33 @@ def test_block_mask_that_favours_a_stream(every, S):
     assert torch.count_nonzero(got[1][:, :130]) == 0 and torch.count_nonzero(got[2][:, :130]) == 0
 
 
+@pytest.mark.parametrize("tiles", [[3], [3, 5], [2, 4], [2, 3, 5], [1, 3, 5, 7, 9], [2, 5, 6, 7, 8, 9, 11]])     # (none to four and more of a stream)
+@pytest.mark.parametrize("H,Hkv", [(2, 2), (2, 1)])
+@pytest.mark.parametrize("family", ["softmax", "sigmoid", "relu"])
+def test_hidden_queries_stay_hidden(tiles, H, Hkv, family):
+    """A gradient of the output that is not finite, in rows that the mask hides from every key: dk and dv have the bits that they
+    have without it."""
+    S = 384
+    g = torch.Generator().manual_seed(len(tiles))
+    q, k, v, dout = (torch.randn(1, S, h, 64, generator=g).bfloat16().cuda() for h in (H, Hkv, Hkv, H))
+    keep = torch.zeros(S, dtype=torch.bool)
+    for t in tiles:
+        keep[32 * t:32 * t + 32] = True
+    em = keep.view(S, 1).expand(S, S).to(torch.uint8).contiguous().view(1, 1, S, S).cuda()
+    emt = em.transpose(2, 3).contiguous()
+    kbm, qbm = (m.view(3, 128, 12, 32).amax(dim=(1, 3)).view(1, 1, 3, 12).contiguous() for m in (em, emt))
+    scale, bias = (0.125, 0.0) if family != "sigmoid" else (0.125, -2.0)
+    run = lambda grad: _run(family, q, k, v, grad, False, scale, bias, elem_mask=em, elem_mask_t=emt, kv_block_mask=kbm, q_block_mask=qbm)
+    want = run(dout)
+    assert all(torch.isfinite(t).all() and torch.count_nonzero(t) > 0 for t in want[1:])
+    for bad in (float("nan"), float("inf")):
+        for head in range(H):
+            grad = dout.clone()
+            grad[0, :, head] = torch.where(keep.view(S, 1).cuda(), grad[0, :, head], bad)
+            got = run(grad)
+            assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2]), f"{bad} in head {head}"
+
+
 def test_both_sides_of_the_rule():
     """512 and 516 key blocks: the same sequences' gradients from two streams and from one."""
     g = torch.Generator().manual_seed(1)
