@@ -1188,8 +1188,7 @@ struct Config {
     size_t need = 0;
     for (int i = 0; i < n; i++) need += ws_bytes(all.s[i], nseg);
     if (query) {
-      // (an automatic choice asks for some workspace also where it is a single pass: 0 is the answer for segments = 1)
-      *query = tail.tail_bg > 0 ? tail_ws_bytes(tail, a.dv_blocks) : need > 0 || want_segments != 0 ? need : 256;
+      *query = tail.tail_bg > 0 ? tail_ws_bytes(tail, a.dv_blocks) : need;
       return 0;
     }
     if (nseg > 1 && (!ws || ws_size < need || ((uintptr_t)ws & 3) != 0)) nseg = 1;   // no workspace: single pass

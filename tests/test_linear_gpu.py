@@ -233,15 +233,19 @@ def test_segments_need_a_workspace_else_single_pass():
 
 
 def test_full_size_mamba2_auto_segments():
-    """B=8 H=64 S=2048 P=64 N=128: the library's own choice of segments against the single pass."""
+    """H=64 S=2048 P=64 N=128: the library's own choice against the single pass.  Three batch entries leave half of the CUs without a
+    workgroup and are cut into segments; eight fill them all, are a single pass and ask for no workspace (cut by hand here)."""
     hb = _hb()
     Cm, Bm, x, dt, A = (t.cuda() for t in inputs.mamba2_inputs(8, 64, 2048, 64, 128, seed=0))
     ldm = dt * A.view(1, 64, 1)
-    assert hb.linear_workspace_bytes(8, 64, 1, 1, 2048, 128, 64) > 0
-    y = hb.linear_fwd(Cm, Bm, x, ldm, v_scale=dt)
     y1 = hb.linear_fwd(Cm, Bm, x, ldm, v_scale=dt, segments=1)
-    torch.cuda.synchronize()
-    torch.testing.assert_close(y.float(), y1.float(), rtol=1e-2, atol=1e-2)
+    assert hb.linear_workspace_bytes(8, 64, 1, 1, 2048, 128, 64) == 0
+    assert torch.equal(hb.linear_fwd(Cm, Bm, x, ldm, v_scale=dt), y1)
+    for B, segments in ((8, 3), (3, 0)):
+        ws = torch.full((hb.linear_workspace_bytes(B, 64, 1, 1, 2048, 128, 64, segments=segments),), 0xA5, dtype=torch.uint8, device="cuda")
+        y = hb.linear_fwd(Cm[:B], Bm[:B], x[:B], ldm[:B], v_scale=dt[:B], segments=segments, workspace=ws)
+        assert ws.numel() > 0 and (ws[-4 * 64:] != 0xA5).any()          # (the last decays that the segments hand over)
+        torch.testing.assert_close(y.float(), y1[:B].float(), rtol=1e-2, atol=1e-2)
 
 
 def test_linear_rejects_bad_arguments():
