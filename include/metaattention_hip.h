@@ -303,6 +303,10 @@ int ma_linear_bwd(const ma_linear_bwd_params* p, ma_stream_t stream);
 /* The gradients of q, k and v alone: dlog_decay and dv_scale are not read and may be NULL.  A workspace of its own query, never more
  * than ma_linear_bwd's. */
 size_t ma_linear_bwd_qkv_workspace_bytes(const ma_linear_bwd_params* p);
+/* The two queries above go by the sizes alone and serve a call with a v_scale and one without.  This one is for the call as *p has it,
+ * v_scale and dv_scale NULL or not (nothing is read through them): what ma_linear_bwd (with_decay not 0) or ma_linear_bwd_qkv takes of the
+ * workspace, and the least that it accepts. */
+size_t ma_linear_bwd_call_workspace_bytes(const ma_linear_bwd_params* p, int32_t with_decay);
 int ma_linear_bwd_qkv(const ma_linear_bwd_params* p, ma_stream_t stream);
 
 /* mla_decode_tl.py:293-303 (`main_split`) */

@@ -433,7 +433,7 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
     p.q_scale = (float)ctx->saved_data["q_scale"].toDouble();
     p.dq = dq.data_ptr(); p.dk = dk.data_ptr(); p.dv = dv.data_ptr(); p.dlog_decay = dg.defined() ? (float*)dg.data_ptr() : nullptr;
     p.dv_scale = dvs.defined() ? (float*)dvs.data_ptr() : nullptr;
-    const size_t need = with_decay ? ma_linear_bwd_workspace_bytes(&p) : ma_linear_bwd_qkv_workspace_bytes(&p);
+    const size_t need = ma_linear_bwd_call_workspace_bytes(&p, with_decay);
     const c10::DataPtr ws = scratch(need);
     p.workspace = ws.get(); p.workspace_bytes = need;
     {

@@ -28,7 +28,7 @@ MA_MASK_NONE, MA_MASK_CAUSAL = 0, 1
 EXPORTED_SYMBOLS = (
     "ma_version", "ma_last_error", "ma_attn_workspace_bytes", "ma_attn_fwd", "ma_attn_bwd_workspace_bytes", "ma_attn_bwd",
     "ma_linear_workspace_bytes", "ma_linear_fwd", "ma_linear_fwd_factors", "ma_linear_bwd_workspace_bytes", "ma_linear_bwd",
-    "ma_linear_bwd_qkv_workspace_bytes", "ma_linear_bwd_qkv",
+    "ma_linear_bwd_qkv_workspace_bytes", "ma_linear_bwd_qkv", "ma_linear_bwd_call_workspace_bytes",
     "ma_mla_choose_split", "ma_mla_workspace_bytes", "ma_mla_decode", "ma_mla_num_sm_parts", "ma_mla_get_metadata",
     "ma_mla_noalloc_max_workspace", "ma_mla_decode_noalloc",
 )
@@ -169,6 +169,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.ma_linear_bwd.restype = c_int
     lib.ma_linear_bwd_qkv_workspace_bytes.argtypes = [POINTER(LinearBwdParams)]
     lib.ma_linear_bwd_qkv_workspace_bytes.restype = c_size_t
+    lib.ma_linear_bwd_call_workspace_bytes.argtypes = [POINTER(LinearBwdParams), c_int32]
+    lib.ma_linear_bwd_call_workspace_bytes.restype = c_size_t
     lib.ma_linear_bwd_qkv.argtypes = [POINTER(LinearBwdParams), c_void_p]
     lib.ma_linear_bwd_qkv.restype = c_int
     lib.ma_mla_choose_split.argtypes = [POINTER(MlaParams)]
@@ -603,13 +605,12 @@ def linear_bwd(q, k, v, log_decay, dout, *, q_scale: float = 1.0, v_scale=None, 
     p.dq, p.dk, p.dv, p.dlog_decay = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dld.data_ptr() if dld is not None else None
     p.dv_scale = dvs.data_ptr() if dvs is not None else None
     lib = load_library()
-    query, call = (lib.ma_linear_bwd_workspace_bytes, lib.ma_linear_bwd) if with_decay else (lib.ma_linear_bwd_qkv_workspace_bytes, lib.ma_linear_bwd_qkv)
-    need = query(ctypes.byref(p))
-    if need > 0:
-        if workspace is None:
-            workspace = torch.empty(need, dtype=torch.uint8, device=v.device)
+    if workspace is None:
+        need = lib.ma_linear_bwd_call_workspace_bytes(ctypes.byref(p), int(with_decay))
+        workspace = torch.empty(need, dtype=torch.uint8, device=v.device) if need > 0 else None
+    if workspace is not None:
         p.workspace, p.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()   # (a small one is refused by the library)
-    _check(call(ctypes.byref(p), _stream()))
+    _check((lib.ma_linear_bwd if with_decay else lib.ma_linear_bwd_qkv)(ctypes.byref(p), _stream()))
     return dq, dk, dv, dld, dvs
 
 

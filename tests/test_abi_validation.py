@@ -194,6 +194,9 @@ def test_workspace_queries_take_bad_arguments():
     assert lib.ma_attn_bwd_workspace_bytes(ctypes.byref(_attn_bwd(batch=big, heads=big, heads_kv=big))) == 0
     assert lib.ma_linear_bwd_workspace_bytes(ctypes.byref(_linear_bwd(batch=big, heads=1 << 24, heads_q=4, heads_k=4, seqlen=65536))) == 0
     assert lib.ma_linear_workspace_bytes(ctypes.byref(_linear(dim_v=big))) == 0
+    for with_decay in (0, 1):
+        assert lib.ma_linear_bwd_call_workspace_bytes(None, with_decay) == 0
+        assert lib.ma_linear_bwd_call_workspace_bytes(ctypes.byref(_linear_bwd(dim_k=96)), with_decay) == 0
     assert lib.ma_mla_workspace_bytes(ctypes.byref(_mla(batch=big, heads_q=big, num_split=4))) == 0
 
 

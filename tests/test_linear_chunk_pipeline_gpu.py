@@ -128,3 +128,47 @@ def test_backward_workspace_is_a_matter_of_sizes(B, Hq, H, T, Dk, Dv):
             got = hb.linear_bwd(q, k, v, ld, torch.ones_like(v), v_scale=scale, workspace=ws, with_decay=with_decay)
             want = hb.linear_bwd(q, k, v, ld, torch.ones_like(v), v_scale=scale, with_decay=with_decay)
             assert all(a is None and b is None or torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("B,Hq,H,T,Dk,Dv", [(1, 1, 4, 300, 128, 64), (8, 16, 16, 256, 256, 512), (1, 2, 2, 100, 64, 128), (2, 4, 4, 200, 128, 128)])
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("with_decay", [False, True])
+def test_backward_call_takes_what_its_query_says(B, Hq, H, T, Dk, Dv, scaled, with_decay):
+    """The query for a call as it is: never more than the one that goes by the sizes, enough for the call, and not a byte too much."""
+    import ctypes
+    hb = _hb()
+    lib, p = hb.load_library(), hb.LinearBwdParams()
+    p.dtype, p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v = hb.MA_BF16, B, H, Hq, Hq, T, Dk, Dv
+    by_sizes = (lib.ma_linear_bwd_workspace_bytes if with_decay else lib.ma_linear_bwd_qkv_workspace_bytes)(ctypes.byref(p))
+    q, k, v, ld, vs = (t.cuda() for t in _case(B, Hq, H, T, Dk, Dv, True, T))
+    vs = vs if scaled else None
+    p.v_scale = p.dv_scale = vs.data_ptr() if scaled else None
+    need = lib.ma_linear_bwd_call_workspace_bytes(ctypes.byref(p), int(with_decay))
+    assert 0 < need <= by_sizes
+    run = lambda n: hb.linear_bwd(q, k, v, ld, torch.ones_like(v), v_scale=vs, with_decay=with_decay, workspace=torch.empty(n, dtype=torch.uint8, device="cuda"))
+    for a, b in zip(run(need), run(by_sizes)):
+        assert a is None and b is None or torch.equal(a, b)
+    with pytest.raises(hb.MetaAttentionError, match=str(need)):
+        run(need - 1)
+
+
+def test_backward_without_the_decays_allocates_what_it_uses():
+    """An operator's backward pass that nobody asks the decay's gradient of, every head with its own q and k: beside the gradients it
+    holds the fp32 sums of dq and dk, and not the copies per half of the value columns and of dv that the decay's gradient would need."""
+    from attn_engine import LinearAttentionEngine
+    from core import CustomIO, meta_tensor
+    B, H, T, Dk, Dv = 8, 16, 512, 256, 512
+    meta = [meta_tensor(B, H, T, d, dtype=torch.bfloat16) for d in (Dk, Dk, Dv)]
+    mod = LinearAttentionEngine(tuple(meta), decay_mod=lambda decay, io: decay.log(), custom_io=CustomIO({}))
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(B, H, T, d, device="cuda", generator=g).mul(0.1).bfloat16().requires_grad_() for d in (Dk, Dk, Dv))
+    decay = torch.rand(B, H, T, device="cuda", generator=g)
+    grad = torch.ones(B, H, T, Dv, device="cuda", dtype=torch.bfloat16)
+    torch.autograd.grad(mod(q, k, v, decay), (q, k, v), grad)
+    out = mod(q, k, v, decay)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    grads = torch.autograd.grad(out, (q, k, v), grad)
+    used = torch.cuda.max_memory_allocated() - before - sum(t.numel() * 2 for t in grads)
+    assert used <= 2 * B * H * T * Dk * 4 + 4 * B * H * T * 4 + (4 << 20)      # dq and dk, values a token, what the allocator rounds up
