@@ -378,7 +378,7 @@ void linear_sizes(const Tensor& q, const Tensor& k, const Tensor& v, int32_t& B,
 }
 
 // fp32, contiguous, the heads and tokens as they are: what the kernels take per-token factors as
-Tensor per_token(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
+Tensor per_token(const Tensor& t) { return t.to(at::kFloat).contiguous().resolve_neg(); }
 
 // g: the log decay, or what the kernel makes it from (decay_kind); vs: fp32 or bf16
 bool linear_forward(const LinearPlan& pl, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& vs, int dev, Tensor& out,
@@ -474,9 +474,11 @@ PyObject* linear_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   for (int i = 0; i < n; i++) wanted = wanted || t[i]->requires_grad();
   if (!(wanted && at::GradMode::is_enabled())) {
     const Tensor* head = pl.decay_kind == DECAY_MUL_HEAD ? t[4 + pl.decay_head_arg] : nullptr;
-    const bool plain = (q.size(3) == 128 || q.size(3) == 256) && decay.scalar_type() == at::kFloat && decay.layout() == at::kStrided && decay.is_contiguous() &&
-                       (!vs.defined() || ((vs.scalar_type() == at::kFloat || vs.scalar_type() == at::kBFloat16) && vs.is_contiguous())) &&
-                       (!head || (head->scalar_type() == at::kFloat && head->is_contiguous() && head->numel() == H));
+    // (its values as they stand in memory: a tensor whose negation is a bit of its own goes the other way)
+    auto as_it_is = [](const Tensor& x) { return x.layout() == at::kStrided && x.is_contiguous() && !x.is_neg(); };
+    const bool plain = (q.size(3) == 128 || q.size(3) == 256) && decay.scalar_type() == at::kFloat && as_it_is(decay) &&
+                       (!vs.defined() || ((vs.scalar_type() == at::kFloat || vs.scalar_type() == at::kBFloat16) && as_it_is(vs))) &&
+                       (!head || (head->scalar_type() == at::kFloat && as_it_is(*head) && head->numel() == H));
     if (plain) {
       Tensor out;
       at::AutoDispatchBelowADInplaceOrView no_autograd;

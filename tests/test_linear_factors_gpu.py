@@ -85,3 +85,23 @@ def test_engine_with_and_without_gradients(Dk):
         assert not got.requires_grad
         assert (got.float() - want.float()).norm() <= 2e-3 * want.float().norm()       # (a unit of bf16's last place here and there)
     assert torch.equal(mod(q, k, v, dt, A, dt.half()), mod(q, k, v, dt.clone(), A.clone(), dt.half()))
+
+
+@pytest.mark.parametrize("Dk", [128, 256])
+def test_negated_views(Dk):
+    """A decay or a value scale whose negation is a bit of the tensor (as the imaginary part of a conjugate has it): its values."""
+    from attn_engine import LinearAttentionEngine
+    from core import CustomIO, meta_tensor
+    B, H, T = 1, 2, 70
+    g = torch.Generator().manual_seed(2)
+    meta = [meta_tensor(B, H, T, d, dtype=torch.bfloat16) for d in (Dk, Dk, 64)]
+    q, k, v = (torch.randn(B, H, T, d, generator=g).mul(0.3).bfloat16().cuda() for d in (Dk, Dk, 64))
+    by_log = LinearAttentionEngine(tuple(meta), decay_mod=lambda decay, io: decay.log(), custom_io=CustomIO({}))
+    decay = torch.rand(B, H, T, generator=g).cuda()
+    assert torch.equal(by_log(q, k, v, torch._neg_view(-decay)), by_log(q, k, v, decay))
+    scaled = LinearAttentionEngine(tuple(meta), decay_mod=lambda decay, io: decay * io.input_tensors["A"], v_mod=lambda v, io: v * io.input_tensors["dt"],
+                                   custom_io=CustomIO({"A": (1, "heads"), "dt": ("batch", "heads", "seq_len")}))
+    A, dt = -torch.rand(1, H, generator=g).cuda(), torch.rand(B, H, T, generator=g).bfloat16().cuda()
+    want = scaled(q, k, v, decay, A, dt)
+    for args in ((torch._neg_view(-decay), A, dt), (decay, torch._neg_view(-A), dt), (decay, A, torch._neg_view(-dt))):
+        assert (scaled(q, k, v, *args).float() - want.float()).norm() <= 2e-3 * want.float().norm()
