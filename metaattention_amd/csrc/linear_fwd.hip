@@ -71,6 +71,26 @@ __device__ __forceinline__ X8 scale_bf16x8(X8 v, const float (&w)[8]) {
   for (int i = 0; i < 8; i++) r[i] = (__bf16)((float)v[i] * w[i]);
   return r;
 }
+
+// The natural logarithm as exactly as the operators that take it in front of the kernel have it.  (-ffast-math makes logf the
+// hardware's log2 times ln 2, one rounded product; here ln 2 is hi + lo and the product's rounding error comes from a fused
+// multiply-add, so that what is left is the error of log2 and one rounding.  The asm statements keep the compiler from reordering
+// the sums as if they were exact.)
+__device__ __forceinline__ float log_f32(float x) {
+  constexpr double kLn2 = 0.693147180559945309417;
+  constexpr float hi = (float)kLn2, lo = (float)(kLn2 - (double)hi);
+  const bool subnormal = x < 0x1p-126f;      // (log2 would take it for 0)
+  const float y = fast_log2(subnormal ? x * 0x1p32f : x);
+  float p = y * hi;
+  asm("" : "+v"(p));
+  float r = p + __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -p));
+  asm("" : "+v"(r));
+  r = __builtin_fabsf(y) < __builtin_inff() ? r : y;      // (of 0 and infinity; NaN)
+  asm("" : "+v"(r));
+  float shifted = subnormal ? r - (float)(32 * kLn2) : r;
+  asm("" : "+v"(shifted));
+  return shifted;
+}
 }  // namespace
 
 // The pipelined chunk loop (P^T shared by the waves of a head and made one chunk ahead): workgroups of four waves or more that
@@ -185,7 +205,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
   };
   auto v_scale_of = [&](float x) { return GEN == 0 && a.v_scale_bf16 ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) << 16) : x; };
   auto log_decay_of = [&](float x, float head_factor) {
-    if (GEN == 0 && a.decay_log) x = logf(x);
+    if (GEN == 0 && a.decay_log) x = log_f32(x);
     return GEN == 0 && a.decay_head ? x * head_factor : x;
   };
   const int n_chunks_all = (Tn + L - 1) / L;

@@ -105,3 +105,30 @@ def test_negated_views(Dk):
     want = scaled(q, k, v, decay, A, dt)
     for args in ((torch._neg_view(-decay), A, dt), (decay, torch._neg_view(-A), dt), (decay, A, torch._neg_view(-dt))):
         assert (scaled(q, k, v, *args).float() - want.float()).norm() <= 2e-3 * want.float().norm()
+
+
+@pytest.mark.parametrize("Hq,H,Dk,Dv", [(2, 2, 256, 256), (2, 2, 256, 64), (1, 3, 128, 128), (1, 4, 128, 64)])
+@pytest.mark.parametrize("segments", [1, 3])
+def test_logarithm(Hq, H, Dk, Dv, segments):
+    """The decay's logarithm that the kernel takes is the one that torch's log rounds to: the same outputs to the bit, for decays over
+    the whole range, close to 1, of 0 and of a subnormal."""
+    from metaattention_amd import hip_backend as hb
+    lib, g, B, T = hb.load_library(), torch.Generator().manual_seed(Dk + Dv), 2, 333
+    q, k = (torch.randn(B, Hq, T, Dk, generator=g).mul(Dk ** -0.5).bfloat16().cuda() for _ in range(2))
+    v = torch.randn(B, H, T, Dv, generator=g).bfloat16().cuda()
+    u = torch.rand(B, H, T, generator=g)
+    some_zero, tiny = u.clone(), u.clone()
+    some_zero[:, :, 100] = 0.0
+    tiny[:, :, 100::40] = 1e-42
+    for decay in (u, 1 - u / 64, 1 + u / 64, some_zero, tiny):
+        decay = decay.cuda()
+        want = hb.linear_fwd(q, k, v, decay.log(), segments=segments, out_fp32=True)
+        out = torch.zeros_like(want)
+        p = hb.LinearParams()
+        p.dtype, p.out_fp32, p.segments, p.q_scale = hb.MA_BF16, 1, segments, 1.0
+        p.batch, p.heads, p.heads_q, p.heads_k, p.seqlen, p.dim_k, p.dim_v = B, H, Hq, Hq, T, Dk, Dv
+        p.q, p.k, p.v, p.o, p.log_decay = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), decay.data_ptr()
+        ws = torch.empty(max(lib.ma_linear_workspace_bytes(ctypes.byref(p)), 1), dtype=torch.uint8, device="cuda")
+        p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        assert lib.ma_linear_fwd_factors(ctypes.byref(p), 1, None, -1, torch.cuda.current_stream().cuda_stream) == 0, lib.ma_last_error()
+        torch.testing.assert_close(out, want, rtol=0, atol=0, equal_nan=True)
