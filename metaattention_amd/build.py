@@ -13,6 +13,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -51,8 +52,16 @@ def _run(cmd: list, what: str, verbose: bool) -> None:
 
 def _compile(src: str, verbose: bool) -> str:
     obj = os.path.join(OBJ_DIR, os.path.basename(src).replace(".hip", ".o"))
-    cmd = [_hipcc(), *HIPCC_FLAGS, *UNIT_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
-    _run(cmd, f"hipcc of {src}", verbose)
+    cmd = [_hipcc(), *HIPCC_FLAGS, "-c", src, "-o", obj]
+    extra = UNIT_FLAGS.get(os.path.basename(src), [])
+    try:
+        _run([*cmd, *extra], f"hipcc of {src}", verbose)
+    except RuntimeError as e:
+        # (an option of the compiler's own, which another version may not have: the kernels are right without it, and slower)
+        if not extra or "nknown command line argument" not in str(e):
+            raise
+        warnings.warn(f"hipcc does not know {' '.join(extra)}: {os.path.basename(src)} is compiled without")
+        _run(cmd, f"hipcc of {src}", verbose)
     return obj
 
 
