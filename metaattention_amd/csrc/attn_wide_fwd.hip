@@ -120,7 +120,8 @@ static constexpr int64_t kWideRowStride = (int64_t)1 << 26;
 // stream is a serial chain of about 0.78 us at 128 / 128 whatever else the CU does, 1.0 with a second wave on the SIMD, so the
 // cut is the one with the shortest schedule in microseconds: the longest workgroup, or all of them over the slots where that is
 // more.  The constants are fitted to all cuts' times at 354 shapes (64/64, 128/128, 192/128; 4 to 128 heads of 64 to 4096 rows,
-// causal and not): the choice costs 0.9 % over the best cut on average, 14 % at the worst.
+// causal and not): the choice costs 0.9 % over the best of the cuts that it may take on average, 14 % at the worst.  (The streams may be
+// taken only below the line drawn in the code; at the line, B1 H16 S4096 128/128 causal, that costs 19 %: 99 us, 83 with streams.)
 // 128 / 256 is always row blocks of 128: the persistent kernel, which takes the value columns in two halves, lost at every size
 // once the general kernel had its registers to itself (B1 H16 S300 28 us and 14.5, B2 H32 S1653 causal 139 and 84, B8 H32 S4096 2087
 // and 1736, without a mask 3710 and 2988); it is left with the rows that are too far apart for the general kernel.
@@ -151,8 +152,9 @@ AttnCut attn_prefill_cut(const AttnArgs& a, int family, bool causal, int dqk, in
   };
   const bool sizes = (dqk == 64 && dv == 64) || (dqk == 128 && dv == 128) || (dqk == 192 && dv == 128);
   consider(AttnCut::kRows128, 4, 1, 4.9);
-  // (only where row blocks of 128 leave slots empty.  With batch x heads in the rule, a row's sums, and so its last bits, may be
-  // formed in another order in a batch than in a call of its own)
+  // (only where row blocks of 128 leave slots empty.  With batch x heads in the rule, a row's sums, and so its last bits, may be formed
+  // in another order in a batch than in a call of its own: at one block a slot too, an entry of 32 heads and 2048 rows would be, and the
+  // calls beyond 4 GiB are compared to the bit with those of their entries)
   if (sizes && bh * (((int64_t)a.Sq + 127) / 128) < (small ? 768 : 512)) {
     consider(AttnCut::kStreams4x2, 4, 2, 8.9);
     if (dqk <= 128) consider(AttnCut::kStreams2x4, 2, 4, 7.3);

@@ -854,8 +854,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       lds_write<float>(lds_scal + (2 * L + ti) * 4, wl);
     }
     // ---- A^T = K Q^T (lane: token i = r, rows j = 8(jj/4) + 4g + jj%4)
-    // two accumulation chains, so that consecutive MFMAs do not wait for each other, where registers
-    // allow (with three waves per SIMD the other waves fill those gaps)
+    // two accumulation chains, so that consecutive MFMAs do not wait for each other, where registers allow
     constexpr bool TWO_CHAINS = HG == 1;
     // (a chain's first MFMA takes the constant zero as its accumulator input: no registers to clear)
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -963,8 +962,8 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
           khi[bb % RING][s] = lds_read_tr4<T>((kta ^ (uint32_t)(((4 * bb) ^ cx ^ Q_X8) << 4)) + (16 * s + 8) * RBQ);
         }
       };
-      // operands are requested one block ahead, except where three waves per SIMD hide the LDS latency
-      // and the registers are needed elsewhere
+      // operands are requested one block ahead, except where three waves per SIMD (two heads a workgroup, states alone) hide the LDS
+      // latency and the registers are needed elsewhere
       constexpr bool AHEAD = HG == 1;
       if (AHEAD) request(0);
 #pragma unroll
