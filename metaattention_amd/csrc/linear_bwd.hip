@@ -342,7 +342,7 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   const bool direct_qk = in_turn || (own_heads && sl.n == 1);
   const int np = side_by_side && !in_turn ? sl.n : 1;
   const int64_t piece_stride = BHT * a.Dk;
-  const size_t part = direct_qk && !in_turn ? 0 : (size_t)np * BHT * a.Dk * 4;
+  const size_t part = in_turn ? (size_t)a.B * a.H * ((a.T + 31) / 32 * 32) * a.Dk * 4 : direct_qk ? 0 : (size_t)np * BHT * a.Dk * 4;
   const size_t o_dqh = take(part), o_dkh = take(part), o_du = take(direct_dv ? 0 : (size_t)BHT * a.Dv * 4);
   const size_t o_dG = take((size_t)BHT * 4), o_grev = take((size_t)BHT * 4);
   // Heads in groups that share q and k, with a v_scale and a contraction of one piece (Mamba2): the dk scan leaves bf16 in
@@ -368,14 +368,14 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   // the columns of piece s that exist (a last piece may reach beyond the value columns: the scan kernel pads with zeros)
   auto piece_cols = [&](int s) { return sl.c0[s] + sl.w[s] <= a.Dv ? 0 : a.Dv - sl.c0[s]; };
   // dq (per head) = LA(do, v, k; v_scale), contraction over the value columns; k is read with its own heads
-  // (direct_qk: dq itself, bf16; in turn: its pieces add up in `out`, and the last leaves dq)
+  // (direct_qk: dq itself, bf16; in turn: its pieces add up in `out`, in the order of the scan's accumulators, and the last leaves dq)
   auto direct = [&](LinArgs la, int s, void* grad, float* out, bool reversed) {
     if (!direct_qk) return la;
     la.rev_o = reversed ? 1 : 0;
-    if (s + 1 < sl.n) return la;
-    la.o = grad;
     la.out_f32 = 0;
-    la.o_add = in_turn ? out : nullptr;
+    if (in_turn && s > 0) la.o_add = out;
+    if (s + 1 < sl.n) la.o_part = out;
+    else la.o = grad;
     return la;
   };
   auto dq_scan = [&](int s, float* out) {
@@ -397,18 +397,34 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   // chains of latencies side by side instead of behind each other.
   const bool whole = sl.n == 1 || side_by_side;
   bool with_du = false;
+  // Two pieces in turn: what they leave and take in makes the launches of dq and dk memory-bound (1.3 and 1.6 GB at 4.9 TB/s at 8 x 16
+  // heads, 2048 tokens, 256 / 512), while the du scan is not (0.8 GB in 230 us).  So the six scans of a head go out two by two, the
+  // lighter beside the heavier ones, and dq's second piece right behind its first: du of half of the heads | dq 0, dq 1 | dk 0,
+  // dk 1 | du of the other heads.  (230 + 270 + 329 us -> 250 + 306 + 273, partial results in whole lines included.)
+  bool mixed = false;
+  auto du_of = [&](LinArgs la, int half) {
+    const int heads = a.B * a.H;
+    la.bg0 = half ? heads / 2 : 0;
+    la.bg_n = half ? heads - heads / 2 : heads / 2;
+    return la;
+  };
   // the scan kernel's workspace (sequence segments): the largest any of the launches asks for
   size_t scan_ws = 0;
   {
     size_t need = 0;
     LinArgs la[3] = {dq_scan(0, nullptr), dk_scan(0, nullptr, nullptr), du_scan(nullptr, nullptr)};
     with_du = whole && !in_turn && sl.w[0] == DKP && linear_scans_together(la, 3, DKP);
+    mixed = in_turn && sl.n == 2 && sl.w[0] == DKP && linear_scans_together(la, 3, DKP);
     if (whole && linear_scans_dispatch(la, with_du ? 3 : 2, sl.w[0], nullptr, 0, nullptr, &need) == 0 && need > scan_ws) scan_ws = need;
     for (int s = 0; s < sl.n && !whole; s++) {
       la[0] = dq_scan(s, nullptr);
       if (linear_fwd_dispatch(la[0], sl.w[s], 0, nullptr, 0, nullptr, &need) == 0 && need > scan_ws) scan_ws = need;
     }
     if (!with_du && linear_fwd_dispatch(la[2], DKP, 0, nullptr, 0, nullptr, &need) == 0 && need > scan_ws) scan_ws = need;
+    for (int half = 0; half < 2 && mixed; half++) {
+      LinArgs two[2] = {la[half], du_of(la[2], half)};
+      if (linear_scans_dispatch(two, 2, DKP, nullptr, 0, nullptr, &need) == 0 && need > scan_ws) scan_ws = need;
+    }
   }
   const size_t o_scan = take(scan_ws);
   if (query) { *query = off; return 0; }
@@ -418,6 +434,13 @@ int linear_bwd_run(const LinBwdArgs& a, void* ws, size_t ws_bytes, hipStream_t s
   void* scan_at = scan_ws ? base + o_scan : nullptr;
   hipLaunchKernelGGL(shift_rev_kernel, dim3((unsigned)((BHT + 255) / 256)), dim3(256), 0, stream, grev, a.log_decay, a.T, BHT);
 
+  if (mixed) {
+    const LinArgs du_all = du_scan(grev, du);
+    const LinArgs turns[3][2] = {{dq_scan(0, dqh), du_of(du_all, 0)}, {dq_scan(1, dqh), dk_scan(0, grev, dkh)}, {dk_scan(1, grev, dkh), du_of(du_all, 1)}};
+    for (const auto& two : turns)
+      if (const int rc = linear_scans_dispatch(two, 2, DKP, scan_at, scan_ws, stream, nullptr)) return rc;
+    return launch_status();
+  }
   // (dk last: the epilogue finds part of what it wrote in the memory-side cache)
   if (!with_du)
     if (const int rc = linear_fwd_dispatch(du_scan(grev, du), DKP, 0, scan_at, scan_ws, stream, nullptr)) return rc;

@@ -32,8 +32,11 @@ struct LinArgs {
   // (fp32) by p * piece_o elements; the caller adds the pieces' outputs up.
   int n_pieces;
   int64_t piece_qk, piece_o;
-  // o_add (general addressing and the pipelined chunk loop only, bf16 outputs; null: none): fp32 [B,H,T,Dv], in the rows' own order where
-  // rev_o says so, added to the outputs before they are rounded (the last piece of a contraction takes in the earlier ones).
+  // o_part, o_add (general addressing and the pipelined chunk loop only; null: none): the pieces of a contraction in turn.  o_part: the
+  // outputs go there, fp32, instead of to o; o_add: what an earlier piece left is added to the outputs (before they are rounded).  Both
+  // in the order of the accumulators, [batch * head][value slice][chunk of 32 tokens][wave][4][64 lanes] x 16 bytes (the last chunk's
+  // missing tokens included): a wave writes and reads whole lines, without a trip through LDS.
+  float* o_part;
   const float* o_add;
   float* ws_state;
   float* ws_decay;

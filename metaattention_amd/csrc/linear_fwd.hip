@@ -605,23 +605,31 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
 
     f32x16 o_out;         // outputs of chunk c - 1, written while chunk c is under way: nobody waits for the stores
     // What is added to a chunk's outputs (o_add) is asked for when they are there and the state loop's operand registers are free
-    // again, and waited for where they are written, behind the next chunk's first reads.
+    // again, and waited for where they are written, behind the next chunk's first reads.  (Asked for in the middle of the state loop,
+    // with V^T P^T behind it, it is no faster: what these passes wait for is memory, 4.5 - 4.9 TB/s.)
     f32x4 add[4];
     const bool adds = GEN && !HELP && a.o_add != nullptr;
-    auto load_add = [&](int t0) {
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
-      const int r = ln & 31, g = ln >> 5, t = min(t0 + r, Tn - 1);
-      const float* src = a.o_add + ((int64_t)bh * Tn + (rev_o ? Tn - 1 - t : t)) * a.Dv + dvb * (32 * NWH) + 32 * (wave % NWH) + 4 * g;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) add[q4] = *(const f32x4*)(src + 8 * q4);
+    // the wave's 32 x 32 block of chunk c in the order of its accumulators: four rows of 64 lanes x 16 bytes
+    auto part_at = [&](const float* part, int c) {
+      return (f32x4*)(part + ((((int64_t)bh * a.dv_blocks + dvb) * n_chunks_all + c) * NW + wave) * (16 * 64));
     };
-    auto finish = [&](int t0, uint32_t vbase) {
+    auto load_add = [&](int c) {
+      const f32x4* src = part_at(a.o_add, c);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) add[q4] = src[64 * q4 + lane];
+    };
+    auto finish = [&](int c, uint32_t vbase) {
       if (adds) {
 #pragma unroll
         for (int j = 0; j < 16; j++) o_out[j] += add[j >> 2][j & 3];
       }
-      write_out(o_out, t0, vbase);
+      if (GEN && !HELP && a.o_part) {
+        f32x4* dst = part_at(a.o_part, c);
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) dst[64 * q4 + lane] = f32x4{o_out[4 * q4], o_out[4 * q4 + 1], o_out[4 * q4 + 2], o_out[4 * q4 + 3]};
+      } else {
+        write_out(o_out, c * L, vbase);
+      }
     };
     // a state wave's work of chunk c
     auto run_chunk = [&](int c, int buf) {
@@ -656,7 +664,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       f32x4 w4[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) w4[i] = lds_read<f32x4>(sh + kScalW + 16 * g + 32 * i);
-      if (!HELP && c > c_begin) finish(t0 - L, vbase);
+      if (!HELP && c > c_begin) finish(c - 1, vbase);
 
       const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       f32x16 o_intra = E::mfma32(vf[0], pf0, zero16);
@@ -675,7 +683,9 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
 
       // ---- per 32-row state block: inter-chunk product with the OLD state (as bf16 operand), decay, state update.  The
       //      conversion and the decay of the next block are dealt into the gaps behind the four MFMAs of this block, operands
-      //      are requested one block ahead.
+      //      are requested one block ahead.  The chunk's loads go out with the first half of the blocks (the last ones of a chunk are
+      //      waited for at its end: over all blocks, 8 x 16 heads, 2048 tokens, 256 / 512 forward and backward took 1017 us, like this 1005;
+      //      not with helpers, which have a stage more to land in: Mamba2's scan 86 and 87 us).
       if (loads && !whole) issue_rows(t2, base2);
       const uint32_t qpa = qbase + r * RBQ + (uint32_t)(((2 * g) ^ swz16(r)) << 4);
       const uint32_t kta = kbase + (4 * g + jr) * RBQ + ((ln >> 1) & 1) * 8 + (uint32_t)(((((ln & 1) << 1) | ((ln >> 4) & 1)) ^ swz16(4 * g + jr)) << 4);
@@ -732,7 +742,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
           }
 #pragma unroll
           for (int x = 0; x < NL; x++)
-            if (x * KB / NL == bb) load_one(x, t2, base2, on);
+            if (x * (HELP ? KB : KB / 2) / NL == bb) load_one(x, t2, base2, on);
         }
       }
 #pragma unroll
@@ -747,7 +757,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
       // chunk c + 2 must be there for P^T of c + 2, made in c + 1: with four stages it was asked for a chunk ago and the loads of this
       // chunk may go on; with three, its V, not read before c + 2, may
       if (adds) {
-        load_add(t0);
+        load_add(c);
       } else {
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++) add[q4] = f32x4{0.f, 0.f, 0.f, 0.f};     // (not carried through the chunk)
@@ -777,7 +787,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
         __syncthreads();
         buf = buf == NST - 1 ? 0 : buf + 1;
       }
-      if (!HELP && c_begin < c_end) finish((c_end - 1) * L, lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE + 2 * QT);
+      if (!HELP && c_begin < c_end) finish(c_end - 1, lds0 + (uint32_t)(buf == 0 ? NST - 1 : buf - 1) * STAGE + 2 * QT);
     }
   }
   if constexpr (!PIPE) {
@@ -1088,7 +1098,7 @@ struct Config {
   }
 
   // workgroups of a single pass
-  static int64_t groups(const LinArgs& a) { return (int64_t)a.B * a.H / HG * (a.Dv / (32 * NWH)) * (a.n_pieces > 1 ? a.n_pieces : 1); }
+  static int64_t groups(const LinArgs& a) { return (a.bg_n > 0 ? a.bg_n : (int64_t)a.B * a.H / HG) * (a.Dv / (32 * NWH)) * (a.n_pieces > 1 ? a.n_pieces : 1); }
 
   // Number of segments and chunks per segment for this problem.  want: 0 = choose, n >= 1 = at most n.
   // Chosen: as many segments as keep every CU's resident workgroup slots busy.  A chunk is a chain of 2 - 4 us however few
@@ -1146,7 +1156,7 @@ struct Config {
   // general operand addressing: defaults for what is left at zero; the row distances must be multiples of the tile
   // rows (the kernel XORs the swizzle of an instruction's first row onto the finished lane offset)
   static bool general(const LinArgs& a) {
-    return a.rev != 0 || a.q_row != 0 || a.k_row != 0 || a.v_row != 0 || (a.Hv != 0 && a.Hv != a.H) || a.qk_cols != 0 || a.n_pieces > 1 || a.rev_o != 0 || a.o_add != nullptr;
+    return a.rev != 0 || a.q_row != 0 || a.k_row != 0 || a.v_row != 0 || (a.Hv != 0 && a.Hv != a.H) || a.qk_cols != 0 || a.n_pieces > 1 || a.rev_o != 0 || a.o_add != nullptr || a.o_part != nullptr;
   }
   static int fill(LinArgs& a) {
     a.dv_blocks = a.Dv / (32 * NWH);
@@ -1158,7 +1168,7 @@ struct Config {
     if (a.qk_cols < 0 || a.qk_cols > DK || a.qk_cols % 32 != 0) return -2;
     if (HG > 1 && a.Hv != a.H) return -2;
     if (a.n_pieces > 1 && !a.out_f32) return -2;
-    if (a.o_add && (!pipelined<NWH, HG, 0>() || helpers<DK, NWH, HG, 0>() > 0 || a.out_f32)) return -2;
+    if ((a.o_add || a.o_part) && (!pipelined<NWH, HG, 0>() || helpers<DK, NWH, HG, 0>() > 0 || a.out_f32)) return -2;
     return 0;
   }
 

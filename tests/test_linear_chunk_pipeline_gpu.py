@@ -93,7 +93,7 @@ def test_later_keys_and_decays_stay_out(layout, bad):
 @pytest.mark.parametrize("T", [1, 33, 96, 130])
 @pytest.mark.parametrize("B,Hq,H,Dk,Dv,scaled", [
     (1, 2, 2, 256, 256, False), (2, 2, 2, 128, 128, False), (1, 2, 2, 64, 64, False), (1, 2, 2, 192, 256, False),   # one piece: the scans write dq and dk
-    (8, 16, 16, 256, 512, False), (4, 32, 32, 128, 512, False), (8, 16, 16, 256, 768, False),                       # equal pieces in turn
+    (8, 16, 16, 256, 512, False), (3, 43, 43, 256, 512, False), (4, 32, 32, 128, 512, False), (8, 16, 16, 256, 768, False),                       # equal pieces in turn
     (1, 2, 2, 256, 512, False), (8, 16, 16, 192, 512, False), (1, 2, 2, 256, 320, False),                           # pieces side by side, unequal pieces
     (2, 1, 4, 128, 64, True), (1, 2, 2, 256, 512, True),                                                            # shared heads, a value scale
 ])
