@@ -114,7 +114,7 @@ constexpr int fused_stages(int dqk, int dv) { return 8 * (32 * (dqk + dv) * 2 + 
 // instructions, LDS latencies and a barrier, and one wave per SIMD waits for most of it: two workgroups (256 registers a wave,
 // lse and delta requested in the step that uses them) take B4 H32 S2048 causal forward + backward from 595 to 438 us (sigmoid)
 // and 557 to 421 us (softmax), B8 H32 S4096 3984 -> 3353 and 3723 -> 3130.  The larger sizes need a SIMD's 512 registers.
-constexpr int fused_per_cu(int dqk, int dv) { return dqk + dv <= 128 ? 2 : 1; }
+constexpr int FUSED_PER_CU = 2;
 // Waits until at most N of this wave's vector-memory loads are outstanding (they complete in order).
 template <int N>
 __device__ __forceinline__ void wait_dma_but() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
@@ -850,12 +850,10 @@ struct PhaseF {
 // stages of their own, as two runs would; at the end one keeps dk and the other dv, and each hands the other one over through LDS.
 // PARTS: n_parts > 1 (an instantiation of its own: the walk over a run's tiles costs the one-run loop 3 % at 64 / 64).
 template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool MASKS, bool PARTS, int STREAMS = 1>
-__global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd_dkv_fused_kernel(const AttnBwdArgs a) {
+__global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fused_kernel(const AttnBwdArgs a) {
   using E = Elem<T>;
   using x8 = typename E::x8;
   using x4 = typename E::x4;
-  // (with a second wave on the SIMD the row values are requested in the step that uses them: 32 registers less)
-  constexpr bool ROWS_AHEAD = fused_per_cu(DQK, DV) == 1;
   constexpr int BNW = 128, BMT = 32;
   constexpr int KS = DQK / 16, VS = DV / 16, QB = DQK / 32, VB = DV / 32;
   constexpr int QROW = pad_width(DQK) * 2, DOROW = DV * 2;   // (LDS rows; 192-wide queries sit in 256-wide rows)
@@ -867,16 +865,13 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
   constexpr int STREAM_LDS = (MASKS ? LIST_N + 4 : ROWVALS + NST * 512) + 1023 & ~1023;
   // the MFMAs of a step and the fragment ring
   constexpr int NF = KS + VS, NV = 2 * VB, NK = 2 * QB, NTOT = NF + NV + NK;
-  // (128 / 128 in runs, whose loop has the registers for it: further ahead, 205 -> 199 us at B2 H32 Hkv8 S2047; without runs the longer
-  // ring moves accumulators about, 161 -> 182 at B2 H32 S1600)
-  constexpr bool LONG = DQK == 128 && DV == 128 && PARTS && !MASKS;
-  constexpr int RING = LONG ? 16 : 8, AH = LONG ? 8 : !ROWS_AHEAD && FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
+  constexpr int RING = 8, AH = FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
   static_assert(NTOT % RING == 0 && AH < RING && AH <= NK && AH <= NF, "fragment ring");
   using PhF = PhaseF<KS, VS>;
 
   extern __shared__ __align__(16) char smem[];
   constexpr bool WALK = PARTS || STREAMS > 1;
-  static_assert(STREAMS == 1 || (STREAMS == 2 && !ROWS_AHEAD), "two streams share a SIMD");
+  static_assert(STREAMS <= 2, "two streams share a SIMD");
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int stream = STREAMS > 1 ? wave_all >> 2 : 0, wave = STREAMS > 1 ? wave_all & 3 : wave_all;   // wave: within its stream
   const uint32_t lds_all = (uint32_t)(uintptr_t)(MA_LDS char*)smem, lds0 = lds_all + (STREAMS > 1 ? stream * (uint32_t)STREAM_LDS : 0u);
@@ -929,16 +924,6 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
     const T* vp = (const T*)a.v + (int64_t)b * a.vsb + (int64_t)n_ld * a.vss + (int64_t)hk * a.vsh + 8 * g;
 #pragma unroll
     for (int sl = 0; sl < VS; sl++) vf[sl] = *(const x8*)(vp + 16 * sl);
-    if constexpr (ROWS_AHEAD && DQK + DV <= 256) {      // (192 / 128, which spills either way, is no faster)
-      // (in accumulation registers, where only MFMAs read them: the scores then get vector registers, which the row function reads
-      // without moves.  One wave on a SIMD issues an instruction at a time, and that bounds the loop: of 412 k clocks a wave at B2
-      // H32 Hkv8 S2047, 250 k were issue, 140 k of those MFMAs' time.  With the MFMAs in their vector-register form, which the build
-      // asks for in this file's unit of 128 / 128: 214 -> 205 us)
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) asm volatile("" : "+a"(kf[ks]));
-#pragma unroll
-      for (int sl = 0; sl < VS; sl++) asm volatile("" : "+a"(vf[sl]));
-    }
   }
   f32x16 dk[QB], dv[VB];
 #pragma unroll
@@ -1049,17 +1034,6 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
 #pragma unroll
       for (int q4 = 0; q4 < 4; q4++) x.td[q4] = lds_read<f32x4>(lds0 + ROWVALS + st * 512 + 256 + (8 * q4 + 4 * g) * 4);
   };
-  auto rowvals = [&](int st, FusedStepRegs<T>& x) {
-    if constexpr (FAMILY == BF_SOFTMAX) {
-      const uint32_t rv = lds0 + ROWVALS + st * 512;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) {
-        x.tl[q4] = lds_read<f32x4>(rv + (8 * q4 + 4 * g) * 4);
-        x.td[q4] = lds_read<f32x4>(rv + 256 + (8 * q4 + 4 * g) * 4);
-      }
-    }
-  };
-
   // the lane's part of the fragment addresses, relative to a tile: row reads (A operands of S and dP) and
   // transposing reads (A operands of dV^T and dK^T: the tile's columns)
   const uint32_t aq_l = (uint32_t)(r * QROW) + (uint32_t)((g ^ swz_tile<QROW / 16>(r)) << 4);
@@ -1123,7 +1097,6 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
     FusedStepRegs<T> ra, rb;
     ra.s = mm_rows<T, DQK>(lds0, r, g, kf);
     ra.dp = mm_rows<T, DV>(lds0 + QTILE, r, g, vf);
-    if (ROWS_AHEAD) rowvals(0, ra);
     x8 fr[RING];
     static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, lds0, lds0 + STAGE); });   // (of step 0)
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1138,8 +1111,7 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
       const uint32_t nn_tile = lds0 + (uint32_t)(((u + 2) & (NST - 1)) * STAGE);
       const int m0 = real ? (t_first + (MASKS ? (int)(c_entry & 0xffffu) : at.t)) * BMT : a.Sq;
       if (!MASKS) at.template next<WALK>(n_runs, t_count, a.kv_group);
-      if (ROWS_AHEAD) rowvals((u + 1) & (NST - 1), nxt);   // (requested here, needed in the next step)
-      else row_lse(u & (NST - 1), cur);
+      row_lse(u & (NST - 1), cur);      // (row values are requested in the step that uses them: 32 registers less, with a second wave on the SIMD)
       // the tiles that touch the diagonal, an end of the sequences or an element-wise mask (the test is wave-uniform)
       const bool by_elem = MASKS && real && a.elem_mask_t && (c_entry >> 31) == 0;
       if ((CAUSAL && n_wave + 31 > m0) || m0 + BMT > a.Sq || n_wave + 32 > a.Skv || by_elem) {
@@ -1192,7 +1164,7 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
           asm volatile("" ::: "memory");
           if (i_n < n_steps) issue_next();
         }
-        if constexpr (!ROWS_AHEAD && j == NF - 2) row_delta(u & (NST - 1), cur);
+        if constexpr (j == NF - 2) row_delta(u & (NST - 1), cur);
         // the fragment of the MFMA AH places on (the last ones of the step: of the next step's first MFMAs)
         if constexpr (j + AH < NTOT) fr[(j + AH) % RING] = fragment(IntC<j + AH>(), cur_tile, nxt_tile);
         else fr[(j + AH) % RING] = fragment(IntC<j + AH - NTOT>(), nxt_tile, nn_tile);
@@ -1277,6 +1249,368 @@ __global__ __launch_bounds__(256 * STREAMS, fused_per_cu(DQK, DV)) void attn_bwd
   store_rows<T, DQK>(dk, a.scale, stage, dkb, a.dkss, n_wave, a.Skv, lane);
   store_rows<T, DV>(dv, 1.f, stage, dvb, a.dvss, n_wave, a.Skv, lane);
   __syncthreads();   // the staged output has left the stages: the next key block's tiles may arrive
+  }   // the item's key blocks
+  }   // items
+}
+
+// ------------------------------------------------------------------------------------------------
+// dk and dv in one launch: two waves per SIMD, one for dv and one for dk
+// ------------------------------------------------------------------------------------------------
+// The work of the kernel above without its masks, where the accumulators of one product and the fragments of one operand fit half a
+// SIMD's registers: eight waves take 128 keys, two waves the same 32 of them, on one SIMD.  For every tile u of 32 query rows
+//   wave A   S(u+1) = Q(u+1) K^T with p(u) behind its MFMAs, p(u) to the partner through LDS (fp32);  dV^T += dO(u)^T P(u)
+//   wave B   dP(u+1) = dO(u+1) V^T with ds(u) behind its MFMAs;                                       dK^T += Q(u)^T dS(u)
+// as many MFMAs each whatever the head sizes.  One barrier a tile, between the two halves of A's step and in front of B's: between
+// two barriers A runs its pure MFMA half beside B's row function and then its own row function beside B's pure MFMA half.
+// What bounded the one-wave kernel was issue: 250 k of 412 k clocks a wave, one instruction at a time, the matrix pipe idle for the rest.
+// B2 H32 Hkv8 S2047 128/128 causal 198 -> 170 us = 0.89 PFLOP/s of MFMAs (40 % of the cycles at 2.07 GHz; the LDS is busy for 32 %, without
+// conflicts).  From there on longer and shorter rings (4, 5 or 7 MFMAs ahead), p written earlier and fewer scalar instructions change
+// 1 % or nothing: the forward kernel's 1.1 PFLOP/s at the clock that random operands leave is near.  Forward + backward B8 H32 S4096
+// 5740 -> 5120 us, B2 H16 S1600 159 -> 144, B2 H32 Hkv8 S1500 sigmoid without a mask 443 -> 389, B4 H16 S1024 192/128 179 -> 163.
+// Ring of NST stages: behind barrier u the tiles u, u + 1 and u + 2 are read, and the stage of tile u - 1 takes tile u + NST - 1.
+// The same products in the same order as the kernel above: the same bits.
+// MASKS: as in the kernel above, from a list of the steps in LDS; wave A reads the mask.
+constexpr int pair_stages(int dqk, int dv, bool masks) { return (pad_width(dqk) + dv <= 256 ? 6 : 5) - masks; }
+constexpr size_t pair_lds(int dqk, int dv, bool masks) {
+  return pair_stages(dqk, dv, masks) * (32 * (size_t)(pad_width(dqk) + dv) * 2 + 512 + (masks ? 4 * 1024 : 0)) + 2 * 4 * 4096 + (masks ? FUSED_LIST_MAX * 4 + 16 : 0);
+}
+
+template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL, bool MASKS, bool PARTS>
+__global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwdArgs a) {
+  using E = Elem<T>;
+  using x8 = typename E::x8;
+  using x4 = typename E::x4;
+  constexpr int BNW = 128, BMT = 32;
+  constexpr int QROW = pad_width(DQK) * 2, DOROW = DV * 2;   // (LDS rows; 192-wide queries sit in 256-wide rows)
+  // a stage: the Q tile, the dO tile, lse (first 128 bytes) and delta (at 256) of its rows
+  constexpr int QTILE = BMT * QROW, DOTILE = BMT * DOROW, ROWVALS = QTILE + DOTILE, STAGE = ROWVALS + 512;
+  constexpr int NST = pair_stages(DQK, DV, MASKS), XCHG = NST * STAGE;
+  // (MASKS) behind the exchanged p: 1 KB of mask bytes per stage and wave, then the step list and its length
+  constexpr int KEEP = XCHG + 2 * 4 * 4096, LIST = KEEP + NST * 4 * 1024, LIST_N = LIST + FUSED_LIST_MAX * 4;
+  static_assert(NST >= 4 && pair_lds(DQK, DV, MASKS) <= 160 * 1024 && STAGE % QROW == 0 && STAGE % DOROW == 0 && 8 * 32 * ((DQK > DV ? DQK : DV) + 16) <= NST * STAGE, "LDS");
+
+  extern __shared__ __align__(16) char smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
+  const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3;
+  const int r = lane & 31, g = lane >> 5, jr = (lane & 15) >> 2, lc = (((lane >> 4) & 1) << 1) | ((lane & 3) >> 1);
+
+  // persistent, items as in the kernel above
+  const int nnb = a.num_blocks, BHK = a.B * a.Hkv, n_parts = PARTS ? a.n_parts : 1;
+  const int per_bh = (CAUSAL ? (nnb + 1) / 2 : nnb) * n_parts, n_items = BHK * per_bh;
+  const float bias = a.bias + (a.bias_ptr ? *a.bias_ptr : 0.f);
+  const float c_scale = a.scale * kLog2e, c_bias = bias * kLog2e;
+  const float s_masked = a.scale >= 0.f ? -__builtin_inff() : __builtin_inff();   // a score whose p is 0
+  const int64_t q_row_bytes = a.qss * 2, do_row_bytes = a.doss * 2;
+  TileDma<QROW, 8, DQK / 8> q_dma;
+  TileDma<DOROW, 8> do_dma;
+  q_dma.init((uint32_t)q_row_bytes, wave_all, lane);
+  do_dma.init((uint32_t)do_row_bytes, wave_all, lane);
+  constexpr int TILE_DMAS = TileDma<QROW, 8>::NJ + TileDma<DOROW, 8>::NJ;   // what a wave issues per tile at least (see above)
+
+  for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+  int bhk, ki, run;
+  if ((BHK & 7) == 0) {
+    const int slot = item >> 3;
+    bhk = (slot / per_bh) * 8 + (item & 7);
+    ki = slot % per_bh;
+    run = ki % n_parts;
+    ki /= n_parts;
+    if (MASKS) ki = (ki + slot / per_bh) % nnb;      // (another key block each time round, see above)
+  } else {
+    bhk = item / per_bh;
+    ki = item % per_bh;
+    run = ki % n_parts;
+    ki /= n_parts;
+    if (MASKS) ki = (ki + bhk) % nnb;
+  }
+  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
+  for (int part = 0; part < (CAUSAL && ki != nnb - 1 - ki ? 2 : 1); part++) {
+  const int nb = part == 0 ? ki : nnb - 1 - ki;
+  const int n_wave = nb * BNW + wave * 32, n_lane = n_wave + r;
+  const int n_ld = min(n_lane, a.Skv - 1);
+
+  const int t_first = CAUSAL ? (nb * BNW) / BMT : 0;
+  const int t_count = (a.Sq + BMT - 1) / BMT - t_first;
+  int n_steps = t_count > 0 ? t_count * a.kv_group : 0;
+  DkvWalk first{0, 0, 0};
+  if (PARTS && !MASKS && n_steps > 0) {
+    const int each = t_count / n_parts, more = t_count % n_parts;
+    first.skip = ((run - t_first) % n_parts + n_parts) % n_parts;
+    n_steps = 0;
+    for (int hg = 0, skip = first.skip; hg < a.kv_group; hg++, skip = skip == 0 ? n_parts - 1 : skip - 1) n_steps += each + (skip < more ? 1 : 0);
+    first.to_tile(first.skip, n_parts, t_count, a.kv_group);
+  }
+  const bool keep_ok = MASKS && a.elem_mask_t && ((a.emt_sk | a.emt_sb | a.emt_sh | (int64_t)(uintptr_t)a.elem_mask_t) & 15) == 0;
+  if constexpr (MASKS) {
+    // the step list: entry = tile | head of the group << 16 | kept in full << 31
+    const uint8_t* qbm = a.q_block_mask ? a.q_block_mask + (int64_t)b * a.qbm_sb + (int64_t)nb * a.qbm_sk : nullptr;
+    if (wave_all == 0) {
+      int count = 0;
+      for (int i0 = 0; i0 < n_steps; i0 += 64) {
+        const int i = i0 + lane;
+        bool keep = false;
+        uint32_t entry = 0;
+        if (i < n_steps) {
+          const int hg = i / t_count, t = i - hg * t_count;
+          const uint8_t e = qbm ? qbm[(int64_t)(hk * a.kv_group + hg) * a.qbm_sh + t] : (uint8_t)1;
+          keep = e != 0 && (!PARTS || (t + hg) % n_parts == run);
+          entry = (uint32_t)t | ((uint32_t)hg << 16) | (e >= 2 || !a.elem_mask_t ? 0x80000000u : 0u);
+        }
+        const uint64_t votes = __ballot(keep);
+        if (keep) lds_write<uint32_t>(lds0 + LIST + 4 * (count + __popcll(votes & ((1ull << lane) - 1ull))), entry);
+        count += __popcll(votes);
+      }
+      if (lane == 0) lds_write<uint32_t>(lds0 + LIST_N, (uint32_t)count);
+    }
+    __syncthreads();
+    n_steps = __builtin_amdgcn_readfirstlane((int)lds_read<uint32_t>(lds0 + LIST_N));
+  }
+  // (list entries are requested a step before they are used and made wave-uniform only then)
+  auto list_request = [&](int i) { return lds_read<uint32_t>(lds0 + LIST + 4 * (i < n_steps ? i : 0)); };
+  auto uniform = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+  auto entry_walk = [&](uint32_t e) { return DkvWalk{(int)((e >> 16) & 0x7fffu), (int)(e & 0xffffu), 0}; };
+  // The next tile to fetch: a run's tiles of a head follow each other at fixed distances, so that its rows' addresses are sums.
+  // (Made anew for every tile they are 48 scalar instructions behind the barrier, where no MFMA is under way.)
+  struct Fetch {
+    DkvWalk w;
+    const char *q, *d;
+    const float *lse, *delta;
+  } fetch;
+  const int64_t q_step = (int64_t)(BMT * n_parts) * q_row_bytes, do_step = (int64_t)(BMT * n_parts) * do_row_bytes;
+  const int t_whole = a.Sq / BMT - t_first;      // (tiles of a head that lie inside the sequence)
+  auto fetch_at = [&](DkvWalk w) {
+    const int h = hk * a.kv_group + w.hg;
+    const int64_t m0 = (int64_t)(t_first + w.t) * BMT, row = ((int64_t)b * a.H + h) * a.Sq + m0;
+    fetch.w = w;
+    fetch.q = (const char*)((const T*)a.q + (int64_t)b * a.qsb + (int64_t)h * a.qsh) + m0 * q_row_bytes;
+    fetch.d = (const char*)((const T*)a.dout + (int64_t)b * a.dosb + (int64_t)h * a.dosh) + m0 * do_row_bytes;
+    fetch.lse = a.lse + row;
+    fetch.delta = (const float*)a.delta + row;
+  };
+  auto issue_tile = [&](uint32_t to, bool full) {
+    if constexpr (MASKS) {
+      // the transposed element-wise keep mask of A's keys: whole tiles of a 16-byte aligned mask come with the Q / dO tile
+      const int m0 = (t_first + fetch.w.t) * BMT, h = hk * a.kv_group + fetch.w.hg;
+      if (wave_all < 4 && keep_ok && !full && m0 + BMT <= a.Sq && n_wave < a.Skv)
+        keep_dma(a.elem_mask_t + (int64_t)b * a.emt_sb + (int64_t)h * a.emt_sh + (int64_t)n_wave * a.emt_sk + m0, a.emt_sk, a.Skv - n_wave,
+                 lds0 + KEEP + ((to - lds0) / STAGE * 4 + wave) * 1024, lane);
+    }
+    const int rows = fetch.w.t < t_whole ? BMT : a.Sq % BMT;   // (wave-uniform)
+    if (rows == BMT) {
+      q_dma.issue(fetch.q, to, wave_all);
+      do_dma.issue(fetch.d, to + QTILE, wave_all);
+    } else {
+      dma_tile<QROW, 8, DQK / 8>(fetch.q, q_row_bytes, 0, rows, to, wave_all, lane);
+      dma_tile<DOROW, 8>(fetch.d, do_row_bytes, 0, rows, to + QTILE, wave_all, lane);
+    }
+    if constexpr (FAMILY == BF_SOFTMAX) {
+      // wave 0 fetches lse, wave 1 delta (the upper lanes repeat the lower ones)
+      if (wave_all < 2) dma4_so(wave_all == 0 ? fetch.lse : fetch.delta, (uint32_t)min(lane & 31, rows - 1) * 4u, to + ROWVALS + wave_all * 256);
+    }
+    if constexpr (MASKS) return;
+    DkvWalk w = fetch.w;
+    w.next<PARTS>(n_parts, t_count, a.kv_group);
+    if (w.hg == fetch.w.hg) {
+      fetch.w = w;
+      fetch.q += q_step;
+      fetch.d += do_step;
+      if constexpr (FAMILY == BF_SOFTMAX) {
+        fetch.lse += BMT * n_parts;
+        fetch.delta += BMT * n_parts;
+      }
+    } else if (w.hg < a.kv_group) {
+      fetch_at(w);
+    }
+  };
+
+  auto work = [&](auto role) __attribute__((always_inline)) {
+    constexpr bool ROLE_B = decltype(role)::value != 0;
+    // rows of one tile against the wave's fragments make the scores, the columns of the other the accumulators
+    constexpr int DR = ROLE_B ? DV : DQK, DC = ROLE_B ? DQK : DV;
+    constexpr int RROW = ROLE_B ? DOROW : QROW, CROW = ROLE_B ? QROW : DOROW, ROFF = ROLE_B ? QTILE : 0, COFF = ROLE_B ? 0 : QTILE;
+    constexpr int NR = DR / 16, CB = DC / 32, NTOT = NR + 2 * CB, RING = NTOT % 8 == 0 ? 8 : 4, AH = RING == 8 ? 5 : 3;
+    static_assert(NTOT % RING == 0 && AH <= NR && AH <= 2 * CB, "fragment ring");
+    x8 wf[NR];
+    {
+      const T* p = ROLE_B ? (const T*)a.v + (int64_t)b * a.vsb + (int64_t)n_ld * a.vss + (int64_t)hk * a.vsh + 8 * g
+                          : (const T*)a.k + (int64_t)b * a.ksb + (int64_t)n_ld * a.kss + (int64_t)hk * a.ksh + 8 * g;
+#pragma unroll
+      for (int i = 0; i < NR; i++) wf[i] = *(const x8*)(p + 16 * i);
+    }
+    f32x16 acc[CB];
+#pragma unroll
+    for (int i = 0; i < CB; i++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) acc[i][j] = 0.f;
+
+    if (n_steps > 0) {
+      const uint32_t row_l = ROFF + (uint32_t)(r * RROW) + (uint32_t)((g ^ swz_tile<RROW / 16>(r)) << 4);
+      const uint32_t col_l = COFF + (uint32_t)((4 * g + jr) * CROW + (lane & 1) * 8) + (uint32_t)((lc ^ swz_tile<CROW / 16>(4 * g + jr)) << 4);
+      // the fragment of MFMA j of a step: the row reads from `rows`, the transposing reads from `cols` (stages)
+      auto fragment = [&](auto jc, uint32_t rows, uint32_t cols) __attribute__((always_inline)) -> x8 {
+        constexpr int j = decltype(jc)::value;
+        if constexpr (j < NR) {
+          return lds_read<x8>((rows + row_l) ^ (uint32_t)(j * 32));
+        } else {
+          constexpr int db = (j - NR) % CB, sl = (j - NR) / CB;
+          const x4 lo = lds_read_tr4<T>(((cols + col_l) ^ (uint32_t)((4 * db) << 4)) + 16 * sl * CROW);
+          const x4 hi = lds_read_tr4<T>(((cols + col_l) ^ (uint32_t)(((4 * db) ^ 2) << 4)) + (16 * sl + 8) * CROW);
+          return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      };
+      const uint32_t x_l = lds0 + XCHG + wave * 4096 + lane * 16;      // p of the even tiles, 16 KB on of the odd ones
+      f32x4 rv[4];      // lse (A) or delta (B) of the rows 8 q4 + 4 g + {0..3} of the step's tile
+      auto row_values = [&](uint32_t tile) {
+        if constexpr (FAMILY == BF_SOFTMAX)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; q4++) rv[q4] = lds_read<f32x4>(tile + ROWVALS + (ROLE_B ? 256 : 0) + (8 * q4 + 4 * g) * 4);
+      };
+
+      DkvWalk at = first;      // the current step's tile
+      if (!MASKS) fetch_at(first);
+      uint32_t i_next = MASKS ? list_request(0) : 0u, c_next = i_next;      // (MASKS) the entries of the next tile to fetch and of the next step
+      int i_n = 0;
+      uint32_t to = lds0;
+      auto after = [&](uint32_t stage) { return stage == lds0 + (NST - 1) * STAGE ? lds0 : stage + STAGE; };
+      auto issue_next = [&]() {
+        bool full = true;
+        if constexpr (MASKS) {
+          const uint32_t e = uniform(i_next);
+          fetch_at(entry_walk(e));
+          full = (e >> 31) != 0;
+        }
+        issue_tile(to, full);
+        to = after(to);
+        i_n++;
+        if constexpr (MASKS) i_next = list_request(i_n);
+      };
+#pragma unroll
+      for (int i = 0; i < NST - 1; i++)
+        if (i_n < n_steps) issue_next();
+      wait_dma();
+      __syncthreads();
+      uint32_t t0 = lds0, t1 = lds0 + STAGE, t2 = lds0 + 2 * STAGE;      // the stages of tiles u, u + 1, u + 2
+      f32x16 sa = mm_rows<T, DR>(t0 + ROFF, r, g, wf), sb;
+      x8 fr[RING];
+      static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, t1, t0); });
+      row_values(t0);
+      const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+      auto body = [&](int u, f32x16& cur, f32x16& nxt) __attribute__((always_inline)) {
+        if constexpr (!ROLE_B) {
+          const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
+          if constexpr (MASKS) {
+            c_next = list_request(u + 1);
+            at = entry_walk(c_entry);
+          }
+          const int m0 = (t_first + at.t) * BMT;
+          if (!MASKS) at.template next<PARTS>(n_parts, t_count, a.kv_group);
+          const bool by_elem = MASKS && a.elem_mask_t && (c_entry >> 31) == 0;
+          if ((CAUSAL && n_wave + 31 > m0) || m0 + BMT > a.Sq || n_wave + 32 > a.Skv || by_elem) {
+            int m0e = m0;
+            asm volatile("; a tile that touches a mask" : "+s"(m0e));      // (see the kernel above)
+            uint32_t keep[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};   // the bytes of this lane's four rows per group
+            if constexpr (MASKS) {
+              if (by_elem) {
+                if (keep_ok && m0e + BMT <= a.Sq && n_wave < a.Skv) {
+#pragma unroll
+                  for (int q4 = 0; q4 < 4; q4++) keep[q4] = keep_read(lds0 + KEEP + ((t0 - lds0) / STAGE * 4 + wave) * 1024, r, g, q4);
+                } else {
+                  // this key's row of the transposed mask, indexed by query position
+                  const uint8_t* emt_row = a.elem_mask_t + (int64_t)b * a.emt_sb + (int64_t)(hk * a.kv_group + at.hg) * a.emt_sh + (int64_t)n_ld * a.emt_sk;
+#pragma unroll
+                  for (int q4 = 0; q4 < 4; q4++) {
+                    const int m = m0e + 8 * q4 + 4 * g;
+                    keep[q4] = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                      if (m + i < a.Sq) keep[q4] |= (uint32_t)emt_row[m + i] << (8 * i);
+                  }
+                }
+              }
+            }
+#pragma unroll
+            for (int jj = 0; jj < 16; jj++) {
+              const int m = m0e + 8 * (jj >> 2) + 4 * g + (jj & 3);
+              if ((CAUSAL && n_lane > m) || m >= a.Sq || n_lane >= a.Skv || (MASKS && ((keep[jj >> 2] >> (8 * (jj & 3))) & 0xffu) == 0)) {
+                cur[jj] = s_masked;
+                // (a row without any kept key has lse = -inf: its masked scores must still give p = 0)
+                if constexpr (FAMILY == BF_SOFTMAX) rv[jj >> 2][jj & 3] = 0.f;
+              }
+            }
+          }
+        }
+        const uint32_t x = x_l + (u & 1) * 16384;
+        x8 f[2];
+        f32x4 p4[4];
+        static_for<0, NTOT>([&](auto jc) __attribute__((always_inline)) {
+          constexpr int j = decltype(jc)::value;
+          if constexpr (j == (ROLE_B ? 0 : NR)) {
+            // tile u + 2 has landed (what may still be in flight: the tiles behind it), p(u) is in LDS, and every wave is done with
+            // tile u - 1, whose stage takes tile u + NST - 1
+            if (u + NST - 2 < n_steps) wait_dma_but<(NST - 4) * TILE_DMAS>();
+            else wait_dma();
+            if constexpr (!ROLE_B) __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if constexpr (ROLE_B) {
+#pragma unroll
+              for (int q4 = 0; q4 < 4; q4++) p4[q4] = lds_read<f32x4>(x + q4 * 1024);
+            }
+          }
+          if constexpr (j == (ROLE_B ? 2 : NR + 2))      // (two MFMAs on: behind the barrier itself, B2 H16 S1600 148 us for 144)
+            if (i_n < n_steps) issue_next();
+          if constexpr (j == NTOT - 4) row_values(t1);
+          // the fragment of the MFMA AH places on (the last ones of the step: of the next step's first MFMAs)
+          if constexpr (j + AH < NTOT) fr[(j + AH) % RING] = fragment(IntC<j + AH>(), t1, t0);
+          else fr[(j + AH) % RING] = fragment(IntC<j + AH - NTOT>(), t2, t1);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (j < NR) nxt = E::mfma32(fr[j % RING], wf[j], j == 0 ? zero16 : nxt);
+          else acc[(j - NR) % CB] = E::mfma32(fr[j % RING], f[(j - NR) / CB], acc[(j - NR) % CB]);
+          // vector work behind the MFMA: p, or ds, of the step's 16 elements (ds from the second MFMA on: its p come from LDS)
+          if constexpr (j < NR) {
+            constexpr int J0 = ROLE_B ? 2 : 0;
+            constexpr int from = j < J0 ? 0 : (j - J0) * 16 / (NR - J0), upto = j < J0 ? 0 : (j + 1 - J0) * 16 / (NR - J0);
+#pragma unroll
+            for (int jj = from; jj < upto; jj++) {
+              if constexpr (!ROLE_B) {
+                p4[jj >> 2][jj & 3] = row_p<FAMILY>(cur[jj], c_scale, c_bias, a.scale, bias, FAMILY == BF_SOFTMAX ? fmaf(rv[jj >> 2][jj & 3], -kLog2e, c_bias) : 0.f);
+                f[jj >> 3][jj & 7] = (T)p4[jj >> 2][jj & 3];
+                if ((jj & 3) == 3) lds_write<f32x4>(x + (jj >> 2) * 1024, p4[jj >> 2]);
+              } else {
+                f[jj >> 3][jj & 7] = (T)row_ds<FAMILY>(p4[jj >> 2][jj & 3], cur[jj], FAMILY == BF_SOFTMAX ? rv[jj >> 2][jj & 3] : 0.f);
+              }
+            }
+            // (evaluated here, behind this MFMA)
+            if constexpr (upto > from) asm volatile("" : "+v"(f[(upto - 1) >> 3]));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        t0 = t1;
+        t1 = t2;
+        t2 = after(t2);
+      };
+      int u = 0;
+      for (; u + 1 < n_steps; u += 2) {
+        body(u, sa, sb);
+        body(u + 1, sb, sa);
+      }
+      if (u < n_steps) body(u, sa, sb);
+    }
+    wait_dma();
+    __syncthreads();   // every wave is done with the tiles: they become output staging
+
+    if constexpr (PARTS) {
+      partial_store<CB>(dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4 + (ROLE_B ? 0 : 32 * DQK), acc);
+    } else {
+      T* base = ROLE_B ? (T*)a.dk + (int64_t)b * a.dksb + (int64_t)hk * a.dksh : (T*)a.dv + (int64_t)b * a.dvsb + (int64_t)hk * a.dvsh;
+      store_rows<T, DC>(acc, ROLE_B ? a.scale : 1.f, lds0 + wave_all * (32 * (DC + 16)), base, ROLE_B ? a.dkss : a.dvss, n_wave, a.Skv, lane);
+      __syncthreads();   // the staged output has left the stages: the next key block's tiles may arrive
+    }
+  };
+  if (wave_all < 4) work(IntC<0>());
+  else work(IntC<1>());
   }   // the item's key blocks
   }   // items
 }
@@ -1393,7 +1727,7 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
       const bool parts = args.n_parts > 1;
       if (CAUSAL && masks) return -2;   // (masks go with MA_MASK_NONE)
       const int64_t workgroups = (int64_t)args.num_blocks * a.B * a.Hkv * args.n_parts;
-      constexpr bool TWO = fused_per_cu(DQK, DV) == 2;
+      constexpr bool TWO = DQK + DV <= 128;
       bool launched = false;
       if constexpr (TWO) {
         if (parts || dkv_two_streams(workgroups, CAUSAL)) {
@@ -1408,19 +1742,25 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
           launched = true;
         }
       }
-      if (!launched) {
-        constexpr bool RUNS = !TWO;      // (at 64 / 64 several runs are always two streams a workgroup)
+      const int cus = device_cus();
+      if (cus <= 0) return -1;
+      const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
+      if constexpr (!TWO) {
+        auto kf = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
+        auto kfp = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, CAUSAL, false, true>;
+        auto km = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, false, true, false>;
+        auto kmp = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, false, true, true>;
+        constexpr size_t plain = pair_lds(DQK, DV, false), with_masks = pair_lds(DQK, DV, true);
+        static std::atomic<uint64_t> plds_ok{0};
+        if (allow_lds(plds_ok, plain > with_masks ? plain : with_masks, kf, kfp, km, kmp) != 0) return -1;
+        hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)(items < cus ? items : cus)), dim3(512), masks ? with_masks : plain, stream, args);
+      } else if (!launched) {
         auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
-        auto kfp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, RUNS>;
         auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false>;
-        auto kmp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, RUNS>;
         static std::atomic<uint64_t> flds_ok{0};
-        if (allow_lds(flds_ok, flds, kf, kfp, km, kmp) != 0) return -1;
-        const int cus = device_cus();
-        if (cus <= 0) return -1;
-        const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
-        const int slots = cus * fused_per_cu(DQK, DV);
-        hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
+        if (allow_lds(flds_ok, flds, kf, km) != 0) return -1;
+        const int slots = cus * FUSED_PER_CU;
+        hipLaunchKernelGGL(masks ? km : kf, dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
       }
       if (parts) {
         const dim3 grid((unsigned)(args.num_blocks * a.B * a.Hkv), 2);
