@@ -11,14 +11,15 @@ int attn_bwd_256_256(const AttnBwdArgs& a, int family, bool causal, bool is_bf16
 int attn_bwd_192_128(const AttnBwdArgs& a, int family, bool causal, bool is_bf16, hipStream_t stream);   // (the reference's DeepSeek-V2-Lite benchmark shape; not the retention family)
 int attn_bwd_256_512(const AttnBwdArgs& a, int family, bool causal, bool is_bf16, hipStream_t stream);   // (256 / 512 is the head size of the retention operator itself, examples/retention_parallel.py)
 
-// The fused dk / dv kernel runs one workgroup per CU on items of a key block (a pair of them under a causal mask).  The number
+// The kernels that make dk and dv in one launch run one workgroup per CU on items of a key block (a pair of them under a causal mask).  The number
 // of runs per item is the one with the shortest schedule: rounds of workgroups x (steps of a run + a workgroup's fixed cost of
 // about six steps), a step taking 1.2 us at 128 / 128, plus the partial sums' way through memory (written and read at about
-// 4 TB/s) and their launch.  B2 H32 Hkv8 S2047 128/128 causal: 128 pairs of 272 steps on 256 CUs.  What element-wise and tile
+// 4 TB/s) and their launch.  B2 H32 Hkv8 S2047 128/128 causal: 128 pairs of 272 steps on 256 CUs; B1 H16 Hkv4 S700
+// 128/256 causal, 12 pairs: forward + backward 187 us in one run, 106 in those that this chooses.  (Steps of 0.7 and 0.9 us: within 3 % either way.)  What element-wise and tile
 // masks keep is not known here: they count as half the pairs, as a causal mask does (and so get as many runs: a triangular mask
 // gives a causal call's bits).
 int attn_bwd_parts(const AttnBwdArgs& a, bool half, int dqk, int dv) {
-  const bool fused = (dqk == 128 && dv == 128) || (dqk == 64 && dv == 64) || (dqk == 192 && dv == 128);
+  const bool fused = (dqk == 128 && dv == 128) || (dqk == 64 && dv == 64) || (dqk == 192 && dv == 128) || (dqk == 128 && dv == 256);
   if (!fused || a.add || a.slope_q || a.slope_kv || a.softcap != 0.f) return 1;
   const int cus = device_cus();
   if (cus <= 0) return 1;

@@ -24,9 +24,9 @@
 //                        directly the B operands of dV^T += dO^T P and dK^T += Q^T dS; lse and delta of
 //                        a tile's rows come with the tile.  dk and dv in one launch or in two (then the
 //                        scores are computed once more), whichever lets two waves share a SIMD.
-//   attn_bwd_dkv_fused_kernel  the same work at head sizes up to 128 / 128 (any mask): dk and dv in one launch,
-//                        one wave per SIMD with the 512-register budget, persistent, the loop pipelined
-//                        inside the wave (see there).
+//   attn_bwd_dkv_pair_kernel  the same work at 128 / 128, 192 / 128 and 128 / 256 (any mask): dk and dv in one launch, two waves
+//                        per SIMD with the same 32 keys, one for dv and one for dk.
+//   attn_bwd_dkv_fused_kernel  the same at 64 / 64: dk and dv in one wave, the loop pipelined inside it (see there).
 // The scores are recomputed in both kernels (7 tile products instead of 5; 8 where dk and dv take two
 // launches), which is what avoiding the fp32 atomics and the post-pass costs.  Tiles of 32 rows arrive by
 // direct-to-LDS DMA (a wave-uniform base in scalar registers plus 32-bit lane offsets computed once),
@@ -1266,7 +1266,8 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
 // B2 H32 Hkv8 S2047 128/128 causal 198 -> 170 us = 0.89 PFLOP/s of MFMAs (40 % of the cycles at 2.07 GHz; the LDS is busy for 32 %, without
 // conflicts).  From there on longer and shorter rings (4, 5 or 7 MFMAs ahead), p written earlier and fewer scalar instructions change
 // 1 % or nothing: the forward kernel's 1.1 PFLOP/s at the clock that random operands leave is near.  Forward + backward B8 H32 S4096
-// 5740 -> 5120 us, B2 H16 S1600 159 -> 144, B2 H32 Hkv8 S1500 sigmoid without a mask 443 -> 389, B4 H16 S1024 192/128 179 -> 163.
+// 5740 -> 5120 us, B2 H16 S1600 159 -> 144, B2 H32 Hkv8 S1500 sigmoid without a mask 443 -> 389, B4 H16 S1024 192/128 179 -> 163; at
+// 128 / 256, which took a launch for dk and one for dv before, B2 H16 S2048 causal 371 -> 286, B4 H32 S2500 1825 -> 1610.
 // Ring of NST stages: behind barrier u the tiles u, u + 1 and u + 2 are read, and the stage of tile u - 1 takes tile u + NST - 1.
 // The same products in the same order as the kernel above: the same bits.
 // MASKS: as in the kernel above, from a list of the steps in LDS; wave A reads the mask.
@@ -1428,7 +1429,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
     // rows of one tile against the wave's fragments make the scores, the columns of the other the accumulators
     constexpr int DR = ROLE_B ? DV : DQK, DC = ROLE_B ? DQK : DV;
     constexpr int RROW = ROLE_B ? DOROW : QROW, CROW = ROLE_B ? QROW : DOROW, ROFF = ROLE_B ? QTILE : 0, COFF = ROLE_B ? 0 : QTILE;
-    constexpr int NR = DR / 16, CB = DC / 32, NTOT = NR + 2 * CB, RING = NTOT % 8 == 0 ? 8 : 4, AH = RING == 8 ? 5 : 3;
+    // (128 / 256: with the longer ring 40 registers spill, B2 H16 S2048 causal 302 us, 286 with four)
+    constexpr int NR = DR / 16, CB = DC / 32, NTOT = NR + 2 * CB, RING = NTOT % 8 == 0 && DQK + DV <= 256 ? 8 : 4, AH = RING == 8 ? 5 : 3;
     static_assert(NTOT % RING == 0 && AH <= NR && AH <= 2 * CB, "fragment ring");
     x8 wf[NR];
     {
@@ -1605,7 +1607,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
       partial_store<CB>(dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4 + (ROLE_B ? 0 : 32 * DQK), acc);
     } else {
       T* base = ROLE_B ? (T*)a.dk + (int64_t)b * a.dksb + (int64_t)hk * a.dksh : (T*)a.dv + (int64_t)b * a.dvsb + (int64_t)hk * a.dvsh;
-      store_rows<T, DC>(acc, ROLE_B ? a.scale : 1.f, lds0 + wave_all * (32 * (DC + 16)), base, ROLE_B ? a.dkss : a.dvss, n_wave, a.Skv, lane);
+      store_rows<T, DC>(acc, ROLE_B ? a.scale : 1.f, lds0 + wave_all * (32 * ((DQK > DV ? DQK : DV) + 16)), base, ROLE_B ? a.dkss : a.dvss, n_wave, a.Skv, lane);
       __syncthreads();   // the staged output has left the stages: the next key block's tiles may arrive
     }
   };
@@ -1715,8 +1717,7 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   }
   if (!dq_done) hipLaunchKernelGGL(masked ? k1m : k1, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(256), lds, stream, args);
   args.num_blocks = (a.Skv + 127) / 128;
-  // (128 / 256 would fit the fused kernel's registers only with 60-90 spilled: measured no faster than its two launches)
-  if constexpr (FAMILY != BF_RETENTION && (DQK + DV <= 256 || (DQK == 192 && DV == 128))) {
+  if constexpr (FAMILY != BF_RETENTION && DQK <= 192 && DV <= 256) {
     // dk and dv by the pipelined single launch (with masks: as long as a key block's steps fit its list)
     const bool masks = a.elem_mask_t || a.q_block_mask;
     if (a.scale != 0.f && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
