@@ -19,7 +19,7 @@ int attn_bwd_256_512(const AttnBwdArgs& a, int family, bool causal, bool is_bf16
 // masks keep is not known here: they count as half the pairs, as a causal mask does (and so get as many runs: a triangular mask
 // gives a causal call's bits).
 int attn_bwd_parts(const AttnBwdArgs& a, bool half, int dqk, int dv) {
-  const bool fused = (dqk == 128 && dv == 128) || (dqk == 64 && dv == 64) || (dqk == 192 && dv == 128) || (dqk == 128 && dv == 256);
+  const bool fused = (dqk == 128 && dv == 128) || (dqk == 64 && dv == 64) || (dqk == 192 && dv == 128) || (dqk == 128 && dv == 256) || (dqk == 256 && dv == 256);
   if (!fused || a.add || a.slope_q || a.slope_kv || a.softcap != 0.f) return 1;
   const int cus = device_cus();
   if (cus <= 0) return 1;

@@ -1267,11 +1267,15 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
 // conflicts).  From there on longer and shorter rings (4, 5 or 7 MFMAs ahead), p written earlier and fewer scalar instructions change
 // 1 % or nothing: the forward kernel's 1.1 PFLOP/s at the clock that random operands leave is near.  Forward + backward B8 H32 S4096
 // 5740 -> 5120 us, B2 H16 S1600 159 -> 144, B2 H32 Hkv8 S1500 sigmoid without a mask 443 -> 389, B4 H16 S1024 192/128 179 -> 163; at
-// 128 / 256, which took a launch for dk and one for dv before, B2 H16 S2048 causal 371 -> 286, B4 H32 S2500 1825 -> 1610.
+// 128 / 256, which took a launch for dk and one for dv before, B2 H16 S2048 causal 371 -> 286, B4 H32 S2500 1825 -> 1610; 256 / 256
+// likewise, B4 H16 S1024 286 -> 263, B4 H12 S1024 sigmoid without a mask 388 -> 318.
 // Ring of NST stages: behind barrier u the tiles u, u + 1 and u + 2 are read, and the stage of tile u - 1 takes tile u + NST - 1.
 // The same products in the same order as the kernel above: the same bits.
 // MASKS: as in the kernel above, from a list of the steps in LDS; wave A reads the mask.
-constexpr int pair_stages(int dqk, int dv, bool masks) { return (pad_width(dqk) + dv <= 256 ? 6 : 5) - masks; }
+// At 256 / 256 fragments, accumulators and one set of scores fill the registers: there a wave's step is its scores, the row function, its
+// accumulators, one after the other, beside the partner's (pair_serial; a tile is then read in two steps, not three).
+constexpr bool pair_serial(int dqk, int dv) { return dqk + dv >= 512; }
+constexpr int pair_stages(int dqk, int dv, bool masks) { return pair_serial(dqk, dv) ? 3 : (pad_width(dqk) + dv <= 256 ? 6 : 5) - masks; }
 constexpr size_t pair_lds(int dqk, int dv, bool masks) {
   return pair_stages(dqk, dv, masks) * (32 * (size_t)(pad_width(dqk) + dv) * 2 + 512 + (masks ? 4 * 1024 : 0)) + 2 * 4 * 4096 + (masks ? FUSED_LIST_MAX * 4 + 16 : 0);
 }
@@ -1288,7 +1292,9 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   constexpr int NST = pair_stages(DQK, DV, MASKS), XCHG = NST * STAGE;
   // (MASKS) behind the exchanged p: 1 KB of mask bytes per stage and wave, then the step list and its length
   constexpr int KEEP = XCHG + 2 * 4 * 4096, LIST = KEEP + NST * 4 * 1024, LIST_N = LIST + FUSED_LIST_MAX * 4;
-  static_assert(NST >= 4 && pair_lds(DQK, DV, MASKS) <= 160 * 1024 && STAGE % QROW == 0 && STAGE % DOROW == 0 && 8 * 32 * ((DQK > DV ? DQK : DV) + 16) <= NST * STAGE, "LDS");
+  constexpr bool SERIAL = pair_serial(DQK, DV);
+  constexpr int READ = SERIAL ? 3 : 4;      // tiles that are read or must have landed
+  static_assert(NST >= READ && pair_lds(DQK, DV, MASKS) <= 160 * 1024 && STAGE % QROW == 0 && STAGE % DOROW == 0 && 8 * 32 * ((DQK > DV ? DQK : DV) + 16) <= NST * STAGE, "LDS");
 
   extern __shared__ __align__(16) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
@@ -1492,70 +1498,76 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
       wait_dma();
       __syncthreads();
       uint32_t t0 = lds0, t1 = lds0 + STAGE, t2 = lds0 + 2 * STAGE;      // the stages of tiles u, u + 1, u + 2
-      f32x16 sa = mm_rows<T, DR>(t0 + ROFF, r, g, wf), sb;
+      f32x16 sa, sb;
+      if constexpr (!SERIAL) sa = mm_rows<T, DR>(t0 + ROFF, r, g, wf);
       x8 fr[RING];
-      static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, t1, t0); });
-      row_values(t0);
+      static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, SERIAL ? t0 : t1, t0); });
+      if constexpr (!SERIAL) row_values(t0);
       const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-      auto body = [&](int u, f32x16& cur, f32x16& nxt) __attribute__((always_inline)) {
-        if constexpr (!ROLE_B) {
-          const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
+      // A: the scores that a mask hides, of the step about to evaluate them
+      auto hide = [&](int u, f32x16& cur) __attribute__((always_inline)) {
+        const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
+        if constexpr (MASKS) {
+          c_next = list_request(u + 1);
+          at = entry_walk(c_entry);
+        }
+        const int m0 = (t_first + at.t) * BMT;
+        if (!MASKS) at.template next<PARTS>(n_parts, t_count, a.kv_group);
+        const bool by_elem = MASKS && a.elem_mask_t && (c_entry >> 31) == 0;
+        if ((CAUSAL && n_wave + 31 > m0) || m0 + BMT > a.Sq || n_wave + 32 > a.Skv || by_elem) {
+          int m0e = m0;
+          asm volatile("; a tile that touches a mask" : "+s"(m0e));      // (see the kernel above)
+          uint32_t keep[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};   // the bytes of this lane's four rows per group
           if constexpr (MASKS) {
-            c_next = list_request(u + 1);
-            at = entry_walk(c_entry);
-          }
-          const int m0 = (t_first + at.t) * BMT;
-          if (!MASKS) at.template next<PARTS>(n_parts, t_count, a.kv_group);
-          const bool by_elem = MASKS && a.elem_mask_t && (c_entry >> 31) == 0;
-          if ((CAUSAL && n_wave + 31 > m0) || m0 + BMT > a.Sq || n_wave + 32 > a.Skv || by_elem) {
-            int m0e = m0;
-            asm volatile("; a tile that touches a mask" : "+s"(m0e));      // (see the kernel above)
-            uint32_t keep[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};   // the bytes of this lane's four rows per group
-            if constexpr (MASKS) {
-              if (by_elem) {
-                if (keep_ok && m0e + BMT <= a.Sq && n_wave < a.Skv) {
+            if (by_elem) {
+              if (keep_ok && m0e + BMT <= a.Sq && n_wave < a.Skv) {
 #pragma unroll
-                  for (int q4 = 0; q4 < 4; q4++) keep[q4] = keep_read(lds0 + KEEP + ((t0 - lds0) / STAGE * 4 + wave) * 1024, r, g, q4);
-                } else {
-                  // this key's row of the transposed mask, indexed by query position
-                  const uint8_t* emt_row = a.elem_mask_t + (int64_t)b * a.emt_sb + (int64_t)(hk * a.kv_group + at.hg) * a.emt_sh + (int64_t)n_ld * a.emt_sk;
+                for (int q4 = 0; q4 < 4; q4++) keep[q4] = keep_read(lds0 + KEEP + ((t0 - lds0) / STAGE * 4 + wave) * 1024, r, g, q4);
+              } else {
+                // this key's row of the transposed mask, indexed by query position
+                const uint8_t* emt_row = a.elem_mask_t + (int64_t)b * a.emt_sb + (int64_t)(hk * a.kv_group + at.hg) * a.emt_sh + (int64_t)n_ld * a.emt_sk;
 #pragma unroll
-                  for (int q4 = 0; q4 < 4; q4++) {
-                    const int m = m0e + 8 * q4 + 4 * g;
-                    keep[q4] = 0;
+                for (int q4 = 0; q4 < 4; q4++) {
+                  const int m = m0e + 8 * q4 + 4 * g;
+                  keep[q4] = 0;
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                      if (m + i < a.Sq) keep[q4] |= (uint32_t)emt_row[m + i] << (8 * i);
-                  }
+                  for (int i = 0; i < 4; i++)
+                    if (m + i < a.Sq) keep[q4] |= (uint32_t)emt_row[m + i] << (8 * i);
                 }
               }
             }
+          }
 #pragma unroll
-            for (int jj = 0; jj < 16; jj++) {
-              const int m = m0e + 8 * (jj >> 2) + 4 * g + (jj & 3);
-              if ((CAUSAL && n_lane > m) || m >= a.Sq || n_lane >= a.Skv || (MASKS && ((keep[jj >> 2] >> (8 * (jj & 3))) & 0xffu) == 0)) {
-                cur[jj] = s_masked;
-                // (a row without any kept key has lse = -inf: its masked scores must still give p = 0)
-                if constexpr (FAMILY == BF_SOFTMAX) rv[jj >> 2][jj & 3] = 0.f;
-              }
+          for (int jj = 0; jj < 16; jj++) {
+            const int m = m0e + 8 * (jj >> 2) + 4 * g + (jj & 3);
+            if ((CAUSAL && n_lane > m) || m >= a.Sq || n_lane >= a.Skv || (MASKS && ((keep[jj >> 2] >> (8 * (jj & 3))) & 0xffu) == 0)) {
+              cur[jj] = s_masked;
+              // (a row without any kept key has lse = -inf: its masked scores must still give p = 0)
+              if constexpr (FAMILY == BF_SOFTMAX) rv[jj >> 2][jj & 3] = 0.f;
             }
           }
         }
+      };
+      // tile u + 2 (SERIAL: u + 1) has landed (what may still be in flight: the tiles behind it), p(u) is in LDS, and every wave is done
+      // with tile u - 1, whose stage takes tile u + NST - 1
+      auto meet = [&](int u) __attribute__((always_inline)) {
+        if (u + NST - 2 < n_steps) wait_dma_but<(NST - READ) * TILE_DMAS>();
+        else wait_dma();
+        if constexpr (!ROLE_B) __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      };
+      auto body = [&](int u, f32x16& cur, f32x16& nxt) __attribute__((always_inline)) {
+        if constexpr (!ROLE_B) hide(u, cur);
         const uint32_t x = x_l + (u & 1) * 16384;
         x8 f[2];
         f32x4 p4[4];
         static_for<0, NTOT>([&](auto jc) __attribute__((always_inline)) {
           constexpr int j = decltype(jc)::value;
           if constexpr (j == (ROLE_B ? 0 : NR)) {
-            // tile u + 2 has landed (what may still be in flight: the tiles behind it), p(u) is in LDS, and every wave is done with
-            // tile u - 1, whose stage takes tile u + NST - 1
-            if (u + NST - 2 < n_steps) wait_dma_but<(NST - 4) * TILE_DMAS>();
-            else wait_dma();
-            if constexpr (!ROLE_B) __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0)
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
+            meet(u);
             if constexpr (ROLE_B) {
 #pragma unroll
               for (int q4 = 0; q4 < 4; q4++) p4[q4] = lds_read<f32x4>(x + q4 * 1024);
@@ -1593,7 +1605,44 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
         t1 = t2;
         t2 = after(t2);
       };
-      int u = 0;
+      auto serial_body = [&](int u) __attribute__((always_inline)) {
+        const uint32_t x = x_l + (u & 1) * 16384;
+        x8 f[2];
+        static_for<0, NTOT>([&](auto jc) __attribute__((always_inline)) {
+          constexpr int j = decltype(jc)::value;
+          if constexpr (ROLE_B && j == 0) meet(u);
+          if constexpr (j == NR - 1) row_values(t0);
+          if constexpr (j == NR) {
+            if constexpr (!ROLE_B) hide(u, sa);
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++) {
+              f32x4 p;
+              if constexpr (ROLE_B) p = lds_read<f32x4>(x + q4 * 1024);
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                const float row = FAMILY == BF_SOFTMAX ? rv[q4][i] : 0.f;
+                if constexpr (!ROLE_B) p[i] = row_p<FAMILY>(sa[4 * q4 + i], c_scale, c_bias, a.scale, bias, FAMILY == BF_SOFTMAX ? fmaf(row, -kLog2e, c_bias) : 0.f);
+                f[q4 >> 1][4 * (q4 & 1) + i] = (T)(ROLE_B ? row_ds<FAMILY>(p[i], sa[4 * q4 + i], row) : p[i]);
+              }
+              if constexpr (!ROLE_B) lds_write<f32x4>(x + q4 * 1024, p);
+            }
+            if constexpr (!ROLE_B) meet(u);
+          }
+          if constexpr (j == (ROLE_B ? 2 : NR + 2))
+            if (i_n < n_steps) issue_next();
+          if constexpr (j + AH < NTOT) fr[(j + AH) % RING] = fragment(IntC<j + AH>(), t0, t0);
+          else fr[(j + AH) % RING] = fragment(IntC<j + AH - NTOT>(), t1, t0);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (j < NR) sa = E::mfma32(fr[j % RING], wf[j], j == 0 ? zero16 : sa);
+          else acc[(j - NR) % CB] = E::mfma32(fr[j % RING], f[(j - NR) / CB], acc[(j - NR) % CB]);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        t0 = t1;
+        t1 = after(t1);
+      };
+      if constexpr (SERIAL)
+        for (int u = 0; u < n_steps; u++) serial_body(u);
+      int u = SERIAL ? n_steps : 0;
       for (; u + 1 < n_steps; u += 2) {
         body(u, sa, sb);
         body(u + 1, sb, sa);
@@ -1717,10 +1766,13 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   }
   if (!dq_done) hipLaunchKernelGGL(masked ? k1m : k1, dim3((unsigned)(args.num_blocks * a.B * a.H)), dim3(256), lds, stream, args);
   args.num_blocks = (a.Skv + 127) / 128;
-  if constexpr (FAMILY != BF_RETENTION && DQK <= 192 && DV <= 256) {
+  if constexpr (FAMILY != BF_RETENTION && DQK <= 256 && DV <= 256) {
     // dk and dv by the pipelined single launch (with masks: as long as a key block's steps fit its list)
     const bool masks = a.elem_mask_t || a.q_block_mask;
-    if (a.scale != 0.f && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
+    // (256 / 256 with masks in one run: 97 registers spill, and its two launches are the faster ones, B2 H16 S1500 with a window of 300
+    // forward + backward 352 and 357 us)
+    const bool two_launches = pair_serial(DQK, DV) && masks && (!a.dkv_part || a.n_parts <= 1);
+    if (a.scale != 0.f && !two_launches && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
       constexpr size_t ftiles = fused_stages(pad_width(DQK), DV) * ((size_t)32 * (pad_width(DQK) + DV) * 2 + 512);
       constexpr size_t mtiles = 4 * ((size_t)32 * (pad_width(DQK) + DV) * 2 + 512 + 4 * 1024) + FUSED_LIST_MAX * 4 + 16;
       constexpr size_t fmax = ftiles > mtiles ? ftiles : mtiles, flds = fmax > ostage ? fmax : ostage;

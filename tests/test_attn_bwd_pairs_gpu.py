@@ -1,4 +1,4 @@
-"""dk and dv by pairs of waves (128 / 128, 192 / 128, 128 / 256), where that can go wrong: one tile, as many tiles as stages and one
+"""dk and dv by pairs of waves (128 / 128, 192 / 128, 128 / 256, 256 / 256), where that can go wrong: one tile, as many tiles as stages and one
 more or fewer, several query heads, runs of steps, and masks that leave a key block nothing."""
 import pytest
 import torch
@@ -35,7 +35,7 @@ def _case(B, H, Hkv, Sq, Skv, D, DV, dtype):
     return [torch.randn(B, s, h, d, generator=g).to(dtype) for s, h, d in ((Sq, H, D), (Skv, Hkv, D), (Skv, Hkv, DV), (Sq, H, DV))]
 
 
-@pytest.mark.parametrize("D,DV", [(128, 128), (192, 128), (128, 256)])
+@pytest.mark.parametrize("D,DV", [(128, 128), (192, 128), (128, 256), (256, 256)])
 @pytest.mark.parametrize("B,H,Hkv,Sq,Skv,causal", [
     (1, 2, 2, 20, 20, True),           # one tile of one block of keys
     (1, 3, 1, 31, 200, False),         # one tile for each of three heads
@@ -55,7 +55,7 @@ def test_pairs(B, H, Hkv, Sq, Skv, causal, D, DV, family, dtype):
     _check(family, q, k, v, dout, allow, scale, bias, got, what)
 
 
-@pytest.mark.parametrize("D,DV", [(128, 128), (192, 128), (128, 256)])
+@pytest.mark.parametrize("D,DV", [(128, 128), (192, 128), (128, 256), (256, 256)])
 @pytest.mark.parametrize("S,first", [(320, 100), (300, 0), (416, 200)])      # (rows of a multiple of 16 bytes come with the tile, others element by element)
 def test_pairs_with_masks(S, first, D, DV):
     """A window of 70 keys over the rows from `first` on: rows and whole key blocks without a score, tiles kept in part and in full."""
