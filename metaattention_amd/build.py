@@ -30,9 +30,9 @@ HIPCC_FLAGS = [
 ]
 
 # -amdgpu-mfma-vgpr-form: kernels of more than 256 registers otherwise put every MFMA's result in accumulation registers, the
-# scores too, which the vector ALU then moves out one by one.  Forward + backward of B2 H32 S1600 256/256 causal 711 us without, 614 with
-# it; 128/128 see attn_bwd_kernels.h
-UNIT_FLAGS = {unit: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for unit in ("attn_bwd_128.hip", "attn_bwd_256.hip")}
+# scores too, which the vector ALU then moves out one by one.  Forward + backward of B2 H32 S1600 256/256 causal by such kernels 711 us
+# without, 614 with it
+UNIT_FLAGS = {unit: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for unit in ("attn_bwd_256.hip",)}
 
 
 def _hipcc() -> str:

@@ -24,7 +24,7 @@
 //                        directly the B operands of dV^T += dO^T P and dK^T += Q^T dS; lse and delta of
 //                        a tile's rows come with the tile.  dk and dv in one launch or in two (then the
 //                        scores are computed once more), whichever lets two waves share a SIMD.
-//   attn_bwd_dkv_pair_kernel  the same work at 128 / 128, 192 / 128 and 128 / 256 (any mask): dk and dv in one launch, two waves
+//   attn_bwd_dkv_pair_kernel  the same work at 128 / 128, 192 / 128, 128 / 256 and 256 / 256: dk and dv in one launch, two waves
 //                        per SIMD with the same 32 keys, one for dv and one for dk.
 //   attn_bwd_dkv_fused_kernel  the same at 64 / 64: dk and dv in one wave, the loop pipelined inside it (see there).
 // The scores are recomputed in both kernels (7 tile products instead of 5; 8 where dk and dv take two
@@ -113,7 +113,7 @@ constexpr int fused_stages(int dqk, int dv) { return 8 * (32 * (dqk + dv) * 2 + 
 // Workgroups of the pipelined dk / dv kernel that a CU holds.  At 64 / 64 a step is 16 MFMAs behind some 200 vector
 // instructions, LDS latencies and a barrier, and one wave per SIMD waits for most of it: two workgroups (256 registers a wave,
 // lse and delta requested in the step that uses them) take B4 H32 S2048 causal forward + backward from 595 to 438 us (sigmoid)
-// and 557 to 421 us (softmax), B8 H32 S4096 3984 -> 3353 and 3723 -> 3130.  The larger sizes need a SIMD's 512 registers.
+// and 557 to 421 us (softmax), B8 H32 S4096 3984 -> 3353 and 3723 -> 3130.
 constexpr int FUSED_PER_CU = 2;
 // Waits until at most N of this wave's vector-memory loads are outstanding (they complete in order).
 template <int N>
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(256, (WHAT == 3 ? (DQK + DV >= 256 ? 1 : 2) : (DQK 
 
 
 // ------------------------------------------------------------------------------------------------
-// dk and dv in one launch: one wave per SIMD, software pipelined
+// dk and dv in one launch at 64 / 64, software pipelined inside the wave
 // ------------------------------------------------------------------------------------------------
 // Few key blocks (short sequences, one or two sequences with grouped-query heads) leave CUs idle: the steps of every key block
 // are then dealt to n_parts runs, taken by workgroups side by side (attn_bwd_parts chooses): tile t of the group's head hg
@@ -800,10 +800,9 @@ __device__ __forceinline__ void partial_store(float* to, const f32x16 (&acc)[N])
       *(f32x4*)(to + (i * 4 + q4) * 256) = f32x4{acc[i][4 * q4], acc[i][4 * q4 + 1], acc[i][4 * q4 + 2], acc[i][4 * q4 + 3]};
 }
 
-// Where the K and V fragments and both [D x 32] accumulators of a wave's 32 keys fit the 512 registers of a wave that has its
-// SIMD to itself, dk and dv share the recomputed scores (7 tile products in all instead of 8).  With no second wave on the
-// SIMD to fill the matrix pipe while one evaluates the row function or waits for LDS, the loop is pipelined inside the
-// wave.  A step is ONE sequence of MFMAs:
+// At 64 / 64 the K and V fragments and both [D x 32] accumulators of a wave's 32 keys fit the registers of one wave of two on a
+// SIMD, and dk and dv share the recomputed scores (7 tile products in all instead of 8).  The loop is pipelined inside the wave.  A
+// step is ONE sequence of MFMAs:
 //   phase F  S(u+1) = Q(u+1) K^T and dP(u+1) = dO(u+1) V^T of the NEXT tile, with p of the current step's 16 score elements
 //            spread behind them,
 //   phase V  dV^T += dO(u)^T P(u), with ds of the 16 elements behind them,
@@ -815,7 +814,8 @@ __device__ __forceinline__ void partial_store(float* to, const f32x16 (&acc)[N])
 // body is written for two steps (the registers of "this" and "the next" step swap roles) so that nothing is copied; an odd
 // number of steps is padded with a step in which everything is masked.  Masked scores are set to -inf (times the sign
 // of scale) before the row function, in the few tiles that touch the diagonal or an end of the sequences: p = 0 and so
-// ds = 0 follow.  The retention family and the larger head sizes take the two-launch kernels above.
+// ds = 0 follow.  Larger head sizes take the pair kernel below; the retention family, 256 / 512, additive score terms, a scale of 0 and
+// masks with more steps than the list holds the kernels above.
 template <int I>
 struct IntC { static constexpr int value = I; };
 template <int I, int N, typename F>
