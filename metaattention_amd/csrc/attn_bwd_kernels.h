@@ -1271,7 +1271,10 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
 // likewise, B4 H16 S1024 286 -> 263, B4 H12 S1024 sigmoid without a mask 388 -> 318.
 // Ring of NST stages: behind barrier u the tiles u, u + 1 and u + 2 are read, and the stage of tile u - 1 takes tile u + NST - 1.
 // The same products in the same order as the kernel above: the same bits.
-// MASKS: as in the kernel above, from a list of the steps in LDS; wave A reads the mask.
+// MASKS: as in the kernel above, from a list of the steps in LDS.  Both waves know what a mask hides: A makes p = 0 of it, and B, where dp or
+// delta is not finite, ds = 0; tiles that a wave's keys do not see under a causal mask stay out of its sums.  (With B's part forward + backward
+// of B2 H32 Hkv8 S2047 128/128 causal 355 -> 360 us, B2 H16 S1600 141.6 -> 142.8; the mask evaluated by B in every tile that it touches
+// cost 6 % under a window.)
 // At 256 / 256 fragments, accumulators and one set of scores fill the registers: there a wave's step is its scores, the row function, its
 // accumulators, one after the other, beside the partner's (pair_serial; a tile is then read in two steps, not three).
 constexpr bool pair_serial(int dqk, int dv) { return dqk + dv >= 512; }
@@ -1299,6 +1302,9 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   extern __shared__ __align__(16) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3;
+  // (where registers are short what is rarely needed is made from the lane's number anew: derived from the one above, the compiler
+  // carries it through the loop in spilled registers, 46 of them at 256 / 256.  128 / 128 has the registers: 201 us for 203, B2 H16 S1500)
+  auto lane_here = [&]() { return DQK + DV > 256 ? lane_anew() : lane; };
   const int r = lane & 31, g = lane >> 5, jr = (lane & 15) >> 2, lc = (((lane >> 4) & 1) << 1) | ((lane & 3) >> 1);
 
   // persistent, items as in the kernel above
@@ -1340,8 +1346,10 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   const int t_count = (a.Sq + BMT - 1) / BMT - t_first;
   int n_steps = t_count > 0 ? t_count * a.kv_group : 0;
   DkvWalk first{0, 0, 0};
+  int each = 0, more = 0;      // a run's tiles of a head: one more than `each` where its first one comes before `more`
   if (PARTS && !MASKS && n_steps > 0) {
-    const int each = t_count / n_parts, more = t_count % n_parts;
+    each = t_count / n_parts;
+    more = t_count % n_parts;
     first.skip = ((run - t_first) % n_parts + n_parts) % n_parts;
     n_steps = 0;
     for (int hg = 0, skip = first.skip; hg < a.kv_group; hg++, skip = skip == 0 ? n_parts - 1 : skip - 1) n_steps += each + (skip < more ? 1 : 0);
@@ -1400,15 +1408,16 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
       const int m0 = (t_first + fetch.w.t) * BMT, h = hk * a.kv_group + fetch.w.hg;
       if (wave_all < 4 && keep_ok && !full && m0 + BMT <= a.Sq && n_wave < a.Skv)
         keep_dma(a.elem_mask_t + (int64_t)b * a.emt_sb + (int64_t)h * a.emt_sh + (int64_t)n_wave * a.emt_sk + m0, a.emt_sk, a.Skv - n_wave,
-                 lds0 + KEEP + ((to - lds0) / STAGE * 4 + wave) * 1024, lane);
+                 lds0 + KEEP + ((to - lds0) / STAGE * 4 + wave) * 1024, lane_here());
     }
     const int rows = fetch.w.t < t_whole ? BMT : a.Sq % BMT;   // (wave-uniform)
     if (rows == BMT) {
       q_dma.issue(fetch.q, to, wave_all);
       do_dma.issue(fetch.d, to + QTILE, wave_all);
     } else {
-      dma_tile<QROW, 8, DQK / 8>(fetch.q, q_row_bytes, 0, rows, to, wave_all, lane);
-      dma_tile<DOROW, 8>(fetch.d, do_row_bytes, 0, rows, to + QTILE, wave_all, lane);
+      const int ln = lane_here();
+      dma_tile<QROW, 8, DQK / 8>(fetch.q, q_row_bytes, 0, rows, to, wave_all, ln);
+      dma_tile<DOROW, 8>(fetch.d, do_row_bytes, 0, rows, to + QTILE, wave_all, ln);
     }
     if constexpr (FAMILY == BF_SOFTMAX) {
       // wave 0 fetches lse, wave 1 delta (the upper lanes repeat the lower ones)
@@ -1499,14 +1508,23 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
       __syncthreads();
       uint32_t t0 = lds0, t1 = lds0 + STAGE, t2 = lds0 + 2 * STAGE;      // the stages of tiles u, u + 1, u + 2
       f32x16 sa, sb;
-      if constexpr (!SERIAL) sa = mm_rows<T, DR>(t0 + ROFF, r, g, wf);
       x8 fr[RING];
-      static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, SERIAL ? t0 : t1, t0); });
-      if constexpr (!SERIAL) row_values(t0);
+      if constexpr (!SERIAL) sa = mm_rows<T, DR>(t0 + ROFF, r, g, wf);
+      // what a step finds ready beside its scores
+      auto fill = [&]() __attribute__((always_inline)) {
+        static_for<0, AH>([&](auto jc) __attribute__((always_inline)) { fr[decltype(jc)::value] = fragment(jc, SERIAL ? t0 : t1, t0); });
+        if constexpr (!SERIAL) row_values(t0);
+      };
       const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-      // A: the scores that a mask hides, of the step about to evaluate them
+      // None of the wave's keys sees the tile at hand: the accumulators are to be left alone (p = 0 times a row of dO that is not finite
+      // is not 0).
+      auto unseen = [&](const DkvWalk& w) { return n_wave >= (t_first + w.t + 1) * BMT; };
+      // The elements that a mask hides: p = 0 (A) and ds = 0 (B, from dp = delta = 0) whatever the rows and keys hold.  B leaves out what
+      // does not matter: relu's ds is 0 where p is, and without a mask all that is hidden is the last row again and keys that do not exist.
+      constexpr bool HIDES = !ROLE_B || ((CAUSAL || MASKS) && FAMILY != BF_RELU);
       auto hide = [&](int u, f32x16& cur) __attribute__((always_inline)) {
+        if constexpr (!HIDES && !CAUSAL) return;
         const uint32_t c_entry = MASKS ? uniform(c_next) : 0u;
         if constexpr (MASKS) {
           c_next = list_request(u + 1);
@@ -1514,10 +1532,19 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
         }
         const int m0 = (t_first + at.t) * BMT;
         if (!MASKS) at.template next<PARTS>(n_parts, t_count, a.kv_group);
+        if constexpr (!HIDES) return;
         const bool by_elem = MASKS && a.elem_mask_t && (c_entry >> 31) == 0;
         if ((CAUSAL && n_wave + 31 > m0) || m0 + BMT > a.Sq || n_wave + 32 > a.Skv || by_elem) {
+          if constexpr (ROLE_B) {
+            // (as a rule nothing here is not finite, and 0 times it is 0: one look at all of it instead of the mask)
+            f32x4 any = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int jj = 0; jj < 16; jj++) any[jj & 3] = FAMILY == BF_SOFTMAX ? fmaf(cur[jj], rv[jj >> 2][jj & 3], any[jj & 3]) : any[jj & 3] + cur[jj];
+            if (__all(__builtin_isfinite((any[0] + any[1]) + (any[2] + any[3])))) return;
+          }
           int m0e = m0;
           asm volatile("; a tile that touches a mask" : "+s"(m0e));      // (see the kernel above)
+          const int ln = lane_here(), r = ln & 31, g = ln >> 5, n_lane = n_wave + r, n_ld = min(n_lane, a.Skv - 1);
           uint32_t keep[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};   // the bytes of this lane's four rows per group
           if constexpr (MASKS) {
             if (by_elem) {
@@ -1542,7 +1569,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
           for (int jj = 0; jj < 16; jj++) {
             const int m = m0e + 8 * (jj >> 2) + 4 * g + (jj & 3);
             if ((CAUSAL && n_lane > m) || m >= a.Sq || n_lane >= a.Skv || (MASKS && ((keep[jj >> 2] >> (8 * (jj & 3))) & 0xffu) == 0)) {
-              cur[jj] = s_masked;
+              cur[jj] = ROLE_B ? 0.f : s_masked;
               // (a row without any kept key has lse = -inf: its masked scores must still give p = 0)
               if constexpr (FAMILY == BF_SOFTMAX) rv[jj >> 2][jj & 3] = 0.f;
             }
@@ -1559,6 +1586,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
       };
+      auto ahead = [&]() {
+        t0 = t1;
+        t1 = SERIAL ? after(t1) : t2;
+        if constexpr (!SERIAL) t2 = after(t2);
+      };
       auto body = [&](int u, f32x16& cur, f32x16& nxt) __attribute__((always_inline)) {
         if constexpr (!ROLE_B) hide(u, cur);
         const uint32_t x = x_l + (u & 1) * 16384;
@@ -1573,6 +1605,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
               for (int q4 = 0; q4 < 4; q4++) p4[q4] = lds_read<f32x4>(x + q4 * 1024);
             }
           }
+          if constexpr (ROLE_B && j == 2) hide(u, cur);
           if constexpr (j == (ROLE_B ? 2 : NR + 2))      // (two MFMAs on: behind the barrier itself, B2 H16 S1600 148 us for 144)
             if (i_n < n_steps) issue_next();
           if constexpr (j == NTOT - 4) row_values(t1);
@@ -1601,9 +1634,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
           }
           __builtin_amdgcn_sched_barrier(0);
         });
-        t0 = t1;
-        t1 = t2;
-        t2 = after(t2);
+        ahead();
       };
       auto serial_body = [&](int u) __attribute__((always_inline)) {
         const uint32_t x = x_l + (u & 1) * 16384;
@@ -1613,7 +1644,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
           if constexpr (ROLE_B && j == 0) meet(u);
           if constexpr (j == NR - 1) row_values(t0);
           if constexpr (j == NR) {
-            if constexpr (!ROLE_B) hide(u, sa);
+            hide(u, sa);
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
               f32x4 p;
@@ -1637,26 +1668,55 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
           else acc[(j - NR) % CB] = E::mfma32(fr[j % RING], f[(j - NR) / CB], acc[(j - NR) % CB]);
           __builtin_amdgcn_sched_barrier(0);
         });
-        t0 = t1;
-        t1 = after(t1);
+        ahead();
       };
-      if constexpr (SERIAL)
-        for (int u = 0; u < n_steps; u++) serial_body(u);
-      int u = SERIAL ? n_steps : 0;
-      for (; u + 1 < n_steps; u += 2) {
-        body(u, sa, sb);
-        body(u + 1, sb, sa);
+      for (int u = 0, upto; u < n_steps; u = upto) {
+        // The tiles in front of the diagonal come first of every head, for the waves of the later keys: those take part in the barriers
+        // and have the next step's scores ready.  (A way round the products inside the step instead makes the compiler spill 60 to 900
+        // registers.)
+        upto = n_steps;
+        if constexpr (CAUSAL) {
+          int passed = 0;      // of the head at hand
+          for (; u < n_steps && unseen(at); u++) {
+            const int hg = at.hg;
+            at.template next<PARTS>(n_parts, t_count, a.kv_group);
+            passed = at.hg == hg ? passed + 1 : 0;
+            if constexpr (!SERIAL)
+              if (!unseen(at)) sa = mm_rows<T, DR>(t1 + ROFF, r, g, wf);
+            meet(u);
+            if (i_n < n_steps) issue_next();
+            ahead();
+          }
+          if (n_wave > t_first * BMT) {
+            upto = u - passed;
+            DkvWalk w = at;
+            do {
+              upto += PARTS ? each + (w.skip < more ? 1 : 0) : t_count;
+              w.to_tile(t_count, n_parts, t_count, a.kv_group);
+            } while (upto < n_steps && !unseen(w));
+            upto = min(upto, n_steps);      // (a run may end in front of the diagonal)
+          }
+        }
+        fill();
+        if constexpr (SERIAL) {
+          for (; u < upto; u++) serial_body(u);
+        } else {
+          for (; u + 1 < upto; u += 2) {
+            body(u, sa, sb);
+            body(u + 1, sb, sa);
+          }
+          if (u < upto) body(u, sa, sb);
+        }
       }
-      if (u < n_steps) body(u, sa, sb);
     }
     wait_dma();
     __syncthreads();   // every wave is done with the tiles: they become output staging
 
     if constexpr (PARTS) {
-      partial_store<CB>(dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4 + (ROLE_B ? 0 : 32 * DQK), acc);
+      partial_store<CB>(dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane_here() * 4 + (ROLE_B ? 0 : 32 * DQK), acc);
     } else {
       T* base = ROLE_B ? (T*)a.dk + (int64_t)b * a.dksb + (int64_t)hk * a.dksh : (T*)a.dv + (int64_t)b * a.dvsb + (int64_t)hk * a.dvsh;
-      store_rows<T, DC>(acc, ROLE_B ? a.scale : 1.f, lds0 + wave_all * (32 * ((DQK > DV ? DQK : DV) + 16)), base, ROLE_B ? a.dkss : a.dvss, n_wave, a.Skv, lane);
+      store_rows<T, DC>(acc, ROLE_B ? a.scale : 1.f, lds0 + wave_all * (32 * ((DQK > DV ? DQK : DV) + 16)), base, ROLE_B ? a.dkss : a.dvss, n_wave, a.Skv, lane_here());
       __syncthreads();   // the staged output has left the stages: the next key block's tiles may arrive
     }
   };

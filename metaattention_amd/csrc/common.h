@@ -69,6 +69,13 @@ __device__ __forceinline__ void lds_write(uint32_t lds_byte_addr, V v) {
   *(MA_LDS V*)(uintptr_t)lds_byte_addr = v;
 }
 
+// the lane's id, made where it is used: nothing derived from it can be moved above this place
+__device__ __forceinline__ int lane_anew() {
+  uint32_t none = 0;
+  asm volatile("" : "+v"(none));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
+}
+
 // value held by lane (l ^ 32)
 __device__ __forceinline__ float xhalf(float x) {
   return __shfl_xor(x, 32, 64);

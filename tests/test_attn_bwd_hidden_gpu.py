@@ -1,0 +1,97 @@
+"""Gradients where a mask hides values that are not finite: what a key does not see leaves dk (and, from tiles that none of a wave's
+32 keys sees, dv) the bits that it has without them.  In one run of steps and in several, with one item a workgroup and with more."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+SIZES = [(128, 128), (192, 128), (128, 256), (256, 256)]
+BAD = [float("nan"), float("inf"), float("-inf")]
+
+
+def _inputs(B, H, Hkv, S, D, DV, dtype=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(S + D + H)
+    return [torch.randn(B, S, h, d, device="cuda", generator=g).to(dtype) for h, d in ((H, D), (Hkv, D), (Hkv, DV), (H, DV))]
+
+
+def backward(family, q, k, v, dout, monkeypatch, one_run, causal=False, seen_v=None, **masks):
+    """(dq, dk, dv), with the library's own choice of runs or in one (a call with only the required workspace).  seen_v: V of the forward
+    pass, where V holds values in keys that it need not read."""
+    from metaattention_amd import hip_backend as hb
+    fam = {"softmax": hb.MA_ATTN_SOFTMAX, "sigmoid": hb.MA_ATTN_SIGMOID, "relu": hb.MA_ATTN_RELU}[family]
+    B, S, H, D = q.shape
+    kw = dict(family=fam, causal=causal, scale=D ** -0.5, bias=-2.0 if family == "sigmoid" else 0.0)
+    lse = torch.empty(B, H, S, device="cuda") if family == "softmax" else None
+    o = hb.attn_fwd(q, k, v if seen_v is None else seen_v, row_scale=lse, elem_mask=masks.get("elem_mask"), **kw)
+    lib = hb.load_library()
+
+    class Lib:
+        def __getattr__(self, name):
+            return (lambda p: 4 * B * H * S if family == "softmax" else 0) if one_run and name == "ma_attn_bwd_workspace_bytes" else getattr(lib, name)
+    with monkeypatch.context() as m:
+        m.setattr(hb, "_lib", Lib())
+        return hb.attn_bwd(q, k, v, o, dout, lse, **masks, **kw)
+
+
+def masks_of(allow):
+    """The masks of a call in the forms that it takes, from which scores are kept (rows padded to 16 bytes)."""
+    S = allow.shape[0]
+    n, rows = (S + 127) // 128 * 128, (S + 31) // 32
+
+    def elem(m):
+        buf = torch.zeros(S, (S + 15) // 16 * 16, dtype=torch.uint8)
+        buf[:, :S] = m
+        return buf.cuda().view(1, 1, S, -1)[..., :S]
+
+    def tiles(m):
+        kept, whole = torch.zeros(n, n, dtype=torch.bool), torch.ones(n, n, dtype=torch.bool)
+        kept[:S, :S], whole[:S, :S] = m, m
+        pool = kept.view(n // 128, 128, n // 32, 32).any(3).any(1).to(torch.uint8) * (1 + whole.view(n // 128, 128, n // 32, 32).all(3).all(1).to(torch.uint8))
+        return pool[:, :rows].contiguous().cuda().view(1, 1, n // 128, rows)
+
+    return dict(elem_mask=elem(allow), elem_mask_t=elem(allow.t()), kv_block_mask=tiles(allow), q_block_mask=tiles(allow.t()))
+
+
+@pytest.mark.parametrize("D,DV", SIZES)
+@pytest.mark.parametrize("family", ["softmax", "sigmoid", "relu"])
+@pytest.mark.parametrize("one_run", [True, False])
+def test_later_keys_do_not_see_a_row_under_a_causal_mask(D, DV, family, one_run, monkeypatch):
+    """A row of dout: the keys of the 32-key groups behind that of the row."""
+    for B, H, Hkv, S, row in ((1, 4, 2, 420, 5), (1, 4, 2, 420, 200), (2, 3, 3, 290, 130), (1, 2, 2, 100, 33)):
+        print(f"causal {family} {D}/{DV} B{B} H{H}/{Hkv} S{S} row {row} one_run={one_run}", flush=True)
+        q, k, v, dout = _inputs(B, H, Hkv, S, D, DV)
+        want = backward(family, q, k, v, dout, monkeypatch, one_run, causal=True)
+        for bad in BAD:
+            grad = dout.clone()
+            grad[0, row, 1] = bad
+            got = backward(family, q, k, v, grad, monkeypatch, one_run, causal=True)
+            behind = row // 32 * 32 + 32
+            for name, a, b in zip(("dk", "dv"), got[1:], want[1:]):
+                assert torch.equal(a[:, behind:], b[:, behind:]) and torch.equal(a[1:], b[1:]), f"{name} {bad}"
+            assert not got[2][0, :row, 1 * Hkv // H].isfinite().any(), "the keys that see the row have it"
+
+
+@pytest.mark.parametrize("D,DV", SIZES)
+@pytest.mark.parametrize("family", ["softmax", "sigmoid", "relu"])
+@pytest.mark.parametrize("one_run", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,S", [(1, 4, 2, 320), (2, 3, 3, 300), (8, 16, 16, 384), (3, 43, 43, 300)])     # (the last two: more items than workgroups)
+def test_hidden_keys_and_rows_under_a_mask(B, H, Hkv, S, D, DV, family, one_run, monkeypatch):
+    """V of 32 padding keys that no row sees, and the gradient of five rows that see no key, in a tile whose other rows do."""
+    print(f"mask {family} {D}/{DV} B{B} H{H}/{Hkv} S{S} one_run={one_run}", flush=True)
+    q, k, v, dout = _inputs(B, H, Hkv, S, D, DV)
+    i, j = torch.arange(S).view(S, 1), torch.arange(S).view(1, S)
+    keys, rows = slice(96, 128), slice(40, 45)
+    allow = (j <= i + 7) & (i - j < 150)
+    allow[:, keys] = False
+    allow[rows] = False
+    m = masks_of(allow)
+    want = backward(family, q, k, v, dout, monkeypatch, one_run, **m)
+    assert all(t.isfinite().all() for t in want) and not want[1][:, keys].any() and not want[2][:, keys].any()
+    for bad in BAD:
+        other = v.clone()
+        other[:, keys] = bad
+        for name, a, b in zip(("dq", "dk", "dv"), backward(family, q, k, other, dout, monkeypatch, one_run, seen_v=v, **m), want):
+            assert torch.equal(a, b), f"{name}, V {bad}"
+        grad = dout.clone()
+        grad[:, rows] = bad
+        got = backward(family, q, k, v, grad, monkeypatch, one_run, **m)
+        assert torch.equal(got[1], want[1]), f"dk, dout {bad}"
