@@ -1145,6 +1145,7 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
           const int m = m0e + 8 * (jj >> 2) + 4 * g + (jj & 3);
           if ((CAUSAL && n_lane > m) || m >= a.Sq || n_lane >= a.Skv || (MASKS && ((keep[jj >> 2] >> (8 * (jj & 3))) & 0xffu) == 0)) {
             cur.s[jj] = s_masked;
+            cur.dp[jj] = 0.f;      // (p = 0 times a hidden key's row of V that is not finite is not 0)
             // (a row without any kept key has lse = -inf: its masked scores must still give p = 0)
             if constexpr (FAMILY == BF_SOFTMAX) cur.tl[jj >> 2][jj & 3] = 0.f;
           }

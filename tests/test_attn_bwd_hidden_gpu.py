@@ -70,12 +70,13 @@ def test_later_keys_do_not_see_a_row_under_a_causal_mask(D, DV, family, one_run,
             assert not got[2][0, :row, 1 * Hkv // H].isfinite().any(), "the keys that see the row have it"
 
 
-@pytest.mark.parametrize("D,DV", SIZES)
+@pytest.mark.parametrize("D,DV", [(64, 64)] + SIZES)
 @pytest.mark.parametrize("family", ["softmax", "sigmoid", "relu"])
 @pytest.mark.parametrize("one_run", [True, False])
 @pytest.mark.parametrize("B,H,Hkv,S", [(1, 4, 2, 320), (2, 3, 3, 300), (8, 16, 16, 384), (3, 43, 43, 300)])     # (the last two: more items than workgroups)
 def test_hidden_keys_and_rows_under_a_mask(B, H, Hkv, S, D, DV, family, one_run, monkeypatch):
-    """V of 32 padding keys that no row sees, and the gradient of five rows that see no key, in a tile whose other rows do."""
+    """V of 32 padding keys that no row sees, and the gradient of five rows that see no key, in a tile whose other rows do (not at 64 / 64,
+    whose one wave has a row's delta only behind the mask)."""
     print(f"mask {family} {D}/{DV} B{B} H{H}/{Hkv} S{S} one_run={one_run}", flush=True)
     q, k, v, dout = _inputs(B, H, Hkv, S, D, DV)
     i, j = torch.arange(S).view(S, 1), torch.arange(S).view(1, S)
@@ -91,6 +92,8 @@ def test_hidden_keys_and_rows_under_a_mask(B, H, Hkv, S, D, DV, family, one_run,
         other[:, keys] = bad
         for name, a, b in zip(("dq", "dk", "dv"), backward(family, q, k, other, dout, monkeypatch, one_run, seen_v=v, **m), want):
             assert torch.equal(a, b), f"{name}, V {bad}"
+        if D == 64:
+            continue
         grad = dout.clone()
         grad[:, rows] = bad
         got = backward(family, q, k, v, grad, monkeypatch, one_run, **m)
