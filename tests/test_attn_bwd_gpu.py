@@ -323,8 +323,7 @@ def test_engine_backward_with_external_block_mask(family, mask, D, S, bq, bk):
 @pytest.mark.parametrize("D,DV", [(128, 128), (192, 128), (128, 256)])
 def test_masked_backward_through_the_c_abi_matches_causal(D, DV):
     """A lower-triangular keep mask through elem_mask / elem_mask_t gives the gradients of the causal flag (bit for bit:
-    the same tiles, the same masked elements), grouped-query heads included; at the head sizes of the fused dk / dv kernel
-    (128 / 128, 192 / 128: its masked form) and of the two-launch kernels (128 / 256)."""
+    the same tiles, the same masked elements), grouped-query heads included."""
     hb = _hb()
     B, H, Hkv, S = 1, 4, 2, 257
     g = torch.Generator().manual_seed(11)

@@ -98,3 +98,36 @@ def test_hidden_keys_and_rows_under_a_mask(B, H, Hkv, S, D, DV, family, one_run,
         grad[:, rows] = bad
         got = backward(family, q, k, v, grad, monkeypatch, one_run, **m)
         assert torch.equal(got[1], want[1]), f"dk, dout {bad}"
+
+
+@pytest.mark.parametrize("D,DV", SIZES)
+@pytest.mark.parametrize("one_run", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,S", [(8, 16, 16, 400), (3, 34, 34, 400), (8, 32, 16, 300), (1, 4, 2, 400)])      # (but for the last: more key blocks than CUs)
+def test_masked_gradients(B, H, Hkv, S, D, DV, one_run, monkeypatch):
+    """A workgroup's key blocks one after the other, a list of steps made for each: a window, and a key block that no row sees."""
+    print(f"masked {D}/{DV} B{B} H{H}/{Hkv} S{S} one_run={one_run}", flush=True)
+    q, k, v, dout = _inputs(B, H, Hkv, S, D, DV)
+    i, j = torch.arange(S).view(S, 1), torch.arange(S).view(1, S)
+    allow = (j <= i) & (i - j < 170) & ((j < 128) | (j >= 256)) & (i >= 20)
+    got = backward("softmax", q, k, v, dout, monkeypatch, one_run, **masks_of(allow))
+    hidden = ~allow.cuda()
+    for b in range(B):      # (an entry at a time: double precision)
+        qd, kd, vd = (t[b].double().transpose(0, 1).contiguous().requires_grad_() for t in (q, k, v))
+        ke, ve = (t.repeat_interleave(H // Hkv, 0) for t in (kd, vd))
+        x = torch.matmul(qd, ke.transpose(1, 2)) * D ** -0.5
+        p = torch.softmax(x.masked_fill(hidden, -1e300), -1) * ~hidden
+        ref = torch.autograd.grad(torch.matmul(p, ve), (qd, kd, vd), dout[b].double().transpose(0, 1))
+        for name, a, want in zip(("dq", "dk", "dv"), got, ref):
+            # p and ds are rounded to bf16 (2^-9 of each, at random): of the 2-norm of a gradient that is well below 1e-2
+            assert (a[b].double().transpose(0, 1) - want).norm() <= 1e-2 * want.norm(), f"{name} {b}"
+    assert not got[1][:, 128:256].any() and not got[2][:, 128:256].any()
+
+
+def test_a_triangular_mask_gives_a_causal_calls_bits_at_256(monkeypatch):
+    """Several runs of steps: the same tiles and masked elements by the masked and the causal form of the kernel."""
+    B, H, Hkv, S = 1, 4, 2, 257
+    q, k, v, dout = _inputs(B, H, Hkv, S, 256, 256)
+    want = backward("softmax", q, k, v, dout, monkeypatch, False, causal=True)
+    elem = {n: m for n, m in masks_of(torch.ones(S, S, dtype=torch.bool).tril()).items() if n.startswith("elem")}
+    for name, a, b in zip(("dq", "dk", "dv"), backward("softmax", q, k, v, dout, monkeypatch, False, **elem), want):
+        assert torch.equal(a, b), name
