@@ -39,7 +39,7 @@ struct AttnBwdArgs {
   const float* slope_q;
   const float* slope_kv;
   float softcap;
-  // the fused dk / dv kernel: n_parts runs of steps per key block, their fp32 partial sums (see attn_bwd_parts); 1 / NULL: one run
+  // the kernels that make dk and dv in one launch: n_parts runs of steps per key block, their fp32 partial sums (see attn_bwd_parts); 1 / NULL: one run
   int n_parts;
   float* dkv_part;
 };

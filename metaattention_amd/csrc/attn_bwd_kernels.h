@@ -108,8 +108,8 @@ __device__ __forceinline__ void dma_tile(const char* src, int64_t row_stride, in
   }
 }
 
-// Stages of the pipelined dk / dv kernel's tile ring: eight (tiles arrive four steps ahead) where they fit the LDS, else four.
-constexpr int fused_stages(int dqk, int dv) { return 8 * (32 * (dqk + dv) * 2 + 512) <= 150 * 1024 ? 8 : 4; }
+// Stages of the pipelined dk / dv kernel's tile ring: with eight, tiles arrive four steps ahead; beside the mask bytes of a stage (4 KB) four fit.
+constexpr int fused_stages(bool masks) { return masks ? 4 : 8; }
 // Workgroups of the pipelined dk / dv kernel that a CU holds.  At 64 / 64 a step is 16 MFMAs behind some 200 vector
 // instructions, LDS latencies and a barrier, and one wave per SIMD waits for most of it: two workgroups (256 registers a wave,
 // lse and delta requested in the step that uses them) take B4 H32 S2048 causal forward + backward from 595 to 438 us (sigmoid)
@@ -812,9 +812,9 @@ __device__ __forceinline__ void partial_store(float* to, const f32x16 (&acc)[N])
 // steps ahead; the step's single barrier sits between phases V and K: behind it tile u+2 is visible to every wave, and
 // every wave is done with tile u-1, whose stage takes tile u+LA.  lse and delta of a tile's rows come with it.  The loop
 // body is written for two steps (the registers of "this" and "the next" step swap roles) so that nothing is copied; an odd
-// number of steps is padded with a step in which everything is masked.  Masked scores are set to -inf (times the sign
-// of scale) before the row function, in the few tiles that touch the diagonal or an end of the sequences: p = 0 and so
-// ds = 0 follow.  Larger head sizes take the pair kernel below; the retention family, 256 / 512, additive score terms, a scale of 0 and
+// number of steps is padded with a step in which everything is masked.  Masked scores are set to -inf and their dp to
+// 0 before the row function, in the few tiles that touch the diagonal or an end of the sequences: p = 0 and so ds = 0 follow.
+// Larger head sizes take the pair kernel below; the retention family, 256 / 512, additive score terms and
 // masks with more steps than the list holds the kernels above.
 template <int I>
 struct IntC { static constexpr int value = I; };
@@ -838,14 +838,6 @@ struct FusedStepRegs {
 // bytes comes with the tile (whole tiles of a 16-byte aligned mask; others are read from global memory), and the
 // masked scores are set to -inf in the same place as for the structural masks.
 constexpr int FUSED_LIST_MAX = 2048;   // steps of a key block that the list holds (the launcher checks)
-// Phase F of a step alternates the k slices of S and dP while both have some left, then finishes the longer contraction:
-// MFMA j of the phase is slice `slice(j)` of S (`is_s(j)`) or of dP.
-template <int KS, int VS>
-struct PhaseF {
-  static constexpr int KMIN = KS < VS ? KS : VS;
-  static constexpr bool is_s(int j) { return j < 2 * KMIN ? j % 2 == 0 : KS > VS; }
-  static constexpr int slice(int j) { return j < 2 * KMIN ? j / 2 : KMIN + (j - 2 * KMIN); }
-};
 // STREAMS 2 (64 / 64, see dkv_two_streams): two streams of four waves walk every other tile of the workgroup's steps each, with
 // stages of their own, as two runs would; at the end one keeps dk and the other dv, and each hands the other one over through LDS.
 // PARTS: n_parts > 1 (an instantiation of its own: the walk over a run's tiles costs the one-run loop 3 % at 64 / 64).
@@ -856,10 +848,10 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
   using x4 = typename E::x4;
   constexpr int BNW = 128, BMT = 32;
   constexpr int KS = DQK / 16, VS = DV / 16, QB = DQK / 32, VB = DV / 32;
-  constexpr int QROW = pad_width(DQK) * 2, DOROW = DV * 2;   // (LDS rows; 192-wide queries sit in 256-wide rows)
+  constexpr int QROW = DQK * 2, DOROW = DV * 2;
   // a stage: the Q tile and the dO tile; behind the stages, 512 bytes per stage: lse (first 128) and delta (at 256) of its rows
   constexpr int QTILE = BMT * QROW, DOTILE = BMT * DOROW, STAGE = QTILE + DOTILE;
-  constexpr int NST = MASKS ? 4 : fused_stages(pad_width(DQK), DV), LA = NST == 8 ? 4 : 3, ROWVALS = NST * STAGE;
+  constexpr int NST = fused_stages(MASKS), LA = NST == 8 ? 4 : 3, ROWVALS = NST * STAGE;
   // (MASKS) behind the row values: 1 KB of mask bytes per stage and wave, then the step list and its length
   constexpr int KEEP = ROWVALS + NST * 512, LIST = KEEP + NST * 4 * 1024, LIST_N = LIST + FUSED_LIST_MAX * 4;
   constexpr int STREAM_LDS = (MASKS ? LIST_N + 4 : ROWVALS + NST * 512) + 1023 & ~1023;
@@ -867,11 +859,12 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
   constexpr int NF = KS + VS, NV = 2 * VB, NK = 2 * QB, NTOT = NF + NV + NK;
   constexpr int RING = 8, AH = FAMILY == BF_SOFTMAX ? 2 : (NK < 6 ? NK : 6);
   static_assert(NTOT % RING == 0 && AH < RING && AH <= NK && AH <= NF, "fragment ring");
-  using PhF = PhaseF<KS, VS>;
+  // phase F alternates the k slices of S and dP: MFMA j is slice j / 2 of S (j even) or of dP
+  static_assert(DQK == DV, "phase F");
 
   extern __shared__ __align__(16) char smem[];
   constexpr bool WALK = PARTS || STREAMS > 1;
-  static_assert(STREAMS <= 2, "two streams share a SIMD");
+  static_assert(STREAMS == 2 || (STREAMS == 1 && !PARTS), "two streams share a SIMD; runs are theirs");
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int stream = STREAMS > 1 ? wave_all >> 2 : 0, wave = STREAMS > 1 ? wave_all & 3 : wave_all;   // wave: within its stream
   const uint32_t lds_all = (uint32_t)(uintptr_t)(MA_LDS char*)smem, lds0 = lds_all + (STREAMS > 1 ? stream * (uint32_t)STREAM_LDS : 0u);
@@ -883,7 +876,7 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
   // same number of query tiles whatever k is: every item weighs the same.  Items that follow each other on an XCD
   // (item % 8) belong to the same (batch, kv head) pairs, whose Q and dO tiles then come from that XCD's L2.
   const int nnb = a.num_blocks, BHK = a.B * a.Hkv, n_parts = PARTS ? a.n_parts : 1;
-  // With n_parts > 1 an item is one of the n_parts runs of each block's steps, whose fp32 sums go to the workspace
+  // With n_parts > 1 (two streams) an item is one of the n_parts runs of each block's steps, whose fp32 sums go to the workspace
   // (attn_bwd_dkv_reduce_kernel adds the runs up).
   const int per_bh = (CAUSAL && STREAMS == 1 ? (nnb + 1) / 2 : nnb) * n_parts, n_items = BHK * per_bh;
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
@@ -936,7 +929,7 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
     for (int j = 0; j < 16; j++) dv[i][j] = 0.f;
   const float bias = a.bias + (a.bias_ptr ? *a.bias_ptr : 0.f);
   const float c_scale = a.scale * kLog2e, c_bias = bias * kLog2e;
-  const float s_masked = a.scale >= 0.f ? -__builtin_inff() : __builtin_inff();   // a score whose p is 0
+  const float s_masked = -__builtin_inff();   // a score whose p is 0 (scale > 0)
 
   // steps: for every query head of the kv head's group, the 32-row tiles that can see this workgroup's keys
   const int t_first = CAUSAL ? (nb * BNW) / BMT : 0;
@@ -993,12 +986,11 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
   auto list_request = [&](int i) { return lds_read<uint32_t>(lds0 + LIST + 4 * (i < n_steps ? i : 0)); };
   auto uniform = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
   const int64_t q_row_bytes = a.qss * 2, do_row_bytes = a.doss * 2;
-  TileDma<QROW, 4, DQK / 8> q_dma;
+  TileDma<QROW, 4> q_dma;
   TileDma<DOROW, 4> do_dma;
   q_dma.init((uint32_t)q_row_bytes, wave, lane);
   do_dma.init((uint32_t)do_row_bytes, wave, lane);
-  // what a wave issues per tile at least (with rows wider than the head size a lane may sit out some of its instructions,
-  // a whole wave never does: the chunks of an instruction's rows are spread over all lanes)
+  // what a wave issues per tile at least
   constexpr int TILE_DMAS = TileDma<QROW, 4>::NJ + TileDma<DOROW, 4>::NJ;
   auto issue_tile = [&](int hg, int t, int st, bool full = true) {
     const int h = hk * a.kv_group + hg, m0 = (t_first + t) * BMT;
@@ -1014,7 +1006,7 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
       q_dma.issue(qb + (int64_t)m0 * q_row_bytes, lds0 + st * STAGE, wave);
       do_dma.issue(dob + (int64_t)m0 * do_row_bytes, lds0 + st * STAGE + QTILE, wave);
     } else {
-      dma_tile<QROW, 4, DQK / 8>(qb, q_row_bytes, m0, a.Sq, lds0 + st * STAGE, wave, lane);
+      dma_tile<QROW, 4>(qb, q_row_bytes, m0, a.Sq, lds0 + st * STAGE, wave, lane);
       dma_tile<DOROW, 4>(dob, do_row_bytes, m0, a.Sq, lds0 + st * STAGE + QTILE, wave, lane);
     }
     if constexpr (FAMILY == BF_SOFTMAX) {
@@ -1046,10 +1038,10 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
     constexpr int j = decltype(jc)::value;
     // (consecutive MFMAs go to different accumulators: with one wave on the SIMD a dependent MFMA waits for the result
     // of the one before it.  Phase F alternates S and dP; phases V and K walk the column blocks before the k slices)
-    if constexpr (j < NF && PhF::is_s(j)) {
-      return lds_read<x8>((nxt + aq_l) ^ (uint32_t)(PhF::slice(j) * 32));
+    if constexpr (j < NF && j % 2 == 0) {
+      return lds_read<x8>((nxt + aq_l) ^ (uint32_t)(j / 2 * 32));
     } else if constexpr (j < NF) {
-      return lds_read<x8>((nxt + QTILE + ad_l) ^ (uint32_t)(PhF::slice(j) * 32));
+      return lds_read<x8>((nxt + QTILE + ad_l) ^ (uint32_t)(j / 2 * 32));
     } else {
       constexpr bool is_v = j < NF + NV;
       constexpr int idx = is_v ? j - NF : j - NF - NV, db = idx % (is_v ? VB : QB), sl = idx / (is_v ? VB : QB);
@@ -1170,8 +1162,8 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
         if constexpr (j + AH < NTOT) fr[(j + AH) % RING] = fragment(IntC<j + AH>(), cur_tile, nxt_tile);
         else fr[(j + AH) % RING] = fragment(IntC<j + AH - NTOT>(), nxt_tile, nn_tile);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (j < NF && PhF::is_s(j)) nxt.s = E::mfma32(fr[j % RING], kf[PhF::slice(j)], j == 0 ? zero16 : nxt.s);
-        else if constexpr (j < NF) nxt.dp = E::mfma32(fr[j % RING], vf[PhF::slice(j)], j == 1 ? zero16 : nxt.dp);
+        if constexpr (j < NF && j % 2 == 0) nxt.s = E::mfma32(fr[j % RING], kf[j / 2], j == 0 ? zero16 : nxt.s);
+        else if constexpr (j < NF) nxt.dp = E::mfma32(fr[j % RING], vf[j / 2], j == 1 ? zero16 : nxt.dp);
         else if constexpr (j < NF + NV) dv[(j - NF) % VB] = E::mfma32(fr[j % RING], pf[(j - NF) / VB], dv[(j - NF) % VB]);
         else dk[(j - NF - NV) % QB] = E::mfma32(fr[j % RING], dsf[(j - NF - NV) / QB], dk[(j - NF - NV) % QB]);
         // vector work behind the MFMA: p of the step's 16 elements in phase F, ds in phase V
@@ -1237,12 +1229,6 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
     __syncthreads();   // the sums have left the stages: the next key block's tiles may arrive
     continue;
   }
-  if constexpr (PARTS) {
-    float* to = dkv_partial<DQK, DV>(a, run, bhk, nb) + wave * (32 * (DQK + DV)) + lane * 4;
-    partial_store<QB>(to, dk);
-    partial_store<VB>(to + 32 * DQK, dv);
-    continue;   // (the stages hold nothing that a wave still reads, see the barrier above)
-  }
   constexpr int DMAX = DQK > DV ? DQK : DV, OROW = DMAX + 16;
   const uint32_t stage = lds0 + wave * 32 * OROW;
   T* dkb = (T*)a.dk + (int64_t)b * a.dksb + (int64_t)hk * a.dksh;
@@ -1257,21 +1243,21 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
 // ------------------------------------------------------------------------------------------------
 // dk and dv in one launch: two waves per SIMD, one for dv and one for dk
 // ------------------------------------------------------------------------------------------------
-// The work of the kernel above without its masks, where the accumulators of one product and the fragments of one operand fit half a
+// The work of the kernel above where the accumulators of one product and the fragments of one operand fit half a
 // SIMD's registers: eight waves take 128 keys, two waves the same 32 of them, on one SIMD.  For every tile u of 32 query rows
 //   wave A   S(u+1) = Q(u+1) K^T with p(u) behind its MFMAs, p(u) to the partner through LDS (fp32);  dV^T += dO(u)^T P(u)
 //   wave B   dP(u+1) = dO(u+1) V^T with ds(u) behind its MFMAs;                                       dK^T += Q(u)^T dS(u)
 // as many MFMAs each whatever the head sizes.  One barrier a tile, between the two halves of A's step and in front of B's: between
 // two barriers A runs its pure MFMA half beside B's row function and then its own row function beside B's pure MFMA half.
 // What bounded the one-wave kernel was issue: 250 k of 412 k clocks a wave, one instruction at a time, the matrix pipe idle for the rest.
-// B2 H32 Hkv8 S2047 128/128 causal 198 -> 170 us = 0.89 PFLOP/s of MFMAs (40 % of the cycles at 2.07 GHz; the LDS is busy for 32 %, without
+// B2 H32 Hkv8 S2047 128/128 causal 198 -> 170 us = 0.865 PFLOP/s of MFMAs (147 GFLOP; 40 % of the cycles at 2.07 GHz; the LDS is busy for 32 %, without
 // conflicts).  From there on longer and shorter rings (4, 5 or 7 MFMAs ahead), p written earlier and fewer scalar instructions change
 // 1 % or nothing: the forward kernel's 1.1 PFLOP/s at the clock that random operands leave is near.  Forward + backward B8 H32 S4096
 // 5740 -> 5120 us, B2 H16 S1600 159 -> 144, B2 H32 Hkv8 S1500 sigmoid without a mask 443 -> 389, B4 H16 S1024 192/128 179 -> 163; at
 // 128 / 256, which took a launch for dk and one for dv before, B2 H16 S2048 causal 371 -> 286, B4 H32 S2500 1825 -> 1610; 256 / 256
 // likewise, B4 H16 S1024 286 -> 263, B4 H12 S1024 sigmoid without a mask 388 -> 318.
 // Ring of NST stages: behind barrier u the tiles u, u + 1 and u + 2 are read, and the stage of tile u - 1 takes tile u + NST - 1.
-// The same products in the same order as the kernel above: the same bits.
+// The same products in the same order as the kernel above: the same bits where everything is finite.
 // MASKS: as in the kernel above, from a list of the steps in LDS.  Both waves know what a mask hides: A makes p = 0 of it, and B, where dp or
 // delta is not finite, ds = 0; tiles that a wave's keys do not see under a causal mask stay out of its sums.  (With B's part forward + backward
 // of B2 H32 Hkv8 S2047 128/128 causal 355 -> 360 us, B2 H16 S1600 141.6 -> 142.8; the mask evaluated by B in every tile that it touches
@@ -1313,7 +1299,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   const int per_bh = (CAUSAL ? (nnb + 1) / 2 : nnb) * n_parts, n_items = BHK * per_bh;
   const float bias = a.bias + (a.bias_ptr ? *a.bias_ptr : 0.f);
   const float c_scale = a.scale * kLog2e, c_bias = bias * kLog2e;
-  const float s_masked = a.scale >= 0.f ? -__builtin_inff() : __builtin_inff();   // a score whose p is 0
+  const float s_masked = -__builtin_inff();   // a score whose p is 0 (scale > 0)
   const int64_t q_row_bytes = a.qss * 2, do_row_bytes = a.doss * 2;
   TileDma<QROW, 8, DQK / 8> q_dma;
   TileDma<DOROW, 8> do_dma;
@@ -1833,17 +1819,18 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
     // (256 / 256 with masks in one run: 97 registers spill, and its two launches are the faster ones, B2 H16 S1500 with a window of 300
     // forward + backward 352 and 357 us)
     const bool two_launches = pair_serial(DQK, DV) && masks && (!a.dkv_part || a.n_parts <= 1);
-    if (a.scale != 0.f && !two_launches && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
-      constexpr size_t ftiles = fused_stages(pad_width(DQK), DV) * ((size_t)32 * (pad_width(DQK) + DV) * 2 + 512);
-      constexpr size_t mtiles = 4 * ((size_t)32 * (pad_width(DQK) + DV) * 2 + 512 + 4 * 1024) + FUSED_LIST_MAX * 4 + 16;
-      constexpr size_t fmax = ftiles > mtiles ? ftiles : mtiles, flds = fmax > ostage ? fmax : ostage;
+    if (!two_launches && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
       if (!a.dkv_part) args.n_parts = 1;
       const bool parts = args.n_parts > 1;
       if (CAUSAL && masks) return -2;   // (masks go with MA_MASK_NONE)
-      const int64_t workgroups = (int64_t)args.num_blocks * a.B * a.Hkv * args.n_parts;
-      constexpr bool TWO = DQK + DV <= 128;
-      bool launched = false;
-      if constexpr (TWO) {
+      const int cus = device_cus();
+      if (cus <= 0) return -1;
+      const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
+      if constexpr (DQK + DV <= 128) {
+        constexpr size_t stage = (size_t)32 * (DQK + DV) * 2 + 512;
+        constexpr size_t ftiles = fused_stages(false) * stage, mtiles = fused_stages(true) * (stage + 4 * 1024) + FUSED_LIST_MAX * 4 + 16;
+        constexpr size_t fmax = ftiles > mtiles ? ftiles : mtiles, flds = fmax > ostage ? fmax : ostage;
+        const int64_t workgroups = (int64_t)args.num_blocks * a.B * a.Hkv * args.n_parts;
         if (parts || dkv_two_streams(workgroups, CAUSAL)) {
           auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false, 2>;
           auto kfp = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, true, 2>;
@@ -1853,28 +1840,23 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
           static std::atomic<uint64_t> slds_ok{0};
           if (allow_lds(slds_ok, slds, kf, kfp, km, kmp) != 0) return -1;
           hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)workgroups), dim3(512), slds, stream, args);
-          launched = true;
+        } else {
+          auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
+          auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false>;
+          static std::atomic<uint64_t> flds_ok{0};
+          if (allow_lds(flds_ok, flds, kf, km) != 0) return -1;
+          const int slots = cus * FUSED_PER_CU;
+          hipLaunchKernelGGL(masks ? km : kf, dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
         }
-      }
-      const int cus = device_cus();
-      if (cus <= 0) return -1;
-      const int items = (CAUSAL ? (args.num_blocks + 1) / 2 : args.num_blocks) * a.B * a.Hkv * args.n_parts;
-      if constexpr (!TWO) {
+      } else {
         auto kf = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
         auto kfp = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, CAUSAL, false, true>;
-        auto km = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, false, true, false>;
+        auto km = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, false, true, pair_serial(DQK, DV)>;      // (pair_serial: never in one run)
         auto kmp = attn_bwd_dkv_pair_kernel<T, DQK, DV, FAMILY, false, true, true>;
         constexpr size_t plain = pair_lds(DQK, DV, false), with_masks = pair_lds(DQK, DV, true);
         static std::atomic<uint64_t> plds_ok{0};
         if (allow_lds(plds_ok, plain > with_masks ? plain : with_masks, kf, kfp, km, kmp) != 0) return -1;
         hipLaunchKernelGGL(masks ? (parts ? kmp : km) : (parts ? kfp : kf), dim3((unsigned)(items < cus ? items : cus)), dim3(512), masks ? with_masks : plain, stream, args);
-      } else if (!launched) {
-        auto kf = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, CAUSAL, false, false>;
-        auto km = attn_bwd_dkv_fused_kernel<T, DQK, DV, FAMILY, false, true, false>;
-        static std::atomic<uint64_t> flds_ok{0};
-        if (allow_lds(flds_ok, flds, kf, km) != 0) return -1;
-        const int slots = cus * FUSED_PER_CU;
-        hipLaunchKernelGGL(masks ? km : kf, dim3((unsigned)(items < slots ? items : slots)), dim3(256), flds, stream, args);
       }
       if (parts) {
         const dim3 grid((unsigned)(args.num_blocks * a.B * a.Hkv), 2);
