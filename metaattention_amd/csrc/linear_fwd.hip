@@ -115,9 +115,13 @@ constexpr int min_waves_per_simd() { return HG > 1 && MODE == 1 ? 3 : NWH == 4 &
 // addressing is the plain one, with compile-time row sizes.
 // GEN 1: one scan, 2: the scans of a LinScans, one blockIdx.y each (with the arguments behind an index the single scan takes 1 %
 // longer: B8 H16 T2048 256 / 512 forward + backward 1516, 1530 us).
+// GEN 3, 4: like 1 and 2, of scans that leave or take in partial results (o_part, o_add): instantiations of their own, because the code for
+// them (and their earlier tile loads) cost the others 1 - 2 %: 8 x 8 heads, 256 / 512, forward + backward, 129 tokens 93.6 -> 92.2 us, 300
+// tokens 140.2 -> 137.4.
+constexpr bool gen_scans(int gen) { return gen == 2 || gen == 4; }
 template <int DK, int NWH, int HG, int MODE, int GEN = 0>
-__global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_waves_per_simd<DK, NWH, HG, MODE>())) void linear_fwd_kernel(const std::conditional_t<GEN == 2, LinScans, LinArgs> all) {
-  const LinArgs& a = one_scan(all, GEN == 2 ? (int)blockIdx.y : 0);
+__global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_waves_per_simd<DK, NWH, HG, MODE>())) void linear_fwd_kernel(const std::conditional_t<gen_scans(GEN), LinScans, LinArgs> all) {
+  const LinArgs& a = one_scan(all, gen_scans(GEN) ? (int)blockIdx.y : 0);
   constexpr int NW = NWH * HG;
   constexpr bool PIPE = pipelined<NWH, HG, MODE>();
   constexpr bool HELP = helpers<DK, NWH, HG, MODE>() > 0;
@@ -608,7 +612,9 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
     // again, and waited for where they are written, behind the next chunk's first reads.  (Asked for in the middle of the state loop,
     // with V^T P^T behind it, it is no faster: what these passes wait for is memory, 4.5 - 4.9 TB/s.)
     f32x4 add[4];
-    const bool adds = GEN && !HELP && a.o_add != nullptr;
+    constexpr bool PARTIAL = GEN >= 3, EARLY = !HELP && (PARTIAL || (GEN == 0 && MODE == 0));
+    static_assert(!PARTIAL || !HELP, "partial results");
+    const bool adds = PARTIAL && a.o_add != nullptr;
     // the wave's 32 x 32 block of chunk c in the order of its accumulators: four rows of 64 lanes x 16 bytes
     auto part_at = [&](const float* part, int c) {
       return (f32x4*)(part + ((((int64_t)bh * a.dv_blocks + dvb) * n_chunks_all + c) * NW + wave) * (16 * 64));
@@ -623,7 +629,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
 #pragma unroll
         for (int j = 0; j < 16; j++) o_out[j] += add[j >> 2][j & 3];
       }
-      if (GEN && !HELP && a.o_part) {
+      if (PARTIAL && a.o_part) {
         f32x4* dst = part_at(a.o_part, c);
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++) dst[64 * q4 + lane] = f32x4{o_out[4 * q4], o_out[4 * q4 + 1], o_out[4 * q4 + 2], o_out[4 * q4 + 3]};
@@ -683,9 +689,12 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
 
       // ---- per 32-row state block: inter-chunk product with the OLD state (as bf16 operand), decay, state update.  The
       //      conversion and the decay of the next block are dealt into the gaps behind the four MFMAs of this block, operands
-      //      are requested one block ahead.  The chunk's loads go out with the first half of the blocks (the last ones of a chunk are
-      //      waited for at its end: over all blocks, 8 x 16 heads, 2048 tokens, 256 / 512 forward and backward took 1017 us, like this 1005;
-      //      not with helpers, which have a stage more to land in: Mamba2's scan 86 and 87 us).
+      //      are requested one block ahead.  The chunk's loads go out behind all blocks, but with the first half of them in a plain scan
+      //      of one pass and with partial results, which fill the device and wait for memory (EARLY; the last
+      //      loads of a chunk are waited for at its end).  Forward + backward, 256 / 512, all early and all late: 8 x 16 heads, 2048 tokens
+      //      1031 and 1042 us; 8 x 8 heads, 300 tokens, whose scans run side by side, 142.7 and 140.6.  A choice made in the kernel, by a
+      //      branch at every load: 1017 and 143 where the early ones alone took 1001 and 140.6, on one box.  Not with helpers, which have
+      //      a stage more to land in: Mamba2's scan 86 us late and 87 early.
       if (loads && !whole) issue_rows(t2, base2);
       const uint32_t qpa = qbase + r * RBQ + (uint32_t)(((2 * g) ^ swz16(r)) << 4);
       const uint32_t kta = kbase + (4 * g + jr) * RBQ + ((ln >> 1) & 1) * 8 + (uint32_t)(((((ln & 1) << 1) | ((ln >> 4) & 1)) ^ swz16(4 * g + jr)) << 4);
@@ -742,7 +751,7 @@ __global__ __launch_bounds__((64 * workgroup_waves<DK, NWH, HG, MODE>()), (min_w
           }
 #pragma unroll
           for (int x = 0; x < NL; x++)
-            if (x * (HELP ? KB : KB / 2) / NL == bb) load_one(x, t2, base2, on);
+            if (x * (EARLY ? KB / 2 : KB) / NL == bb) load_one(x, t2, base2, on);
         }
       }
 #pragma unroll
@@ -1076,6 +1085,8 @@ struct Config {
   static_assert(lds <= 160 * 1024, "a workgroup's LDS");
   static constexpr int64_t ws_wave_floats = (int64_t)(DK / 32) * 16 * 64;
 
+  // partial results (o_part, o_add): by the pipelined chunk loop without helpers
+  static constexpr bool can_leave_parts = pipelined<NWH, HG, 0>() && helpers<DK, NWH, HG, 0>() == 0;
   static bool prepare(int& resident, int& cus) {
     // (threads that meet in a first call compute the same numbers; a device other than the first one asked is assumed to
     // be of the same kind)
@@ -1085,6 +1096,12 @@ struct Config {
                   linear_fwd_kernel<DK, NWH, HG, 0, 1>, linear_fwd_kernel<DK, NWH, HG, 1, 1>, linear_fwd_kernel<DK, NWH, HG, 2, 1>,
                   linear_fwd_kernel<DK, NWH, HG, 0, 2>, linear_fwd_kernel<DK, NWH, HG, 1, 2>, linear_fwd_kernel<DK, NWH, HG, 2, 2>) != 0)
       return false;
+    if constexpr (can_leave_parts) {
+      static std::atomic<uint64_t> parts_ok{0};
+      if (allow_lds(parts_ok, lds, linear_fwd_kernel<DK, NWH, HG, 0, 3>, linear_fwd_kernel<DK, NWH, HG, 2, 3>,
+                    linear_fwd_kernel<DK, NWH, HG, 0, 4>, linear_fwd_kernel<DK, NWH, HG, 2, 4>) != 0)
+        return false;
+    }
     cus = device_cus();
     if (cus <= 0) return false;
     int r = s_resident.load(std::memory_order_relaxed);
@@ -1168,7 +1185,7 @@ struct Config {
     if (a.qk_cols < 0 || a.qk_cols > DK || a.qk_cols % 32 != 0) return -2;
     if (HG > 1 && a.Hv != a.H) return -2;
     if (a.n_pieces > 1 && !a.out_f32) return -2;
-    if ((a.o_add || a.o_part) && (!pipelined<NWH, HG, 0>() || helpers<DK, NWH, HG, 0>() > 0 || a.out_f32)) return -2;
+    if ((a.o_add || a.o_part) && (!can_leave_parts || a.out_f32)) return -2;
     return 0;
   }
 
@@ -1182,9 +1199,20 @@ struct Config {
       const unsigned w = (unsigned)(heads * a.dv_blocks * (a.n_pieces > 1 ? a.n_pieces : 1) * (MODE == 0 ? 1 : MODE == 1 ? a.nseg - 1 : a.nseg));
       width = w > width ? w : width;
     }
-    if (n > 1) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 2>), dim3(width, (unsigned)n), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all);
-    else if (gen) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 1>), dim3(width), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all.s[0]);
-    else hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE>), dim3(width), dim3(64 * (MODE == 1 ? NW : waves)), MODE == 1 ? lds_states : lds, stream, all.s[0]);
+    const dim3 grid(width, (unsigned)n), block(64 * (MODE == 1 ? NW : waves));
+    const size_t l = MODE == 1 ? lds_states : lds;
+    if constexpr (can_leave_parts && MODE != 1) {
+      bool parts = false;
+      for (int i = 0; i < n; i++) parts = parts || all.s[i].o_add || all.s[i].o_part;
+      if (parts) {
+        if (n > 1) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 4>), grid, block, l, stream, all);
+        else hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 3>), grid, block, l, stream, all.s[0]);
+        return;
+      }
+    }
+    if (n > 1) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 2>), grid, block, l, stream, all);
+    else if (gen) hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE, 1>), grid, block, l, stream, all.s[0]);
+    else hipLaunchKernelGGL((linear_fwd_kernel<DK, NWH, HG, MODE>), grid, block, l, stream, all.s[0]);
   }
 
   // n scans side by side (see linear_scans_dispatch; more than one: all with the general addressing).
