@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   TileDma<DOROW, 8> do_dma;
   q_dma.init((uint32_t)q_row_bytes, wave_all, lane);
   do_dma.init((uint32_t)do_row_bytes, wave_all, lane);
-  constexpr int TILE_DMAS = TileDma<QROW, 8>::NJ + TileDma<DOROW, 8>::NJ;   // what a wave issues per tile at least (see above)
+  constexpr int TILE_DMAS = TileDma<QROW, 8>::NJ + TileDma<DOROW, 8>::NJ;   // what a wave issues per tile at least (a lane may sit out instructions at 192, a whole wave never does)
 
   for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
   int bhk, ki, run;
