@@ -1263,7 +1263,11 @@ __global__ __launch_bounds__(256 * STREAMS, FUSED_PER_CU) void attn_bwd_dkv_fuse
 // of B2 H32 Hkv8 S2047 128/128 causal 355 -> 360 us, B2 H16 S1600 141.6 -> 142.8; the mask evaluated by B in every tile that it touches
 // cost 6 % under a window.)
 // At 256 / 256 fragments, accumulators and one set of scores fill the registers: there a wave's step is its scores, the row function, its
-// accumulators, one after the other, beside the partner's (pair_serial; a tile is then read in two steps, not three).
+// accumulators, one after the other, beside the partner's (pair_serial; a tile is then read in two steps, not three).  There a softmax step
+// reads its operand fragments two MFMAs ahead instead of three, and the lane's part of every address but the fragments' is made where it is
+// used: held in registers they were spilled, and a reload waits for all loads under way, the next tiles' among them (causal: 8 of them a
+// step; now none).  Forward + backward, B8 H12 S829 causal 366 -> 304 us, B8 H16 S600 302 -> 253, B4 H16 S4096 3020 -> 2725, without a mask
+// 5345 -> 4912; with three fragments ahead, one reload left, 318, 262, 2740 and 5003.
 constexpr bool pair_serial(int dqk, int dv) { return dqk + dv >= 512; }
 constexpr int pair_stages(int dqk, int dv, bool masks) { return pair_serial(dqk, dv) ? 3 : (pad_width(dqk) + dv <= 256 ? 6 : 5) - masks; }
 constexpr size_t pair_lds(int dqk, int dv, bool masks) {
@@ -1290,7 +1294,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MA_LDS char*)smem;
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all & 3;
   // (where registers are short what is rarely needed is made from the lane's number anew: derived from the one above, the compiler
-  // carries it through the loop in spilled registers, 46 of them at 256 / 256.  128 / 128 has the registers: 201 us for 203, B2 H16 S1500)
+  // carries it through the loop in spilled registers.  128 / 128 has the registers: 201 us for 203, B2 H16 S1500)
   auto lane_here = [&]() { return DQK + DV > 256 ? lane_anew() : lane; };
   const int r = lane & 31, g = lane >> 5, jr = (lane & 15) >> 2, lc = (((lane >> 4) & 1) << 1) | ((lane & 3) >> 1);
 
@@ -1399,6 +1403,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
     }
     const int rows = fetch.w.t < t_whole ? BMT : a.Sq % BMT;   // (wave-uniform)
     if (rows == BMT) {
+      if constexpr (SERIAL) {
+        const int ln = lane_anew();
+        q_dma.init((uint32_t)q_row_bytes, wave_all, ln);
+        do_dma.init((uint32_t)do_row_bytes, wave_all, ln);
+      }
       q_dma.issue(fetch.q, to, wave_all);
       do_dma.issue(fetch.d, to + QTILE, wave_all);
     } else {
@@ -1432,7 +1441,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
     constexpr int DR = ROLE_B ? DV : DQK, DC = ROLE_B ? DQK : DV;
     constexpr int RROW = ROLE_B ? DOROW : QROW, CROW = ROLE_B ? QROW : DOROW, ROFF = ROLE_B ? QTILE : 0, COFF = ROLE_B ? 0 : QTILE;
     // (128 / 256: with the longer ring 40 registers spill, B2 H16 S2048 causal 302 us, 286 with four)
-    constexpr int NR = DR / 16, CB = DC / 32, NTOT = NR + 2 * CB, RING = NTOT % 8 == 0 && DQK + DV <= 256 ? 8 : 4, AH = RING == 8 ? 5 : 3;
+    constexpr int NR = DR / 16, CB = DC / 32, NTOT = NR + 2 * CB, RING = NTOT % 8 == 0 && DQK + DV <= 256 ? 8 : 4, AH = RING == 8 ? 5 : SERIAL && FAMILY == BF_SOFTMAX ? 2 : 3;
     static_assert(NTOT % RING == 0 && AH <= NR && AH <= 2 * CB, "fragment ring");
     x8 wf[NR];
     {
@@ -1465,9 +1474,15 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
       const uint32_t x_l = lds0 + XCHG + wave * 4096 + lane * 16;      // p of the even tiles, 16 KB on of the odd ones
       f32x4 rv[4];      // lse (A) or delta (B) of the rows 8 q4 + 4 g + {0..3} of the step's tile
       auto row_values = [&](uint32_t tile) {
-        if constexpr (FAMILY == BF_SOFTMAX)
+        if constexpr (FAMILY == BF_SOFTMAX) {
+          uint32_t at = tile + ROWVALS + (ROLE_B ? 256 : 0);
+          if constexpr (SERIAL) {
+            at += lane_anew() >> 5 << 4;
+            asm volatile("" : "+v"(at));      // (one address and four offsets, not four addresses)
+          }
 #pragma unroll
-          for (int q4 = 0; q4 < 4; q4++) rv[q4] = lds_read<f32x4>(tile + ROWVALS + (ROLE_B ? 256 : 0) + (8 * q4 + 4 * g) * 4);
+          for (int q4 = 0; q4 < 4; q4++) rv[q4] = lds_read<f32x4>(at + (SERIAL ? 8 * q4 : 8 * q4 + 4 * g) * 4);
+        }
       };
 
       DkvWalk at = first;      // the current step's tile
@@ -1624,7 +1639,6 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
         ahead();
       };
       auto serial_body = [&](int u) __attribute__((always_inline)) {
-        const uint32_t x = x_l + (u & 1) * 16384;
         x8 f[2];
         static_for<0, NTOT>([&](auto jc) __attribute__((always_inline)) {
           constexpr int j = decltype(jc)::value;
@@ -1632,6 +1646,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkv_pair_kernel(const AttnBwd
           if constexpr (j == NR - 1) row_values(t0);
           if constexpr (j == NR) {
             hide(u, sa);
+            const uint32_t x = lds0 + XCHG + wave * 4096 + (u & 1) * 16384 + lane_anew() * 16;
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
               f32x4 p;
