@@ -1776,6 +1776,17 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_reduce_kernel(const AttnBwdA
 // 0.94, 0.97, 0.98).  Without a mask, at 192, 256 and 288: 128/128 0.97, 0.99, 1.08, 64/64 0.92, 0.91, 1.06.
 inline bool dq_two_streams(int64_t blocks, bool causal) { return 2 * blocks <= (causal ? 3 : 2) * (int64_t)device_cus(); }
 
+// Masked calls at 128 / 256 in one run, where key blocks have few steps: the pair kernel holds one workgroup a CU, so that its list of steps, first
+// tiles and outputs stand alone and a last round that is nearly empty costs a whole one; the two-launch kernels hold two.  Forward + backward,
+// two launches and pairs, windows of 147 and 600, S1115 (35 steps, 9 key blocks a head), by key blocks a CU: 1.1 156, 172 and 221, 240 us; 1.4
+// 159, 174 and 234, 242; 2.0 168, 181 and 243, 248; 2.25 232, 258 and 314, 345; 2.5 267, 272; 2.8 283, 281; 3.1 295, 329.  Full rounds: 3.0, S679
+// 249, 246; 4.0, S400 226, 204; 5.0, S1200 598, 492.  More steps: 1.1, S2300 (72) 192, 197; 1.5, S3000 (94) 229, 222; 2.0, S2000 in groups of
+// four heads (252) 538, 425.
+inline bool masked_two_launches(int64_t key_blocks, int64_t steps) {
+  const int64_t cus = device_cus(), rounds = cus > 0 ? (key_blocks + cus - 1) / cus : 1;
+  return steps <= 72 && rounds > 1 && (rounds == 2 || 10 * key_blocks < 8 * rounds * cus);
+}
+
 template <typename T, int DQK, int DV, int FAMILY, bool CAUSAL>
 static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   constexpr int DMAX = DQK > DV ? DQK : DV;
@@ -1831,10 +1842,12 @@ static int launch_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   if constexpr (FAMILY != BF_RETENTION && DQK <= 256 && DV <= 256) {
     // dk and dv by the pipelined single launch (with masks: as long as a key block's steps fit its list)
     const bool masks = a.elem_mask_t || a.q_block_mask;
-    // (256 / 256 with masks in one run: 97 registers spill, and its two launches are the faster ones, B2 H16 S1500 with a window of 300
-    // forward + backward 352 and 357 us)
-    const bool two_launches = pair_serial(DQK, DV) && masks && (!a.dkv_part || a.n_parts <= 1);
-    if (!two_launches && (!masks || (int64_t)((a.Sq + 31) / 32) * a.kv_group <= FUSED_LIST_MAX)) {
+    // (256 / 256 with masks in one run: the list's loop has no registers to spare, and its two launches were the faster ones, B2 H16 S1500 with
+    // a window of 300 forward + backward 352 and 357 us)
+    const int64_t steps = (int64_t)((a.Sq + 31) / 32) * a.kv_group;
+    const bool one_run = !a.dkv_part || a.n_parts <= 1;
+    const bool two_launches = masks && one_run && (pair_serial(DQK, DV) || (DQK + DV == 384 && masked_two_launches((int64_t)args.num_blocks * a.B * a.Hkv, steps)));
+    if (!two_launches && (!masks || steps <= FUSED_LIST_MAX)) {
       if (!a.dkv_part) args.n_parts = 1;
       const bool parts = args.n_parts > 1;
       if (CAUSAL && masks) return -2;   // (masks go with MA_MASK_NONE)

@@ -102,7 +102,8 @@ def test_hidden_keys_and_rows_under_a_mask(B, H, Hkv, S, D, DV, family, one_run,
 
 @pytest.mark.parametrize("D,DV", SIZES)
 @pytest.mark.parametrize("one_run", [True, False])
-@pytest.mark.parametrize("B,H,Hkv,S", [(8, 16, 16, 400), (3, 34, 34, 400), (8, 32, 16, 300), (1, 4, 2, 400)])      # (but for the last: more key blocks than CUs)
+# (but for the last: more key blocks than CUs, in 1.5 to 2 rounds, in 3 and almost 4 full ones and in 2.25)
+@pytest.mark.parametrize("B,H,Hkv,S", [(8, 16, 16, 400), (3, 34, 34, 400), (8, 32, 16, 300), (8, 32, 32, 384), (5, 51, 51, 400), (9, 16, 16, 400), (1, 4, 2, 400)])
 def test_masked_gradients(B, H, Hkv, S, D, DV, one_run, monkeypatch):
     """A workgroup's key blocks one after the other, a list of steps made for each: a window, and a key block that no row sees."""
     print(f"masked {D}/{DV} B{B} H{H}/{Hkv} S{S} one_run={one_run}", flush=True)
